@@ -281,10 +281,11 @@ def _prompts(c):
     return out
 
 
-def _prepare_forward(c, seed):
+def _forward_inputs(c, seed):
+    """Every sequence's (token ids, k, v), then the queries.  k and v are views of buffers that the
+    next sequence's private tokens overwrite."""
     g, h = _gen(seed), c["heads"]
     prompts = _prompts(c)
-    attn = _cache(c, sum(len(ids) // c["chunk"] + 2 for ids, _ in prompts))
     longest = max(len(ids) for ids, _ in prompts)
     k, v = (torch.empty((longest, h, D), dtype=HALF, device=DEV) for _ in range(2))
     root, group = c["root"], c["group"]
@@ -295,12 +296,20 @@ def _prepare_forward(c, seed):
             if group and s % c["per_group"] == 0:
                 t[root:root + group].normal_(generator=g)
             t[root + group:len(ids)].normal_(generator=g)
-        attn.add_seq(ids, k[:len(ids)], v[:len(ids)])
+        yield ids, k[:len(ids)], v[:len(ids)]
+    yield _normal(g, c["batch"], h, D)
+
+
+def _prepare_forward(c, seed):
+    attn = _cache(c, sum(len(ids) // c["chunk"] + 2 for ids, _ in _prompts(c)))
+    inputs = _forward_inputs(c, seed)
+    for _ in range(c["batch"]):
+        attn.add_seq(*next(inputs))
     attn.refresh_kernel_context()
-    return {"kind": "forward", "attn": attn, "q": _normal(g, c["batch"], h, D)}
+    return {"kind": "forward", "attn": attn, "q": next(inputs)}
 
 
-def _prepare_generate(c, seed):
+def _generate_inputs(c, seed):
     g, h, n = _gen(seed), c["heads"], c["batch"]
     prompts = _prompts(c)
     root_k, root_v = _normal(g, c["root"], h, D), _normal(g, c["root"], h, D)
@@ -309,11 +318,16 @@ def _prepare_generate(c, seed):
         requests.append((ids, torch.cat([root_k, _normal(g, own, h, D)]), torch.cat([root_v, _normal(g, own, h, D)])))
     steps = [([20_000_000 + 1000 * t + s for s in range(n)], _normal(g, n, h, D), _normal(g, n, h, D), _normal(g, n, h, D))
              for t in range(c["steps"])]
-    chunks = sum((len(ids) + c["steps"]) // c["chunk"] + 2 for ids, _ in prompts)
+    return requests, steps
+
+
+def _prepare_generate(c, seed):
+    requests, steps = _generate_inputs(c, seed)
+    chunks = sum((len(ids) + c["steps"]) // c["chunk"] + 2 for ids, _, _ in requests)
     return {"kind": "generate", "attn": _cache(c, chunks), "requests": requests, "steps": steps}
 
 
-def _prepare_beam(c, seed):
+def _beam_inputs(c, seed):
     g, h, width = _gen(seed), c["heads"], c["width"]
     prompt = (list(range(c["prompt"])), _normal(g, c["prompt"], h, D), _normal(g, c["prompt"], h, D))
     steps = []
@@ -326,7 +340,12 @@ def _prepare_beam(c, seed):
         for b, m in enumerate(counts):
             parts.append(([1_000_000 + 1000 * t + 10 * b + i for i in range(m)], _normal(g, m, h, D), _normal(g, m, h, D)))
         steps.append((parts, None if first else (11 * t + 3) % (width + 1), _normal(g, width, h, D)))
-    chunks = c["prompt"] // c["chunk"] + (width + 2) * (c["steps"] // c["chunk"] + 3)
+    return prompt, steps
+
+
+def _prepare_beam(c, seed):
+    prompt, steps = _beam_inputs(c, seed)
+    chunks = c["prompt"] // c["chunk"] + (c["width"] + 2) * (c["steps"] // c["chunk"] + 3)
     return {"kind": "beam", "attn": _cache(c, chunks), "prompt": prompt, "steps": steps}
 
 
@@ -443,3 +462,106 @@ def _run_ops(s):
 def run(state):
     return {"forward": _run_forward, "generate": _run_generate, "beam": _run_beam, "layer": _run_layer,
             "model": _run_model, "ops": _run_ops}[state["kind"]](state)
+
+
+# ---- the same in 64 bits ---------------------------------------------------------------------------------
+
+def _attend(q, k, v):
+    """q [h, d], k and v [n, h, d] -> [h, d]."""
+    q, k, v = (t.double() for t in (q, k, v))
+    p = torch.softmax((k * q).sum(-1) / math.sqrt(D), dim=0)
+    return (p[:, :, None] * v).sum(0)
+
+
+def _exact_forward(c, seed):
+    def one(attended):       # the queries come last: two passes over the same draws
+        inputs = _forward_inputs(c, seed)
+        rows = [attended(s, *next(inputs)[1:]) for s in range(c["batch"])]
+        return rows, next(inputs)
+    _, q = one(lambda s, k, v: None)
+    return torch.stack(one(lambda s, k, v: _attend(q[s], k, v))[0])
+
+
+def _exact_generate(c, seed):
+    requests, steps = _generate_inputs(c, seed)
+    out = []
+    for s, (_, k, v) in enumerate(requests):
+        k = torch.cat([k] + [step[2][s:s + 1] for step in steps])
+        v = torch.cat([v] + [step[3][s:s + 1] for step in steps])
+        n = k.shape[0] - len(steps)
+        out.append(torch.stack([_attend(step[1][s], k[:n + t + 1], v[:n + t + 1]) for t, step in enumerate(steps)]))
+    return list(torch.stack(out, dim=1))
+
+
+def _exact_beam(c, seed):
+    (_, k, v), steps = _beam_inputs(c, seed)
+    beams, out = [(k, v)], []
+    for parts, lost, q in steps:
+        grown = []
+        for (bk, bv), (tokens, k, v) in zip(beams, parts):
+            grown += [(torch.cat([bk, k[i:i + 1]]), torch.cat([bv, v[i:i + 1]])) for i in range(len(tokens))]
+        if lost is not None:
+            del grown[lost]
+        beams = grown
+        out.append(torch.stack([_attend(q[b], bk, bv) for b, (bk, bv) in enumerate(beams)]))
+    return out
+
+
+def _rotated(x, positions, table, neox):
+    """x [n, heads, d] turned by the angles that `table` has for `positions`."""
+    cos, sin = table.double()[positions].chunk(2, dim=-1)
+    cos, sin = cos[:, None], sin[:, None]
+    if neox:
+        a, b = x.chunk(2, dim=-1)
+        return torch.cat([a * cos - b * sin, b * cos + a * sin], dim=-1)
+    a, b = x[..., 0::2], x[..., 1::2]
+    return torch.stack([a * cos - b * sin, b * cos + a * sin], dim=-1).flatten(-2)
+
+
+def _normed(x, weight, eps):
+    return x * torch.rsqrt((x * x).mean(-1, keepdim=True) + eps) * weight.double()
+
+
+def _causal_layer(layer, x):
+    """One attention layer over a whole sequence, x [n, hidden]."""
+    n, h = x.shape[0], x.shape[1] // D
+    q, k, v = ((x @ p.weight.double().t()).view(n, h, D) for p in (layer.q_proj, layer.k_proj, layer.v_proj))
+    positions = torch.arange(n, device=x.device)
+    q, k = (_rotated(t, positions, layer.rotary_emb.cos_sin_cache, True) for t in (q, k))
+    future = torch.ones(n, n, dtype=torch.bool, device=x.device).triu(1)
+    heads = [torch.softmax((q[:, i] @ k[:, i].t() / math.sqrt(D)).masked_fill(future, float("-inf")), dim=-1) @ v[:, i]
+             for i in range(h)]
+    return torch.cat(heads, dim=-1) @ layer.o_proj.weight.double().t()
+
+
+@torch.no_grad()
+def _exact_layer(c, seed):
+    s = _prepare_layer(c, seed)
+    n, x = c["prompt"], torch.cat([s["prompt"][0]] + [step[0] for step in s["steps"]], dim=1).double()
+    whole = torch.stack([_causal_layer(s["layer"], row) for row in x])
+    return [whole[:, :n]] + [whole[:, n + t:n + t + 1] for t in range(c["steps"])]
+
+
+@torch.no_grad()
+def _exact_model(c, seed):
+    s = _prepare_model(c, seed)
+    model, n = s["model"], c["root"] + c["unique"]
+    each = []
+    for prompt, answer in zip(s["prompts"], s["answers"]):
+        x = model.embed_tokens.weight[torch.tensor(prompt + answer, device=DEV)].double()
+        for norm, layer in zip(model.input_norms, model.layers):
+            x = x + _causal_layer(layer, _normed(x, norm.weight, norm.eps))
+        each.append(_normed(x[n - 1:], model.norm.weight, model.norm.eps) @ model.lm_head.weight.double().t())
+    return [e[:1] for e in each] + [torch.stack([e[t + 1] for e in each]) for t in range(c["steps"])]
+
+
+def _exact_ops(c, seed):
+    s = _prepare_ops(c, seed)
+    residual = s["residual"].double() + s["x"].double()
+    q, k = (_rotated(s[t].double().view(c["tokens"], -1, D), s["positions"], s["cos_sin"], c["neox"]).flatten(1) for t in "qk")
+    return {"x": _normed(residual, s["weight"], 1e-6), "residual": residual, "q": q, "k": k}
+
+
+def exact(case, seed):
+    return {"forward": _exact_forward, "generate": _exact_generate, "beam": _exact_beam, "layer": _exact_layer,
+            "model": _exact_model, "ops": _exact_ops}[case["kind"]](case, seed)

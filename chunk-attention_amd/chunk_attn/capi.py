@@ -73,6 +73,8 @@ SIGNATURES = {
                                    ctypes.c_int64, ctypes.c_int, ctypes.c_void_p]),
     "ca_fused_add_rms_norm": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_float,
                                              ctypes.c_int64, ctypes.c_int, ctypes.c_void_p]),
+    "ca_causal_attention": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
+                                           ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p]),
     "ca_rope_append_kv": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
                                          ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_int,
                                          ctypes.c_int, ctypes.c_int, ctypes.c_void_p]),
@@ -377,6 +379,31 @@ def fused_add_rms_norm(input, residual, weight, epsilon: float) -> None:
     with torch.cuda.device(input.device):
         _check(load().ca_fused_add_rms_norm(input.data_ptr(), residual.data_ptr(), weight.data_ptr(), float(epsilon),
                                             n, hidden, torch.cuda.current_stream(input.device).cuda_stream))
+
+
+def causal_attention_takes(*tensors) -> bool:
+    """Whether causal_attention computes on these: fp16 GPU tensors [batch, n, heads, 128] of one shape,
+    contiguous and 16-byte aligned, no gradient asked for (the kernel has no backward)."""
+    import torch
+    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
+        return False
+    shape, device = tensors[0].shape, tensors[0].device
+    return len(shape) == 4 and shape[3] == 128 and device.type == "cuda" and all(
+        t.dtype == torch.float16 and t.shape == shape and t.device == device and t.is_contiguous() and
+        t.data_ptr() % 16 == 0 for t in tensors)
+
+
+def causal_attention(q, k, v):
+    """Causal attention of whole prompts, [batch, n, heads, 128] each; returns a tensor like q."""
+    import torch
+    if not causal_attention_takes(q, k, v):
+        raise RuntimeError("causal_attention: contiguous, 16-byte aligned fp16 GPU tensors [batch, n, heads, 128] "
+                           "of one shape, without gradients")
+    out = torch.empty_like(q)
+    with torch.cuda.device(q.device):
+        _check(load().ca_causal_attention(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), q.shape[0], q.shape[1],
+                                          q.shape[2], q.shape[3], torch.cuda.current_stream(q.device).cuda_stream))
+    return out
 
 
 def max_chunks_for(memory_mb: int, chunk_size: int, n_heads: int, d_head: int, elem_bytes: int = 2) -> int:

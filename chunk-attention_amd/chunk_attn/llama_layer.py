@@ -71,12 +71,15 @@ class LlamaChunkAttention(nn.Module):
             q, k = self.rotary_emb(position_ids.contiguous(), q, k)
             shape = (batch, n_tokens, self.num_heads, self.head_dim)
             q4, k4, v4 = q.view(shape), k.view(shape), v.view(shape)
-            # causal attention over the prompt (not the decode path: plain fp32 torch math)
-            qh, kh, vh = (t.transpose(1, 2).float() for t in (q4, k4, v4))
-            scores = qh @ kh.transpose(-1, -2) / math.sqrt(self.head_dim)
-            future = torch.ones(n_tokens, n_tokens, dtype=torch.bool, device=scores.device).triu(1)
-            attn = torch.softmax(scores.masked_fill(future, float("-inf")), dim=-1) @ vh
-            attn_output = attn.transpose(1, 2).reshape(batch, n_tokens, d_hidden).to(hidden_states.dtype)
+            if hidden_states.dtype == torch.float16 and capi.causal_attention_takes(q4, k4, v4):
+                attn_output = capi.causal_attention(q4, k4, v4).view(batch, n_tokens, d_hidden)
+            else:
+                # what the kernel does not take (a gradient is wanted, another head size): plain fp32 torch math
+                qh, kh, vh = (t.transpose(1, 2).float() for t in (q4, k4, v4))
+                scores = qh @ kh.transpose(-1, -2) / math.sqrt(self.head_dim)
+                future = torch.ones(n_tokens, n_tokens, dtype=torch.bool, device=scores.device).triu(1)
+                attn = torch.softmax(scores.masked_fill(future, float("-inf")), dim=-1) @ vh
+                attn_output = attn.transpose(1, 2).reshape(batch, n_tokens, d_hidden).to(hidden_states.dtype)
             self.last_indices = [kv_cache.add_seq(list(seqs[i]), k4[i].contiguous(), v4[i].contiguous())
                                  for i in range(batch)]
         else:

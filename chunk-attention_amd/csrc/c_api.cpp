@@ -775,6 +775,20 @@ int ca_fused_add_rms_norm(void* input, void* residual, const void* weight, float
                                          static_cast<hipStream_t>(stream)), "fused_add_rms_norm launch");
 }
 
+int ca_causal_attention(const void* q, const void* k, const void* v, void* out, int batch, int n_tokens,
+                        int n_heads, int d_head, void* stream) {
+    if (batch < 0 || n_tokens < 0 || n_heads <= 0) return fail(CA_ERR_INVALID, "bad argument");
+    if (d_head != 128) return fail(CA_ERR_INVALID, "causal attention needs d_head 128");
+    if (batch == 0 || n_tokens == 0) return CA_OK;
+    if (!q || !k || !v || !out) return fail(CA_ERR_INVALID, "null device pointer");
+    if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(out)) {
+        return fail(CA_ERR_INVALID, "q, k, v and out must be 16-byte aligned");
+    }
+    const float scale_log2 = 1.4426950408889634f / std::sqrt(float(d_head));
+    return launch_rc(ca::launch_causal_attention(q, k, v, out, batch, n_tokens, n_heads, scale_log2,
+                                                 static_cast<hipStream_t>(stream)), "causal attention launch");
+}
+
 int ca_rope_append_kv(ca_ctx* c, const int64_t* positions, void* q, const void* k, const void* v,
                       const void* cos_sin_cache, int max_position, int rot_dim, int is_neox,
                       int n_seqs, void* stream) {

@@ -118,4 +118,9 @@ int launch_rope_append(const LaunchArgs& a, const RotaryArgs& r, const void* k, 
 int launch_rms_norm(void* out, void* input, void* residual, const void* weight, float epsilon,
                     int64_t n_tokens, int hidden, bool vec8, hipStream_t st);
 
+// Causal attention of whole prompts: q, k, v, out [batch, n_tokens, n_heads, 128] fp16, contiguous and
+// 16-byte aligned; out must not overlap the inputs.
+int launch_causal_attention(const void* q, const void* k, const void* v, void* out, int batch, int n_tokens, int n_heads,
+                            float scale_log2, hipStream_t st);
+
 }  // namespace ca

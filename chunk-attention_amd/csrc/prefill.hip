@@ -1,0 +1,309 @@
+// Causal attention over whole prompts for gfx950 (MI355X): the prefill branch of the attention layer
+// (the reference computes it with an external attention library,
+// src/chunk_attn/models/llama_hf/modeling_llama.py:64-84).  fp16 q/k/v [batch, n, heads, 128], fp32
+// scores, softmax and sums, fp16 output rounded once; d_head 128.
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+#include <type_traits>
+
+#include "kernels.h"
+
+namespace ca {
+namespace {
+
+typedef _Float16 half_t;
+typedef half_t h2 __attribute__((ext_vector_type(2)));
+typedef half_t h4 __attribute__((ext_vector_type(4)));
+typedef half_t h8 __attribute__((ext_vector_type(8)));
+typedef float f4 __attribute__((ext_vector_type(4)));
+
+constexpr int D = 128;
+constexpr int WG = 256;
+constexpr int TILE = 64;            // keys per tile
+constexpr float NEG_INF = -__builtin_huge_valf();
+constexpr float kShift = 8.f;       // probabilities are kept as 2^8 times their value (see below)
+
+__device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
+
+__device__ __forceinline__ h4 lds_read_tr(const half_t* p) {
+    typedef short s4v __attribute__((ext_vector_type(4)));
+    const s4v raw = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s4v __attribute__((address_space(3)))*)p);
+    return __builtin_bit_cast(h4, raw);
+}
+
+// maximum over lanes l, l^16, l^32, l^48 (the four 16-lane groups), in all four
+__device__ __forceinline__ float max_over_groups(float v) {
+    const unsigned u = __builtin_bit_cast(unsigned, v);
+    const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    const unsigned a0 = a[0], a1 = a[1];
+    const float m16 = fmaxf(__builtin_bit_cast(float, a0), __builtin_bit_cast(float, a1));
+    const unsigned w = __builtin_bit_cast(unsigned, m16);
+    const auto b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+    const unsigned b0 = b[0], b1 = b[1];
+    return fmaxf(__builtin_bit_cast(float, b0), __builtin_bit_cast(float, b1));
+}
+
+// K and V tiles in LDS, rows of 256 B without padding (the direct global -> LDS loads write 64
+// consecutive 16-byte pieces): piece c of row r stands at place c ^ (r & 15), so that the 16 rows a
+// read touches at one column lie in 16 different bank groups.
+struct CausalLds {
+    half_t k[2][TILE * D];
+    half_t v[2][TILE * D];
+};
+__device__ __forceinline__ int place(int row, int piece) { return row * D + ((piece ^ (row & 15)) << 3); }
+
+__device__ __forceinline__ void load_to_lds16(const half_t* src, half_t* dst) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                     (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+}
+
+// A workgroup attends 64 * MB query rows of one (sequence, head): wave w owns 16 * MB of them and
+// keeps their Q^T operands and output accumulators in registers; 64-key tiles of K and V go through
+// LDS, the next tile on its way into a second buffer.  S^T = K.Q^T leaves each lane with four keys of one row,
+// which is the operand layout O^T = V^T.P^T needs, so probabilities never leave registers.
+//
+// The probabilities are fp32; the matrix cores take fp16.  p = hi + lo with hi = fp16(p) and
+// lo = fp16(p - hi) carries 21 bits of p at the price of a second P.V product, and p is scaled by 2^8
+// (the row sum likewise, so it cancels) to keep lo of small p above fp16's smallest step.  Against 64
+// bits the output is as far off as with fp32 products: its own rounding to fp16 is what remains.
+template <int MB>
+__global__ __launch_bounds__(WG, 2) void causal_attention_kernel(const half_t* __restrict__ q, const half_t* __restrict__ k,
+                                                                 const half_t* __restrict__ v, half_t* __restrict__ out,
+                                                                 int n, int H, int n_bh, int n_blocks, float scale_log2) {
+    __shared__ __attribute__((aligned(16))) CausalLds sm;
+    // Query blocks in descending order (the last ones attend most).  Workgroup b runs on XCD b % 8:
+    // with a multiple of 8 heads every head stays on one XCD, whose L2 then holds its K and V.
+    // Every second 256 workgroups (one per compute unit) are taken in reverse, in steps of 8 so that the
+    // XCD does not change: a compute unit gets a long and a short block instead of two long ones.
+    int b = blockIdx.x;
+    if (((b >> 8) & 1) && (b | 255) < int(gridDim.x)) b = (b & ~255) | ((31 - ((b >> 3) & 31)) << 3) | (b & 7);
+    const int bh = b % n_bh;
+    const int block = n_blocks - 1 - b / n_bh;
+    const int seq = bh / H, h = bh - seq * H;
+    const size_t stride = size_t(H) * D;                       // halves between tokens
+    const size_t base = size_t(seq) * n * stride + size_t(h) * D;
+
+    const int tid = threadIdx.x;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l = tid & 63, g = l >> 4, i = l & 15;
+    const int q0 = block * 64 * MB;                            // first row of the workgroup
+    const int row0 = q0 + 16 * MB * w;                         // first row of the wave
+
+    h8 qreg[MB][4];
+#pragma unroll
+    for (int mb = 0; mb < MB; mb++) {
+        const int row = row0 + 16 * mb + i;
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++) {
+            qreg[mb][ks] = (row < n) ? *reinterpret_cast<const h8*>(q + base + size_t(row) * stride + 32 * ks + 8 * g)
+                                     : h8{ 0, 0, 0, 0, 0, 0, 0, 0 };
+        }
+    }
+    float m_run[MB], l_lane[MB];
+    f4 oacc[MB][8];
+#pragma unroll
+    for (int mb = 0; mb < MB; mb++) {
+        m_run[mb] = NEG_INF;
+        l_lane[mb] = 0.f;
+#pragma unroll
+        for (int db = 0; db < 8; db++) oacc[mb][db] = f4{ 0.f, 0.f, 0.f, 0.f };
+    }
+
+    // Wave w brings rows 16w .. 16w+15 of a tile, four per load: lane l writes piece l of those 1024 B,
+    // i.e. place l & 15 of row l >> 4, and therefore reads piece (l & 15) ^ (row & 15).  Rows past the last
+    // token repeat it (valid memory; their scores are masked for every row).
+    auto fetch_tile = [&](int t, int buf) {
+        const half_t* __restrict__ kg = k + base + size_t(TILE * t) * stride;   // uniform; the lane's part is 32 bits
+        const half_t* __restrict__ vg = v + base + size_t(TILE * t) * stride;
+        const int left = n - 1 - TILE * t;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int row = 16 * w + 4 * r + g;
+            const unsigned off = unsigned(row < left ? row : left) * unsigned(stride) + 8 * (i ^ (row & 15));
+            load_to_lds16(kg + off, &sm.k[buf][(16 * w + 4 * r) * D]);
+            load_to_lds16(vg + off, &sm.v[buf][(16 * w + 4 * r) * D]);
+        }
+    };
+
+    const int last = (q0 + 64 * MB < n ? q0 + 64 * MB : n) - 1;  // last query row of the workgroup
+    const int n_tiles = last / TILE + 1;
+
+    auto tile_body = [&](int t, const half_t* __restrict__ kt, const half_t* __restrict__ vt, auto masked_tag) {
+        constexpr bool MASKED = decltype(masked_tag)::value;   // some key of the tile lies after some row of the wave
+        f4 sc[MB][4];
+#pragma unroll
+        for (int tb = 0; tb < 4; tb++) {
+            h8 kop[4];
+#pragma unroll
+            for (int ks = 0; ks < 4; ks++) {
+                kop[ks] = *reinterpret_cast<const h8*>(&kt[place(16 * tb + i, 4 * ks + g)]);
+            }
+#pragma unroll
+            for (int mb = 0; mb < MB; mb++) {
+                f4 acc = f4{ 0.f, 0.f, 0.f, 0.f };
+#pragma unroll
+                for (int ks = 0; ks < 4; ks++) {
+                    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(kop[ks], qreg[mb][ks], acc, 0, 0, 0);
+                }
+                sc[mb][tb] = acc;
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (MASKED) {  // selects, not branches, between a matrix op and its first reader
+#pragma unroll
+            for (int mb = 0; mb < MB; mb++) {
+                const int row = row0 + 16 * mb + i;
+#pragma unroll
+                for (int tb = 0; tb < 4; tb++) {
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        if (TILE * t + 16 * tb + 4 * g + r > row) sc[mb][tb][r] = NEG_INF;
+                    }
+                }
+            }
+        }
+        // online softmax: the scale is positive and rides in the exponent's multiply-add
+        float m_new[MB];
+        bool grew = false;
+#pragma unroll
+        for (int mb = 0; mb < MB; mb++) {
+            float mx = fmaxf(fmaxf(sc[mb][0][0], sc[mb][0][1]), fmaxf(sc[mb][0][2], sc[mb][0][3]));
+#pragma unroll
+            for (int tb = 1; tb < 4; tb++) {
+                mx = fmaxf(mx, fmaxf(fmaxf(sc[mb][tb][0], sc[mb][tb][1]), fmaxf(sc[mb][tb][2], sc[mb][tb][3])));
+            }
+            mx = max_over_groups(mx);
+            m_new[mb] = fmaxf(m_run[mb], mx * scale_log2);
+            grew |= m_new[mb] > m_run[mb];
+        }
+        if (__builtin_amdgcn_ballot_w64(grew) != 0) {
+#pragma unroll
+            for (int mb = 0; mb < MB; mb++) {
+                const float alpha = (m_run[mb] == NEG_INF) ? 0.f : fast_exp2(m_run[mb] - m_new[mb]);
+                m_run[mb] = m_new[mb];
+                l_lane[mb] *= alpha;
+#pragma unroll
+                for (int db = 0; db < 8; db++) oacc[mb][db] *= alpha;
+            }
+        }
+        h8 hi[MB][2], lo[MB][2];
+        auto probabilities = [&](int tp) {
+#pragma unroll
+            for (int mb = 0; mb < MB; mb++) {
+                // a row whose scores are all -inf so far has no maximum to subtract
+                const float nm = kShift - (m_run[mb] == NEG_INF ? 0.f : m_run[mb]);
+                float sum = 0.f;
+#pragma unroll
+                for (int e = 0; e < 8; e += 2) {
+                    const float p0 = fast_exp2(__builtin_fmaf(sc[mb][2 * tp + (e >> 2)][e & 3], scale_log2, nm));
+                    const float p1 = fast_exp2(__builtin_fmaf(sc[mb][2 * tp + (e >> 2)][(e & 3) + 1], scale_log2, nm));
+                    const h2 a = __builtin_bit_cast(h2, __builtin_amdgcn_cvt_pkrtz(p0, p1));
+                    const h2 c = __builtin_bit_cast(h2, __builtin_amdgcn_cvt_pkrtz(p0 - float(a[0]), p1 - float(a[1])));
+                    hi[mb][tp][e] = a[0];
+                    hi[mb][tp][e + 1] = a[1];
+                    lo[mb][tp][e] = c[0];
+                    lo[mb][tp][e + 1] = c[1];
+                    sum += p0 + p1;
+                }
+                l_lane[mb] += sum;
+            }
+        };
+        probabilities(0);
+#pragma unroll
+        for (int tp = 0; tp < 2; tp++) {
+            __builtin_amdgcn_sched_barrier(0);
+            h8 a[8];
+#pragma unroll
+            for (int db = 0; db < 8; db++) {
+                const int key = 32 * tp + 4 * g + (i >> 2);     // rows key and key + 16 are swizzled alike
+                const half_t* p0 = &vt[place(key, 2 * db + ((i >> 1) & 1)) + 4 * (i & 1)];
+                const h4 x = lds_read_tr(p0), y = lds_read_tr(p0 + 16 * D);
+                a[db] = h8{ x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3] };
+            }
+            if (tp == 0) probabilities(1);
+#pragma unroll
+            for (int db = 0; db < 8; db++) {
+#pragma unroll
+                for (int mb = 0; mb < MB; mb++) {
+                    oacc[mb][db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[db], hi[mb][tp], oacc[mb][db], 0, 0, 0);
+                }
+            }
+#pragma unroll
+            for (int db = 0; db < 8; db++) {
+#pragma unroll
+                for (int mb = 0; mb < MB; mb++) {
+                    oacc[mb][db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[db], lo[mb][tp], oacc[mb][db], 0, 0, 0);
+                }
+            }
+        }
+    };
+
+    // this wave's pieces of tile t have landed; behind the barrier everyone's have, and everyone is done
+    // with the other buffer
+    auto arrive = [&](int t) {
+        __builtin_amdgcn_s_waitcnt(0x0f70);                    // vmcnt(0)
+        __syncthreads();
+        if (t + 1 < n_tiles) fetch_tile(t + 1, (t + 1) & 1);
+    };
+    fetch_tile(0, 0);
+    const int n_whole = q0 / TILE;                             // tiles that lie before every row of the workgroup
+    for (int t = 0; t < n_whole; t++) {
+        arrive(t);
+        tile_body(t, sm.k[t & 1], sm.v[t & 1], std::false_type{});
+    }
+    // The diagonal, MB tiles: waves whose rows all lie before a tile skip it.  Waves begin at multiples of
+    // 16 * MB, which divides the tile: a wave that takes part has the tile's first key before or at every
+    // one of its rows.
+    for (int t = n_whole; t < n_tiles; t++) {
+        arrive(t);
+        if (TILE * t <= row0) tile_body(t, sm.k[t & 1], sm.v[t & 1], std::true_type{});
+    }
+
+#pragma unroll
+    for (int mb = 0; mb < MB; mb++) {
+        float sum = l_lane[mb];
+        sum += __shfl_xor(sum, 16, 64);
+        sum += __shfl_xor(sum, 32, 64);
+        const int row = row0 + 16 * mb + i;
+        const float r = 1.f / sum;
+        if (row < n) {
+            half_t* dst = out + base + size_t(row) * stride + 4 * g;
+#pragma unroll
+            for (int db = 0; db < 8; db++) {
+                const f4 o = oacc[mb][db];
+                *reinterpret_cast<h4*>(dst + 16 * db) = h4{ half_t(o[0] * r), half_t(o[1] * r), half_t(o[2] * r), half_t(o[3] * r) };
+            }
+        }
+    }
+}
+
+}  // namespace
+
+int launch_causal_attention(const void* q, const void* k, const void* v, void* out, int batch, int n_tokens, int n_heads,
+                            float scale_log2, hipStream_t st) {
+    if (batch <= 0 || n_tokens <= 0 || n_heads <= 0) return 0;
+    const int64_t n_bh = int64_t(batch) * n_heads;
+    // 128 query rows per workgroup reuse a K/V tile twice as often; where that leaves compute units without a
+    // workgroup, 64
+    const bool wide = n_bh * ((n_tokens + 127) / 128) >= 256;
+    const int rows = wide ? 128 : 64;
+    const int64_t blocks = (n_tokens + rows - 1) / rows;
+    if (n_bh * blocks > 0x7fffff00 || n_tokens > 0x7fffff00 - 128) return -1;
+    const dim3 grid(static_cast<unsigned>(n_bh * blocks)), block(WG);
+    const half_t* qh = static_cast<const half_t*>(q);
+    const half_t* kh = static_cast<const half_t*>(k);
+    const half_t* vh = static_cast<const half_t*>(v);
+    half_t* oh = static_cast<half_t*>(out);
+    if (wide) {
+        hipLaunchKernelGGL(causal_attention_kernel<2>, grid, block, 0, st, qh, kh, vh, oh, n_tokens, n_heads, int(n_bh),
+                           int(blocks), scale_log2);
+    } else {
+        hipLaunchKernelGGL(causal_attention_kernel<1>, grid, block, 0, st, qh, kh, vh, oh, n_tokens, n_heads, int(n_bh),
+                           int(blocks), scale_log2);
+    }
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? 0 : static_cast<int>(e);
+}
+
+}  // namespace ca

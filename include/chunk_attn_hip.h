@@ -163,6 +163,14 @@ int ca_rms_norm(void* out, const void* input, const void* weight, float epsilon,
 int ca_fused_add_rms_norm(void* input, void* residual, const void* weight, float epsilon,
                           int64_t n_tokens, int hidden_size, void* stream);
 
+/* Causal attention of whole prompts, the prefill branch of the reference's attention layer
+ * (src/chunk_attn/models/llama_hf/modeling_llama.py:64-84): q, k, v and out are
+ * [batch, n_tokens, n_heads, d_head] fp16 on the device, contiguous, 16-byte aligned, d_head 128;
+ * token t attends tokens 0 .. t of its own sequence, scores scaled by 1/sqrt(d_head), scores, softmax and
+ * sums in fp32, the output rounded to fp16 once.  out must not overlap the inputs. */
+int ca_causal_attention(const void* q, const void* k, const void* v, void* out, int batch, int n_tokens,
+                        int n_heads, int d_head, void* stream);
+
 /* The decode step of the reference's attention layer
  * (src/chunk_attn/models/llama_hf/modeling_llama.py:62,91-95: rotary_embedding on the new
  * query/key rows, then append_token -> append_kv) as one launch: q [n_seqs, n_heads, d_head]

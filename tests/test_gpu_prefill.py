@@ -1,0 +1,59 @@
+"""Causal attention of whole prompts against fp64 on the CPU, at the sizes where the kernel's tiles end:
+64-key tiles, 64- and 128-row workgroups (128 from 256 workgroups on), 32 rows per wave."""
+import math
+
+import pytest
+import torch
+
+from chunk_attn import capi
+
+pytestmark = pytest.mark.gpu
+
+
+def reference(q, k, v):
+    q, k, v = (t.double().transpose(1, 2).contiguous() for t in (q, k, v))
+    n = q.shape[2]
+    scores = (q @ k.transpose(-1, -2).contiguous()) / math.sqrt(q.shape[3])
+    future = torch.ones(n, n, dtype=torch.bool).triu(1)
+    return (torch.softmax(scores.masked_fill(future, float("-inf")), dim=-1) @ v).transpose(1, 2)
+
+
+@pytest.mark.parametrize("batch,n,heads", [
+    (1, 1, 1), (2, 15, 3), (1, 16, 8), (3, 63, 2), (1, 64, 8), (2, 65, 5), (1, 127, 2), (1, 129, 8),
+    (1, 192, 8), (2, 193, 1),
+    (8, 130, 16), (16, 128, 16), (37, 33, 8), (2, 513, 32), (1, 1025, 32)])
+def test_causal_attention_at_tile_edges(batch, n, heads):
+    g = torch.Generator().manual_seed(n * 100 + heads)
+    # scores of a few units either way: the running maximum moves, and small probabilities matter
+    q, k, v = (torch.randn(batch, n, heads, 128, generator=g).half() for _ in range(3))
+    q *= 2
+    out = capi.causal_attention(q.cuda(), k.cuda(), v.cuda()).cpu().double()
+    want = reference(q, k, v)
+    # the output's own rounding is 2^-12 of it at most; sums of n fp32 terms add less than 2^-16 of max |v| < 6
+    assert ((out - want).abs() <= want.abs() * 2.0 ** -11 + 6 * 2.0 ** -16).all()
+
+
+def test_what_a_row_must_not_see_and_extreme_scores():
+    """Tokens after a row change nothing in it; scores of +-3e4 neither overflow nor lose the row."""
+    g = torch.Generator().manual_seed(5)
+    q, k, v = (torch.randn(1, 200, 8, 128, generator=g).half() for _ in range(3))
+    q[:, 50:] *= 60
+    k[:, 50:] *= 60
+    whole = capi.causal_attention(q.cuda(), k.cuda(), v.cuda()).cpu()
+    assert torch.isfinite(whole).all()
+    first = capi.causal_attention(*(t[:, :70].contiguous().cuda() for t in (q, k, v))).cpu()
+    assert torch.equal(whole[:, :70], first)
+    want = reference(q, k, v)
+    # scores of |s| <= 3e4 carry an fp32 rounding of 2^-24 |s| sqrt(128): at most 2^-6 of a probability
+    assert ((whole.double() - want).abs() <= want.abs() * 2.0 ** -6 + 6 * 2.0 ** -6).all()
+    assert torch.equal(whole[:, :50], capi.causal_attention(*(t[:, :50].contiguous().cuda() for t in (q, k, v))).cpu())
+
+
+def test_refused_inputs():
+    q = torch.zeros(1, 8, 2, 128, dtype=torch.float16, device="cuda")
+    for bad in (q.float(), q[:, ::2], torch.zeros(1, 8, 2, 64, dtype=torch.float16, device="cuda"), q.cpu(),
+                torch.zeros(8 * 256 + 1, dtype=torch.float16, device="cuda")[1:].view(1, 8, 2, 128)):
+        assert not capi.causal_attention_takes(bad, bad, bad)
+        with pytest.raises(RuntimeError):
+            capi.causal_attention(bad, bad, bad)
+    assert not capi.causal_attention_takes(q, q, torch.zeros_like(q, requires_grad=True))

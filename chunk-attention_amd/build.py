@@ -37,7 +37,7 @@ def _run(cmd):
 def build_hip_lib() -> str:
     os.makedirs(LIBDIR, exist_ok=True)
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
-    srcs = [os.path.join(CSRC, f) for f in ("kernels.hip", "rotary.hip", "norm.hip", "prefill.hip", "c_api.cpp", "c_api_host.cpp", "tables.cpp", "prefix_tree.cpp")]
+    srcs = [os.path.join(CSRC, f) for f in ("kernels.hip", "rotary.hip", "norm.hip", "prefill.hip", "project.hip", "c_api.cpp", "c_api_host.cpp", "tables.cpp", "prefix_tree.cpp")]
     cmd = [hipcc] + HIP_FLAGS + ["-shared", "-I" + os.path.join(ROOT, "include"), "-I" + CSRC,
                                   "-o", HIP_LIB] + srcs
     _run(cmd)

@@ -3,9 +3,10 @@
 Mirrors the reference's `LlamaChunkAttention`
 (src/chunk_attn/models/llama_hf/modeling_llama.py:16-113) and its rotary module
 (src/chunk_attn/models/llama_hf/rotary_embedding_vllm.py:43-147) with the same argument
-meaning.  The projections are plain torch matmuls; what differs is the decode branch: the
-rotary embedding of the new query/key rows and the KV append are one launch
-(`Attention.append_token_rotary`) instead of a rotary launch followed by an append launch.
+meaning.  For few rows (a decode batch, a short prompt) the three input projections and the rotary
+embedding are one launch, in the decode branch the KV append too; for many the projections are plain
+torch matmuls, and the rotary embedding of a decode step's query/key rows and the KV append are one
+launch (`Attention.append_token_rotary`).
 Weights are whatever the caller loads; tests use seeded random ones.
 """
 from __future__ import annotations
@@ -64,11 +65,24 @@ class LlamaChunkAttention(nn.Module):
         into kv_cache (their cache indices are returned in self.last_indices); decode expects
         batch row i to be cache sequence i."""
         batch, n_tokens, d_hidden = hidden_states.shape
-        q = self.q_proj(hidden_states)
-        k = self.k_proj(hidden_states)
-        v = self.v_proj(hidden_states)
+        projections = (self.q_proj, self.k_proj, self.v_proj)
+        few_rows = self.head_dim == 128 and self._plain_rotary() and capi.projection_takes(hidden_states, *projections)
+        if few_rows:
+            weights = [p.weight for p in projections]
+        if few_rows and not prefill and type(kv_cache) is capi.Attention:   # other caches have append_token_rotary only
+            assert n_tokens == 1
+            q3 = kv_cache.project_append_rotary([s[-1] for s in seqs], hidden_states, *weights,
+                                                self.rotary_emb.cos_sin_cache, position_ids.reshape(batch).contiguous())
+            return self._output(kv_cache.forward(q3).view(batch, 1, d_hidden), kv_cache)
+        if few_rows and prefill:
+            q, k, v = capi.qkv_rotary(hidden_states, *weights, position_ids.contiguous(), self.rotary_emb.cos_sin_cache)
+        else:
+            q = self.q_proj(hidden_states)
+            k = self.k_proj(hidden_states)
+            v = self.v_proj(hidden_states)
         if prefill:
-            q, k = self.rotary_emb(position_ids.contiguous(), q, k)
+            if not few_rows:
+                q, k = self.rotary_emb(position_ids.contiguous(), q, k)
             shape = (batch, n_tokens, self.num_heads, self.head_dim)
             q4, k4, v4 = q.view(shape), k.view(shape), v.view(shape)
             if hidden_states.dtype == torch.float16 and capi.causal_attention_takes(q4, k4, v4):
@@ -89,7 +103,20 @@ class LlamaChunkAttention(nn.Module):
             kv_cache.append_token_rotary([s[-1] for s in seqs], q3, k3, v3, self.rotary_emb.cos_sin_cache,
                                          self.rotary_emb.is_neox_style, position_ids.reshape(batch).contiguous())
             attn_output = kv_cache.forward(q3).view(batch, 1, d_hidden)
-        output = self.o_proj(attn_output)
+        return self._output(attn_output, kv_cache)
+
+    def _plain_rotary(self) -> bool:
+        """The rotary module is the one this layer was built with, over whole heads, and nothing hangs on it."""
+        r = self.rotary_emb
+        return type(r) is RotaryEmbedding and r.is_neox_style and r.rotary_dim == r.head_size == self.head_dim and \
+            not (r._forward_hooks or r._forward_pre_hooks or r._backward_hooks or r._backward_pre_hooks) and \
+            "forward" not in r.__dict__
+
+    def _output(self, attn_output: torch.Tensor, kv_cache: capi.Attention) -> torch.Tensor:
+        if capi.projection_takes(attn_output, self.o_proj):
+            output = capi.linear(attn_output, self.o_proj.weight)
+        else:
+            output = self.o_proj(attn_output)
         kv_cache.reserve()
         kv_cache.refresh_kernel_context(force=False)
         return output

@@ -79,7 +79,10 @@ class AttentionOnlyLM(nn.Module):
             if prefill:
                 for s, idx in zip(seqs, layer.last_indices):
                     s.index = idx
-        return self.lm_head(self.norm(hidden[:, -1]))
+        last = self.norm(hidden[:, -1])
+        if capi.projection_takes(last, self.lm_head):
+            return capi.linear(last, self.lm_head.weight)
+        return self.lm_head(last)
 
     @torch.no_grad()
     def forward(self, seqs: List[Sequence], kv_caches, prefill: bool) -> List[int]:

@@ -789,6 +789,76 @@ int ca_causal_attention(const void* q, const void* k, const void* v, void* out, 
                                                  static_cast<hipStream_t>(stream)), "causal attention launch");
 }
 
+namespace {
+int project(ca::ProjectArgs& a, const void* x, int M, int N, int K, void* stream) {
+    if (M < 0 || N <= 0 || K <= 0 || K % 64 != 0) return fail(CA_ERR_INVALID, "projection: n_in must be a multiple of 64");
+    if (M == 0) return CA_OK;
+    a.x = x;
+    a.M = M;
+    a.N = N;
+    a.K = K;
+    bool ok = x && aligned16(x);
+    a.vec8 = N % 8 == 0;
+    for (int j = 0; j < a.n_w; j++) {
+        ok = ok && a.w[j] && aligned16(a.w[j]) && a.y[j];
+        a.vec8 = a.vec8 && aligned16(a.y[j]);
+    }
+    if (!ok) return fail(CA_ERR_INVALID, "projection: null or misaligned device pointer");
+    if (a.positions && (!a.vec8 || !a.cos_sin_cache || !aligned16(a.cos_sin_cache) || a.max_position <= 0)) {
+        return fail(CA_ERR_INVALID, "projection: misaligned output or no cos/sin cache");
+    }
+    return launch_rc(ca::launch_project(a, static_cast<hipStream_t>(stream)), "projection launch");
+}
+}  // namespace
+
+int ca_linear(const void* x, const void* w, void* y, int n_rows, int n_out, int n_in, void* stream) {
+    ca::ProjectArgs a;
+    a.n_w = 1;
+    a.w[0] = w;
+    a.y[0] = y;
+    return project(a, x, n_rows, n_out, n_in, stream);
+}
+
+int ca_qkv_rotary(const void* x, const void* wq, const void* wk, const void* wv, const int64_t* positions,
+                  const void* cos_sin_cache, int max_position, void* q, void* k, void* v, int n_rows, int n_heads,
+                  int n_in, void* stream) {
+    if (n_heads <= 0 || n_heads > (1 << 20) || (n_rows > 0 && !positions)) return fail(CA_ERR_INVALID, "bad argument");
+    ca::ProjectArgs a;
+    a.n_w = 3;
+    a.w[0] = wq; a.w[1] = wk; a.w[2] = wv;
+    a.y[0] = q; a.y[1] = k; a.y[2] = v;
+    a.positions = positions;
+    a.cos_sin_cache = cos_sin_cache;
+    a.max_position = max_position;
+    return project(a, x, n_rows, n_heads * 128, n_in, stream);
+}
+
+int ca_qkv_rotary_append_kv(ca_ctx* c, const void* x, const void* wq, const void* wk, const void* wv,
+                            const int64_t* positions, const void* cos_sin_cache, int max_position, void* q,
+                            int n_in, int n_seqs, void* stream) {
+    if (int rc = check_ready(c, q, n_seqs)) return rc;
+    if (c->d != 128) return fail(CA_ERR_INVALID, "fused projection and append need d_head 128");
+    if (n_seqs > 0 && !positions) return fail(CA_ERR_INVALID, "null device pointer");
+    if (c->delta_tokens < 0) return fail(CA_ERR_STATE, "delta_tokens is negative");
+    for (int s = 0; s < n_seqs; s++) {
+        if (c->plan.tail_fill[s] + c->delta_tokens >= c->C) {
+            return fail(CA_ERR_STATE, "sequence " + std::to_string(s) + " has no free row in its last chunk: reserve and refresh first");
+        }
+    }
+    ca::ProjectArgs a;
+    a.n_w = 3;
+    a.w[0] = wq; a.w[1] = wk; a.w[2] = wv;
+    a.y[0] = q; a.y[1] = c->k_pool; a.y[2] = c->v_pool;
+    a.positions = positions;
+    a.cos_sin_cache = cos_sin_cache;
+    a.max_position = max_position;
+    a.tail_slot = reinterpret_cast<const int32_t*>(c->dev_blob + c->off_tail_slot);
+    a.tail_fill = reinterpret_cast<const int32_t*>(c->dev_blob + c->off_tail_fill);
+    a.delta_tokens = c->delta_tokens;
+    a.C = c->C;
+    return project(a, x, n_seqs, c->H * 128, n_in, stream);
+}
+
 int ca_rope_append_kv(ca_ctx* c, const int64_t* positions, void* q, const void* k, const void* v,
                       const void* cos_sin_cache, int max_position, int rot_dim, int is_neox,
                       int n_seqs, void* stream) {

@@ -123,4 +123,24 @@ int launch_rms_norm(void* out, void* input, void* residual, const void* weight, 
 int launch_causal_attention(const void* q, const void* k, const void* v, void* out, int batch, int n_tokens, int n_heads,
                             float scale_log2, hipStream_t st);
 
+// y[j] = x . w[j]^T for up to three weights: x [M, K], w[j] [N, K], fp16, contiguous and 16-byte aligned, K a
+// multiple of 64; fp32 sums.  positions == nullptr: y[j] is [M, N].  Otherwise (three weights, N a multiple of
+// 128) the heads of y[0] and y[1] are turned by the angles of the rows' positions (NeoX style over the
+// whole head of 128, cos_sin_cache [max_position, 128]) before they are rounded; with tail_slot set, y[1] and
+// y[2] are the K and the V pool and row m goes to row tail_fill[m] + delta_tokens of chunk tail_slot[m].
+struct ProjectArgs {
+    const void* x = nullptr;
+    const void* w[3] = { nullptr, nullptr, nullptr };
+    void* y[3] = { nullptr, nullptr, nullptr };
+    int M = 0, N = 0, K = 0, n_w = 0;
+    int vec8 = 0;                        // rows of y are whole 16-byte pieces (positions == nullptr only)
+    const int64_t* positions = nullptr;  // [M]
+    const void* cos_sin_cache = nullptr;
+    int max_position = 0;
+    const int32_t* tail_slot = nullptr;  // [M]
+    const int32_t* tail_fill = nullptr;
+    int delta_tokens = 0, C = 0;
+};
+int launch_project(const ProjectArgs& a, hipStream_t st);
+
 }  // namespace ca

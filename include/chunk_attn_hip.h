@@ -171,6 +171,24 @@ int ca_fused_add_rms_norm(void* input, void* residual, const void* weight, float
 int ca_causal_attention(const void* q, const void* k, const void* v, void* out, int batch, int n_tokens,
                         int n_heads, int d_head, void* stream);
 
+/* Projections of n_rows token rows (the torch linear layers of
+ * src/chunk_attn/models/llama_hf/modeling_llama.py:52-62,111): x [n_rows, n_in], weights [n_out, n_in], fp16,
+ * contiguous, 16-byte aligned, n_in a multiple of 64; fp32 sums rounded to fp16 once.  Meant for row
+ * counts at which reading the weights is the work; any count is computed.
+ *   ca_linear:        y [n_rows, n_out] = x . w^T
+ *   ca_qkv_rotary:    q, k, v [n_rows, n_heads, 128] = x . wq^T, x . wk^T, x . wv^T in one launch; the heads of q
+ *                     and k are rotated (NeoX pairs over the whole head, cos_sin_cache [max_position, 128],
+ *                     positions int64 [n_rows]) before they are rounded.
+ *   ca_qkv_rotary_append_kv: the same for one decode step: k and v go to the free row of each sequence's
+ *                     last chunk.  Preconditions and delta_tokens behaviour of ca_append_kv. */
+int ca_linear(const void* x, const void* w, void* y, int n_rows, int n_out, int n_in, void* stream);
+int ca_qkv_rotary(const void* x, const void* wq, const void* wk, const void* wv, const int64_t* positions_dev,
+                  const void* cos_sin_cache, int max_position, void* q, void* k, void* v, int n_rows,
+                  int n_heads, int n_in, void* stream);
+int ca_qkv_rotary_append_kv(ca_ctx* ctx, const void* x, const void* wq, const void* wk, const void* wv,
+                            const int64_t* positions_dev, const void* cos_sin_cache, int max_position, void* q,
+                            int n_in, int n_seqs, void* stream);
+
 /* The decode step of the reference's attention layer
  * (src/chunk_attn/models/llama_hf/modeling_llama.py:62,91-95: rotary_embedding on the new
  * query/key rows, then append_token -> append_kv) as one launch: q [n_seqs, n_heads, d_head]

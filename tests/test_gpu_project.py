@@ -1,0 +1,132 @@
+"""The projection kernel against fp64 at the edges of its tiles: 16, 32 and 64 rows, columns past the last whole
+tile, one to many units of 64 elements for each of the eight waves."""
+import pytest
+import torch
+
+from chunk_attn import capi
+from chunk_attn.llama_layer import LlamaChunkAttention
+
+pytestmark = pytest.mark.gpu
+
+
+def _draw(g, *shape, sigma=1.0):
+    return (torch.randn(*shape, generator=g) * sigma).half().cuda()
+
+
+def _close(got, want, n_in):
+    # one rounding to fp16 (2^-11 of the value), and n_in fp32 products of unit variance summed in any order:
+    # at most 2^-24 * n_in of their absolute sum, which is below n_in * n_in ** -0.5
+    assert got.shape == want.shape
+    assert ((got.double() - want).abs() <= want.abs() * 2.0 ** -11 + n_in ** 1.5 * 2.0 ** -24 + 2.0 ** -20).all()
+
+
+@pytest.mark.parametrize("rows,n_out,n_in", [
+    (1, 1, 64), (1, 17, 128), (3, 500, 256), (8, 8000, 1024), (15, 128, 448), (16, 130, 512), (16, 64, 1088),
+    (16, 48, 1536), (9, 40, 4096), (17, 33, 64), (32, 96, 576), (33, 31, 1024), (64, 512, 256), (65, 130, 320),
+    (252, 1024, 1024), (100, 4100, 1024), (129, 8192, 192), (2048, 512, 512)])
+def test_linear_at_tile_edges(rows, n_out, n_in):
+    g = torch.Generator().manual_seed(rows * 7 + n_out)
+    x, w = _draw(g, rows, n_in), _draw(g, n_out, n_in, sigma=n_in ** -0.5)
+    layer = torch.nn.Linear(n_in, n_out, bias=False, dtype=torch.float16, device="cuda")
+    with torch.no_grad():
+        layer.weight.copy_(w)
+        assert capi.projection_takes(x, layer)
+    guard = torch.full((rows * n_out + 64,), 3.0, dtype=torch.float16, device="cuda")
+    out = guard[:rows * n_out].view(rows, n_out)
+    capi._check(capi.load().ca_linear(x.data_ptr(), w.data_ptr(), out.data_ptr(), rows, n_out, n_in,
+                                      torch.cuda.current_stream().cuda_stream))
+    _close(out, x.double() @ w.double().t(), n_in)
+    assert (guard[rows * n_out:] == 3.0).all()
+    assert torch.equal(capi.linear(x, w), out)
+
+
+@pytest.mark.parametrize("rows,heads,n_in", [(1, 1, 128), (5, 3, 384), (16, 8, 1024), (8, 12, 1536), (17, 2, 256),
+                                             (63, 3, 1024), (252, 8, 1024), (130, 32, 4096), (700, 12, 1472)])
+def test_qkv_rotary(rows, heads, n_in):
+    g = torch.Generator().manual_seed(rows + heads)
+    x = _draw(g, rows, n_in)
+    ws = [_draw(g, heads * 128, n_in, sigma=n_in ** -0.5) for _ in range(3)]
+    angles = torch.rand(300, 64, generator=g) * 6.3
+    table = torch.cat([angles.cos(), angles.sin()], dim=1).half().cuda()
+    positions = torch.randint(-3, 303, (rows,), generator=g)           # outside the table: clamped into it
+    q, k, v = capi.qkv_rotary(x, *ws, positions.cuda(), table)
+    cos, sin = table.double()[positions.clamp(0, 299).cuda()].chunk(2, dim=-1)
+    for got, w, turned in ((q, ws[0], True), (k, ws[1], True), (v, ws[2], False)):
+        want = (x.double() @ w.double().t()).view(rows, heads, 128)
+        if turned:
+            a, b = want.chunk(2, dim=-1)
+            want = torch.cat([a * cos[:, None] - b * sin[:, None], b * cos[:, None] + a * sin[:, None]], dim=-1)
+        _close(got, want.reshape(rows, -1), 2 * n_in)
+
+
+@pytest.mark.parametrize("batch,heads,chunk", [(1, 2, 32), (9, 8, 64), (17, 2, 128)])
+def test_layer_decode_writes_the_pool_as_the_library_path_does(batch, heads, chunk):
+    """The folded step and the one with torch projections leave the same cache (but for fp16 roundings), over
+    steps in which last chunks fill up, and refuse the same calls."""
+    hidden, n = heads * 128, chunk - 2
+    outs, caches = [], []
+    for folded in (True, False):
+        g = torch.Generator().manual_seed(batch)
+        layer = LlamaChunkAttention(hidden, heads, device="cuda")
+        with torch.no_grad():
+            for p in (layer.q_proj, layer.k_proj, layer.v_proj, layer.o_proj):
+                p.weight.copy_(_draw(g, hidden, hidden, sigma=hidden ** -0.5))
+        if not folded:
+            for p in (layer.q_proj, layer.o_proj):
+                p.register_forward_hook(lambda module, args, out: out)   # something hangs on the module
+        kv = capi.Attention(heads, 128, chunk, memory_mb=64, dtype=torch.float16, device=torch.device("cuda:0"))
+        seqs = [[100 * s + t for t in range(n)] for s in range(batch)]
+        out = []
+        with torch.inference_mode():
+            pos = torch.arange(n).repeat(batch, 1).cuda()
+            out.append(layer(_draw(g, batch, n, hidden), seqs, pos, kv, True))
+            for t in range(4):
+                seqs = [s + [7] for s in seqs]
+                out.append(layer(_draw(g, batch, 1, hidden), seqs, torch.full((batch, 1), n + t).cuda(), kv, False))
+            with pytest.raises(RuntimeError, match="num of seqs"):
+                layer(_draw(g, batch + 1, 1, hidden), seqs + [[1]], torch.zeros(batch + 1, 1, dtype=torch.int64).cuda(), kv, False)
+        outs.append(out)
+        caches.append((kv.tree.get_chunks(), [p.float() for p in kv.pool_views()]))
+    assert (caches[0][0] == caches[1][0]).all()
+    for a, b in zip(*outs):
+        assert (a.float() - b.float()).norm() <= 4e-3 * b.float().norm()
+    for slot, n_tokens, _, _ in caches[0][0]:
+        for a, b in zip(caches[0][1], caches[1][1]):
+            a, b = a[slot][:, :n_tokens], b[slot][:, :n_tokens]
+            # the library path rounds the projection, then the rotation: two roundings of 2^-11 against one
+            assert ((a - b).abs() <= 2.0 ** -9 * b.abs().amax()).all()
+
+
+def test_layer_takes_the_pybind_cache_too():
+    from chunk_attn import Attention
+    outs = []
+    for cls in (capi.Attention, Attention):
+        g = torch.Generator().manual_seed(3)
+        layer = LlamaChunkAttention(256, 2, device="cuda")
+        kv = cls(2, 128, 64, memory_mb=16, dtype=torch.float16, device=torch.device("cuda:0"))
+        with torch.inference_mode():
+            pos = torch.arange(20).repeat(3, 1).cuda()
+            x, y = _draw(g, 3, 20, 256), _draw(g, 3, 1, 256)
+            for p, w in zip((layer.q_proj, layer.k_proj, layer.v_proj, layer.o_proj), (_draw(g, 256, 256, sigma=0.06) for _ in range(4))):
+                p.weight.copy_(w)
+            layer(x, [[s] * 20 for s in range(3)], pos, kv, True)
+            outs.append(layer(y, [[s] * 21 for s in range(3)], torch.full((3, 1), 20).cuda(), kv, False).float())
+    assert (outs[0] - outs[1]).norm() <= 4e-3 * outs[1].norm()
+
+
+def test_what_the_projection_leaves_to_torch():
+    x = torch.zeros(4, 256, dtype=torch.float16, device="cuda")
+    lin = torch.nn.Linear(256, 128, bias=False, dtype=torch.float16, device="cuda")
+    assert not capi.projection_takes(x, lin)                            # a gradient is wanted
+    with torch.no_grad():
+        assert capi.projection_takes(x, lin)
+        assert not capi.projection_takes(x.float(), lin)
+        assert not capi.projection_takes(torch.zeros(4, 512, dtype=torch.float16, device="cuda")[:, ::2], lin)
+        assert not capi.projection_takes(torch.zeros(8192, 256, dtype=torch.float16, device="cuda"), lin)
+        assert not capi.projection_takes(x, torch.nn.Linear(256, 128, dtype=torch.float16, device="cuda"))
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            assert not capi.projection_takes(x, lin)
+        handle = lin.register_forward_hook(lambda *a: None)
+        assert not capi.projection_takes(x, lin)
+        handle.remove()
+        assert capi.projection_takes(x, lin)

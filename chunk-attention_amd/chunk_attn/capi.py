@@ -10,6 +10,7 @@ entry point reports an error when no HIP device is present.
 """
 from __future__ import annotations
 
+import array
 import ctypes
 import os
 from typing import List, Optional, Sequence, Tuple
@@ -81,6 +82,9 @@ SIGNATURES = {
                       [ctypes.c_int] * 3 + [ctypes.c_void_p]),
     "ca_qkv_rotary_append_kv": (ctypes.c_int, [ctypes.c_void_p] * 7 + [ctypes.c_int, ctypes.c_void_p, ctypes.c_int,
                                                                        ctypes.c_int, ctypes.c_void_p]),
+    "ca_layer_decode": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, c_i32_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_int] +
+                        [ctypes.c_void_p] * 4 + [ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int] +
+                        [ctypes.c_void_p] * 4),
     "ca_rope_append_kv": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
                                          ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_int,
                                          ctypes.c_int, ctypes.c_int, ctypes.c_void_p]),
@@ -181,12 +185,29 @@ def _check(rc: int) -> None:
         raise ChunkAttnError(rc, load().ca_last_error().decode())
 
 
+def _launch(device, fn, *args) -> None:
+    """fn(*args, stream): the current stream of `device`, with that device current."""
+    import torch
+    if device.index is None or torch._C._cuda_getDevice() == device.index:
+        index = device.index if device.index is not None else torch._C._cuda_getDevice()
+        _check(fn(*args, torch._C._cuda_getCurrentRawStream(index)))
+    else:
+        with torch.cuda.device(device):
+            _check(fn(*args, torch._C._cuda_getCurrentRawStream(device.index)))
+
+
 def set_markers(enable: bool) -> None:
     """Named ranges (roctx) around refreshes, patches, attention calls and appends; off by default."""
     _check(load().ca_set_markers(1 if enable else 0))
 
 
 def _i32(values: Sequence[int]):
+    if type(values) is list and values:
+        try:
+            flat = array.array("i", values)          # several times as fast as numpy for lists of Python ints
+            return flat, (ctypes.c_int32 * len(flat)).from_buffer(flat)
+        except TypeError:                            # other things that convert: numpy's business
+            pass
     arr = np.ascontiguousarray(np.asarray(values, dtype=np.int32))
     return arr, arr.ctypes.data_as(c_i32_p)
 
@@ -347,12 +368,9 @@ def rotary_embedding(positions, query, key, head_size: int, cos_sin_cache, is_ne
     k_stride = key.shape[-1] if k2 is not None else key.stride(-2)
     if (q2 is None or k2 is None) and query.dim() != 2:
         raise RuntimeError("strided query/key must be two-dimensional")
-    with torch.cuda.device(query.device):
-        stream = torch.cuda.current_stream(query.device).cuda_stream
-        _check(load().ca_rotary_embedding(positions.data_ptr(), query.data_ptr(), key.data_ptr(),
-                                          cos_sin_cache.data_ptr(), n_tokens, query.shape[-1] // head_size,
-                                          key.shape[-1] // head_size, head_size, cos_sin_cache.shape[1],
-                                          cos_sin_cache.shape[0], q_stride, k_stride, int(is_neox), stream))
+    _launch(query.device, load().ca_rotary_embedding, positions.data_ptr(), query.data_ptr(), key.data_ptr(),
+            cos_sin_cache.data_ptr(), n_tokens, query.shape[-1] // head_size, key.shape[-1] // head_size, head_size,
+            cos_sin_cache.shape[1], cos_sin_cache.shape[0], q_stride, k_stride, int(is_neox))
 
 
 def _norm_args(name, tensors, weight):
@@ -370,21 +388,16 @@ def _norm_args(name, tensors, weight):
 def rms_norm(out, input, weight, epsilon: float) -> None:
     """out = rms_norm(input) * weight on torch fp16 tensors, the reference's
     `chunk_attn.ops.rms_norm` (python_exports_ops.cpp:16)."""
-    import torch
     n, hidden = _norm_args("rms_norm", [input, out], weight)
-    with torch.cuda.device(input.device):
-        _check(load().ca_rms_norm(out.data_ptr(), input.data_ptr(), weight.data_ptr(), float(epsilon), n, hidden,
-                                  torch.cuda.current_stream(input.device).cuda_stream))
+    _launch(input.device, load().ca_rms_norm, out.data_ptr(), input.data_ptr(), weight.data_ptr(), float(epsilon), n, hidden)
 
 
 def fused_add_rms_norm(input, residual, weight, epsilon: float) -> None:
     """In place: residual += input; input = rms_norm(residual) * weight, the reference's
     `chunk_attn.ops.fused_add_rms_norm` (python_exports_ops.cpp:17)."""
-    import torch
     n, hidden = _norm_args("fused_add_rms_norm", [input, residual], weight)
-    with torch.cuda.device(input.device):
-        _check(load().ca_fused_add_rms_norm(input.data_ptr(), residual.data_ptr(), weight.data_ptr(), float(epsilon),
-                                            n, hidden, torch.cuda.current_stream(input.device).cuda_stream))
+    _launch(input.device, load().ca_fused_add_rms_norm, input.data_ptr(), residual.data_ptr(), weight.data_ptr(),
+            float(epsilon), n, hidden)
 
 
 def causal_attention_takes(*tensors) -> bool:
@@ -406,9 +419,7 @@ def causal_attention(q, k, v):
         raise RuntimeError("causal_attention: contiguous, 16-byte aligned fp16 GPU tensors [batch, n, heads, 128] "
                            "of one shape, without gradients")
     out = torch.empty_like(q)
-    with torch.cuda.device(q.device):
-        _check(load().ca_causal_attention(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), q.shape[0], q.shape[1],
-                                          q.shape[2], q.shape[3], torch.cuda.current_stream(q.device).cuda_stream))
+    _launch(q.device, load().ca_causal_attention, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), *q.shape)
     return out
 
 
@@ -431,13 +442,16 @@ def projection_takes(x, *linears) -> bool:
             torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack() or \
             torch.nn.modules.module._has_any_global_hook() or torch.autograd.forward_ad._current_level >= 0:
         return False
+    device = x.device
     for m in linears:
-        if type(m) is not torch.nn.Linear or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or \
-                m._backward_pre_hooks or "forward" in m.__dict__:
+        own = m.__dict__
+        if type(m) is not torch.nn.Linear or own["_forward_hooks"] or own["_forward_pre_hooks"] or \
+                own["_backward_hooks"] or own["_backward_pre_hooks"] or "forward" in own:
             return False
-        w = m.weight
-        if type(w) not in (torch.nn.Parameter, torch.Tensor) or m.bias is not None or w.dtype != torch.float16 or \
-                w.device != x.device or w.dim() != 2 or w.shape[1] != n_in or not w.is_contiguous() or \
+        parameters = own["_parameters"]
+        w = parameters.get("weight")
+        if type(w) is not torch.nn.Parameter or parameters.get("bias", w) is not None or w.dtype != torch.float16 or \
+                w.device != device or w.dim() != 2 or w.shape[1] != n_in or not w.is_contiguous() or \
                 w.data_ptr() % 16 or (grad and w.requires_grad):
             return False
     return True
@@ -448,9 +462,7 @@ def linear(x, weight):
     import torch
     out = torch.empty(x.shape[:-1] + (weight.shape[0],), dtype=x.dtype, device=x.device)
     n_in = x.shape[-1]
-    with torch.cuda.device(x.device):
-        _check(load().ca_linear(x.data_ptr(), weight.data_ptr(), out.data_ptr(), x.numel() // n_in, weight.shape[0], n_in,
-                                torch.cuda.current_stream(x.device).cuda_stream))
+    _launch(x.device, load().ca_linear, x.data_ptr(), weight.data_ptr(), out.data_ptr(), x.numel() // n_in, weight.shape[0], n_in)
     return out
 
 
@@ -474,11 +486,8 @@ def qkv_rotary(x, wq, wk, wv, positions, cos_sin_cache):
     if n % 128 or wk.shape != wq.shape or wv.shape != wq.shape:
         raise RuntimeError("q, k and v weights must have one shape of whole heads of 128")
     q, k, v = torch.empty((3,) + tuple(x.shape[:-1]) + (n,), dtype=x.dtype, device=x.device).unbind(0)
-    with torch.cuda.device(x.device):
-        _check(load().ca_qkv_rotary(x.data_ptr(), wq.data_ptr(), wk.data_ptr(), wv.data_ptr(), positions.data_ptr(),
-                                    cos_sin_cache.data_ptr(), cos_sin_cache.shape[0], q.data_ptr(), k.data_ptr(),
-                                    v.data_ptr(), rows, n // 128, n_in,
-                                    torch.cuda.current_stream(x.device).cuda_stream))
+    _launch(x.device, load().ca_qkv_rotary, x.data_ptr(), wq.data_ptr(), wk.data_ptr(), wv.data_ptr(), positions.data_ptr(),
+            cos_sin_cache.data_ptr(), cos_sin_cache.shape[0], q.data_ptr(), k.data_ptr(), v.data_ptr(), rows, n // 128, n_in)
     return q, k, v
 
 
@@ -796,7 +805,8 @@ class Attention:
 
     def _stream(self) -> int:
         import torch
-        return torch.cuda.current_stream(self.device).cuda_stream
+        index = self.device.index
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice() if index is None else index)
 
     def _check_kv(self, t, rows: int, name: str):
         import torch
@@ -893,6 +903,27 @@ class Attention:
         self.tree.append_token(tokens)
         self.ctx.delta_tokens = self.ctx.delta_tokens + 1
         return n_new
+
+    def layer_decode(self, tokens: Sequence[int], x, wq, wk, wv, wo, cos_sin_cache, positions):
+        """project_append_rotary, forward and the output projection, then room for the next step's token
+        (reserve, refresh_kernel_context): a layer's decode pass as one native call.  Returns [n, n_out]."""
+        import torch
+        n = len(tokens)
+        if self.tree.n_seqs != n:
+            raise RuntimeError("num of seqs is not equal to num of tokens")
+        n_in, width = x.shape[-1], self.n_heads * 128
+        if self.d_head != 128 or x.device != self.device or x.numel() != n * n_in or wo.dim() != 2 or wo.shape[1] != width or \
+                wo.data_ptr() % 16 or any(w.shape != (width, n_in) for w in (wq, wk, wv)):
+            raise RuntimeError(f"x must be [{n}, n_in] and the weights [{width}, n_in] and [n_out, {width}] on {self.device}, d_head 128")
+        _check_rotary(positions, n, cos_sin_cache, self.device)
+        rows = torch.empty((2, n, width), dtype=x.dtype, device=x.device)     # q, then the attention's output
+        y = torch.empty((n, wo.shape[0]), dtype=x.dtype, device=x.device)
+        arr, ptr = _i32(tokens)
+        q = rows.data_ptr()
+        _launch(x.device, self.ctx._lib.ca_layer_decode, self.ctx._h, self.tree._h, ptr, n, x.data_ptr(), n_in, wq.data_ptr(),
+                wk.data_ptr(), wv.data_ptr(), wo.data_ptr(), wo.shape[0], positions.data_ptr(), cos_sin_cache.data_ptr(),
+                cos_sin_cache.shape[0], q, q + 2 * n * width, y.data_ptr())
+        return y
 
     def project_append_rotary(self, tokens: Sequence[int], x, wq, wk, wv, cos_sin_cache, positions):
         """append_token_rotary with the projections folded in: the rows of x (what projection_takes accepts)

@@ -66,14 +66,20 @@ class LlamaChunkAttention(nn.Module):
         batch row i to be cache sequence i."""
         batch, n_tokens, d_hidden = hidden_states.shape
         projections = (self.q_proj, self.k_proj, self.v_proj)
-        few_rows = self.head_dim == 128 and self._plain_rotary() and capi.projection_takes(hidden_states, *projections)
+        own_output = few_rows = False                  # which projections the framework's own kernel computes
+        if self.head_dim == 128 and self._plain_rotary():
+            own_output = capi.projection_takes(hidden_states, *projections, self.o_proj)
+            few_rows = own_output or capi.projection_takes(hidden_states, *projections)
         if few_rows:
             weights = [p.weight for p in projections]
         if few_rows and not prefill and type(kv_cache) is capi.Attention:   # other caches have append_token_rotary only
             assert n_tokens == 1
-            q3 = kv_cache.project_append_rotary([s[-1] for s in seqs], hidden_states, *weights,
-                                                self.rotary_emb.cos_sin_cache, position_ids.reshape(batch).contiguous())
-            return self._output(kv_cache.forward(q3).view(batch, 1, d_hidden), kv_cache)
+            step = ([s[-1] for s in seqs], hidden_states, *weights)
+            rotary = (self.rotary_emb.cos_sin_cache, position_ids.reshape(batch).contiguous())
+            if own_output:
+                return kv_cache.layer_decode(*step, self.o_proj.weight, *rotary).view(batch, 1, -1)
+            q3 = kv_cache.project_append_rotary(*step, *rotary)
+            return self._output(kv_cache.forward(q3).view(batch, 1, d_hidden), kv_cache, False)
         if few_rows and prefill:
             q, k, v = capi.qkv_rotary(hidden_states, *weights, position_ids.contiguous(), self.rotary_emb.cos_sin_cache)
         else:
@@ -103,7 +109,7 @@ class LlamaChunkAttention(nn.Module):
             kv_cache.append_token_rotary([s[-1] for s in seqs], q3, k3, v3, self.rotary_emb.cos_sin_cache,
                                          self.rotary_emb.is_neox_style, position_ids.reshape(batch).contiguous())
             attn_output = kv_cache.forward(q3).view(batch, 1, d_hidden)
-        return self._output(attn_output, kv_cache)
+        return self._output(attn_output, kv_cache, own_output and attn_output.is_contiguous())
 
     def _plain_rotary(self) -> bool:
         """The rotary module is the one this layer was built with, over whole heads, and nothing hangs on it."""
@@ -112,11 +118,8 @@ class LlamaChunkAttention(nn.Module):
             not (r._forward_hooks or r._forward_pre_hooks or r._backward_hooks or r._backward_pre_hooks) and \
             "forward" not in r.__dict__
 
-    def _output(self, attn_output: torch.Tensor, kv_cache: capi.Attention) -> torch.Tensor:
-        if capi.projection_takes(attn_output, self.o_proj):
-            output = capi.linear(attn_output, self.o_proj.weight)
-        else:
-            output = self.o_proj(attn_output)
+    def _output(self, attn_output: torch.Tensor, kv_cache: capi.Attention, own: bool) -> torch.Tensor:
+        output = capi.linear(attn_output, self.o_proj.weight) if own else self.o_proj(attn_output)
         kv_cache.reserve()
         kv_cache.refresh_kernel_context(force=False)
         return output

@@ -26,7 +26,7 @@ class RMSNorm(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         x = x.contiguous()
         out = torch.empty_like(x)
-        capi.rms_norm(out, x, self.weight.detach(), self.eps)
+        capi.rms_norm(out, x, self.weight, self.eps)
         return out
 
 
@@ -70,8 +70,8 @@ class AttentionOnlyLM(nn.Module):
             input_ids = [[s[-1]] for s in seqs]
             position_ids = [[len(s) - 1] for s in seqs]
         dev = self.embed_tokens.weight.device
-        ids = torch.tensor(input_ids, dtype=torch.long, device=dev)
-        pos = torch.tensor(position_ids, dtype=torch.int64, device=dev)
+        # one upload, from pinned memory: the host does not wait for what the GPU still has to do
+        ids, pos = torch.tensor([input_ids, position_ids], dtype=torch.int64, pin_memory=dev.type == "cuda").to(dev, non_blocking=True)
         hidden = self.embed_tokens(ids)
         token_lists = [s.tokens for s in seqs]
         for i, layer in enumerate(self.layers):

@@ -859,6 +859,47 @@ int ca_qkv_rotary_append_kv(ca_ctx* c, const void* x, const void* wq, const void
     return project(a, x, n_seqs, c->H * 128, n_in, stream);
 }
 
+namespace {
+// A free row in every last chunk, and device tables that know it.
+int settle(ca_ctx* c, ca_tree* tree, int n_seqs, void* stream) {
+    std::vector<int32_t> seqs(n_seqs), slots(n_seqs);
+    int n = 0;
+    if (int rc = ca_tree_reserve_tails(tree, seqs.data(), slots.data(), n_seqs, &n)) return rc;
+    if (n > 0 && c->valid) {
+        const int rc = ca_ctx_roll_tails(c, seqs.data(), slots.data(), n, stream);
+        if (rc != CA_OK && rc != CA_ERR_STATE) {
+            ca_ctx_invalidate(c);                   // the tree has the new chunks, the tables do not
+            return rc;
+        }
+        if (rc != CA_OK) ca_ctx_invalidate(c);      // not patchable: built anew below
+    }
+    if (c->valid) return CA_OK;
+    int n_rows = 0;
+    if (int rc = ca_tree_get_chunks(tree, nullptr, 0, &n_rows)) return rc;
+    std::vector<ca_chunk_row> rows(std::max(n_rows, 1));
+    if (int rc = ca_tree_get_chunks(tree, rows.data(), n_rows, &n_rows)) return rc;
+    return ca_refresh_kernel_context(c, rows.data(), n_rows, n_seqs, stream);
+}
+}  // namespace
+
+int ca_layer_decode(ca_ctx* c, ca_tree* tree, const int32_t* tokens, int n_seqs, const void* x, int n_in,
+                    const void* wq, const void* wk, const void* wv, const void* wo, int n_out,
+                    const int64_t* positions, const void* cos_sin_cache, int max_position, void* q, void* attn,
+                    void* y, void* stream) {
+    if (!c || !tree || !tokens || n_seqs <= 0) return fail(CA_ERR_INVALID, "bad argument");
+    if (ca_tree_n_seqs(tree) != n_seqs) return fail(CA_ERR_INVALID, "num of seqs is not equal to num of tokens");
+    return guarded([&]() -> int {
+        if (int rc = settle(c, tree, n_seqs, stream)) return rc;
+        if (int rc = ca_qkv_rotary_append_kv(c, x, wq, wk, wv, positions, cos_sin_cache, max_position, q, n_in, n_seqs, stream)) return rc;
+        int fresh = 0;
+        if (int rc = ca_tree_append_token(tree, tokens, n_seqs, &fresh)) return rc;
+        if (int rc = ca_ctx_set_delta_tokens(c, c->delta_tokens + 1)) return rc;
+        if (int rc = ca_attention(c, q, attn, n_seqs, 0, stream)) return rc;
+        if (int rc = ca_linear(attn, wo, y, n_seqs, n_out, c->H * 128, stream)) return rc;
+        return settle(c, tree, n_seqs, stream);
+    });
+}
+
 int ca_rope_append_kv(ca_ctx* c, const int64_t* positions, void* q, const void* k, const void* v,
                       const void* cos_sin_cache, int max_position, int rot_dim, int is_neox,
                       int n_seqs, void* stream) {

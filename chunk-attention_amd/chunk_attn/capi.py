@@ -423,6 +423,13 @@ def causal_attention(q, k, v):
     return out
 
 
+def is_bare(module, cls) -> bool:
+    """The module is a `cls` and nothing hangs on it that a call would also run (hooks, a patched forward)."""
+    own = module.__dict__
+    return type(module) is cls and not (own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"] or
+                                        own["_backward_pre_hooks"] or "forward" in own)
+
+
 def projection_takes(x, *linears) -> bool:
     """Whether the projection kernel stands in for these torch.nn.Linear modules on the rows of x: nothing but
     x . W^T in fp16 on one GPU is asked of them, and the product is small enough.
@@ -444,11 +451,9 @@ def projection_takes(x, *linears) -> bool:
         return False
     device = x.device
     for m in linears:
-        own = m.__dict__
-        if type(m) is not torch.nn.Linear or own["_forward_hooks"] or own["_forward_pre_hooks"] or \
-                own["_backward_hooks"] or own["_backward_pre_hooks"] or "forward" in own:
+        if not is_bare(m, torch.nn.Linear):
             return False
-        parameters = own["_parameters"]
+        parameters = m.__dict__["_parameters"]
         w = parameters.get("weight")
         if type(w) is not torch.nn.Parameter or parameters.get("bias", w) is not None or w.dtype != torch.float16 or \
                 w.device != device or w.dim() != 2 or w.shape[1] != n_in or not w.is_contiguous() or \

@@ -114,9 +114,7 @@ class LlamaChunkAttention(nn.Module):
     def _plain_rotary(self) -> bool:
         """The rotary module is the one this layer was built with, over whole heads, and nothing hangs on it."""
         r = self.rotary_emb
-        return type(r) is RotaryEmbedding and r.is_neox_style and r.rotary_dim == r.head_size == self.head_dim and \
-            not (r._forward_hooks or r._forward_pre_hooks or r._backward_hooks or r._backward_pre_hooks) and \
-            "forward" not in r.__dict__
+        return capi.is_bare(r, RotaryEmbedding) and r.is_neox_style and r.rotary_dim == r.head_size == self.head_dim
 
     def _output(self, attn_output: torch.Tensor, kv_cache: capi.Attention, own: bool) -> torch.Tensor:
         output = capi.linear(attn_output, self.o_proj.weight) if own else self.o_proj(attn_output)

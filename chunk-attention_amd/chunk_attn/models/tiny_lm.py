@@ -74,15 +74,36 @@ class AttentionOnlyLM(nn.Module):
         ids, pos = torch.tensor([input_ids, position_ids], dtype=torch.int64, pin_memory=dev.type == "cuda").to(dev, non_blocking=True)
         hidden = self.embed_tokens(ids)
         token_lists = [s.tokens for s in seqs]
+        joined = self._adds_in_norms()
+        normed = self.input_norms[0](hidden) if len(self.layers) else None
         for i, layer in enumerate(self.layers):
-            hidden = hidden + layer(self.input_norms[i](hidden), token_lists, pos, kv_caches[i], prefill)
+            out = layer(normed, token_lists, pos, kv_caches[i], prefill)
             if prefill:
                 for s, idx in zip(seqs, layer.last_indices):
                     s.index = idx
-        last = self.norm(hidden[:, -1])
+            final = i + 1 == len(self.layers)
+            norm = self.norm if final else self.input_norms[i + 1]
+            if final:   # from here on the last positions alone
+                out, hidden = out[:, -1], hidden[:, -1]
+            if joined:  # hidden += out, out = norm(hidden): one launch over both
+                out, hidden = out.contiguous(), hidden.contiguous()
+                capi.fused_add_rms_norm(out, hidden, norm.weight, norm.eps)
+                normed = out
+            else:
+                hidden = hidden + out
+                normed = norm(hidden)
+        last = self.norm(hidden[:, -1]) if normed is None else normed
         if capi.projection_takes(last, self.lm_head):
             return capi.linear(last, self.lm_head.weight)
         return self.lm_head(last)
+
+    def _adds_in_norms(self) -> bool:
+        """A layer's residual is added in the norm behind it, in place: nothing may want the tensors it overwrites
+        (a gradient, a hook), and the norms must be the plain ones."""
+        return not torch.is_grad_enabled() and capi.is_bare(self.embed_tokens, nn.Embedding) and \
+            all(capi.is_bare(m, LlamaChunkAttention) for m in self.layers) and \
+            all(capi.is_bare(m, RMSNorm) for m in self.input_norms) and capi.is_bare(self.norm, RMSNorm) and \
+            not torch.nn.modules.module._has_any_global_hook() and not torch._C._len_torch_dispatch_stack()
 
     @torch.no_grad()
     def forward(self, seqs: List[Sequence], kv_caches, prefill: bool) -> List[int]:

@@ -114,6 +114,33 @@ def test_layer_takes_the_pybind_cache_too():
     assert (outs[0] - outs[1]).norm() <= 4e-3 * outs[1].norm()
 
 
+def test_model_with_its_adds_in_the_norms():
+    """A hook on a norm keeps the adds on their own: the same logits but for the roundings of the residual."""
+    from chunk_attn.models.sequence import Sequence
+    from chunk_attn.models.tiny_lm import AttentionOnlyLM
+    runs = []
+    for hooked in (False, True):
+        model = AttentionOnlyLM(300, 256, 2, 3, chunk_size=32, memory_mb=16, seed=4)
+        seen = []
+        if hooked:
+            model.input_norms[1].register_forward_hook(lambda m, a, out: seen.append(out.clone()))
+        caches, out = model.create_kv_caches(), []
+        with torch.inference_mode():
+            seqs = [Sequence([5 * s + t for t in range(40)]) for s in range(3)]
+            out.append(model.logits(seqs, caches, True))
+            seqs.sort(key=lambda s: s.index)
+            for t in range(3):
+                for s in seqs:
+                    s.append(7 + t)
+                out.append(model.logits(seqs, caches, False))
+        assert len(seen) == (4 if hooked else 0)
+        runs.append(out)
+    for a, b in zip(*runs):
+        # each norm's input differs by one fp16 rounding (2^-11) of the residual at most
+        assert (a.float() - b.float()).norm() <= 4e-3 * b.float().norm()
+    assert AttentionOnlyLM(50, 128, 1, 0, memory_mb=1).logits([Sequence([1, 2])], [], True).shape == (1, 50)
+
+
 def test_what_the_projection_leaves_to_torch():
     x = torch.zeros(4, 256, dtype=torch.float16, device="cuda")
     lin = torch.nn.Linear(256, 128, bias=False, dtype=torch.float16, device="cuda")

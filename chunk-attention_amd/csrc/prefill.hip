@@ -20,9 +20,11 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 
 constexpr int D = 128;
 constexpr int WG = 256;
-constexpr int TILE = 64;            // keys per tile
+constexpr int NW = WG / 64;
+constexpr int ROWS = 64;            // query rows of a workgroup
 constexpr float NEG_INF = -__builtin_huge_valf();
 constexpr float kShift = 8.f;       // probabilities are kept as 2^8 times their value (see below)
+constexpr float kSlack = 7.f;       // a row's maximum moves when it grows by more than 2^7 (see below)
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
@@ -32,46 +34,73 @@ __device__ __forceinline__ h4 lds_read_tr(const half_t* p) {
     return __builtin_bit_cast(h4, raw);
 }
 
+// what fp16 leaves of p: p - a, a the lower or upper half of a register (one instruction; written out, the
+// compiler widens the half first)
+template <bool UPPER>
+__device__ __forceinline__ float rest_of(float p, h2 a) {
+    float r;
+    if constexpr (UPPER) asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(a), "v"(p));
+    else asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(a), "v"(p));
+    return r;
+}
+
+// IEEE maximum: unlike fmaxf it needs no canonical inputs, and three of them fit one instruction
+__device__ __forceinline__ float max2(float a, float b) { return __builtin_elementwise_maximum(a, b); }
+
 // maximum over lanes l, l^16, l^32, l^48 (the four 16-lane groups), in all four
 __device__ __forceinline__ float max_over_groups(float v) {
     const unsigned u = __builtin_bit_cast(unsigned, v);
     const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
     const unsigned a0 = a[0], a1 = a[1];
-    const float m16 = fmaxf(__builtin_bit_cast(float, a0), __builtin_bit_cast(float, a1));
+    const float m16 = max2(__builtin_bit_cast(float, a0), __builtin_bit_cast(float, a1));
     const unsigned w = __builtin_bit_cast(unsigned, m16);
     const auto b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
     const unsigned b0 = b[0], b1 = b[1];
-    return fmaxf(__builtin_bit_cast(float, b0), __builtin_bit_cast(float, b1));
+    return max2(__builtin_bit_cast(float, b0), __builtin_bit_cast(float, b1));
 }
 
 // K and V tiles in LDS, rows of 256 B without padding (the direct global -> LDS loads write 64
-// consecutive 16-byte pieces): piece c of row r stands at place c ^ (r & 15), so that the 16 rows a
-// read touches at one column lie in 16 different bank groups.
+// consecutive 16-byte pieces): piece c of row r stands at place c ^ swizzle(r).  A 16-byte read is served for
+// eight lanes of two neighbouring 16-lane groups at a time, i.e. eight rows at two neighbouring pieces, a
+// transposed read for eight rows at two pieces too: the swizzle leaves the lowest bit of the piece alone within
+// eight rows, so that those sixteen places are all different.
+template <int TILE>
 struct CausalLds {
     half_t k[2][TILE * D];
     half_t v[2][TILE * D];
 };
-__device__ __forceinline__ int place(int row, int piece) { return row * D + ((piece ^ (row & 15)) << 3); }
-
-__device__ __forceinline__ void load_to_lds16(const half_t* src, half_t* dst) {
+__device__ __forceinline__ int swizzle(int row) { return ((row & 7) << 1) | ((row >> 3) & 1); }
+__device__ __forceinline__ int place(int row, int piece) { return row * D + ((piece ^ swizzle(row)) << 3); }
+__device__ __forceinline__ void load_to_lds16(const char* src, half_t* dst) {
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
                                      (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
 }
 
-// A workgroup attends 64 * MB query rows of one (sequence, head): wave w owns 16 * MB of them and
-// keeps their Q^T operands and output accumulators in registers; 64-key tiles of K and V go through
-// LDS, the next tile on its way into a second buffer.  S^T = K.Q^T leaves each lane with four keys of one row,
-// which is the operand layout O^T = V^T.P^T needs, so probabilities never leave registers.
+// A workgroup attends 64 query rows of one (sequence, head): wave w owns 16 of them and keeps their Q^T
+// operands and output accumulators in registers; TILE-key tiles of K and V go through LDS, the next tile on
+// its way into a second buffer.  S^T = K.Q^T leaves each lane with four keys of one row, which is the operand
+// layout O^T = V^T.P^T needs, so probabilities never leave registers.
+//
+// What bounds it: matrix ops (half of them the second P.V product below) and the vector ops of the softmax are
+// about equal, and each wave's run of them is one dependent chain; what hides a chain is another wave.  TILE 32
+// holds four workgroups a compute unit (118 registers, 32 KB), 64 two.  32 heads, 2048 tokens: 68 us, 8 x 300
+// tokens 25 us; 16 heads, 8 x 1000 tokens 69 us (32 rows a wave, 64 keys a tile, two workgroups a unit: 81, 40 and
+// 85).  Long runs of large ones are held back by the clock, which falls with what they draw (about 1.7 GHz).
 //
 // The probabilities are fp32; the matrix cores take fp16.  p = hi + lo with hi = fp16(p) and
 // lo = fp16(p - hi) carries 21 bits of p at the price of a second P.V product, and p is scaled by 2^8
 // (the row sum likewise, so it cancels) to keep lo of small p above fp16's smallest step.  Against 64
 // bits the output is as far off as with fp32 products: its own rounding to fp16 is what remains.
-template <int MB>
-__global__ __launch_bounds__(WG, 2) void causal_attention_kernel(const half_t* __restrict__ q, const half_t* __restrict__ k,
-                                                                 const half_t* __restrict__ v, half_t* __restrict__ out,
-                                                                 int n, int H, int n_bh, int n_blocks, float scale_log2) {
-    __shared__ __attribute__((aligned(16))) CausalLds sm;
+// The maximum a row's scores are taken relative to moves only when it would grow by more than 2^7 (p stays
+// below 2^15, inside fp16): the accumulators are rescaled a few times a row instead of at most tiles.
+template <int TILE>
+__global__ __launch_bounds__(WG, TILE == 32 ? 4 : 2) void causal_attention_kernel(
+    const half_t* __restrict__ q, const half_t* __restrict__ k, const half_t* __restrict__ v, half_t* __restrict__ out,
+    int n, int H, int n_bh, int n_blocks, float scale_log2) {
+    constexpr int TB = TILE / 16;                              // 16-key blocks of a tile
+    constexpr int TP = TILE / 32;                              // pairs of them
+    constexpr int RPW = TILE / NW;                             // rows of a tile that a wave brings
+    __shared__ __attribute__((aligned(16))) CausalLds<TILE> sm;
     // Query blocks in descending order (the last ones attend most).  Workgroup b runs on XCD b % 8:
     // with a multiple of 8 heads every head stays on one XCD, whose L2 then holds its K and V.
     // Every second 256 workgroups (one per compute unit) are taken in reverse, in steps of 8 so that the
@@ -87,154 +116,120 @@ __global__ __launch_bounds__(WG, 2) void causal_attention_kernel(const half_t* _
     const int tid = threadIdx.x;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l = tid & 63, g = l >> 4, i = l & 15;
-    const int q0 = block * 64 * MB;                            // first row of the workgroup
-    const int row0 = q0 + 16 * MB * w;                         // first row of the wave
+    const int q0 = block * ROWS;                               // first row of the workgroup
+    const int row0 = q0 + 16 * w;                              // first row of the wave
+    const int row = row0 + i;                                  // the lane's row
 
-    h8 qreg[MB][4];
+    h8 qreg[4];
 #pragma unroll
-    for (int mb = 0; mb < MB; mb++) {
-        const int row = row0 + 16 * mb + i;
-#pragma unroll
-        for (int ks = 0; ks < 4; ks++) {
-            qreg[mb][ks] = (row < n) ? *reinterpret_cast<const h8*>(q + base + size_t(row) * stride + 32 * ks + 8 * g)
-                                     : h8{ 0, 0, 0, 0, 0, 0, 0, 0 };
-        }
+    for (int ks = 0; ks < 4; ks++) {
+        qreg[ks] = (row < n) ? *reinterpret_cast<const h8*>(q + base + size_t(row) * stride + 32 * ks + 8 * g)
+                             : h8{ 0, 0, 0, 0, 0, 0, 0, 0 };
     }
-    float m_run[MB], l_lane[MB];
-    f4 oacc[MB][8];
+    float m_run = NEG_INF, l_lane = 0.f;
+    f4 oacc[8];
 #pragma unroll
-    for (int mb = 0; mb < MB; mb++) {
-        m_run[mb] = NEG_INF;
-        l_lane[mb] = 0.f;
-#pragma unroll
-        for (int db = 0; db < 8; db++) oacc[mb][db] = f4{ 0.f, 0.f, 0.f, 0.f };
-    }
+    for (int db = 0; db < 8; db++) oacc[db] = f4{ 0.f, 0.f, 0.f, 0.f };
 
-    // Wave w brings rows 16w .. 16w+15 of a tile, four per load: lane l writes piece l of those 1024 B,
-    // i.e. place l & 15 of row l >> 4, and therefore reads piece (l & 15) ^ (row & 15).  Rows past the last
+    // Wave w brings rows RPW * w and on of a tile, four per load: lane l writes piece l of those 1024 B,
+    // i.e. place l & 15 of row l >> 4, and therefore reads piece (l & 15) ^ swizzle(row).  Rows past the last
     // token repeat it (valid memory; their scores are masked for every row).
+    unsigned whole[RPW / 4];                                   // bytes from the tile's first row
+#pragma unroll
+    for (int r = 0; r < RPW / 4; r++) {
+        const int kr = RPW * w + 4 * r + g;
+        whole[r] = (unsigned(kr) * unsigned(stride) + 8 * (i ^ swizzle(kr))) * 2;
+    }
     auto fetch_tile = [&](int t, int buf) {
-        const half_t* __restrict__ kg = k + base + size_t(TILE * t) * stride;   // uniform; the lane's part is 32 bits
-        const half_t* __restrict__ vg = v + base + size_t(TILE * t) * stride;
+        const char* __restrict__ kg = reinterpret_cast<const char*>(k + base + size_t(TILE * t) * stride);
+        const char* __restrict__ vg = reinterpret_cast<const char*>(v + base + size_t(TILE * t) * stride);
         const int left = n - 1 - TILE * t;
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int row = 16 * w + 4 * r + g;
-            const unsigned off = unsigned(row < left ? row : left) * unsigned(stride) + 8 * (i ^ (row & 15));
-            load_to_lds16(kg + off, &sm.k[buf][(16 * w + 4 * r) * D]);
-            load_to_lds16(vg + off, &sm.v[buf][(16 * w + 4 * r) * D]);
+        for (int r = 0; r < RPW / 4; r++) {
+            unsigned off = whole[r];
+            const int kr = RPW * w + 4 * r + g;
+            if (left < TILE - 1 && kr > left) off -= unsigned(kr - left) * unsigned(stride) * 2;
+            load_to_lds16(kg + off, &sm.k[buf][(RPW * w + 4 * r) * D]);
+            load_to_lds16(vg + off, &sm.v[buf][(RPW * w + 4 * r) * D]);
         }
     };
 
-    const int last = (q0 + 64 * MB < n ? q0 + 64 * MB : n) - 1;  // last query row of the workgroup
+    const int last = (q0 + ROWS < n ? q0 + ROWS : n) - 1;      // last query row of the workgroup
     const int n_tiles = last / TILE + 1;
 
     auto tile_body = [&](int t, const half_t* __restrict__ kt, const half_t* __restrict__ vt, auto masked_tag) {
         constexpr bool MASKED = decltype(masked_tag)::value;   // some key of the tile lies after some row of the wave
-        f4 sc[MB][4];
+        // The places of a row's pieces differ in a few bits of the address: one base a lane, the others by
+        // exclusive or, formed where they are used (hoisted out of the loop they cost twelve registers).
+        int kbase = place(i, g), vbase = place(4 * g + (i >> 2), (i >> 1) & 1) + 4 * (i & 1);
+        asm volatile("" : "+v"(kbase), "+v"(vbase));
+        f4 sc[TB];
 #pragma unroll
-        for (int tb = 0; tb < 4; tb++) {
+        for (int tb = 0; tb < TB; tb++) {
             h8 kop[4];
 #pragma unroll
-            for (int ks = 0; ks < 4; ks++) {
-                kop[ks] = *reinterpret_cast<const h8*>(&kt[place(16 * tb + i, 4 * ks + g)]);
-            }
+            for (int ks = 0; ks < 4; ks++) kop[ks] = *reinterpret_cast<const h8*>(&kt[16 * D * tb + (kbase ^ (32 * ks))]);
+            f4 acc = f4{ 0.f, 0.f, 0.f, 0.f };
 #pragma unroll
-            for (int mb = 0; mb < MB; mb++) {
-                f4 acc = f4{ 0.f, 0.f, 0.f, 0.f };
-#pragma unroll
-                for (int ks = 0; ks < 4; ks++) {
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(kop[ks], qreg[mb][ks], acc, 0, 0, 0);
-                }
-                sc[mb][tb] = acc;
-            }
+            for (int ks = 0; ks < 4; ks++) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(kop[ks], qreg[ks], acc, 0, 0, 0);
+            sc[tb] = acc;
             __builtin_amdgcn_sched_barrier(0);
         }
         if constexpr (MASKED) {  // selects, not branches, between a matrix op and its first reader
 #pragma unroll
-            for (int mb = 0; mb < MB; mb++) {
-                const int row = row0 + 16 * mb + i;
+            for (int tb = 0; tb < TB; tb++) {
 #pragma unroll
-                for (int tb = 0; tb < 4; tb++) {
-#pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        if (TILE * t + 16 * tb + 4 * g + r > row) sc[mb][tb][r] = NEG_INF;
-                    }
+                for (int r = 0; r < 4; r++) {
+                    if (TILE * t + 16 * tb + 4 * g + r > row) sc[tb][r] = NEG_INF;
                 }
             }
         }
         // online softmax: the scale is positive and rides in the exponent's multiply-add
-        float m_new[MB];
-        bool grew = false;
+        float mx = sc[0][0];
 #pragma unroll
-        for (int mb = 0; mb < MB; mb++) {
-            float mx = fmaxf(fmaxf(sc[mb][0][0], sc[mb][0][1]), fmaxf(sc[mb][0][2], sc[mb][0][3]));
+        for (int e = 1; e < 4 * TB - 1; e += 2) mx = max2(max2(mx, sc[e >> 2][e & 3]), sc[(e + 1) >> 2][(e + 1) & 3]);
+        mx = max_over_groups(max2(mx, sc[TB - 1][3]));
+        const float m_new = max2(m_run, mx * scale_log2);
+        if (__builtin_amdgcn_ballot_w64(m_new > m_run + kSlack) != 0) {
+            const float alpha = (m_run == NEG_INF) ? 0.f : fast_exp2(m_run - m_new);
+            m_run = m_new;
+            l_lane *= alpha;
 #pragma unroll
-            for (int tb = 1; tb < 4; tb++) {
-                mx = fmaxf(mx, fmaxf(fmaxf(sc[mb][tb][0], sc[mb][tb][1]), fmaxf(sc[mb][tb][2], sc[mb][tb][3])));
-            }
-            mx = max_over_groups(mx);
-            m_new[mb] = fmaxf(m_run[mb], mx * scale_log2);
-            grew |= m_new[mb] > m_run[mb];
+            for (int db = 0; db < 8; db++) oacc[db] *= alpha;
         }
-        if (__builtin_amdgcn_ballot_w64(grew) != 0) {
+        // a row whose scores are all -inf so far has no maximum to subtract
+        const float nm = kShift - (m_run == NEG_INF ? 0.f : m_run);
 #pragma unroll
-            for (int mb = 0; mb < MB; mb++) {
-                const float alpha = (m_run[mb] == NEG_INF) ? 0.f : fast_exp2(m_run[mb] - m_new[mb]);
-                m_run[mb] = m_new[mb];
-                l_lane[mb] *= alpha;
+        for (int tp = 0; tp < TP; tp++) {
+            h8 hi, lo;
+            float sum = 0.f;
 #pragma unroll
-                for (int db = 0; db < 8; db++) oacc[mb][db] *= alpha;
+            for (int e = 0; e < 8; e += 2) {
+                const float p0 = fast_exp2(__builtin_fmaf(sc[2 * tp + (e >> 2)][e & 3], scale_log2, nm));
+                const float p1 = fast_exp2(__builtin_fmaf(sc[2 * tp + (e >> 2)][(e & 3) + 1], scale_log2, nm));
+                const h2 a = __builtin_bit_cast(h2, __builtin_amdgcn_cvt_pkrtz(p0, p1));
+                const h2 c = __builtin_bit_cast(h2, __builtin_amdgcn_cvt_pkrtz(rest_of<false>(p0, a), rest_of<true>(p1, a)));
+                hi[e] = a[0];
+                hi[e + 1] = a[1];
+                lo[e] = c[0];
+                lo[e + 1] = c[1];
+                sum += p0 + p1;
             }
-        }
-        h8 hi[MB][2], lo[MB][2];
-        auto probabilities = [&](int tp) {
+            l_lane += sum;
 #pragma unroll
-            for (int mb = 0; mb < MB; mb++) {
-                // a row whose scores are all -inf so far has no maximum to subtract
-                const float nm = kShift - (m_run[mb] == NEG_INF ? 0.f : m_run[mb]);
-                float sum = 0.f;
+            for (int half = 0; half < 2; half++) {             // V operands of four dim blocks at a time
+                __builtin_amdgcn_sched_barrier(0);
+                h8 a[4];
 #pragma unroll
-                for (int e = 0; e < 8; e += 2) {
-                    const float p0 = fast_exp2(__builtin_fmaf(sc[mb][2 * tp + (e >> 2)][e & 3], scale_log2, nm));
-                    const float p1 = fast_exp2(__builtin_fmaf(sc[mb][2 * tp + (e >> 2)][(e & 3) + 1], scale_log2, nm));
-                    const h2 a = __builtin_bit_cast(h2, __builtin_amdgcn_cvt_pkrtz(p0, p1));
-                    const h2 c = __builtin_bit_cast(h2, __builtin_amdgcn_cvt_pkrtz(p0 - float(a[0]), p1 - float(a[1])));
-                    hi[mb][tp][e] = a[0];
-                    hi[mb][tp][e + 1] = a[1];
-                    lo[mb][tp][e] = c[0];
-                    lo[mb][tp][e + 1] = c[1];
-                    sum += p0 + p1;
+                for (int d = 0; d < 4; d++) {                  // rows key and key + 16 are swizzled alike
+                    const half_t* p0 = &vt[32 * D * tp + (vbase ^ (16 * (4 * half + d)))];
+                    const h4 x = lds_read_tr(p0), y = lds_read_tr(p0 + 16 * D);
+                    a[d] = h8{ x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3] };
                 }
-                l_lane[mb] += sum;
-            }
-        };
-        probabilities(0);
 #pragma unroll
-        for (int tp = 0; tp < 2; tp++) {
-            __builtin_amdgcn_sched_barrier(0);
-            h8 a[8];
+                for (int d = 0; d < 4; d++) oacc[4 * half + d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[d], hi, oacc[4 * half + d], 0, 0, 0);
 #pragma unroll
-            for (int db = 0; db < 8; db++) {
-                const int key = 32 * tp + 4 * g + (i >> 2);     // rows key and key + 16 are swizzled alike
-                const half_t* p0 = &vt[place(key, 2 * db + ((i >> 1) & 1)) + 4 * (i & 1)];
-                const h4 x = lds_read_tr(p0), y = lds_read_tr(p0 + 16 * D);
-                a[db] = h8{ x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3] };
-            }
-            if (tp == 0) probabilities(1);
-#pragma unroll
-            for (int db = 0; db < 8; db++) {
-#pragma unroll
-                for (int mb = 0; mb < MB; mb++) {
-                    oacc[mb][db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[db], hi[mb][tp], oacc[mb][db], 0, 0, 0);
-                }
-            }
-#pragma unroll
-            for (int db = 0; db < 8; db++) {
-#pragma unroll
-                for (int mb = 0; mb < MB; mb++) {
-                    oacc[mb][db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[db], lo[mb][tp], oacc[mb][db], 0, 0, 0);
-                }
+                for (int d = 0; d < 4; d++) oacc[4 * half + d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[d], lo, oacc[4 * half + d], 0, 0, 0);
             }
         }
     };
@@ -252,28 +247,23 @@ __global__ __launch_bounds__(WG, 2) void causal_attention_kernel(const half_t* _
         arrive(t);
         tile_body(t, sm.k[t & 1], sm.v[t & 1], std::false_type{});
     }
-    // The diagonal, MB tiles: waves whose rows all lie before a tile skip it.  Waves begin at multiples of
-    // 16 * MB, which divides the tile: a wave that takes part has the tile's first key before or at every
-    // one of its rows.
+    // The diagonal: waves whose rows all lie before a tile skip it.  Waves begin at multiples of 16, which
+    // divides the tile: a wave that takes part has the tile's first key before or at every one of its rows.
     for (int t = n_whole; t < n_tiles; t++) {
         arrive(t);
         if (TILE * t <= row0) tile_body(t, sm.k[t & 1], sm.v[t & 1], std::true_type{});
     }
 
+    float sum = l_lane;
+    sum += __shfl_xor(sum, 16, 64);
+    sum += __shfl_xor(sum, 32, 64);
+    const float r = 1.f / sum;
+    if (row < n) {
+        half_t* dst = out + base + size_t(row) * stride + 4 * g;
 #pragma unroll
-    for (int mb = 0; mb < MB; mb++) {
-        float sum = l_lane[mb];
-        sum += __shfl_xor(sum, 16, 64);
-        sum += __shfl_xor(sum, 32, 64);
-        const int row = row0 + 16 * mb + i;
-        const float r = 1.f / sum;
-        if (row < n) {
-            half_t* dst = out + base + size_t(row) * stride + 4 * g;
-#pragma unroll
-            for (int db = 0; db < 8; db++) {
-                const f4 o = oacc[mb][db];
-                *reinterpret_cast<h4*>(dst + 16 * db) = h4{ half_t(o[0] * r), half_t(o[1] * r), half_t(o[2] * r), half_t(o[3] * r) };
-            }
+        for (int db = 0; db < 8; db++) {
+            const f4 o = oacc[db];
+            *reinterpret_cast<h4*>(dst + 16 * db) = h4{ half_t(o[0] * r), half_t(o[1] * r), half_t(o[2] * r), half_t(o[3] * r) };
         }
     }
 }
@@ -284,22 +274,21 @@ int launch_causal_attention(const void* q, const void* k, const void* v, void* o
                             float scale_log2, hipStream_t st) {
     if (batch <= 0 || n_tokens <= 0 || n_heads <= 0) return 0;
     const int64_t n_bh = int64_t(batch) * n_heads;
-    // 128 query rows per workgroup reuse a K/V tile twice as often; where that leaves compute units without a
-    // workgroup, 64
-    const bool wide = n_bh * ((n_tokens + 127) / 128) >= 256;
-    const int rows = wide ? 128 : 64;
-    const int64_t blocks = (n_tokens + rows - 1) / rows;
-    if (n_bh * blocks > 0x7fffff00 || n_tokens > 0x7fffff00 - 128) return -1;
+    const int64_t blocks = (n_tokens + ROWS - 1) / ROWS;
+    if (n_bh * blocks > 0x7fffff00 || n_tokens > 0x7fffff00 - ROWS) return -1;
     const dim3 grid(static_cast<unsigned>(n_bh * blocks)), block(WG);
     const half_t* qh = static_cast<const half_t*>(q);
     const half_t* kh = static_cast<const half_t*>(k);
     const half_t* vh = static_cast<const half_t*>(v);
     half_t* oh = static_cast<half_t*>(out);
-    if (wide) {
-        hipLaunchKernelGGL(causal_attention_kernel<2>, grid, block, 0, st, qh, kh, vh, oh, n_tokens, n_heads, int(n_bh),
+    // Tiles of 32 keys let four workgroups share a compute unit; with fewer workgroups than two a unit there is
+    // nobody to share with, and half as many barriers are worth more (1000 tokens, 8 heads: 23.7 us with 64 keys
+    // a tile, 26.1 with 32; 400 x 32 heads 12.8, 13.3; 1000 x 32 heads, 512 workgroups: 29.9 with 32 keys).
+    if (n_bh * blocks >= 400) {
+        hipLaunchKernelGGL(causal_attention_kernel<32>, grid, block, 0, st, qh, kh, vh, oh, n_tokens, n_heads, int(n_bh),
                            int(blocks), scale_log2);
     } else {
-        hipLaunchKernelGGL(causal_attention_kernel<1>, grid, block, 0, st, qh, kh, vh, oh, n_tokens, n_heads, int(n_bh),
+        hipLaunchKernelGGL(causal_attention_kernel<64>, grid, block, 0, st, qh, kh, vh, oh, n_tokens, n_heads, int(n_bh),
                            int(blocks), scale_log2);
     }
     const hipError_t e = hipGetLastError();

@@ -252,7 +252,35 @@ void build_plan(const ChunkRow* rows, int n_rows, int n_seqs, int chunk_size,
         }
         return wgs;
     };
-    int base_tiles = std::max(static_cast<int>(0.3 * step_us), 4);
+    // Four tiles are the least (one block of each tile a wave and the fixed cost of a workgroup and of its
+    // partial rows), unless the whole launch is so small that its workgroups have compute units to themselves: a
+    // short step is as long as its longest chain, and with two tiles a segment that chain is half as long
+    // (one shared prefix, 64 private tokens, us a forward with 4 -> 2 tiles: 4 sequences x 12 heads, 256 shared
+    // tokens 8.65 -> 7.65, 512 tokens 8.81 -> 7.81, 1024 tokens 9.37 -> 8.52; 16 x 32 heads, 512 tokens
+    // 11.7 -> 10.95).  Not for more than half a workgroup per compute unit (2 x 32 heads, 1024 tokens
+    // 10.4 -> 10.9), not where the streaming fills the device's slots anyway (64 x 12 heads, 512 tokens 13.4 ->
+    // 14.5), and not for more than eight segments on a path (12 heads, 2048 tokens 9.6 -> 10.1: their rows are
+    // merged one by one); for more than four only while every workgroup finds a place at once, on a compute unit of
+    // its own where none covers more than 16 sequences (8 x 12 heads, 1024 tokens 9.84 -> 9.36, but 16 x 12 heads
+    // 11.55 -> 11.92), in one of two otherwise (32 x 12 heads 15.5 -> 14.3, but 64 x 8 heads 16.2 -> 16.7).  One
+    // tile is too little for any of it (4 x 12 heads, 1024 tokens 9.7).
+    bool tiny = int64_t(n_seqs) * std::max(params.n_heads, 1) <= int64_t(2) * params.n_cus && 2 * shared_wgs_with(2) <= params.n_cus;
+    if (tiny) {
+        std::vector<int> path_segs(n_seqs, 0);
+        int longest = 0, widest = 0;
+        for (const Run& run : runs) {
+            const ChunkRow& r0 = rows[run.first_row];
+            const int seg = std::max(2 * 64 / chunk_size, 1);
+            for (int s = r0.seq_begin; s < r0.seq_end; s++) {
+                path_segs[s] += ceil_div(run.count, seg);
+                longest = std::max(longest, path_segs[s]);
+            }
+            widest = std::max(widest, r0.seq_end - r0.seq_begin);
+        }
+        const int64_t wgs = shared_wgs_with(2) + int64_t(n_seqs) * std::max(params.n_heads, 1);
+        tiny = longest <= 4 || (longest <= 8 && wgs <= int64_t(widest <= 16 ? 1 : 2) * params.n_cus);
+    }
+    int base_tiles = std::max(static_cast<int>(0.3 * step_us), tiny ? 2 : 4);
     while (base_tiles < 32 && shared_wgs_with(base_tiles) > int64_t(2) * params.n_cus) base_tiles++;
     if (params.keep) base_tiles = params.keep->base_tiles;
     p.hints.base_tiles = base_tiles;

@@ -405,3 +405,18 @@ def test_replanning_policy_keeps_patched_tables_near_fresh_ones(cfg, steps):
     assert worst <= 0.10, worst
     if cfg == 0:
         assert worst_never > 0.3
+
+
+@pytest.mark.parametrize("n_seqs,heads,root,want", [
+    (4, 12, 256, 2), (4, 12, 64, 1), (2, 8, 1024, 8), (16, 32, 512, 4), (17, 32, 512, 2), (2, 32, 1024, 4),
+    (16, 12, 1024, 4), (32, 12, 1024, 8), (64, 8, 1024, 4), (64, 8, 512, 4), (2, 8, 2048, 8), (2, 8, 1088, 4)])
+def test_tiny_launches_cut_shared_runs_into_two_tiles(n_seqs, heads, root, want):
+    """Segments of 128 shared tokens while the launch has compute units to spare, of 256 otherwise; each segment
+    is attended once for every covered sequence either way."""
+    rows = [(i, 64, 0, n_seqs) for i in range(root // 64)] + [(100 + s, 30, s, s + 1) for s in range(n_seqs)]
+    plan = capi.build_tables(np.array(rows, np.int32), n_seqs, 64, n_heads=heads, n_cus=256)["plan"]
+    items = plan["shared_items"]
+    assert len(set(items[:, 4])) == want                       # ordinals of partial rows = segments
+    for s in range(n_seqs):
+        covering = items[(items[:, 0] <= s) & (s < items[:, 0] + items[:, 1])]
+        assert sorted(covering[:, 4]) == list(range(want)) and covering[:, 3].sum() == root // 64

@@ -285,8 +285,10 @@ constexpr int OPITCH = D + 4;  // floats per row of the cross-wave accumulation 
 // MBT: 16-row blocks per shared item (2: items of up to 32 sequences, 1: up to 16)
 template <int MBT>
 struct SharedPathLds {
-    half_t v[NW][16 * VPITCH];
-    float o[16 * MBT * OPITCH];
+    union {
+        half_t v[NW][16 * VPITCH];
+        float o[NW][16 * MBT * OPITCH];   // every wave's sums, when all are done with their V blocks
+    };
     float m[NW][16 * MBT];
     float l[NW][16 * MBT];
     int last[16 * MBT];
@@ -852,26 +854,26 @@ __device__ __forceinline__ void shared_path(const DecodeArgs& A, const WorkItem*
 #pragma unroll
         for (int db = 0; db < 8; db++) oacc[mb][db] *= f;
     }
-    for (int k = 0; k < NW; k++) {
-        if (w == k) {
+    // Every wave leaves its sums in a buffer of its own, and the threads that write the partial rows add
+    // the four up: one barrier (adding in turn into one buffer took four; 4 sequences x 12 heads, 512 shared
+    // tokens 7.79 -> 7.15 us a forward).
 #pragma unroll
-            for (int mb = 0; mb < MB; mb++) {
+    for (int mb = 0; mb < MB; mb++) {
 #pragma unroll
-                for (int db = 0; db < 8; db++) {
-                    // lane owns dims 16*db + 4*g .. +3 of sequence row mb*16 + i
-                    f4* dst = reinterpret_cast<f4*>(&sm.o[(mb * 16 + i) * OPITCH + 16 * db + 4 * g]);
-                    *dst = (k == 0) ? oacc[mb][db] : (*dst + oacc[mb][db]);
-                }
-            }
+        for (int db = 0; db < 8; db++) {
+            // lane owns dims 16*db + 4*g .. +3 of sequence row mb*16 + i
+            *reinterpret_cast<f4*>(&sm.o[w][(mb * 16 + i) * OPITCH + 16 * db + 4 * g]) = oacc[mb][db];
         }
-        __syncthreads();
     }
+    __syncthreads();
 
     // ---- write the partial rows ------------------------------------------------------------
     for (int idx = tid; idx < it.n_rows * (D / 4); idx += WG) {
         const int row = idx / (D / 4), c4 = idx % (D / 4);
         float* dst = A.part + (size_t(sm.row[row]) * H + h) * PART_STRIDE + 4 + 4 * c4;
-        const f4 v = *reinterpret_cast<const f4*>(&sm.o[row * OPITCH + 4 * c4]);
+        f4 v = *reinterpret_cast<const f4*>(&sm.o[0][row * OPITCH + 4 * c4]);
+#pragma unroll
+        for (int k = 1; k < NW; k++) v += *reinterpret_cast<const f4*>(&sm.o[k][row * OPITCH + 4 * c4]);
         part_store2(dst, v[0], v[1], coh);
         part_store2(dst + 2, v[2], v[3], coh);
     }

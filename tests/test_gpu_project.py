@@ -157,3 +157,15 @@ def test_what_the_projection_leaves_to_torch():
         assert not capi.projection_takes(x, lin)
         handle.remove()
         assert capi.projection_takes(x, lin)
+
+
+def test_model_keeps_what_a_hook_on_an_output_projection_holds():
+    """The tensor a hook keeps is the projection's output still, not the sum or norm that followed it."""
+    from chunk_attn.models.sequence import Sequence
+    from chunk_attn.models.tiny_lm import AttentionOnlyLM
+    model = AttentionOnlyLM(300, 256, 2, 2, chunk_size=32, memory_mb=16, seed=5)
+    kept, copies = [], []
+    model.layers[0].o_proj.register_forward_hook(lambda m, a, out: (kept.append(out), copies.append(out.clone())) and None)
+    with torch.inference_mode():
+        model.logits([Sequence(list(range(40)))], model.create_kv_caches(), True)
+    assert len(kept) == 1 and (kept[0] == copies[0]).all()

@@ -400,11 +400,19 @@ def fused_add_rms_norm(input, residual, weight, epsilon: float) -> None:
             float(epsilon), n, hidden)
 
 
+def plain_call() -> bool:
+    """Nothing stands between a call and its kernel: no tracing, no mode that intercepts tensor operations, no
+    forward-mode level whose tangents a kernel would drop."""
+    import torch
+    return not (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() or
+                torch._C._len_torch_function_stack() or torch.autograd.forward_ad._current_level >= 0)
+
+
 def causal_attention_takes(*tensors) -> bool:
     """Whether causal_attention computes on these: fp16 GPU tensors [batch, n, heads, 128] of one shape,
-    contiguous and 16-byte aligned, no gradient asked for (the kernel has no backward)."""
+    contiguous and 16-byte aligned, no derivative asked for (the kernel has none)."""
     import torch
-    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
+    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors) or not plain_call():
         return False
     shape, device = tensors[0].shape, tensors[0].device
     return len(shape) == 4 and shape[3] == 128 and device.type == "cuda" and all(
@@ -445,9 +453,8 @@ def projection_takes(x, *linears) -> bool:
         return False
     grad = torch.is_grad_enabled()
     # whatever else may stand between a module and its product: hooks, subclasses, patched forwards, modes
-    if grad and x.requires_grad or torch.is_autocast_enabled() or torch.compiler.is_compiling() or torch.jit.is_tracing() or \
-            torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack() or \
-            torch.nn.modules.module._has_any_global_hook() or torch.autograd.forward_ad._current_level >= 0:
+    if grad and x.requires_grad or torch.is_autocast_enabled() or not plain_call() or \
+            torch.nn.modules.module._has_any_global_hook():
         return False
     device = x.device
     for m in linears:

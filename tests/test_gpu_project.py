@@ -169,3 +169,12 @@ def test_model_keeps_what_a_hook_on_an_output_projection_holds():
     with torch.inference_mode():
         model.logits([Sequence(list(range(40)))], model.create_kv_caches(), True)
     assert len(kept) == 1 and (kept[0] == copies[0]).all()
+
+
+def test_causal_attention_leaves_forward_mode_to_torch():
+    from torch.autograd import forward_ad
+    q = torch.zeros(1, 8, 2, 128, dtype=torch.float16, device="cuda")
+    assert capi.causal_attention_takes(q, q, q)
+    with forward_ad.dual_level():
+        assert not capi.causal_attention_takes(q, q, q)
+    assert capi.causal_attention_takes(q, q, q)

@@ -70,8 +70,10 @@ class AttentionOnlyLM(nn.Module):
             input_ids = [[s[-1]] for s in seqs]
             position_ids = [[len(s) - 1] for s in seqs]
         dev = self.embed_tokens.weight.device
-        # one upload, from pinned memory: the host does not wait for what the GPU still has to do
-        ids, pos = torch.tensor([input_ids, position_ids], dtype=torch.int64, pin_memory=dev.type == "cuda").to(dev, non_blocking=True)
+        # one upload, from pinned memory: the host does not wait for what the GPU still has to do (the device is
+        # named: only host memory can be pinned, whatever the default device is)
+        ids, pos = torch.tensor([input_ids, position_ids], dtype=torch.int64, device="cpu",
+                                pin_memory=dev.type == "cuda").to(dev, non_blocking=True)
         hidden = self.embed_tokens(ids)
         token_lists = [s.tokens for s in seqs]
         joined = self._adds_in_norms()

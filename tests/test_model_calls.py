@@ -1,0 +1,72 @@
+"""The small model's and the layer's Python on the CPU: the native operators are emulated through raw addresses,
+as the kernels write (past autograd, modes and hooks), and a cache that only counts stands in for the real one."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from chunk_attn import capi
+from chunk_attn.models.sequence import Sequence
+from chunk_attn.models.tiny_lm import AttentionOnlyLM
+
+
+def raw(t):
+    """The tensor's memory, with nothing of torch in between."""
+    return np.ctypeslib.as_array((ctypes.c_uint16 * t.numel()).from_address(t.data_ptr())).view(np.float16).reshape(t.shape)
+
+
+def normed(x, weight, eps):
+    x = x.astype(np.float32)
+    return (x / np.sqrt((x * x).mean(-1, keepdims=True) + eps)).astype(np.float16) * weight
+
+
+class CountingCache:
+    def __init__(self):
+        self.n = 0
+
+    def add_seq(self, tokens, k, v):
+        self.n += 1
+        return self.n - 1
+
+    def reserve(self):
+        return 0
+
+    def refresh_kernel_context(self, force=False):
+        pass
+
+
+@pytest.fixture
+def fused(monkeypatch):
+    """Emulated operators; the list has one entry a fused add and norm."""
+    calls = []
+
+    def rms_norm(out, x, weight, eps):
+        raw(out)[...] = normed(raw(x), raw(weight), eps)
+
+    def fused_add_rms_norm(x, residual, weight, eps):
+        calls.append(x.shape)
+        raw(residual)[...] = raw(residual) + raw(x)
+        raw(x)[...] = normed(raw(residual), raw(weight), eps)
+
+    monkeypatch.setattr(capi, "rms_norm", rms_norm)
+    monkeypatch.setattr(capi, "fused_add_rms_norm", fused_add_rms_norm)
+    monkeypatch.setattr(capi, "rotary_embedding", lambda *a: None)
+    return calls
+
+
+def model(layers=2):
+    return AttentionOnlyLM(50, 32, 2, layers, max_position_embeddings=64, seed=3, device="cpu")
+
+
+def logits(m):
+    return m.logits([Sequence([3, 1, 4, 1, 5])], [CountingCache() for _ in m.layers], True)
+
+
+def test_default_device_places_nothing_of_a_pass(fused):
+    m = model()
+    with torch.no_grad():
+        want = logits(m)
+        with torch.device("meta"):
+            got = logits(m)
+    assert torch.equal(got, want)

@@ -30,6 +30,12 @@ class RMSNorm(nn.Module):
         return out
 
 
+def _pins(device: torch.device) -> bool:
+    """Whether ids for `device` go through pinned memory.  Not under stream capture: a replay would read whatever
+    the staging buffer holds by then; the copy from ordinary memory is refused there."""
+    return device.type == "cuda" and not torch.cuda.is_current_stream_capturing()
+
+
 class AttentionOnlyLM(nn.Module):
     def __init__(self, vocab_size: int, hidden_size: int, num_heads: int, num_layers: int,
                  max_position_embeddings: int = 4096, chunk_size: int = 64, memory_mb: int = 256,
@@ -72,8 +78,9 @@ class AttentionOnlyLM(nn.Module):
         dev = self.embed_tokens.weight.device
         # one upload, from pinned memory: the host does not wait for what the GPU still has to do (the device is
         # named: only host memory can be pinned, whatever the default device is)
+        pinned = _pins(dev)
         ids, pos = torch.tensor([input_ids, position_ids], dtype=torch.int64, device="cpu",
-                                pin_memory=dev.type == "cuda").to(dev, non_blocking=True)
+                                pin_memory=pinned).to(dev, non_blocking=pinned)
         hidden = self.embed_tokens(ids)
         token_lists = [s.tokens for s in seqs]
         joined = self._adds_in_norms()

@@ -8,6 +8,7 @@ import torch
 
 from chunk_attn import capi
 from chunk_attn.models.sequence import Sequence
+from chunk_attn.models import tiny_lm
 from chunk_attn.models.tiny_lm import AttentionOnlyLM
 
 
@@ -70,3 +71,11 @@ def test_default_device_places_nothing_of_a_pass(fused):
         with torch.device("meta"):
             got = logits(m)
     assert torch.equal(got, want)
+
+
+def test_no_pinned_upload_is_captured(monkeypatch):
+    """A captured copy would read its staging buffer again on every replay, long after it was given back."""
+    for capturing in (False, True):
+        monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing)
+        assert tiny_lm._pins(torch.device("cuda:0")) is not capturing
+        assert not tiny_lm._pins(torch.device("cpu"))

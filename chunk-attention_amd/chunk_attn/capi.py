@@ -401,11 +401,15 @@ def fused_add_rms_norm(input, residual, weight, epsilon: float) -> None:
 
 
 def plain_call() -> bool:
-    """Nothing stands between a call and its kernel: no tracing, no mode that intercepts tensor operations, no
-    forward-mode level whose tangents a kernel would drop."""
+    """Nothing stands between a call and its kernel: no tracing, no mode that intercepts tensor operations (one that
+    only places new tensors, as torch.set_default_device leaves on the stack, does not), no forward-mode level
+    whose tangents a kernel would drop."""
     import torch
-    return not (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() or
-                torch._C._len_torch_function_stack() or torch.autograd.forward_ad._current_level >= 0)
+    if torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() or \
+            torch.autograd.forward_ad._current_level >= 0:
+        return False
+    return all(type(torch._C._get_function_stack_at(i)) is torch.utils._device.DeviceContext
+               for i in range(torch._C._len_torch_function_stack()))
 
 
 def causal_attention_takes(*tensors) -> bool:

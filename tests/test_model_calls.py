@@ -79,3 +79,22 @@ def test_no_pinned_upload_is_captured(monkeypatch):
         monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing)
         assert tiny_lm._pins(torch.device("cuda:0")) is not capturing
         assert not tiny_lm._pins(torch.device("cpu"))
+
+
+def test_what_stands_between_a_call_and_its_kernel():
+    """A default device does not; a mode that sees the operations does, alone and beside a default device."""
+    class Watching(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    assert capi.plain_call()
+    with torch.device("cpu"):
+        assert capi.plain_call()
+        with Watching():
+            seen = capi.plain_call()
+        assert not seen
+    with Watching(), torch.device("cpu"):
+        seen = capi.plain_call()
+    assert not seen
+    with torch.autograd.forward_ad.dual_level():
+        assert not capi.plain_call()

@@ -98,3 +98,34 @@ def test_what_stands_between_a_call_and_its_kernel():
     assert not seen
     with torch.autograd.forward_ad.dual_level():
         assert not capi.plain_call()
+
+
+def test_tensors_that_a_mode_saw_are_not_overwritten(fused):
+    class Keeping(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            out = func(*args, **(kwargs or {}))
+            if func is torch.nn.functional.linear:
+                kept.append((out, out.clone()))
+            return out
+
+    m, kept = model(), []
+    with torch.no_grad():
+        want = logits(m)
+        assert len(fused) == 2
+        with Keeping():
+            got = logits(m)
+    assert len(kept) == 2 * 4 + 1 and all(torch.equal(a, b) for a, b in kept)
+    assert torch.allclose(got, want, rtol=2e-3, atol=2e-3)              # fp16 roundings of the residual
+
+
+def test_no_tangent_of_an_overwritten_tensor_reaches_the_logits(fused):
+    """The norms drop tangents (they are native calls): logits of a dual output projection have none."""
+    from torch.autograd import forward_ad
+    m = model()
+    with torch.no_grad(), forward_ad.dual_level():
+        w = m.layers[1].o_proj.weight
+        dual = forward_ad.make_dual(w.detach(), torch.ones_like(w))
+        del m.layers[1].o_proj.weight
+        m.layers[1].o_proj.weight = dual
+        assert forward_ad.unpack_dual(logits(m)).tangent is None
+    assert not fused

@@ -74,6 +74,8 @@ SIGNATURES = {
                                    ctypes.c_int64, ctypes.c_int, ctypes.c_void_p]),
     "ca_fused_add_rms_norm": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_float,
                                              ctypes.c_int64, ctypes.c_int, ctypes.c_void_p]),
+    "ca_add_rms_norm": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_float,
+                                       ctypes.c_int64, ctypes.c_int, ctypes.c_void_p]),
     "ca_causal_attention": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
                                            ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p]),
     "ca_linear": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_int,
@@ -397,6 +399,14 @@ def fused_add_rms_norm(input, residual, weight, epsilon: float) -> None:
     `chunk_attn.ops.fused_add_rms_norm` (python_exports_ops.cpp:17)."""
     n, hidden = _norm_args("fused_add_rms_norm", [input, residual], weight)
     _launch(input.device, load().ca_fused_add_rms_norm, input.data_ptr(), residual.data_ptr(), weight.data_ptr(),
+            float(epsilon), n, hidden)
+
+
+def add_rms_norm(input, residual, weight, epsilon: float) -> None:
+    """In place: residual += input in fp16; input = rms_norm(residual) * weight.  One launch for the two operations,
+    the same bits (fused_add_rms_norm takes its mean over the unrounded sums)."""
+    n, hidden = _norm_args("add_rms_norm", [input, residual], weight)
+    _launch(input.device, load().ca_add_rms_norm, input.data_ptr(), residual.data_ptr(), weight.data_ptr(),
             float(epsilon), n, hidden)
 
 

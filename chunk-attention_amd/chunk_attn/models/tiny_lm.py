@@ -94,9 +94,9 @@ class AttentionOnlyLM(nn.Module):
             norm = self.norm if final else self.input_norms[i + 1]
             if final:   # from here on the last positions alone
                 out, hidden = out[:, -1], hidden[:, -1]
-            if joined:  # hidden += out, out = norm(hidden): one launch over both
+            if joined:  # hidden += out, out = norm(hidden): one launch over both, the same bits
                 out, hidden = out.contiguous(), hidden.contiguous()
-                capi.fused_add_rms_norm(out, hidden, norm.weight, norm.eps)
+                capi.add_rms_norm(out, hidden, norm.weight, norm.eps)
                 normed = out
             else:
                 hidden = hidden + out

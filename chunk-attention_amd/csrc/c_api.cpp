@@ -761,18 +761,30 @@ int ca_rms_norm(void* out, const void* input, const void* weight, float epsilon,
     if (!out || !input || !weight) return fail(CA_ERR_INVALID, "null device pointer");
     const bool vec8 = hidden_size % 8 == 0 && aligned16(out) && aligned16(input) && aligned16(weight);
     return launch_rc(ca::launch_rms_norm(out, const_cast<void*>(input), nullptr, weight, epsilon, n_tokens,
-                                         hidden_size, vec8, static_cast<hipStream_t>(stream)), "rms_norm launch");
+                                         hidden_size, vec8, false, static_cast<hipStream_t>(stream)), "rms_norm launch");
 }
 
-int ca_fused_add_rms_norm(void* input, void* residual, const void* weight, float epsilon, int64_t n_tokens,
-                          int hidden_size, void* stream) {
+namespace {
+int add_and_norm(void* input, void* residual, const void* weight, float epsilon, int64_t n_tokens, int hidden_size,
+                 bool mean_of_rounded, void* stream) {
     if (n_tokens < 0 || hidden_size <= 0 || !(epsilon >= 0.f)) return fail(CA_ERR_INVALID, "bad argument");
     if (n_tokens == 0) return CA_OK;
     if (!input || !residual || !weight) return fail(CA_ERR_INVALID, "null device pointer");
     if (input == residual) return fail(CA_ERR_INVALID, "input and residual must be different buffers");
     const bool vec8 = hidden_size % 8 == 0 && aligned16(input) && aligned16(residual) && aligned16(weight);
     return launch_rc(ca::launch_rms_norm(nullptr, input, residual, weight, epsilon, n_tokens, hidden_size, vec8,
-                                         static_cast<hipStream_t>(stream)), "fused_add_rms_norm launch");
+                                         mean_of_rounded, static_cast<hipStream_t>(stream)), "fused_add_rms_norm launch");
+}
+}  // namespace
+
+int ca_fused_add_rms_norm(void* input, void* residual, const void* weight, float epsilon, int64_t n_tokens,
+                          int hidden_size, void* stream) {
+    return add_and_norm(input, residual, weight, epsilon, n_tokens, hidden_size, false, stream);
+}
+
+int ca_add_rms_norm(void* input, void* residual, const void* weight, float epsilon, int64_t n_tokens, int hidden_size,
+                    void* stream) {
+    return add_and_norm(input, residual, weight, epsilon, n_tokens, hidden_size, true, stream);
 }
 
 int ca_causal_attention(const void* q, const void* k, const void* v, void* out, int batch, int n_tokens,

@@ -116,7 +116,7 @@ int launch_rope_append(const LaunchArgs& a, const RotaryArgs& r, const void* k, 
 // input = norm(residual) * weight, `out` unused.  vec8: hidden % 8 == 0 and all pointers 16-byte
 // aligned.
 int launch_rms_norm(void* out, void* input, void* residual, const void* weight, float epsilon,
-                    int64_t n_tokens, int hidden, bool vec8, hipStream_t st);
+                    int64_t n_tokens, int hidden, bool vec8, bool mean_of_rounded, hipStream_t st);
 
 // Causal attention of whole prompts: q, k, v, out [batch, n_tokens, n_heads, 128] fp16, contiguous and
 // 16-byte aligned; out must not overlap the inputs.

@@ -6,6 +6,8 @@
 //   rms_norm            out = fp16(x * rsqrt(mean(x^2) + eps)) * weight
 //   fused_add_rms_norm  residual = fp16(input + residual);  input = fp16(residual * rsqrt(...)) * weight
 //                       with the mean taken over the unrounded fp32 sums, as the reference does
+//   add_rms_norm        the same with the mean over the rounded sums: bit for bit what an fp16 addition
+//                       and rms_norm give in two launches
 // Rounding points are the reference's: the normalised value is rounded to fp16, then multiplied
 // by the weight in fp16.
 #include <hip/hip_runtime.h>
@@ -21,6 +23,7 @@ typedef _Float16 half_t;
 typedef half_t h8 __attribute__((ext_vector_type(8)));
 
 constexpr int WG = 256;
+enum { kNoAdd = 0, kAdd = 1, kAddRounded = 2 };   // what a row is added to first, and which sums the mean is of
 
 __device__ __forceinline__ float block_sum(float v, float* sm) {
 #pragma unroll
@@ -39,16 +42,16 @@ constexpr int KEEP = 4;
 
 // One 8-element piece of the first pass: returns its contribution to the sum of squares and
 // leaves in x what the second pass normalises (with ADD: the rounded sum, also written to residual).
-template <bool ADD>
+template <int ADD>
 __device__ __forceinline__ float first_pass8(h8& x, half_t* __restrict__ residual_piece) {
     float ss = 0.f;
-    if constexpr (ADD) {
+    if constexpr (ADD != kNoAdd) {
         const h8 r = *reinterpret_cast<const h8*>(residual_piece);
 #pragma unroll
         for (int e = 0; e < 8; e++) {
             const float s = float(x[e]) + float(r[e]);
-            ss += s * s;
             x[e] = half_t(s);
+            ss += (ADD == kAdd) ? s * s : float(x[e]) * float(x[e]);
         }
         *reinterpret_cast<h8*>(residual_piece) = x;
     } else {
@@ -65,7 +68,7 @@ __device__ __forceinline__ h8 second_pass8(const h8 x, const h8 w, float inv) {
     return y;
 }
 
-template <int VEC, bool ADD>
+template <int VEC, int ADD>
 __global__ __launch_bounds__(WG) void rms_norm_kernel(half_t* __restrict__ out, half_t* __restrict__ input,
                                                       half_t* __restrict__ residual,
                                                       const half_t* __restrict__ weight, float epsilon,
@@ -111,6 +114,7 @@ __global__ __launch_bounds__(WG) void rms_norm_kernel(half_t* __restrict__ out, 
             if constexpr (ADD) {
                 s += float(residual[row + idx]);
                 residual[row + idx] = half_t(s);
+                if (ADD == kAddRounded) s = float(half_t(s));
             }
             ss += s * s;
         }
@@ -124,7 +128,7 @@ __global__ __launch_bounds__(WG) void rms_norm_kernel(half_t* __restrict__ out, 
 }  // namespace
 
 int launch_rms_norm(void* out, void* input, void* residual, const void* weight, float epsilon,
-                    int64_t n_tokens, int hidden, bool vec8, hipStream_t st) {
+                    int64_t n_tokens, int hidden, bool vec8, bool mean_of_rounded, hipStream_t st) {
     if (n_tokens <= 0 || hidden <= 0) return 0;
     if (n_tokens > 0x7fffffff) return -1;
     const dim3 grid(static_cast<unsigned>(n_tokens)), block(WG);
@@ -132,12 +136,15 @@ int launch_rms_norm(void* out, void* input, void* residual, const void* weight, 
     half_t* in = static_cast<half_t*>(input);
     half_t* res = static_cast<half_t*>(residual);
     const half_t* w = static_cast<const half_t*>(weight);
-    if (residual) {
-        if (vec8) hipLaunchKernelGGL((rms_norm_kernel<8, true>), grid, block, 0, st, o, in, res, w, epsilon, hidden);
-        else hipLaunchKernelGGL((rms_norm_kernel<1, true>), grid, block, 0, st, o, in, res, w, epsilon, hidden);
+    if (residual && mean_of_rounded) {
+        if (vec8) hipLaunchKernelGGL((rms_norm_kernel<8, kAddRounded>), grid, block, 0, st, o, in, res, w, epsilon, hidden);
+        else hipLaunchKernelGGL((rms_norm_kernel<1, kAddRounded>), grid, block, 0, st, o, in, res, w, epsilon, hidden);
+    } else if (residual) {
+        if (vec8) hipLaunchKernelGGL((rms_norm_kernel<8, kAdd>), grid, block, 0, st, o, in, res, w, epsilon, hidden);
+        else hipLaunchKernelGGL((rms_norm_kernel<1, kAdd>), grid, block, 0, st, o, in, res, w, epsilon, hidden);
     } else {
-        if (vec8) hipLaunchKernelGGL((rms_norm_kernel<8, false>), grid, block, 0, st, o, in, res, w, epsilon, hidden);
-        else hipLaunchKernelGGL((rms_norm_kernel<1, false>), grid, block, 0, st, o, in, res, w, epsilon, hidden);
+        if (vec8) hipLaunchKernelGGL((rms_norm_kernel<8, kNoAdd>), grid, block, 0, st, o, in, res, w, epsilon, hidden);
+        else hipLaunchKernelGGL((rms_norm_kernel<1, kNoAdd>), grid, block, 0, st, o, in, res, w, epsilon, hidden);
     }
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? 0 : static_cast<int>(e);

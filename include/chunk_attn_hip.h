@@ -162,6 +162,10 @@ int ca_rms_norm(void* out, const void* input, const void* weight, float epsilon,
                 int hidden_size, void* stream);
 int ca_fused_add_rms_norm(void* input, void* residual, const void* weight, float epsilon,
                           int64_t n_tokens, int hidden_size, void* stream);
+/* The same with the mean taken over the rounded sums: what an fp16 addition into residual followed by ca_rms_norm
+ * of it gives, bit for bit, in one launch. */
+int ca_add_rms_norm(void* input, void* residual, const void* weight, float epsilon,
+                    int64_t n_tokens, int hidden_size, void* stream);
 
 /* Causal attention of whole prompts, the prefill branch of the reference's attention layer
  * (src/chunk_attn/models/llama_hf/modeling_llama.py:64-84): q, k, v and out are

@@ -66,3 +66,13 @@ def test_pybind_ops_and_errors():
         capi.rms_norm(out[:, :256], tx, tw, 1e-6)
     with pytest.raises(capi.ChunkAttnError, match="different buffers"):
         capi.fused_add_rms_norm(tx, tx, tw, 1e-6)
+
+
+@pytest.mark.parametrize("n,hidden", [(1, 8), (3, 256), (2, 1024), (3, 4096), (3, 8200), (5, 4099)])
+def test_add_rms_norm_is_the_addition_and_the_norm_bit_for_bit(n, hidden):
+    g = torch.Generator().manual_seed(hidden)
+    x, r, w = (torch.randn(*shape, generator=g).half().cuda() for shape in ((n, hidden), (n, hidden), (hidden,)))
+    summed, out = r + x, torch.empty_like(x)
+    capi.rms_norm(out, summed, w, 1e-6)
+    capi.add_rms_norm(x, r, w, 1e-6)
+    assert torch.equal(r, summed) and torch.equal(x, out)

@@ -178,3 +178,20 @@ def test_causal_attention_leaves_forward_mode_to_torch():
     with forward_ad.dual_level():
         assert not capi.causal_attention_takes(q, q, q)
     assert capi.causal_attention_takes(q, q, q)
+
+
+def test_model_with_its_adds_in_the_norms_keeps_every_bit():
+    from chunk_attn.models.sequence import Sequence
+    from chunk_attn.models.tiny_lm import AttentionOnlyLM
+    out = []
+    for hooked in (False, True):
+        model = AttentionOnlyLM(300, 1024, 8, 3, chunk_size=32, memory_mb=16, seed=4)
+        if hooked:
+            model.input_norms[1].register_forward_hook(lambda m, a, out: None)
+        caches = model.create_kv_caches()
+        with torch.inference_mode():
+            seq = Sequence(list(range(200)))
+            out.append([model.logits([seq], caches, True)])
+            seq.append(7)
+            out[-1].append(model.logits([seq], caches, False))
+    assert all(torch.equal(a, b) for a, b in zip(*out))

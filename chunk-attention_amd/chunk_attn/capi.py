@@ -418,8 +418,9 @@ def plain_call() -> bool:
     if torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() or \
             torch.autograd.forward_ad._current_level >= 0:
         return False
-    return all(type(torch._C._get_function_stack_at(i)) is torch.utils._device.DeviceContext
-               for i in range(torch._C._len_torch_function_stack()))
+    modes = torch._C._len_torch_function_stack()
+    return modes == 0 or all(type(torch._C._get_function_stack_at(i)) is torch.utils._device.DeviceContext
+                             for i in range(modes))
 
 
 def causal_attention_takes(*tensors) -> bool:
@@ -483,8 +484,37 @@ def projection_takes(x, *linears) -> bool:
     return True
 
 
+def _check_projection(x, *weights) -> None:
+    """Raises unless the projection kernels can read these: x [..., n_in] and weights [n_out, n_in], fp16, contiguous
+    and 16-byte aligned on one GPU, n_in a multiple of 64 (they are handed on as bare addresses)."""
+    n_in = x.shape[-1] if x.dim() else 0
+    if x.device.type != "cuda" or n_in == 0 or n_in % 64:
+        raise RuntimeError(f"projection: rows of a multiple of 64 elements on the GPU, got {tuple(x.shape)} on {x.device}")
+    _check_operand(x, x.device)
+    for w in weights:
+        _check_weight(w, n_in, x.device)
+
+
+def _check_operand(t, device) -> None:
+    import torch
+    if t.dtype != torch.float16 or t.device != device or not t.is_contiguous() or t.data_ptr() % 16:
+        raise RuntimeError("projection: rows and weights must be contiguous, 16-byte aligned fp16 tensors on one GPU")
+
+
+def _check_weight(w, n_in: int, device) -> None:
+    _check_operand(w, device)
+    if w.dim() != 2 or w.shape[1] != n_in:
+        raise RuntimeError(f"projection: weights must be [n_out, {n_in}], got {tuple(w.shape)}")
+
+
 def linear(x, weight):
-    """x . weight^T for what projection_takes accepts."""
+    """x . weight^T in fp16 with fp32 sums; what _check_projection lets through."""
+    _check_projection(x, weight)
+    return _linear(x, weight)
+
+
+def _linear(x, weight):
+    """linear() of what projection_takes has accepted."""
     import torch
     out = torch.empty(x.shape[:-1] + (weight.shape[0],), dtype=x.dtype, device=x.device)
     n_in = x.shape[-1]
@@ -505,6 +535,12 @@ def _check_rotary(positions, rows: int, cos_sin_cache, device) -> None:
 def qkv_rotary(x, wq, wk, wv, positions, cos_sin_cache):
     """(q, k, v) = x . W^T for the three weights [n, n_in] in one launch, n a multiple of 128; q and k are
     rotated for `positions` (NeoX pairs over whole heads of 128) before they are rounded."""
+    _check_projection(x, wq, wk, wv)
+    return _qkv_rotary(x, wq, wk, wv, positions, cos_sin_cache)
+
+
+def _qkv_rotary(x, wq, wk, wv, positions, cos_sin_cache):
+    """qkv_rotary() of rows and weights that projection_takes has accepted."""
     import torch
     n, n_in = wq.shape
     rows = x.numel() // n_in
@@ -933,13 +969,19 @@ class Attention:
     def layer_decode(self, tokens: Sequence[int], x, wq, wk, wv, wo, cos_sin_cache, positions):
         """project_append_rotary, forward and the output projection, then room for the next step's token
         (reserve, refresh_kernel_context): a layer's decode pass as one native call.  Returns [n, n_out]."""
+        _check_projection(x, wq, wk, wv)
+        _check_weight(wo, self.n_heads * 128, x.device)
+        return self._layer_decode(tokens, x, wq, wk, wv, wo, cos_sin_cache, positions)
+
+    def _layer_decode(self, tokens, x, wq, wk, wv, wo, cos_sin_cache, positions):
+        """layer_decode() of rows and weights that projection_takes has accepted."""
         import torch
         n = len(tokens)
         if self.tree.n_seqs != n:
             raise RuntimeError("num of seqs is not equal to num of tokens")
         n_in, width = x.shape[-1], self.n_heads * 128
         if self.d_head != 128 or x.device != self.device or x.numel() != n * n_in or wo.dim() != 2 or wo.shape[1] != width or \
-                wo.data_ptr() % 16 or any(w.shape != (width, n_in) for w in (wq, wk, wv)):
+                any(w.shape != (width, n_in) for w in (wq, wk, wv)):
             raise RuntimeError(f"x must be [{n}, n_in] and the weights [{width}, n_in] and [n_out, {width}] on {self.device}, d_head 128")
         _check_rotary(positions, n, cos_sin_cache, self.device)
         rows = torch.empty((2, n, width), dtype=x.dtype, device=x.device)     # q, then the attention's output
@@ -954,13 +996,18 @@ class Attention:
     def project_append_rotary(self, tokens: Sequence[int], x, wq, wk, wv, cos_sin_cache, positions):
         """append_token_rotary with the projections folded in: the rows of x (what projection_takes accepts)
         times the three weights, q and k rotated, k and v written into the cache.  Returns q."""
+        _check_projection(x, wq, wk, wv)
+        return self._project_append_rotary(tokens, x, wq, wk, wv, cos_sin_cache, positions)
+
+    def _project_append_rotary(self, tokens, x, wq, wk, wv, cos_sin_cache, positions):
+        """project_append_rotary() of rows and weights that projection_takes has accepted."""
         import torch
         n = len(tokens)
         if self.tree.n_seqs != n:
             raise RuntimeError("num of seqs is not equal to num of tokens")
         n_in = x.shape[-1]
         if self.d_head != 128 or x.device != self.device or x.numel() != n * n_in or \
-                any(tuple(w.shape) != (self.n_heads * 128, n_in) for w in (wq, wk, wv)):
+                any(w.shape != (self.n_heads * 128, n_in) for w in (wq, wk, wv)):
             raise RuntimeError(f"x must be [{n}, n_in] and the weights [{self.n_heads * 128}, n_in] on {self.device}, d_head 128")
         _check_rotary(positions, n, cos_sin_cache, self.device)
         self.reserve()

@@ -77,11 +77,11 @@ class LlamaChunkAttention(nn.Module):
             step = ([s[-1] for s in seqs], hidden_states, *weights)
             rotary = (self.rotary_emb.cos_sin_cache, position_ids.reshape(batch).contiguous())
             if own_output:
-                return kv_cache.layer_decode(*step, self.o_proj.weight, *rotary).view(batch, 1, -1)
-            q3 = kv_cache.project_append_rotary(*step, *rotary)
+                return kv_cache._layer_decode(*step, self.o_proj.weight, *rotary).view(batch, 1, -1)
+            q3 = kv_cache._project_append_rotary(*step, *rotary)
             return self._output(kv_cache.forward(q3).view(batch, 1, d_hidden), kv_cache, False)
         if few_rows and prefill:
-            q, k, v = capi.qkv_rotary(hidden_states, *weights, position_ids.contiguous(), self.rotary_emb.cos_sin_cache)
+            q, k, v = capi._qkv_rotary(hidden_states, *weights, position_ids.contiguous(), self.rotary_emb.cos_sin_cache)
         else:
             q = self.q_proj(hidden_states)
             k = self.k_proj(hidden_states)
@@ -117,7 +117,7 @@ class LlamaChunkAttention(nn.Module):
         return capi.is_bare(r, RotaryEmbedding) and r.is_neox_style and r.rotary_dim == r.head_size == self.head_dim
 
     def _output(self, attn_output: torch.Tensor, kv_cache: capi.Attention, own: bool) -> torch.Tensor:
-        output = capi.linear(attn_output, self.o_proj.weight) if own else self.o_proj(attn_output)
+        output = capi._linear(attn_output, self.o_proj.weight) if own else self.o_proj(attn_output)
         kv_cache.reserve()
         kv_cache.refresh_kernel_context(force=False)
         return output

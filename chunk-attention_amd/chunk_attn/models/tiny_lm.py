@@ -103,7 +103,7 @@ class AttentionOnlyLM(nn.Module):
                 normed = norm(hidden)
         last = self.norm(hidden[:, -1]) if normed is None else normed
         if capi.projection_takes(last, self.lm_head):
-            return capi.linear(last, self.lm_head.weight)
+            return capi._linear(last, self.lm_head.weight)
         return self.lm_head(last)
 
     def _adds_in_norms(self) -> bool:

@@ -195,3 +195,33 @@ def test_model_with_its_adds_in_the_norms_keeps_every_bit():
             seq.append(7)
             out[-1].append(model.logits([seq], caches, False))
     assert all(torch.equal(a, b) for a, b in zip(*out))
+
+
+def test_projections_refuse_what_their_kernels_cannot_read():
+    """Fewer columns, other types, strides, alignments and devices: refused before anything is launched or kept."""
+    heads, n_in, n = 2, 256, 3
+    x = torch.zeros(n, n_in, dtype=torch.float16, device="cuda")
+    w = torch.zeros(n_in, n_in, dtype=torch.float16, device="cuda")
+    flat = torch.zeros(n_in * n_in + 1, dtype=torch.float16, device="cuda")
+    bad_x = [x.float(), x.cpu(), x.t().contiguous().t(), flat[1:1 + n * n_in].view(n, n_in), x[:, :100].contiguous(), x[:, :0]]
+    bad_w = [w[:, :128].contiguous(), w.float(), w.bfloat16(), torch.empty(n_in, n_in, dtype=torch.float16, device="cuda").t(),
+             w.cpu(), flat[1:].view(n_in, n_in), w.view(-1)]
+    table = torch.zeros(64, 128, dtype=torch.float16, device="cuda")
+    pos = torch.zeros(n, dtype=torch.int64, device="cuda")
+    kv = capi.Attention(heads, 128, 32, memory_mb=4, dtype=torch.float16, device=torch.device("cuda:0"))
+    for s in range(n):
+        kv.add_seq([s] * 5, *(torch.zeros(5, heads, 128, dtype=torch.float16, device="cuda") for _ in range(2)))
+    kv.refresh_kernel_context()
+    calls = [(lambda a, b: capi.linear(a, b), 1), (lambda a, *b: capi.qkv_rotary(a, *b, pos, table), 3),
+             (lambda a, *b: kv.project_append_rotary([7] * n, a, *b, table, pos), 3),
+             (lambda a, *b: kv.layer_decode([7] * n, a, *b, table, pos), 4)]
+    before = kv.tree.dump()
+    for call, count in calls:
+        cases = [(bad, *[w] * count) for bad in bad_x]
+        cases += [(x, *[w] * at, bad, *[w] * (count - at - 1)) for bad in bad_w for at in range(count)]
+        for case in cases:
+            with pytest.raises(RuntimeError):
+                call(*case)
+    assert kv.tree.dump() == before and kv.ctx.delta_tokens == 0
+    for call, count in calls:
+        call(x, *[w] * count)

@@ -802,8 +802,11 @@ int ca_causal_attention(const void* q, const void* k, const void* v, void* out, 
 }
 
 namespace {
-int project(ca::ProjectArgs& a, const void* x, int M, int N, int K, void* stream) {
-    if (M < 0 || N <= 0 || K <= 0 || K % 64 != 0) return fail(CA_ERR_INVALID, "projection: n_in must be a multiple of 64");
+// Completes the arguments, or says what is wrong with them; nothing is launched.
+int check_project(ca::ProjectArgs& a, const void* x, int M, int N, int K) {
+    if (M < 0 || N <= 0 || K <= 0 || K % 64 != 0) {
+        return fail(CA_ERR_INVALID, "projection: n_out must be positive and n_in a multiple of 64");
+    }
     if (M == 0) return CA_OK;
     a.x = x;
     a.M = M;
@@ -819,6 +822,12 @@ int project(ca::ProjectArgs& a, const void* x, int M, int N, int K, void* stream
     if (a.positions && (!a.vec8 || !a.cos_sin_cache || !aligned16(a.cos_sin_cache) || a.max_position <= 0)) {
         return fail(CA_ERR_INVALID, "projection: misaligned output or no cos/sin cache");
     }
+    return CA_OK;
+}
+
+int project(ca::ProjectArgs& a, const void* x, int M, int N, int K, void* stream) {
+    if (int rc = check_project(a, x, M, N, K)) return rc;
+    if (M == 0) return CA_OK;
     return launch_rc(ca::launch_project(a, static_cast<hipStream_t>(stream)), "projection launch");
 }
 }  // namespace
@@ -845,6 +854,20 @@ int ca_qkv_rotary(const void* x, const void* wq, const void* wk, const void* wv,
     return project(a, x, n_rows, n_heads * 128, n_in, stream);
 }
 
+namespace {
+ca::ProjectArgs qkv_append_args(const ca_ctx* c, const void* wq, const void* wk, const void* wv, const int64_t* positions,
+                                const void* cos_sin_cache, int max_position, void* q) {
+    ca::ProjectArgs a;
+    a.n_w = 3;
+    a.w[0] = wq; a.w[1] = wk; a.w[2] = wv;
+    a.y[0] = q; a.y[1] = c->k_pool; a.y[2] = c->v_pool;
+    a.positions = positions;
+    a.cos_sin_cache = cos_sin_cache;
+    a.max_position = max_position;
+    return a;
+}
+}  // namespace
+
 int ca_qkv_rotary_append_kv(ca_ctx* c, const void* x, const void* wq, const void* wk, const void* wv,
                             const int64_t* positions, const void* cos_sin_cache, int max_position, void* q,
                             int n_in, int n_seqs, void* stream) {
@@ -857,13 +880,7 @@ int ca_qkv_rotary_append_kv(ca_ctx* c, const void* x, const void* wq, const void
             return fail(CA_ERR_STATE, "sequence " + std::to_string(s) + " has no free row in its last chunk: reserve and refresh first");
         }
     }
-    ca::ProjectArgs a;
-    a.n_w = 3;
-    a.w[0] = wq; a.w[1] = wk; a.w[2] = wv;
-    a.y[0] = q; a.y[1] = c->k_pool; a.y[2] = c->v_pool;
-    a.positions = positions;
-    a.cos_sin_cache = cos_sin_cache;
-    a.max_position = max_position;
+    ca::ProjectArgs a = qkv_append_args(c, wq, wk, wv, positions, cos_sin_cache, max_position, q);
     a.tail_slot = reinterpret_cast<const int32_t*>(c->dev_blob + c->off_tail_slot);
     a.tail_fill = reinterpret_cast<const int32_t*>(c->dev_blob + c->off_tail_fill);
     a.delta_tokens = c->delta_tokens;
@@ -900,6 +917,17 @@ int ca_layer_decode(ca_ctx* c, ca_tree* tree, const int32_t* tokens, int n_seqs,
                     void* y, void* stream) {
     if (!c || !tree || !tokens || n_seqs <= 0) return fail(CA_ERR_INVALID, "bad argument");
     if (ca_tree_n_seqs(tree) != n_seqs) return fail(CA_ERR_INVALID, "num of seqs is not equal to num of tokens");
+    // everything its calls would refuse, before the cache moves on: a refused call can be made again
+    if (int rc = check_attention_shape(c)) return rc;
+    if (!positions || !q || !attn || !y) return fail(CA_ERR_INVALID, "null device pointer");
+    if (c->valid && c->delta_tokens < 0) return fail(CA_ERR_STATE, "delta_tokens is negative");
+    ca::ProjectArgs in = qkv_append_args(c, wq, wk, wv, positions, cos_sin_cache, max_position, q);
+    if (int rc = check_project(in, x, n_seqs, c->H * 128, n_in)) return rc;
+    ca::ProjectArgs out;
+    out.n_w = 1;
+    out.w[0] = wo;
+    out.y[0] = y;
+    if (int rc = check_project(out, attn, n_seqs, n_out, c->H * 128)) return rc;
     return guarded([&]() -> int {
         if (int rc = settle(c, tree, n_seqs, stream)) return rc;
         if (int rc = ca_qkv_rotary_append_kv(c, x, wq, wk, wv, positions, cos_sin_cache, max_position, q, n_in, n_seqs, stream)) return rc;

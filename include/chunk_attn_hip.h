@@ -440,7 +440,7 @@ int ca_tree_dump(const ca_tree* tree, int32_t* nodes, int node_cap, int* n_nodes
  * (ca_tree_reserve_tails, ca_ctx_roll_tails, ca_refresh_kernel_context as needed), ca_qkv_rotary_append_kv,
  * ca_tree_append_token, ca_attention, ca_linear with wo [n_out, n_heads * 128], room for the next token.
  * x [n_seqs, n_in]; q and attn [n_seqs, n_heads * 128] and y [n_seqs, n_out] are written; tokens: host, one
- * per sequence. */
+ * per sequence.  Arguments are checked first: a call refused for one leaves cache, tree and tables as they were. */
 int ca_layer_decode(ca_ctx* ctx, ca_tree* tree, const int32_t* tokens, int n_seqs, const void* x, int n_in,
                     const void* wq, const void* wk, const void* wv, const void* wo, int n_out,
                     const int64_t* positions_dev, const void* cos_sin_cache, int max_position, void* q,

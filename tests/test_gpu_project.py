@@ -225,3 +225,40 @@ def test_projections_refuse_what_their_kernels_cannot_read():
     assert kv.tree.dump() == before and kv.ctx.delta_tokens == 0
     for call, count in calls:
         call(x, *[w] * count)
+
+
+def test_a_refused_decode_pass_leaves_the_cache_as_it_was():
+    """Every argument of ca_layer_decode is looked at before the tree, the pool and the tables move on."""
+    import ctypes
+    heads, n = 2, 3
+    t = lambda *shape: torch.ones(shape, dtype=torch.float16, device="cuda")
+    x, w, q, y, table = t(n, 256), t(256 * 256 + 8) / 256, t(2, n, 256), t(n, 256), t(64, 128)   # products of 1
+    pos = torch.zeros(n, dtype=torch.int64, device="cuda")
+    tokens = (ctypes.c_int32 * n)(7, 7, 7)
+
+    def cache(chunk):
+        kv = capi.Attention(heads, 128, chunk, memory_mb=4, dtype=torch.float16, device=torch.device("cuda:0"))
+        for s in range(n):
+            kv.add_seq([s] * chunk, t(chunk, heads, 128), t(chunk, heads, 128))   # full: a pass needs new last chunks
+        return kv
+
+    def args(**changed):
+        a = dict(x=x.data_ptr(), n_in=256, wq=w.data_ptr(), wk=w.data_ptr(), wv=w.data_ptr(), wo=w.data_ptr(), n_out=256,
+                 positions=pos.data_ptr(), table=table.data_ptr(), max_position=64, q=q[0].data_ptr(), attn=q[1].data_ptr(), y=y.data_ptr())
+        assert set(changed) <= set(a)
+        return list(dict(a, **changed).values())
+
+    def call(kv, a):
+        return kv.ctx._lib.ca_layer_decode(kv.ctx._h, kv.tree._h, tokens, n, *a, torch.cuda.current_stream().cuda_stream)
+
+    bad = [{k: 0} for k in ("x", "wq", "wk", "wv", "wo", "n_in", "n_out", "positions", "table", "max_position", "q", "attn", "y")]
+    bad += [{"n_in": 100}, {"n_out": -5}, {"wo": w.data_ptr() + 2}, {"attn": q[1].data_ptr() + 2}, {"wq": w.data_ptr() + 4},
+            {"q": q.data_ptr() + 2}, {"table": table.data_ptr() + 2}]
+    for kv, changes in ((cache(32), bad), (cache(48), [{}])):               # chunks of 48: no attention kernel
+        before, pools = kv.tree.dump(), [p.clone() for p in kv.pool_views()]
+        for change in changes:
+            assert call(kv, args(**change)) < 0, change
+        assert kv.tree.dump() == before and kv.ctx.delta_tokens == 0
+        assert all(torch.equal(a, b) for a, b in zip(pools, kv.pool_views()))
+    kv = cache(32)
+    assert call(kv, args()) == 0 and kv.tree.n_seqs == n and torch.isfinite(y).all()

@@ -190,9 +190,11 @@ __global__ __launch_bounds__(WG, TILE == 32 ? 4 : 2) void causal_attention_kerne
         for (int e = 1; e < 4 * TB - 1; e += 2) mx = max2(max2(mx, sc[e >> 2][e & 3]), sc[(e + 1) >> 2][(e + 1) & 3]);
         mx = max_over_groups(max2(mx, sc[TB - 1][3]));
         const float m_new = max2(m_run, mx * scale_log2);
-        if (__builtin_amdgcn_ballot_w64(m_new > m_run + kSlack) != 0) {
-            const float alpha = (m_run == NEG_INF) ? 0.f : fast_exp2(m_run - m_new);
-            m_run = m_new;
+        const bool grew = m_new > m_run + kSlack;
+        if (__builtin_amdgcn_ballot_w64(grew) != 0) {
+            // only the rows that grew: what a row gives must not depend on the rows behind it
+            const float alpha = !grew ? 1.f : (m_run == NEG_INF) ? 0.f : fast_exp2(m_run - m_new);
+            m_run = grew ? m_new : m_run;
             l_lane *= alpha;
 #pragma unroll
             for (int db = 0; db < 8; db++) oacc[db] *= alpha;

@@ -57,3 +57,15 @@ def test_refused_inputs():
         with pytest.raises(RuntimeError):
             capi.causal_attention(bad, bad, bad)
     assert not capi.causal_attention_takes(q, q, torch.zeros_like(q, requires_grad=True))
+
+
+@pytest.mark.parametrize("batch,n,heads", [(1, 200, 8), (8, 300, 16)])       # 64-key tiles, 32-key tiles
+def test_later_rows_of_a_wave_change_nothing_in_earlier_ones(batch, n, heads):
+    """Ordinary scores, whose running maxima move by less than the kernel's slack, beside rows of the same 16
+    whose maxima jump."""
+    g = torch.Generator().manual_seed(n)
+    q, k, v = (torch.randn(batch, n, heads, 128, generator=g).half().cuda() for _ in range(3))
+    first = capi.causal_attention(q, k, v)
+    q[:, 150:] *= 8                                                       # rows 150 .. 159 share a wave with 144 .. 149
+    second = capi.causal_attention(q, k, v)
+    assert torch.equal(first[:, :150], second[:, :150]) and not torch.equal(first[:, 150:], second[:, 150:])

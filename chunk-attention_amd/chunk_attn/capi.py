@@ -13,6 +13,7 @@ from __future__ import annotations
 import array
 import ctypes
 import os
+import sys
 from typing import List, Optional, Sequence, Tuple
 
 import numpy as np
@@ -415,7 +416,7 @@ def plain_call() -> bool:
     only places new tensors, as torch.set_default_device leaves on the stack, does not), no forward-mode level
     whose tangents a kernel would drop."""
     import torch
-    if torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() or \
+    if torch.compiler.is_compiling() or torch._C._is_tracing() or torch._C._len_torch_dispatch_stack() or \
             torch.autograd.forward_ad._current_level >= 0:
         return False
     modes = torch._C._len_torch_function_stack()
@@ -450,7 +451,29 @@ def is_bare(module, cls) -> bool:
     """The module is a `cls` and nothing hangs on it that a call would also run (hooks, a patched forward)."""
     own = module.__dict__
     return type(module) is cls and not (own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"] or
-                                        own["_backward_pre_hooks"] or "forward" in own)
+                                        own["_backward_pre_hooks"] or "forward" in own or "_call_impl" in own)
+
+
+def are_unpatched(*classes) -> bool:
+    """Nobody has replaced the forwards of these module classes, what a module call goes through before them, or the
+    functions that torch's own compute with (adapters and profilers do): each still belongs to the file that
+    defines it."""
+    import torch
+    nn = torch.nn
+    try:
+        module = nn.modules.module.__dict__
+        call, impl = nn.Module.__call__, nn.Module._call_impl
+        if call.__globals__ is not module or impl.__globals__ is not module:
+            return False
+        for cls in classes:
+            if cls.forward.__globals__ is not sys.modules[cls.__module__].__dict__ or cls.__call__ is not call or cls._call_impl is not impl:
+                return False
+            if cls is nn.Linear and nn.functional.linear is not torch._C._nn.linear or \
+                    cls is nn.Embedding and nn.functional.embedding.__globals__ is not nn.functional.__dict__:
+                return False
+    except AttributeError:                                # something that is no Python function
+        return False
+    return True
 
 
 def projection_takes(x, *linears) -> bool:
@@ -469,7 +492,7 @@ def projection_takes(x, *linears) -> bool:
     grad = torch.is_grad_enabled()
     # whatever else may stand between a module and its product: hooks, subclasses, patched forwards, modes
     if grad and x.requires_grad or torch.is_autocast_enabled() or not plain_call() or \
-            torch.nn.modules.module._has_any_global_hook():
+            torch.nn.modules.module._has_any_global_hook() or not are_unpatched(torch.nn.Linear):
         return False
     device = x.device
     for m in linears:
@@ -980,8 +1003,8 @@ class Attention:
         if self.tree.n_seqs != n:
             raise RuntimeError("num of seqs is not equal to num of tokens")
         n_in, width = x.shape[-1], self.n_heads * 128
-        if self.d_head != 128 or x.device != self.device or x.numel() != n * n_in or wo.dim() != 2 or wo.shape[1] != width or \
-                any(w.shape != (width, n_in) for w in (wq, wk, wv)):
+        if self.d_head != 128 or x.device != self.device or x.numel() != n * n_in or wq.size(0) != width or \
+                wk.size(0) != width or wv.size(0) != width or wo.size(1) != width:
             raise RuntimeError(f"x must be [{n}, n_in] and the weights [{width}, n_in] and [n_out, {width}] on {self.device}, d_head 128")
         _check_rotary(positions, n, cos_sin_cache, self.device)
         rows = torch.empty((2, n, width), dtype=x.dtype, device=x.device)     # q, then the attention's output
@@ -1005,10 +1028,10 @@ class Attention:
         n = len(tokens)
         if self.tree.n_seqs != n:
             raise RuntimeError("num of seqs is not equal to num of tokens")
-        n_in = x.shape[-1]
-        if self.d_head != 128 or x.device != self.device or x.numel() != n * n_in or \
-                any(w.shape != (self.n_heads * 128, n_in) for w in (wq, wk, wv)):
-            raise RuntimeError(f"x must be [{n}, n_in] and the weights [{self.n_heads * 128}, n_in] on {self.device}, d_head 128")
+        n_in, width = x.shape[-1], self.n_heads * 128
+        if self.d_head != 128 or x.device != self.device or x.numel() != n * n_in or wq.size(0) != width or \
+                wk.size(0) != width or wv.size(0) != width:
+            raise RuntimeError(f"x must be [{n}, n_in] and the weights [{width}, n_in] on {self.device}, d_head 128")
         _check_rotary(positions, n, cos_sin_cache, self.device)
         self.reserve()
         self.refresh_kernel_context()
@@ -1058,3 +1081,17 @@ class Attention:
         """(K, V) pool tensors viewed as [max_chunks, H, c, d]."""
         shape = (self.max_chunks, self.n_heads, self.chunk_size, self.d_head)
         return self.key_storage.view(shape), self.value_storage.view(shape)
+
+
+def is_plain_cache(cache) -> bool:
+    """An `Attention` of this module whose steps of a decode pass nobody has replaced, on the class or the object."""
+    if type(cache) is not Attention:
+        return False
+    own, here = cache.__dict__, globals()
+    try:
+        for name in ("append_token_rotary", "forward", "reserve", "refresh_kernel_context"):
+            if name in own or getattr(Attention, name).__globals__ is not here:
+                return False
+    except AttributeError:
+        return False
+    return True

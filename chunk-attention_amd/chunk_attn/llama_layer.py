@@ -72,7 +72,7 @@ class LlamaChunkAttention(nn.Module):
             few_rows = own_output or capi.projection_takes(hidden_states, *projections)
         if few_rows:
             weights = [p.weight for p in projections]
-        if few_rows and not prefill and type(kv_cache) is capi.Attention:   # other caches have append_token_rotary only
+        if few_rows and not prefill and capi.is_plain_cache(kv_cache):      # other caches have append_token_rotary only
             assert n_tokens == 1
             step = ([s[-1] for s in seqs], hidden_states, *weights)
             rotary = (self.rotary_emb.cos_sin_cache, position_ids.reshape(batch).contiguous())
@@ -114,7 +114,7 @@ class LlamaChunkAttention(nn.Module):
     def _plain_rotary(self) -> bool:
         """The rotary module is the one this layer was built with, over whole heads, and nothing hangs on it."""
         r = self.rotary_emb
-        return capi.is_bare(r, RotaryEmbedding) and r.is_neox_style and r.rotary_dim == r.head_size == self.head_dim
+        return capi.is_bare(r, RotaryEmbedding) and capi.are_unpatched(RotaryEmbedding) and r.is_neox_style and r.rotary_dim == r.head_size == self.head_dim
 
     def _output(self, attn_output: torch.Tensor, kv_cache: capi.Attention, own: bool) -> torch.Tensor:
         output = capi._linear(attn_output, self.o_proj.weight) if own else self.o_proj(attn_output)

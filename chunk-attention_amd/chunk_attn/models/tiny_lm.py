@@ -110,7 +110,9 @@ class AttentionOnlyLM(nn.Module):
         """A layer's residual is added in the norm behind it, in place: nothing may want the tensors it overwrites
         (a gradient, a hook, a mode that sees them, a forward-mode tangent of them), and the norms must be the plain
         ones."""
-        return capi.plain_call() and not torch.is_grad_enabled() and capi.is_bare(self.embed_tokens, nn.Embedding) and \
+        return capi.plain_call() and not torch.is_grad_enabled() and \
+            capi.are_unpatched(nn.Embedding, nn.Linear, LlamaChunkAttention, RMSNorm) and \
+            capi.is_bare(self.embed_tokens, nn.Embedding) and \
             all(capi.is_bare(m, LlamaChunkAttention) and capi.is_bare(m.o_proj, nn.Linear) for m in self.layers) and \
             all(capi.is_bare(m, RMSNorm) for m in self.input_norms) and capi.is_bare(self.norm, RMSNorm) and \
             not torch.nn.modules.module._has_any_global_hook()

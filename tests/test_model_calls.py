@@ -129,3 +129,36 @@ def test_no_tangent_of_an_overwritten_tensor_reaches_the_logits(fused):
         m.layers[1].o_proj.weight = dual
         assert forward_ad.unpack_dual(logits(m)).tangent is None
     assert not fused
+
+
+def test_replaced_classes_and_functions_are_seen(monkeypatch, fused):
+    from chunk_attn.llama_layer import LlamaChunkAttention, RotaryEmbedding
+    nn = torch.nn
+    classes = (nn.Linear, nn.Embedding, RotaryEmbedding, LlamaChunkAttention, tiny_lm.RMSNorm)
+    m = model()
+
+    def joined():
+        with torch.no_grad():
+            return m._adds_in_norms()
+
+    assert all(map(capi.are_unpatched, classes)) and joined()
+    for cls in classes:
+        with monkeypatch.context() as mp:
+            forward = cls.forward
+            mp.setattr(cls, "forward", lambda *a: forward(*a))
+            assert not capi.are_unpatched(cls) and joined() == (cls is RotaryEmbedding)
+    for owner, name in ((nn.Module, "__call__"), (nn.Module, "_call_impl")):
+        with monkeypatch.context() as mp:
+            mp.setattr(owner, name, lambda *a, **k: None)
+            assert not any(map(capi.are_unpatched, classes))
+    for name, cls in (("linear", nn.Linear), ("embedding", nn.Embedding)):
+        with monkeypatch.context() as mp:
+            mp.setattr(nn.functional, name, lambda *a: None)
+            assert [capi.are_unpatched(c) for c in classes] == [c is not cls for c in classes] and not joined()
+    cache = object.__new__(capi.Attention)
+    assert capi.is_plain_cache(cache) and not capi.is_plain_cache(CountingCache())
+    with monkeypatch.context() as mp:
+        mp.setattr(capi.Attention, "forward", lambda self, q: q)
+        assert not capi.is_plain_cache(cache)
+    cache.append_token_rotary = lambda *a: None
+    assert not capi.is_plain_cache(cache)

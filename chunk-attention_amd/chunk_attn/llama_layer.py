@@ -66,17 +66,19 @@ class LlamaChunkAttention(nn.Module):
         batch row i to be cache sequence i."""
         batch, n_tokens, d_hidden = hidden_states.shape
         projections = (self.q_proj, self.k_proj, self.v_proj)
-        own_output = few_rows = False                  # which projections the framework's own kernel computes
+        few_rows = folded = False       # q, k and v by the framework's own kernel; a decode pass as one native call
+        # (caches of other classes have append_token_rotary only)
+        plain_cache = not prefill and capi.is_plain_cache(kv_cache)
         if self.head_dim == 128 and self._plain_rotary():
-            own_output = capi.projection_takes(hidden_states, *projections, self.o_proj)
-            few_rows = own_output or capi.projection_takes(hidden_states, *projections)
+            folded = plain_cache and capi.projection_takes(hidden_states, *projections, self.o_proj)
+            few_rows = folded or capi.projection_takes(hidden_states, *projections)
         if few_rows:
             weights = [p.weight for p in projections]
-        if few_rows and not prefill and capi.is_plain_cache(kv_cache):      # other caches have append_token_rotary only
+        if few_rows and plain_cache:
             assert n_tokens == 1
             step = ([s[-1] for s in seqs], hidden_states, *weights)
             rotary = (self.rotary_emb.cos_sin_cache, position_ids.reshape(batch).contiguous())
-            if own_output:
+            if folded:
                 return kv_cache._layer_decode(*step, self.o_proj.weight, *rotary).view(batch, 1, -1)
             q3 = kv_cache._project_append_rotary(*step, *rotary)
             return self._output(kv_cache.forward(q3).view(batch, 1, d_hidden), kv_cache, False)
@@ -109,14 +111,16 @@ class LlamaChunkAttention(nn.Module):
             kv_cache.append_token_rotary([s[-1] for s in seqs], q3, k3, v3, self.rotary_emb.cos_sin_cache,
                                          self.rotary_emb.is_neox_style, position_ids.reshape(batch).contiguous())
             attn_output = kv_cache.forward(q3).view(batch, 1, d_hidden)
-        return self._output(attn_output, kv_cache, own_output and attn_output.is_contiguous())
+        return self._output(attn_output, kv_cache, few_rows)
 
     def _plain_rotary(self) -> bool:
         """The rotary module is the one this layer was built with, over whole heads, and nothing hangs on it."""
         r = self.rotary_emb
         return capi.is_bare(r, RotaryEmbedding) and capi.are_unpatched(RotaryEmbedding) and r.is_neox_style and r.rotary_dim == r.head_size == self.head_dim
 
-    def _output(self, attn_output: torch.Tensor, kv_cache: capi.Attention, own: bool) -> torch.Tensor:
+    def _output(self, attn_output: torch.Tensor, kv_cache: capi.Attention, few_rows: bool) -> torch.Tensor:
+        # what the attention gave is looked at itself: a cache of another class may return anything
+        own = few_rows and capi.projection_takes(attn_output, self.o_proj)
         output = capi._linear(attn_output, self.o_proj.weight) if own else self.o_proj(attn_output)
         kv_cache.reserve()
         kv_cache.refresh_kernel_context(force=False)

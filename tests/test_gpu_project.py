@@ -262,3 +262,17 @@ def test_a_refused_decode_pass_leaves_the_cache_as_it_was():
         assert all(torch.equal(a, b) for a, b in zip(pools, kv.pool_views()))
     kv = cache(32)
     assert call(kv, args()) == 0 and kv.tree.n_seqs == n and torch.isfinite(y).all()
+
+
+def test_output_of_another_cache_is_not_taken_for_granted():
+    """A cache of another class may return another type: torch's product refuses it, the kernel must not read it."""
+    class Wide(capi.Attention):
+        def forward(self, q, partition=0):
+            return super().forward(q, partition).float()
+
+    layer = LlamaChunkAttention(256, 2, device="cuda")
+    kv = Wide(2, 128, 64, memory_mb=16, dtype=torch.float16, device=torch.device("cuda:0"))
+    with torch.inference_mode():
+        layer(_draw(torch.Generator().manual_seed(1), 1, 5, 256), [[1] * 5], torch.arange(5)[None].cuda(), kv, True)
+        with pytest.raises(RuntimeError):
+            layer(torch.zeros(1, 1, 256, dtype=torch.float16, device="cuda"), [[1] * 6], torch.full((1, 1), 5).cuda(), kv, False)

@@ -478,11 +478,8 @@ def are_unpatched(*classes) -> bool:
 
 def projection_takes(x, *linears) -> bool:
     """Whether the projection kernel stands in for these torch.nn.Linear modules on the rows of x: nothing but
-    x . W^T in fp16 on one GPU is asked of them, and the product is small enough.
-
-    The line: rows * n_in up to 2^20.  Beyond it the library's products win (a layer of 4096 on 252 rows: q, k and v
-    68 us here, 58 + 4 for the library and the rotary launch; on 512 rows 131 against 79; a layer of 1024 on
-    768 rows 22.6 against 27.4, on 1024 rows 24.5 against 27.9, on 2048 rows 45 against 33)."""
+    x . W^T in fp16 on one GPU is asked of them, on at most 2^20 elements.  Whether that is also the better choice is
+    projection_pays's business."""
     import torch
     if type(x) is not torch.Tensor or x.dtype != torch.float16 or x.device.type != "cuda" or not x.is_contiguous():
         return False
@@ -505,6 +502,25 @@ def projection_takes(x, *linears) -> bool:
                 w.data_ptr() % 16 or (grad and w.requires_grad):
             return False
     return True
+
+
+def projection_pays(rows: int, n_in: int, n_out: int) -> bool:
+    """Whether rows [rows, n_in] times one weight [n_out, n_in], or times a layer's three with the rotation, are better
+    computed here than by the library's products.
+
+    A product of the library costs the host 20 us, one here 11 with its checks, q, k and v with their rotation 16 where
+    the library's four launches take 70; a layer or model pass of such row counts is bound by the host.  On the GPU
+    this kernel wins where reading the weights is the work (us here against the library's: 1024 x 1024 on 8 rows 3.2
+    to 4.3, 8000 x 1024 on 8 rows 4.9 to 10.1; q, k, v and rotation of 1024 on 252 rows 8.7 to 26.7, of 4096 on 16
+    rows 25 to 40) and loses to tiles that waves share as the rows grow.  The lines keep the loss below what the host
+    saves: rows * n_out up to 2^20 (4096 x 4096 on 252 rows 19.7 to 19.2, q, k and v 68 to 72; 8000 x 1024 on 128 rows
+    10.6 to 9.6 but on 252 rows 19.8 to 11.2, 32000 x 1024 on 252 rows 69 to 25); 16 rows for weights of more than
+    2^25 elements (8192 x 8192 on 16 rows 26 to 22, on 48 rows 46 to 26, q, k and v 86 to 89 and 95 to 100, on 65 rows
+    139 to 122; 32000 x 4096 on 16 rows 59 to 58, on 65 rows 102 to 62); none of more than 2^27, which were not
+    measured.  Below 2^25, with rows * n_in up to 2^20 as projection_takes has it, the largest losses are 1536 x 1536 on
+    682 rows, 19 to 12, and 5120 x 5120 on 128 rows, 30 to 25 (q, k and v 64 to 99)."""
+    weights = n_in * n_out
+    return rows * n_out <= 1 << 20 and (weights <= 1 << 25 or rows <= 16 and weights <= 1 << 27)
 
 
 def _check_projection(x, *weights) -> None:

@@ -69,7 +69,7 @@ class LlamaChunkAttention(nn.Module):
         few_rows = folded = False       # q, k and v by the framework's own kernel; a decode pass as one native call
         # (caches of other classes have append_token_rotary only)
         plain_cache = not prefill and capi.is_plain_cache(kv_cache)
-        if self.head_dim == 128 and self._plain_rotary():
+        if self.head_dim == 128 and capi.projection_pays(batch * n_tokens, d_hidden, d_hidden) and self._plain_rotary():
             folded = plain_cache and capi.projection_takes(hidden_states, *projections, self.o_proj)
             few_rows = folded or capi.projection_takes(hidden_states, *projections)
         if few_rows:

@@ -102,7 +102,7 @@ class AttentionOnlyLM(nn.Module):
                 hidden = hidden + out
                 normed = norm(hidden)
         last = self.norm(hidden[:, -1]) if normed is None else normed
-        if capi.projection_takes(last, self.lm_head):
+        if capi.projection_pays(len(seqs), self.hidden_size, self.vocab_size) and capi.projection_takes(last, self.lm_head):
             return capi._linear(last, self.lm_head.weight)
         return self.lm_head(last)
 

@@ -37,7 +37,7 @@ enum { kPlain = 0, kRotary = 1, kAppend = 2 };
 // library 44), below that the launch and two round trips to memory (1024 x 1024: 3.3 us, the library 4.4; q, k
 // and v together 4.3, as three library calls 13.3, the rotary launch not counted); with hundreds of rows
 // LDS, which every wave fills and reads for itself, and from some n_rows * n_in on a library product that
-// shares its tiles between waves is faster (projection_takes in capi.py has the line).
+// shares its tiles between waves is faster (projection_pays in capi.py has the line).
 //
 // Columns of a rotary tile: half of them from the first half of a head, half their partners 64 further on.
 template <int MB, int NB, int R, int MODE>

@@ -162,3 +162,20 @@ def test_replaced_classes_and_functions_are_seen(monkeypatch, fused):
         assert not capi.is_plain_cache(cache)
     cache.append_token_rotary = lambda *a: None
     assert not capi.is_plain_cache(cache)
+
+
+# us on one GPU (MI355X), weights from memory
+@pytest.mark.parametrize("rows,n_in,n_out,here,library,pays", [
+    (2048, 128, 128, 3.1, 4.2, True), (1024, 512, 512, 5.8, 6.1, True), (252, 1024, 1024, 4.4, 8.0, True),
+    (1024, 1024, 1024, 8.8, 9.0, True), (1536, 1024, 1024, 15.6, 9.9, False), (512, 1536, 1536, 10.9, 9.3, True),
+    (1024, 1536, 1536, 20.2, 13.0, False), (512, 2048, 2048, 13.7, 11.4, True), (16, 4096, 4096, 8.3, 9.0, True),
+    (252, 4096, 4096, 19.7, 19.2, True), (320, 4096, 4096, 34.0, 22.4, False), (128, 5120, 5120, 30.2, 25.0, True),
+    (252, 5120, 5120, 41.9, 27.4, False), (16, 8192, 8192, 26.2, 22.0, True), (48, 8192, 8192, 46.4, 25.6, False),
+    (65, 1024, 4000, 7.4, 8.5, True), (512, 1024, 4000, 20.0, 11.7, False), (128, 1024, 8000, 10.6, 9.6, True),
+    (160, 1024, 8000, 17.4, 10.4, False), (252, 1024, 8000, 19.8, 11.2, False), (32, 1024, 32000, 21.2, 23.6, True),
+    (252, 1024, 32000, 69.3, 25.4, False), (16, 4096, 32000, 58.6, 57.7, True), (252, 4096, 32000, 193.8, 75.4, False),
+    (16, 4096, 11008, 23.7, 20.8, True), (64, 4096, 11008, 37.9, 27.5, False)])
+def test_projections_are_computed_here_while_the_host_gains_more(rows, n_in, n_out, here, library, pays):
+    """A library call costs the host 9 us more than one here."""
+    assert capi.projection_pays(rows, n_in, n_out) == pays
+    assert here <= library + 9 if pays else here > library + 5

@@ -13,7 +13,6 @@ from __future__ import annotations
 import array
 import ctypes
 import os
-import sys
 from typing import List, Optional, Sequence, Tuple
 
 import numpy as np
@@ -438,10 +437,15 @@ def causal_attention_takes(*tensors) -> bool:
 
 def causal_attention(q, k, v):
     """Causal attention of whole prompts, [batch, n, heads, 128] each; returns a tensor like q."""
-    import torch
     if not causal_attention_takes(q, k, v):
         raise RuntimeError("causal_attention: contiguous, 16-byte aligned fp16 GPU tensors [batch, n, heads, 128] "
                            "of one shape, without gradients")
+    return _causal_attention(q, k, v)
+
+
+def _causal_attention(q, k, v):
+    """causal_attention() of what causal_attention_takes has accepted."""
+    import torch
     out = torch.empty_like(q)
     _launch(q.device, load().ca_causal_attention, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), *q.shape)
     return out
@@ -454,32 +458,16 @@ def is_bare(module, cls) -> bool:
                                         own["_backward_pre_hooks"] or "forward" in own or "_call_impl" in own)
 
 
-def are_unpatched(*classes) -> bool:
-    """Nobody has replaced the forwards of these module classes, what a module call goes through before them, or the
-    functions that torch's own compute with (adapters and profilers do): each still belongs to the file that
-    defines it."""
-    import torch
-    nn = torch.nn
-    try:
-        module = nn.modules.module.__dict__
-        call, impl = nn.Module.__call__, nn.Module._call_impl
-        if call.__globals__ is not module or impl.__globals__ is not module:
-            return False
-        for cls in classes:
-            if cls.forward.__globals__ is not sys.modules[cls.__module__].__dict__ or cls.__call__ is not call or cls._call_impl is not impl:
-                return False
-            if cls is nn.Linear and nn.functional.linear is not torch._C._nn.linear or \
-                    cls is nn.Embedding and nn.functional.embedding.__globals__ is not nn.functional.__dict__:
-                return False
-    except AttributeError:                                # something that is no Python function
-        return False
-    return True
-
-
 def projection_takes(x, *linears) -> bool:
     """Whether the projection kernel stands in for these torch.nn.Linear modules on the rows of x: nothing but
     x . W^T in fp16 on one GPU is asked of them, on at most 2^20 elements.  Whether that is also the better choice is
     projection_pays's business."""
+    from .stock import linear_is_stock
+    return linear_is_stock() and _projection_takes(x, *linears)
+
+
+def _projection_takes(x, *linears) -> bool:
+    """projection_takes() once torch.nn.Linear is known to be as torch wrote it."""
     import torch
     if type(x) is not torch.Tensor or x.dtype != torch.float16 or x.device.type != "cuda" or not x.is_contiguous():
         return False
@@ -489,15 +477,15 @@ def projection_takes(x, *linears) -> bool:
     grad = torch.is_grad_enabled()
     # whatever else may stand between a module and its product: hooks, subclasses, patched forwards, modes
     if grad and x.requires_grad or torch.is_autocast_enabled() or not plain_call() or \
-            torch.nn.modules.module._has_any_global_hook() or not are_unpatched(torch.nn.Linear):
+            torch.nn.modules.module._has_any_global_hook():
         return False
-    device = x.device
+    device, Linear, Parameter, half = x.device, torch.nn.Linear, torch.nn.Parameter, torch.float16
     for m in linears:
-        if not is_bare(m, torch.nn.Linear):
+        if not is_bare(m, Linear):
             return False
         parameters = m.__dict__["_parameters"]
         w = parameters.get("weight")
-        if type(w) is not torch.nn.Parameter or parameters.get("bias", w) is not None or w.dtype != torch.float16 or \
+        if type(w) is not Parameter or parameters.get("bias", w) is not None or w.dtype is not half or \
                 w.device != device or w.dim() != 2 or w.shape[1] != n_in or not w.is_contiguous() or \
                 w.data_ptr() % 16 or (grad and w.requires_grad):
             return False
@@ -534,9 +522,13 @@ def _check_projection(x, *weights) -> None:
         _check_weight(w, n_in, x.device)
 
 
-def _check_operand(t, device) -> None:
+def _is_operand(t, device) -> bool:
     import torch
-    if t.dtype != torch.float16 or t.device != device or not t.is_contiguous() or t.data_ptr() % 16:
+    return t.dtype == torch.float16 and t.device == device and t.is_contiguous() and t.data_ptr() % 16 == 0
+
+
+def _check_operand(t, device) -> None:
+    if not _is_operand(t, device):
         raise RuntimeError("projection: rows and weights must be contiguous, 16-byte aligned fp16 tensors on one GPU")
 
 
@@ -1013,11 +1005,10 @@ class Attention:
         return self._layer_decode(tokens, x, wq, wk, wv, wo, cos_sin_cache, positions)
 
     def _layer_decode(self, tokens, x, wq, wk, wv, wo, cos_sin_cache, positions):
-        """layer_decode() of rows and weights that projection_takes has accepted."""
+        """layer_decode() of rows and weights that projection_takes has accepted.  (The native call compares the number
+        of tokens with the tree's sequences.)"""
         import torch
         n = len(tokens)
-        if self.tree.n_seqs != n:
-            raise RuntimeError("num of seqs is not equal to num of tokens")
         n_in, width = x.shape[-1], self.n_heads * 128
         if self.d_head != 128 or x.device != self.device or x.numel() != n * n_in or wq.size(0) != width or \
                 wk.size(0) != width or wv.size(0) != width or wo.size(1) != width:
@@ -1099,15 +1090,11 @@ class Attention:
         return self.key_storage.view(shape), self.value_storage.view(shape)
 
 
+_STEPS = ("append_token_rotary", "forward", "reserve", "refresh_kernel_context")      # of a decode pass
+_STEP_FUNCTIONS = tuple(getattr(Attention, name) for name in _STEPS)
+
+
 def is_plain_cache(cache) -> bool:
     """An `Attention` of this module whose steps of a decode pass nobody has replaced, on the class or the object."""
-    if type(cache) is not Attention:
-        return False
-    own, here = cache.__dict__, globals()
-    try:
-        for name in ("append_token_rotary", "forward", "reserve", "refresh_kernel_context"):
-            if name in own or getattr(Attention, name).__globals__ is not here:
-                return False
-    except AttributeError:
-        return False
-    return True
+    return type(cache) is Attention and cache.__dict__.keys().isdisjoint(_STEPS) and _STEP_FUNCTIONS == (
+        Attention.append_token_rotary, Attention.forward, Attention.reserve, Attention.refresh_kernel_context)

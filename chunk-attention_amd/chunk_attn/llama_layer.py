@@ -17,7 +17,7 @@ from typing import List, Sequence
 import torch
 from torch import nn
 
-from . import capi
+from . import capi, stock
 
 
 class RotaryEmbedding(nn.Module):
@@ -37,6 +37,9 @@ class RotaryEmbedding(nn.Module):
     def forward(self, positions: torch.Tensor, query: torch.Tensor, key: torch.Tensor):
         capi.rotary_embedding(positions, query, key, self.head_size, self.cos_sin_cache, self.is_neox_style)
         return query, key
+
+
+_ROTARY_FORWARD = RotaryEmbedding.forward
 
 
 class LlamaChunkAttention(nn.Module):
@@ -66,19 +69,18 @@ class LlamaChunkAttention(nn.Module):
         batch row i to be cache sequence i."""
         batch, n_tokens, d_hidden = hidden_states.shape
         projections = (self.q_proj, self.k_proj, self.v_proj)
-        few_rows = folded = False       # q, k and v by the framework's own kernel; a decode pass as one native call
-        # (caches of other classes have append_token_rotary only)
-        plain_cache = not prefill and capi.is_plain_cache(kv_cache)
-        if self.head_dim == 128 and capi.projection_pays(batch * n_tokens, d_hidden, d_hidden) and self._plain_rotary():
-            folded = plain_cache and capi.projection_takes(hidden_states, *projections, self.o_proj)
-            few_rows = folded or capi.projection_takes(hidden_states, *projections)
+        own_output = few_rows = False                  # which projections the framework's own kernel computes
+        if self.head_dim == 128 and capi.projection_pays(batch * n_tokens, d_hidden, d_hidden) and \
+                self._plain_rotary() and stock.linear_is_stock():
+            own_output = capi._projection_takes(hidden_states, *projections, self.o_proj)
+            few_rows = own_output or capi._projection_takes(hidden_states, *projections)
         if few_rows:
             weights = [p.weight for p in projections]
-        if few_rows and plain_cache:
+        if few_rows and not prefill and capi.is_plain_cache(kv_cache):      # other caches have append_token_rotary only
             assert n_tokens == 1
             step = ([s[-1] for s in seqs], hidden_states, *weights)
             rotary = (self.rotary_emb.cos_sin_cache, position_ids.reshape(batch).contiguous())
-            if folded:
+            if own_output:
                 return kv_cache._layer_decode(*step, self.o_proj.weight, *rotary).view(batch, 1, -1)
             q3 = kv_cache._project_append_rotary(*step, *rotary)
             return self._output(kv_cache.forward(q3).view(batch, 1, d_hidden), kv_cache, False)
@@ -94,7 +96,7 @@ class LlamaChunkAttention(nn.Module):
             shape = (batch, n_tokens, self.num_heads, self.head_dim)
             q4, k4, v4 = q.view(shape), k.view(shape), v.view(shape)
             if hidden_states.dtype == torch.float16 and capi.causal_attention_takes(q4, k4, v4):
-                attn_output = capi.causal_attention(q4, k4, v4).view(batch, n_tokens, d_hidden)
+                attn_output = capi._causal_attention(q4, k4, v4).view(batch, n_tokens, d_hidden)
             else:
                 # what the kernel does not take (a gradient is wanted, another head size): plain fp32 torch math
                 qh, kh, vh = (t.transpose(1, 2).float() for t in (q4, k4, v4))
@@ -111,17 +113,23 @@ class LlamaChunkAttention(nn.Module):
             kv_cache.append_token_rotary([s[-1] for s in seqs], q3, k3, v3, self.rotary_emb.cos_sin_cache,
                                          self.rotary_emb.is_neox_style, position_ids.reshape(batch).contiguous())
             attn_output = kv_cache.forward(q3).view(batch, 1, d_hidden)
-        return self._output(attn_output, kv_cache, few_rows)
+        # (a cache of another class may return anything)
+        return self._output(attn_output, kv_cache, own_output and capi._is_operand(attn_output, hidden_states.device))
 
     def _plain_rotary(self) -> bool:
         """The rotary module is the one this layer was built with, over whole heads, and nothing hangs on it."""
         r = self.rotary_emb
-        return capi.is_bare(r, RotaryEmbedding) and capi.are_unpatched(RotaryEmbedding) and r.is_neox_style and r.rotary_dim == r.head_size == self.head_dim
+        return capi.is_bare(r, RotaryEmbedding) and stock.is_stock(RotaryEmbedding, _ROTARY_FORWARD) and r.is_neox_style and r.rotary_dim == r.head_size == self.head_dim
 
-    def _output(self, attn_output: torch.Tensor, kv_cache: capi.Attention, few_rows: bool) -> torch.Tensor:
-        # what the attention gave is looked at itself: a cache of another class may return anything
-        own = few_rows and capi.projection_takes(attn_output, self.o_proj)
+    def _output(self, attn_output: torch.Tensor, kv_cache: capi.Attention, own: bool) -> torch.Tensor:
         output = capi._linear(attn_output, self.o_proj.weight) if own else self.o_proj(attn_output)
         kv_cache.reserve()
         kv_cache.refresh_kernel_context(force=False)
         return output
+
+
+_LAYER_FORWARD = LlamaChunkAttention.forward
+
+
+def layer_is_stock() -> bool:
+    return stock.is_stock(LlamaChunkAttention, _LAYER_FORWARD)

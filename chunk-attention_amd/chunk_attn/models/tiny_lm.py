@@ -12,8 +12,8 @@ from typing import List
 import torch
 from torch import nn
 
-from .. import capi
-from ..llama_layer import LlamaChunkAttention
+from .. import capi, stock
+from ..llama_layer import LlamaChunkAttention, layer_is_stock
 from .sequence import Sequence
 
 
@@ -28,6 +28,9 @@ class RMSNorm(nn.Module):
         out = torch.empty_like(x)
         capi.rms_norm(out, x, self.weight, self.eps)
         return out
+
+
+_NORM_FORWARD = RMSNorm.forward
 
 
 def _pins(device: torch.device) -> bool:
@@ -102,7 +105,8 @@ class AttentionOnlyLM(nn.Module):
                 hidden = hidden + out
                 normed = norm(hidden)
         last = self.norm(hidden[:, -1]) if normed is None else normed
-        if capi.projection_pays(len(seqs), self.hidden_size, self.vocab_size) and capi.projection_takes(last, self.lm_head):
+        if capi.projection_pays(len(seqs), self.hidden_size, self.vocab_size) and stock.linear_is_stock() and \
+                capi._projection_takes(last, self.lm_head):
             return capi._linear(last, self.lm_head.weight)
         return self.lm_head(last)
 
@@ -111,11 +115,11 @@ class AttentionOnlyLM(nn.Module):
         (a gradient, a hook, a mode that sees them, a forward-mode tangent of them), and the norms must be the plain
         ones."""
         return capi.plain_call() and not torch.is_grad_enabled() and \
-            capi.are_unpatched(nn.Embedding, nn.Linear, LlamaChunkAttention, RMSNorm) and \
-            capi.is_bare(self.embed_tokens, nn.Embedding) and \
-            all(capi.is_bare(m, LlamaChunkAttention) and capi.is_bare(m.o_proj, nn.Linear) for m in self.layers) and \
-            all(capi.is_bare(m, RMSNorm) for m in self.input_norms) and capi.is_bare(self.norm, RMSNorm) and \
-            not torch.nn.modules.module._has_any_global_hook()
+            stock.embedding_is_stock() and stock.linear_is_stock() and layer_is_stock() and \
+            stock.is_stock(RMSNorm, _NORM_FORWARD) and \
+            not torch.nn.modules.module._has_any_global_hook() and capi.is_bare(self.embed_tokens, nn.Embedding) and \
+            all([capi.is_bare(m, LlamaChunkAttention) and capi.is_bare(m.o_proj, nn.Linear) for m in self.layers]) and \
+            all([capi.is_bare(m, RMSNorm) for m in (*self.input_norms, self.norm)])
 
     @torch.no_grad()
     def forward(self, seqs: List[Sequence], kv_caches, prefill: bool) -> List[int]:

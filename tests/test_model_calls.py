@@ -132,29 +132,34 @@ def test_no_tangent_of_an_overwritten_tensor_reaches_the_logits(fused):
 
 
 def test_replaced_classes_and_functions_are_seen(monkeypatch, fused):
+    from chunk_attn import llama_layer, stock
     from chunk_attn.llama_layer import LlamaChunkAttention, RotaryEmbedding
-    nn = torch.nn
-    classes = (nn.Linear, nn.Embedding, RotaryEmbedding, LlamaChunkAttention, tiny_lm.RMSNorm)
+    nn, F = torch.nn, torch.nn.functional
+    checks = {nn.Linear: stock.linear_is_stock, nn.Embedding: stock.embedding_is_stock, LlamaChunkAttention: llama_layer.layer_is_stock,
+              RotaryEmbedding: lambda: stock.is_stock(RotaryEmbedding, llama_layer._ROTARY_FORWARD),
+              tiny_lm.RMSNorm: lambda: stock.is_stock(tiny_lm.RMSNorm, tiny_lm._NORM_FORWARD)}
     m = model()
 
-    def joined():
+    def seen():
+        """The classes found changed; whether the model still overwrites."""
         with torch.no_grad():
-            return m._adds_in_norms()
+            return [cls for cls, check in checks.items() if not check()], m._adds_in_norms()
 
-    assert all(map(capi.are_unpatched, classes)) and joined()
-    for cls in classes:
+    assert seen() == ([], True)
+    for cls in checks:
         with monkeypatch.context() as mp:
             forward = cls.forward
             mp.setattr(cls, "forward", lambda *a: forward(*a))
-            assert not capi.are_unpatched(cls) and joined() == (cls is RotaryEmbedding)
-    for owner, name in ((nn.Module, "__call__"), (nn.Module, "_call_impl")):
+            assert seen() == ([cls], cls is RotaryEmbedding)
+    for name in ("__call__", "_call_impl"):
         with monkeypatch.context() as mp:
-            mp.setattr(owner, name, lambda *a, **k: None)
-            assert not any(map(capi.are_unpatched, classes))
+            mp.setattr(nn.Module, name, lambda *a, **k: None)
+            assert seen() == (list(checks), False)
     for name, cls in (("linear", nn.Linear), ("embedding", nn.Embedding)):
         with monkeypatch.context() as mp:
-            mp.setattr(nn.functional, name, lambda *a: None)
-            assert [capi.are_unpatched(c) for c in classes] == [c is not cls for c in classes] and not joined()
+            mp.setattr(F, name, lambda *a: None)
+            assert seen() == ([cls], False)
+    assert stock._at_home(seen, nn) is None and stock._at_home(F.embedding, F) is F.embedding
     cache = object.__new__(capi.Attention)
     assert capi.is_plain_cache(cache) and not capi.is_plain_cache(CountingCache())
     with monkeypatch.context() as mp:

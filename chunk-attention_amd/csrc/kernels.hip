@@ -282,12 +282,14 @@ constexpr int VPITCH = D + 16;  // halves per LDS row of a V block: 288 B puts t
                                 // four consecutive token rows into four different bank groups,
                                 // and rows stay 16-byte aligned for whole-vector writes
 constexpr int OPITCH = D + 4;  // floats per row of the cross-wave accumulation buffer
-// MBT: 16-row blocks per shared item (2: items of up to 32 sequences, 1: up to 16)
-template <int MBT>
+// MBT: 16-row blocks per shared item (2: items of up to 32 sequences, 1: up to 16); OB: buffers for the waves' sums,
+// one for all (added up in turn) or one for each
+template <int MBT, int OB>
 struct SharedPathLds {
+    static_assert(OB == 1 || OB == NW, "one buffer for all waves or one for each");
     union {
         half_t v[NW][16 * VPITCH];
-        float o[NW][16 * MBT * OPITCH];   // every wave's sums, when all are done with their V blocks
+        float o[OB][16 * MBT * OPITCH];   // the sums, when all waves are done with their V blocks
     };
     float m[NW][16 * MBT];
     float l[NW][16 * MBT];
@@ -322,16 +324,17 @@ constexpr int kMixFull = 0, kMixStream = 1, kMixNarrow = 2;
 constexpr int kNarrowLookahead = 1;  // blocks on their way in the narrow form (three workgroups per CU: 168 registers)
 template <int MIX> union DecodeLds;
 template <> union __attribute__((aligned(16))) DecodeLds<kMixFull> {
-    SharedPathLds<2> sh;
-    SharedPathLds<1> sh1;
+    SharedPathLds<2, 1> sh;
+    SharedPathLds<1, 1> sh1;
     StreamPathLds st;
     WidePathLds wd;
 };
+static_assert(sizeof(DecodeLds<kMixFull>) <= 38 << 10, "the tiles of the wide path decide what a full launch's workgroups hold");
 template <> union __attribute__((aligned(16))) DecodeLds<kMixStream> {
     StreamPathLds st;
 };
 template <> union __attribute__((aligned(16))) DecodeLds<kMixNarrow> {
-    SharedPathLds<1> sh;
+    SharedPathLds<1, NW> sh;
     StreamPathLds st;
 };
 
@@ -670,9 +673,9 @@ __device__ __forceinline__ void stream_path(const DecodeArgs& A, const WorkItem*
 //   tokens), so probabilities never leave registers.  V^T comes from a wave-private LDS copy
 //   of the 16 x 128 V block through the LDS transpose read (lds_read_tr).
 // ---------------------------------------------------------------------------------------
-template <int C, int MBT, int LA>
+template <int C, int MBT, int LA, int OB>
 __device__ __forceinline__ void shared_path(const DecodeArgs& A, const WorkItem* __restrict__ gi,
-                                            int h, SharedPathLds<MBT>& sm) {
+                                            int h, SharedPathLds<MBT, OB>& sm) {
     constexpr int MB = MBT;  // 16-row blocks of the item
     constexpr int R = LA + 1;  // register sets
     WorkItem it;
@@ -854,18 +857,26 @@ __device__ __forceinline__ void shared_path(const DecodeArgs& A, const WorkItem*
 #pragma unroll
         for (int db = 0; db < 8; db++) oacc[mb][db] *= f;
     }
-    // Every wave leaves its sums in a buffer of its own, and the threads that write the partial rows add
-    // the four up: one barrier (adding in turn into one buffer took four; 4 sequences x 12 heads, 512 shared
-    // tokens 7.79 -> 7.15 us a forward).
+    // Small launches (the narrow form) are as long as their longest chain: every wave leaves its sums in a buffer of
+    // its own, and the threads that write the partial rows add the four up, one barrier instead of four (4
+    // sequences x 12 heads, 512 shared tokens 7.79 -> 7.15 us a forward).  In the full form the waves add in turn into
+    // one buffer: four would raise every workgroup's LDS from 37 to 69 KB, and 64 sequences in two levels
+    // take 50.2 us with them, 50.2 with two buffers in two rounds, 49.8 in turn.
 #pragma unroll
-    for (int mb = 0; mb < MB; mb++) {
+    for (int k = 0; k < (OB == 1 ? NW : 1); k++) {
+        if (OB == NW || w == k) {
 #pragma unroll
-        for (int db = 0; db < 8; db++) {
-            // lane owns dims 16*db + 4*g .. +3 of sequence row mb*16 + i
-            *reinterpret_cast<f4*>(&sm.o[w][(mb * 16 + i) * OPITCH + 16 * db + 4 * g]) = oacc[mb][db];
+            for (int mb = 0; mb < MB; mb++) {
+#pragma unroll
+                for (int db = 0; db < 8; db++) {
+                    // lane owns dims 16*db + 4*g .. +3 of sequence row mb*16 + i
+                    f4* dst = reinterpret_cast<f4*>(&sm.o[OB == 1 ? 0 : w][(mb * 16 + i) * OPITCH + 16 * db + 4 * g]);
+                    *dst = (k == 0) ? oacc[mb][db] : (*dst + oacc[mb][db]);
+                }
+            }
         }
+        __syncthreads();
     }
-    __syncthreads();
 
     // ---- write the partial rows ------------------------------------------------------------
     for (int idx = tid; idx < it.n_rows * (D / 4); idx += WG) {
@@ -873,7 +884,7 @@ __device__ __forceinline__ void shared_path(const DecodeArgs& A, const WorkItem*
         float* dst = A.part + (size_t(sm.row[row]) * H + h) * PART_STRIDE + 4 + 4 * c4;
         f4 v = *reinterpret_cast<const f4*>(&sm.o[0][row * OPITCH + 4 * c4]);
 #pragma unroll
-        for (int k = 1; k < NW; k++) v += *reinterpret_cast<const f4*>(&sm.o[k][row * OPITCH + 4 * c4]);
+        for (int k = 1; k < OB; k++) v += *reinterpret_cast<const f4*>(&sm.o[k][row * OPITCH + 4 * c4]);
         part_store2(dst, v[0], v[1], coh);
         part_store2(dst + 2, v[2], v[3], coh);
     }
@@ -1273,12 +1284,12 @@ __global__ __launch_bounds__(WG, (MIX == kMixFull || C == 128 || STEP != kForwar
                         wide_path<C, 2>(A, gi, h, lds.wd);
                     }
                 } else if (gi->n_rows <= 16) {
-                    shared_path<C, 1, 3>(A, gi, h, lds.sh1);
+                    shared_path<C, 1, 3, 1>(A, gi, h, lds.sh1);
                 } else {
-                    shared_path<C, 2, 1>(A, gi, h, lds.sh);
+                    shared_path<C, 2, 1, 1>(A, gi, h, lds.sh);
                 }
             } else {
-                shared_path<C, 1, kNarrowLookahead>(A, gi, h, lds.sh);
+                shared_path<C, 1, kNarrowLookahead, NW>(A, gi, h, lds.sh);
             }
         }
     } else {

@@ -239,12 +239,16 @@ void build_plan(const ChunkRow* rows, int n_rows, int n_seqs, int chunk_size,
         all_tokens += int64_t(rows[i].n_tokens) * (is_shared(rows[i]) ? 1 : rows[i].seq_end - rows[i].seq_begin);
     }
     const double step_us = double(all_tokens) * 4.0 * std::max(params.n_heads, 1) * 128.0 / 6.4e6;
+    // segments of a run: nearest, not ceiling; but never more chunks in a segment than an item holds
+    auto segs_of = [&](const Run& run, int seg_chunks) {
+        return std::max({ 1, (run.count + seg_chunks / 2) / seg_chunks, ceil_div(run.count, kMaxItemChunks) });
+    };
+    auto seg_of_tiles = [&](int n_tiles) { return std::clamp(n_tiles * 64 / chunk_size, 1, kMaxItemChunks); };
     auto shared_wgs_with = [&](int n_tiles) {   // shared workgroups if every run used n_tiles per segment
         int64_t wgs = 0;
         for (const Run& run : runs) {
             const int n = rows[run.first_row].seq_end - rows[run.first_row].seq_begin;
-            const int seg = std::clamp(n_tiles * 64 / chunk_size, 1, kMaxItemChunks);
-            const int n_segs = std::max({ 1, (run.count + seg / 2) / seg, ceil_div(run.count, kMaxItemChunks) });
+            const int n_segs = segs_of(run, seg_of_tiles(n_tiles));
             // a wide workgroup counts for two: it keeps a compute unit's vector and matrix units
             // busy by itself, and a second one beside it only makes both take twice as long
             const bool wide = run_wide(run);
@@ -270,9 +274,9 @@ void build_plan(const ChunkRow* rows, int n_rows, int n_seqs, int chunk_size,
         int longest = 0, widest = 0;
         for (const Run& run : runs) {
             const ChunkRow& r0 = rows[run.first_row];
-            const int seg = std::max(2 * 64 / chunk_size, 1);
+            const int n_segs = segs_of(run, seg_of_tiles(2));
             for (int s = r0.seq_begin; s < r0.seq_end; s++) {
-                path_segs[s] += ceil_div(run.count, seg);
+                path_segs[s] += n_segs;
                 longest = std::max(longest, path_segs[s]);
             }
             widest = std::max(widest, r0.seq_end - r0.seq_begin);
@@ -287,17 +291,12 @@ void build_plan(const ChunkRow* rows, int n_rows, int n_seqs, int chunk_size,
     p.hints.built_tokens = params.keep ? params.keep->built_tokens : all_tokens;
     auto seg_chunks_for = [&](bool wide) {
         if (params.shared_seg_chunks > 0) return std::min(params.shared_seg_chunks, kMaxItemChunks);
-        const int n_tiles = std::min(base_tiles, wide ? 64 : 32);  // 64-token tiles
-        return std::clamp(n_tiles * 64 / chunk_size, 1, kMaxItemChunks);
+        return seg_of_tiles(std::min(base_tiles, wide ? 64 : 32));  // 64-token tiles
     };
 
     std::vector<int32_t> n_parts(n_seqs, 0);  // partial rows handed out per sequence so far
-    // segments per run: nearest, not ceiling; but never more chunks in a segment than an item holds
     std::vector<int> run_segs(runs.size());
-    for (size_t r = 0; r < runs.size(); r++) {
-        const int seg = seg_chunks_for(run_wide(runs[r]));
-        run_segs[r] = std::max({ 1, (runs[r].count + seg / 2) / seg, ceil_div(runs[r].count, kMaxItemChunks) });
-    }
+    for (size_t r = 0; r < runs.size(); r++) run_segs[r] = segs_of(runs[r], seg_chunks_for(run_wide(runs[r])));
     // Runs of different widths (a root shared by everyone, groups below it): a tile costs more
     // with more sequences on it (relative, alone: 1.0 up to 16 rows, 1.4 up to 32, 2.0 in the wide
     // form), and the workgroups with the longest chains keep their slots from the streaming

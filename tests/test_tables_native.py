@@ -420,3 +420,11 @@ def test_tiny_launches_cut_shared_runs_into_two_tiles(n_seqs, heads, root, want)
     for s in range(n_seqs):
         covering = items[(items[:, 0] <= s) & (s < items[:, 0] + items[:, 1])]
         assert sorted(covering[:, 4]) == list(range(want)) and covering[:, 3].sum() == root // 64
+
+
+def test_tiny_launches_count_the_segments_that_are_cut():
+    """Chunks of 32: 17 make four segments of two tiles (the nearest number), which is not more than four, though a
+    fifth begins."""
+    rows = [(i, 32, 0, 16) for i in range(17)] + [(100 + s, 20, s, s + 1) for s in range(16)]
+    plan = capi.build_tables(np.array(rows, np.int32), 16, 32, n_heads=16, n_cus=256)["plan"]
+    assert len(set(plan["shared_items"][:, 4])) == 4

@@ -188,6 +188,7 @@ ca::LaunchArgs launch_args(const ca_ctx* c, const void* q, void* out) {
     a.H = c->H;
     a.C = c->C;
     a.d = c->d;
+    a.n_cus = c->n_cus;
     a.scale_log2 = 1.4426950408889634f / std::sqrt(static_cast<float>(c->d));
     a.stream_per_wave = c->plan.stream_per_wave;
     a.shared_narrow = c->plan.shared_narrow;

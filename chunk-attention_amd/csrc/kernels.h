@@ -26,6 +26,7 @@ struct LaunchArgs {
     int H = 0;
     int C = 0;
     int d = 128;
+    int n_cus = 256;         // compute units of the device
     float scale_log2 = 0.f;  // log2(e) / sqrt(d_head)
     // Read the per-sequence (private) chunks with the non-temporal hint.  Worth it when one
     // forward streams more than the last-level cache holds: the data cannot be found there

@@ -319,13 +319,20 @@ struct WidePathLds {
 // (two workgroups per compute unit) and run three per compute unit instead:
 //   kMixFull    every path;
 //   kMixStream  stream items only (nothing shared, or partition 2);
-//   kMixNarrow  stream items and shared items of at most 16 sequences, none wide.
-constexpr int kMixFull = 0, kMixStream = 1, kMixNarrow = 2;
+//   kMixNarrow  stream items and shared items of at most 16 sequences, none wide;
+//   kMixFullSmall  every path, for launches whose workgroups all run at once: more LDS for shorter chains.
+constexpr int kMixFull = 0, kMixStream = 1, kMixNarrow = 2, kMixFullSmall = 3;
 constexpr int kNarrowLookahead = 1;  // blocks on their way in the narrow form (three workgroups per CU: 168 registers)
 template <int MIX> union DecodeLds;
 template <> union __attribute__((aligned(16))) DecodeLds<kMixFull> {
     SharedPathLds<2, 1> sh;
     SharedPathLds<1, 1> sh1;
+    StreamPathLds st;
+    WidePathLds wd;
+};
+template <> union __attribute__((aligned(16))) DecodeLds<kMixFullSmall> {
+    SharedPathLds<2, NW> sh;
+    SharedPathLds<1, NW> sh1;
     StreamPathLds st;
     WidePathLds wd;
 };
@@ -857,11 +864,12 @@ __device__ __forceinline__ void shared_path(const DecodeArgs& A, const WorkItem*
 #pragma unroll
         for (int db = 0; db < 8; db++) oacc[mb][db] *= f;
     }
-    // Small launches (the narrow form) are as long as their longest chain: every wave leaves its sums in a buffer of
-    // its own, and the threads that write the partial rows add the four up, one barrier instead of four (4
-    // sequences x 12 heads, 512 shared tokens 7.79 -> 7.15 us a forward).  In the full form the waves add in turn into
-    // one buffer: four would raise every workgroup's LDS from 37 to 69 KB, and 64 sequences in two levels
-    // take 50.2 us with them, 50.2 with two buffers in two rounds, 49.8 in turn.
+    // Small launches are as long as their longest chain: every wave leaves its sums in a buffer of its own, and the
+    // threads that write the partial rows add the four up, one barrier instead of four (4 sequences x 12 heads, 512
+    // shared tokens 7.79 -> 7.15 us a forward; 20 x 12 heads, 576 shared tokens in chunks of 32, 10.9 -> 10.0).  In
+    // the full form's other launches the waves add in turn into one buffer: four would raise every workgroup's LDS
+    // from 37 to 69 KB, and 64 sequences in two levels take 50.2 us with them, 50.2 with two buffers in two
+    // rounds, 49.8 in turn.
 #pragma unroll
     for (int k = 0; k < (OB == 1 ? NW : 1); k++) {
         if (OB == NW || w == k) {
@@ -1251,7 +1259,7 @@ __device__ __forceinline__ int xcd_unit(int b, int n) {
 }
 
 template <int C, int MIX, int STEP>
-__global__ __launch_bounds__(WG, (MIX == kMixFull || C == 128 || STEP != kForward) ? 2 : 3) void decode_kernel(
+__global__ __launch_bounds__(WG, (MIX == kMixFull || MIX == kMixFullSmall || C == 128 || STEP != kForward) ? 2 : 3) void decode_kernel(
     const WorkItem* stream_items, const WorkItem* shared_items, const half_t* kpool, const half_t* vpool,
     const half_t* q, int n_shared_wgs, int H, int delta_tokens, int flags, float scale_log2,
     int n_stream_items, const DecodeRest rest) {
@@ -1275,7 +1283,8 @@ __global__ __launch_bounds__(WG, (MIX == kMixFull || C == 128 || STEP != kForwar
             const int n_items = A.n_shared_wgs / A.H;
             const int h = unit / n_items;
             const WorkItem* gi = A.shared_items + (unit - h * n_items);
-            if constexpr (MIX == kMixFull) {
+            if constexpr (MIX == kMixFull || MIX == kMixFullSmall) {
+                constexpr int OB = MIX == kMixFull ? 1 : NW;
                 if (gi->flags & kItemWide) {
                     // up to 64 sequences: 16 rows per wave keep all four waves busy
                     if (gi->n_rows <= 64) {
@@ -1284,9 +1293,9 @@ __global__ __launch_bounds__(WG, (MIX == kMixFull || C == 128 || STEP != kForwar
                         wide_path<C, 2>(A, gi, h, lds.wd);
                     }
                 } else if (gi->n_rows <= 16) {
-                    shared_path<C, 1, 3, 1>(A, gi, h, lds.sh1);
+                    shared_path<C, 1, 3, OB>(A, gi, h, lds.sh1);
                 } else {
-                    shared_path<C, 2, 1, 1>(A, gi, h, lds.sh);
+                    shared_path<C, 2, 1, OB>(A, gi, h, lds.sh);
                 }
             } else {
                 shared_path<C, 1, kNarrowLookahead, NW>(A, gi, h, lds.sh);
@@ -1579,7 +1588,9 @@ int launch_decode(const LaunchArgs& a, int n_shared_items, int n_stream_items, b
     const int flags = (d.fuse_merge ? kFlagFuseMerge : 0) | (d.stream_per_wave ? kFlagPerWave : 0) |
                       (d.stream_nt ? kFlagStreamNt : 0);
     // the lightest form of the kernel that holds every path this launch takes
-    const int mix = (n_shared_items == 0) ? kMixStream : (a.shared_narrow ? kMixNarrow : kMixFull);
+    // (two workgroups of the full forms fit a compute unit; up to a quarter more than that still gain: 48 sequences x
+    // 12 heads, 512 shared tokens, 624 workgroups 12.65 -> 12.35 us, but 24 x 32 heads, 1024, 832 workgroups 15.0 -> 15.3)
+    const int mix = (n_shared_items == 0) ? kMixStream : a.shared_narrow ? kMixNarrow : 2 * wgs <= 5 * a.n_cus ? kMixFullSmall : kMixFull;
 #define CA_DECODE_LAUNCH(CS, MIX, STEP)                                                                    \
     hipLaunchKernelGGL((decode_kernel<CS, MIX, STEP>), grid, block, 0, st, d.stream_items, d.shared_items, \
                        d.kpool, d.vpool, d.q, d.n_shared_wgs, d.H, d.delta_tokens, flags, d.scale_log2,     \
@@ -1593,6 +1604,7 @@ int launch_decode(const LaunchArgs& a, int n_shared_items, int n_stream_items, b
     do {                                                                  \
         if (mix == kMixStream) CA_DECODE_STEP(CS, kMixStream);            \
         else if (mix == kMixNarrow) CA_DECODE_STEP(CS, kMixNarrow);       \
+        else if (mix == kMixFullSmall) CA_DECODE_STEP(CS, kMixFullSmall); \
         else CA_DECODE_STEP(CS, kMixFull);                                \
     } while (0)
     switch (a.C) {

@@ -85,3 +85,25 @@ def test_head_counts_that_are_no_multiple_of_eight(H):
             out = attn.forward(tq, partition)
             assert attn.ctx.plan_info().n_shared_items > 0
             assert_close(out, want)
+
+
+@pytest.mark.parametrize("c", [32, 64, 128])
+@pytest.mark.parametrize("H,small", [(1, True), (24, False)])
+def test_small_and_large_launches_of_wide_mixes(c, H, small):
+    """Launches with items of more than 16 sequences come in two forms, up to and beyond two and a half workgroups a
+    compute unit, which differ in how an item's four waves are added up."""
+    rng = np.random.default_rng(c + H)
+    attn, n, _ = build(c, rng, H)
+    q = rng.standard_normal((n, H, 128)).astype(np.float16)
+    rows, kpool, vpool = host_state(attn)
+    want = textbook_attention(q.astype(np.float32), rows.tolist(), kpool, vpool)
+    line = 5 * torch.cuda.get_device_properties(0).multi_processor_count // 2
+    for schedule in (0, 1):
+        attn.ctx.set_schedule(schedule)
+        attn.refresh_kernel_context()
+        assert_close(attn.forward(to_dev(q)), want)
+        info = attn.ctx.plan_info()
+        if small:
+            assert (info.n_shared_items + info.n_stream_items) * H <= line
+        else:   # (four stream items a workgroup at most)
+            assert (info.n_shared_items + info.n_stream_items // 4) * H > line

@@ -117,9 +117,14 @@ class LlamaChunkAttention(nn.Module):
         return self._output(attn_output, kv_cache, own_output and capi._is_operand(attn_output, hidden_states.device))
 
     def _plain_rotary(self) -> bool:
-        """The rotary module is the one this layer was built with, over whole heads, and nothing hangs on it."""
+        """The rotary module is the one this layer was built with, over whole heads, nothing hangs on it, and its table
+        is one that the projection kernels read (the operator takes narrower ones and any alignment)."""
         r = self.rotary_emb
-        return capi.is_bare(r, RotaryEmbedding) and stock.is_stock(RotaryEmbedding, _ROTARY_FORWARD) and r.is_neox_style and r.rotary_dim == r.head_size == self.head_dim
+        if not (capi.is_bare(r, RotaryEmbedding) and stock.is_stock(RotaryEmbedding, _ROTARY_FORWARD) and r.is_neox_style and
+                r.rotary_dim == r.head_size == self.head_dim):
+            return False
+        table = r.cos_sin_cache
+        return table.dim() == 2 and table.shape[1] == self.head_dim and table.data_ptr() % 16 == 0
 
     def _output(self, attn_output: torch.Tensor, kv_cache: capi.Attention, own: bool) -> torch.Tensor:
         output = capi._linear(attn_output, self.o_proj.weight) if own else self.o_proj(attn_output)

@@ -169,6 +169,17 @@ def test_replaced_classes_and_functions_are_seen(monkeypatch, fused):
     assert not capi.is_plain_cache(cache)
 
 
+def test_tables_that_only_the_operator_takes():
+    """A rotary table put in by the user: narrower rows or an odd address are the operator's, not the kernels'."""
+    from chunk_attn.llama_layer import LlamaChunkAttention
+    layer = LlamaChunkAttention(256, 2, max_position_embeddings=8, device="cpu")
+    flat = torch.zeros(8 * 128 + 1, dtype=torch.float16)
+    assert layer._plain_rotary()
+    for table, plain in ((flat[:-1].view(8, 128), True), (flat[1:].view(8, 128), False), (flat[:512].view(8, 64), False)):
+        layer.rotary_emb.cos_sin_cache = table
+        assert layer._plain_rotary() == plain
+
+
 # us on one GPU (MI355X), weights from memory
 @pytest.mark.parametrize("rows,n_in,n_out,here,library,pays", [
     (2048, 128, 128, 3.1, 4.2, True), (1024, 512, 512, 5.8, 6.1, True), (252, 1024, 1024, 4.4, 8.0, True),

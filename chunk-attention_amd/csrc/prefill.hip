@@ -83,8 +83,8 @@ __device__ __forceinline__ void load_to_lds16(const char* src, half_t* dst) {
 //
 // What bounds it: matrix ops (half of them the second P.V product below) and the vector ops of the softmax are
 // about equal, and each wave's run of them is one dependent chain; what hides a chain is another wave.  TILE 32
-// holds four workgroups a compute unit (118 registers, 32 KB), 64 two.  32 heads, 2048 tokens: 68 us, 8 x 300
-// tokens 25 us; 16 heads, 8 x 1000 tokens 69 us (32 rows a wave, 64 keys a tile, two workgroups a unit: 81, 40 and
+// holds four workgroups a compute unit (118 registers, 32 KB), 64 two.  32 heads, 2048 tokens: 66 us, 8 x 300
+// tokens 22 us; 16 heads, 8 x 1000 tokens 66 us (32 rows a wave, 64 keys a tile, two workgroups a unit: 81, 40 and
 // 85).  Long runs of large ones are held back by the clock, which falls with what they draw (about 1.7 GHz).
 //
 // The probabilities are fp32; the matrix cores take fp16.  p = hi + lo with hi = fp16(p) and
@@ -283,10 +283,13 @@ int launch_causal_attention(const void* q, const void* k, const void* v, void* o
     const half_t* kh = static_cast<const half_t*>(k);
     const half_t* vh = static_cast<const half_t*>(v);
     half_t* oh = static_cast<half_t*>(out);
-    // Tiles of 32 keys let four workgroups share a compute unit; with fewer workgroups than two a unit there is
-    // nobody to share with, and half as many barriers are worth more (1000 tokens, 8 heads: 23.7 us with 64 keys
-    // a tile, 26.1 with 32; 400 x 32 heads 12.8, 13.3; 1000 x 32 heads, 512 workgroups: 29.9 with 32 keys).
-    if (n_bh * blocks >= 400) {
+    // Tiles of 32 keys let four workgroups share a compute unit, tiles of 64 two, with half as many barriers: worth
+    // more while few workgroups are left over from two a unit, the longer the prompt the more (us with 64 and 32 keys
+    // a tile, workgroups in brackets: 1004 tokens x 16 heads [256] 21.9, 24.8; 1516 x 16 [384] 33.5, 37.6; 1004 x 32
+    // [512] 23.5, 25.8; 4 x 236 x 32 [512] 9.5, 9.3; 4 x 556 x 16 [576] 15.8, 17.1; 4 x 300 x 32 [640] 12.4, 11.8;
+    // 4 x 620 x 16 [640] 17.6, 18.9; 4 x 364 x 32 [768] 15.9, 14.3; 1516 x 32 [768] 37.7, 42.0; 2028 x 32 [1024]
+    // 64.0, 61.5).
+    if (n_bh * blocks > (n_tokens < 600 ? 576 : 768)) {
         hipLaunchKernelGGL(causal_attention_kernel<32>, grid, block, 0, st, qh, kh, vh, oh, n_tokens, n_heads, int(n_bh),
                            int(blocks), scale_log2);
     } else {

@@ -1,5 +1,5 @@
 """Causal attention of whole prompts against fp64 on the CPU, at the sizes where the kernel's tiles end:
-64-key tiles, from 400 workgroups of 64 rows on 32-key tiles, 16 rows per wave."""
+64-key tiles, in launches of more workgroups of 64 rows 32-key tiles, 16 rows per wave."""
 import math
 
 import pytest
@@ -29,8 +29,17 @@ def test_causal_attention_at_tile_edges(batch, n, heads):
     q *= 2
     out = capi.causal_attention(q.cuda(), k.cuda(), v.cuda()).cpu().double()
     want = reference(q, k, v)
-    # the output's own rounding is 2^-12 of it at most; sums of n fp32 terms add less than 2^-16 of max |v| < 6
+    # the output's own rounding is 2^-11 of it at most; sums of n fp32 terms add less than 2^-16 of max |v| < 6
     assert ((out - want).abs() <= want.abs() * 2.0 ** -11 + 6 * 2.0 ** -16).all()
+
+
+@pytest.mark.parametrize("batch,n,heads", [
+    (37, 31, 16), (52, 64, 12), (26, 65, 12), (13, 97, 24), (20, 129, 10), (5, 193, 42), (13, 513, 8), (2, 600, 39), (1, 1633, 30),
+    (1, 577, 64), (9, 64, 64), (3, 601, 25)])
+def test_causal_attention_of_many_workgroups(batch, n, heads):
+    """32-key tiles: from 577 workgroups on, from 769 for prompts of 600 tokens and more (the last two lie before
+    the lines)."""
+    test_causal_attention_at_tile_edges(batch, n, heads)
 
 
 def test_what_a_row_must_not_see_and_extreme_scores():

@@ -78,3 +78,20 @@ def test_later_rows_of_a_wave_change_nothing_in_earlier_ones(batch, n, heads):
     q[:, 150:] *= 8                                                       # rows 150 .. 159 share a wave with 144 .. 149
     second = capi.causal_attention(q, k, v)
     assert torch.equal(first[:, :150], second[:, :150]) and not torch.equal(first[:, 150:], second[:, 150:])
+
+
+@pytest.mark.parametrize("batch,n,heads", [(1, 200, 8), (8, 300, 16)])       # 64-key tiles, 32-key tiles
+def test_infinite_and_undefined_scores(batch, n, heads):
+    """A key of minus infinity is not attended, one of infinity or NaN spoils the rows that see it; rows before stay
+    as they were."""
+    g = torch.Generator().manual_seed(n)
+    q, k, v = (torch.randn(batch, n, heads, 128, generator=g).half() for _ in range(3))
+    q[..., 0] = 1
+    inf = float("inf")
+    k[0, 100, 1, 0], k[0, 120, 2, 0], k[0, 130, 3, 5], k[0, 0, 4, 0], k[0, 63:66, 5, 0] = -inf, inf, float("nan"), -inf, -inf
+    out = capi.causal_attention(q.cuda(), k.cuda(), v.cuda()).cpu().double()
+    want = reference(q, k, v)
+    assert torch.equal(torch.isnan(out), torch.isnan(want))
+    assert torch.isnan(want).any(-1).sum() == (n - 120) + (n - 130) + 1
+    ok = ~torch.isnan(want)
+    assert ((out - want).abs() <= want.abs() * 2.0 ** -11 + 6 * 2.0 ** -16)[ok].all()

@@ -276,3 +276,68 @@ def test_output_of_another_cache_is_not_taken_for_granted():
         layer(_draw(torch.Generator().manual_seed(1), 1, 5, 256), [[1] * 5], torch.arange(5)[None].cuda(), kv, True)
         with pytest.raises(RuntimeError):
             layer(torch.zeros(1, 1, 256, dtype=torch.float16, device="cuda"), [[1] * 6], torch.full((1, 1), 5).cuda(), kv, False)
+
+
+@pytest.mark.parametrize("batch,heads,chunk", [(1, 2, 32), (9, 8, 64)])
+def test_folded_projections_with_the_output_projection_on_its_own(batch, heads, chunk):
+    """A hook on the output projection alone: q, k and v still come from one launch with their append, in steps of
+    their own.  The cache is the whole pass's bit for bit, last chunks that fill up on the way included."""
+    hidden, n = heads * 128, chunk - 2
+    outs, caches, seen = [], [], []
+    for hooked in (False, True):
+        g = torch.Generator().manual_seed(batch)
+        layer = LlamaChunkAttention(hidden, heads, device="cuda")
+        with torch.no_grad():
+            for p in (layer.q_proj, layer.k_proj, layer.v_proj, layer.o_proj):
+                p.weight.copy_(_draw(g, hidden, hidden, sigma=hidden ** -0.5))
+        if hooked:
+            layer.o_proj.register_forward_hook(lambda module, args, out: seen.append(out))
+        kv = capi.Attention(heads, 128, chunk, memory_mb=64, dtype=torch.float16, device=torch.device("cuda:0"))
+        seqs = [[100 * s + t for t in range(n)] for s in range(batch)]
+        with torch.inference_mode():
+            out = [layer(_draw(g, batch, n, hidden), seqs, torch.arange(n).repeat(batch, 1).cuda(), kv, True)]
+            for t in range(5):
+                seqs = [s + [7] for s in seqs]
+                out.append(layer(_draw(g, batch, 1, hidden), seqs, torch.full((batch, 1), n + t).cuda(), kv, False))
+        outs.append(out)
+        caches.append((kv.tree.dump(), kv.tree.get_chunks(), kv.pool_views()))
+    assert len(seen) == 6 and caches[0][0] == caches[1][0]
+    for slot, n_tokens, _, _ in caches[0][1]:
+        assert all(torch.equal(a[slot][:, :n_tokens], b[slot][:, :n_tokens]) for a, b in zip(caches[0][2], caches[1][2]))
+    for a, b in zip(*outs):
+        # the two output projections sum in different orders and round once: a few units of 2^-11 at most
+        assert (a.float() - b.float()).norm() <= 2e-3 * b.float().norm()
+
+
+def test_infinities_and_nans_stay_in_their_rows():
+    g = torch.Generator().manual_seed(2)
+    x, w = _draw(g, 20, 256), _draw(g, 70, 256, sigma=0.06)
+    x[3, 10], x[5, 200], x[19, 0] = float("inf"), float("nan"), float("-inf")
+    x[7] = 60000.0
+    want = (x.double() @ w.double().t())
+    got = capi.linear(x, w).double()
+    finite = want.abs() < 65504
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and (got[want > 65520] == float("inf")).all() and (got[want < -65520] == float("-inf")).all()
+    assert ((got - want).abs() <= want.abs() * 2.0 ** -11 + 60000 * 256 ** 1.5 * 2.0 ** -24)[finite].all()
+
+
+def test_launches_follow_the_current_stream():
+    """The rows are written on a side stream behind a long wait: a launch anywhere else would read the old ones."""
+    side = torch.cuda.Stream()
+    g = torch.Generator().manual_seed(6)
+    layer = LlamaChunkAttention(256, 2, device="cuda")
+    x, y = _draw(g, 2, 30, 256), _draw(g, 2, 1, 256)
+    pos, last = torch.arange(30).repeat(2, 1).cuda(), torch.full((2, 1), 30).cuda()
+    outs = []
+    for stream in (torch.cuda.current_stream(), side):
+        kv = capi.Attention(2, 128, 64, memory_mb=16, dtype=torch.float16, device=torch.device("cuda:0"))
+        a, b = torch.zeros_like(x), torch.zeros_like(y)
+        torch.cuda.synchronize()
+        with torch.inference_mode(), torch.cuda.stream(stream):
+            torch.cuda._sleep(20_000_000)
+            a.copy_(x)
+            b.copy_(y)
+            outs.append([layer(a, [[s] * 30 for s in range(2)], pos, kv, True), layer(b, [[s] * 31 for s in range(2)], last, kv, False),
+                         capi.linear(b, layer.o_proj.weight)])
+        torch.cuda.synchronize()
+    assert all(torch.equal(s, t) and t.abs().max() > 0 for s, t in zip(*outs))

@@ -16,6 +16,9 @@ import os
 from typing import List, Optional, Sequence, Tuple
 
 import numpy as np
+import torch
+
+from . import stock
 
 _LIB_PATH = os.environ.get("CHUNK_ATTN_HIP_LIB") or os.path.join(
     os.path.dirname(os.path.abspath(__file__)), "lib", "libchunkattn_hip.so")
@@ -189,7 +192,6 @@ def _check(rc: int) -> None:
 
 def _launch(device, fn, *args) -> None:
     """fn(*args, stream): the current stream of `device`, with that device current."""
-    import torch
     if device.index is None or torch._C._cuda_getDevice() == device.index:
         index = device.index if device.index is not None else torch._C._cuda_getDevice()
         _check(fn(*args, torch._C._cuda_getCurrentRawStream(index)))
@@ -351,7 +353,6 @@ def rotary_embedding(positions, query, key, head_size: int, cos_sin_cache, is_ne
     `chunk_attn.ops.rotary_embedding` (python_exports_ops.cpp:13): positions int64 [n_tokens] (or
     [batch, seq]), query [..., n_heads*head_size], key [..., n_kv_heads*head_size], rows
     contiguous, cos_sin_cache [max_position, rot_dim]."""
-    import torch
     for name, t in (("query", query), ("key", key), ("cos_sin_cache", cos_sin_cache)):
         if t.dtype != torch.float16 or t.device.type != "cuda":
             raise RuntimeError(f"{name} must be an fp16 tensor on the GPU")
@@ -376,7 +377,6 @@ def rotary_embedding(positions, query, key, head_size: int, cos_sin_cache, is_ne
 
 
 def _norm_args(name, tensors, weight):
-    import torch
     hidden = weight.numel()
     for t in tensors + [weight]:
         if t.dtype != torch.float16 or t.device.type != "cuda" or not t.is_contiguous():
@@ -414,7 +414,6 @@ def plain_call() -> bool:
     """Nothing stands between a call and its kernel: no tracing, no mode that intercepts tensor operations (one that
     only places new tensors, as torch.set_default_device leaves on the stack, does not), no forward-mode level
     whose tangents a kernel would drop."""
-    import torch
     if torch.compiler.is_compiling() or torch._C._is_tracing() or torch._C._len_torch_dispatch_stack() or \
             torch.autograd.forward_ad._current_level >= 0:
         return False
@@ -426,7 +425,6 @@ def plain_call() -> bool:
 def causal_attention_takes(*tensors) -> bool:
     """Whether causal_attention computes on these: fp16 GPU tensors [batch, n, heads, 128] of one shape,
     contiguous and 16-byte aligned, no derivative asked for (the kernel has none)."""
-    import torch
     if torch.is_grad_enabled() and any(t.requires_grad for t in tensors) or not plain_call():
         return False
     shape, device = tensors[0].shape, tensors[0].device
@@ -445,7 +443,6 @@ def causal_attention(q, k, v):
 
 def _causal_attention(q, k, v):
     """causal_attention() of what causal_attention_takes has accepted."""
-    import torch
     out = torch.empty_like(q)
     _launch(q.device, load().ca_causal_attention, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), *q.shape)
     return out
@@ -455,20 +452,18 @@ def is_bare(module, cls) -> bool:
     """The module is a `cls` and nothing hangs on it that a call would also run (hooks, a patched forward)."""
     own = module.__dict__
     return type(module) is cls and not (own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"] or
-                                        own["_backward_pre_hooks"] or "forward" in own or "_call_impl" in own)
+                                        own["_backward_pre_hooks"] or "forward" in own)
 
 
 def projection_takes(x, *linears) -> bool:
     """Whether the projection kernel stands in for these torch.nn.Linear modules on the rows of x: nothing but
     x . W^T in fp16 on one GPU is asked of them, on at most 2^20 elements.  Whether that is also the better choice is
     projection_pays's business."""
-    from .stock import linear_is_stock
-    return linear_is_stock() and _projection_takes(x, *linears)
+    return stock.linear_is_stock() and _projection_takes(x, *linears)
 
 
 def _projection_takes(x, *linears) -> bool:
     """projection_takes() once torch.nn.Linear is known to be as torch wrote it."""
-    import torch
     if type(x) is not torch.Tensor or x.dtype != torch.float16 or x.device.type != "cuda" or not x.is_contiguous():
         return False
     n_in = x.shape[-1]
@@ -523,7 +518,6 @@ def _check_projection(x, *weights) -> None:
 
 
 def _is_operand(t, device) -> bool:
-    import torch
     return t.dtype == torch.float16 and t.device == device and t.is_contiguous() and t.data_ptr() % 16 == 0
 
 
@@ -546,36 +540,41 @@ def linear(x, weight):
 
 def _linear(x, weight):
     """linear() of what projection_takes has accepted."""
-    import torch
     out = torch.empty(x.shape[:-1] + (weight.shape[0],), dtype=x.dtype, device=x.device)
     n_in = x.shape[-1]
     _launch(x.device, load().ca_linear, x.data_ptr(), weight.data_ptr(), out.data_ptr(), x.numel() // n_in, weight.shape[0], n_in)
     return out
 
 
-def _check_rotary(positions, rows: int, cos_sin_cache, device) -> None:
-    import torch
+def _check_positions(positions, rows: int, device) -> None:
     if positions.dtype != torch.int64 or positions.device != device or positions.numel() != rows or \
             not positions.is_contiguous():
         raise RuntimeError(f"positions must be contiguous int64 [{rows}] on {device}")
-    if cos_sin_cache.dtype != torch.float16 or cos_sin_cache.device != device or cos_sin_cache.dim() != 2 or \
-            cos_sin_cache.shape[1] != 128 or not cos_sin_cache.is_contiguous():
-        raise RuntimeError("cos_sin_cache must be contiguous fp16 [max_position, 128] on the GPU of the rows")
+
+
+def is_rotary_table(table, device) -> bool:
+    """What the projection kernels read as a cos/sin cache: contiguous, 16-byte aligned fp16 [max_position, 128]."""
+    return _is_operand(table, device) and table.dim() == 2 and table.shape[1] == 128
+
+
+def _check_rotary_table(table, device) -> None:
+    if not is_rotary_table(table, device):
+        raise RuntimeError(f"cos_sin_cache must be contiguous, 16-byte aligned fp16 [max_position, 128] on {device}")
 
 
 def qkv_rotary(x, wq, wk, wv, positions, cos_sin_cache):
     """(q, k, v) = x . W^T for the three weights [n, n_in] in one launch, n a multiple of 128; q and k are
     rotated for `positions` (NeoX pairs over whole heads of 128) before they are rounded."""
     _check_projection(x, wq, wk, wv)
+    _check_rotary_table(cos_sin_cache, x.device)
     return _qkv_rotary(x, wq, wk, wv, positions, cos_sin_cache)
 
 
 def _qkv_rotary(x, wq, wk, wv, positions, cos_sin_cache):
-    """qkv_rotary() of rows and weights that projection_takes has accepted."""
-    import torch
+    """qkv_rotary() of rows and weights that projection_takes has accepted, and of such a table."""
     n, n_in = wq.shape
     rows = x.numel() // n_in
-    _check_rotary(positions, rows, cos_sin_cache, x.device)
+    _check_positions(positions, rows, x.device)
     if n % 128 or wk.shape != wq.shape or wv.shape != wq.shape:
         raise RuntimeError("q, k and v weights must have one shape of whole heads of 128")
     q, k, v = torch.empty((3,) + tuple(x.shape[:-1]) + (n,), dtype=x.dtype, device=x.device).unbind(0)
@@ -874,7 +873,6 @@ class Attention:
 
     def __init__(self, n_heads: int = 12, d_head: int = 64, chunk_size: int = 64, memory_mb: int = 1024,
                  share_prefix: bool = True, tpp_threshold: int = 1, dtype=None, device=None):
-        import torch
         dtype = dtype or torch.get_default_dtype()
         device = torch.device(device) if device is not None else torch.randn(1).device
         if dtype != torch.float16:
@@ -897,12 +895,10 @@ class Attention:
         self._tables_version = 0
 
     def _stream(self) -> int:
-        import torch
         index = self.device.index
         return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice() if index is None else index)
 
     def _check_kv(self, t, rows: int, name: str):
-        import torch
         if t.dtype != torch.float16 or t.device != self.device or tuple(t.shape) != (rows, self.n_heads, self.d_head):
             raise RuntimeError(f"{name} must be fp16 [{rows}, {self.n_heads}, {self.d_head}] on {self.device}")
         return t.contiguous()
@@ -952,7 +948,6 @@ class Attention:
     def decode_step(self, tokens: Sequence[int], q, k, v):
         """append_token(tokens, k, v) followed by forward(q) as one call (same results, bit for bit):
         the new K/V rows are written by the attention launch itself.  Returns the output."""
-        import torch
         n = len(tokens)
         if self.tree.n_seqs != n:
             raise RuntimeError("num of seqs is not equal to num of tokens")
@@ -971,7 +966,6 @@ class Attention:
         """append_token with the rotary embedding of the new rows folded in: q is rotated in
         place, k is rotated on its way into the cache (k itself is left as it is), v is copied.
         Without `positions` (int64 [n_seqs] on the device) a sequence's position is its length."""
-        import torch
         if self.tree.n_seqs != len(tokens):
             raise RuntimeError("num of seqs is not equal to num of tokens")
         n = len(tokens)
@@ -1001,19 +995,19 @@ class Attention:
         """project_append_rotary, forward and the output projection, then room for the next step's token
         (reserve, refresh_kernel_context): a layer's decode pass as one native call.  Returns [n, n_out]."""
         _check_projection(x, wq, wk, wv)
+        _check_rotary_table(cos_sin_cache, x.device)
         _check_weight(wo, self.n_heads * 128, x.device)
         return self._layer_decode(tokens, x, wq, wk, wv, wo, cos_sin_cache, positions)
 
     def _layer_decode(self, tokens, x, wq, wk, wv, wo, cos_sin_cache, positions):
         """layer_decode() of rows and weights that projection_takes has accepted.  (The native call compares the number
         of tokens with the tree's sequences.)"""
-        import torch
         n = len(tokens)
         n_in, width = x.shape[-1], self.n_heads * 128
         if self.d_head != 128 or x.device != self.device or x.numel() != n * n_in or wq.size(0) != width or \
                 wk.size(0) != width or wv.size(0) != width or wo.size(1) != width:
             raise RuntimeError(f"x must be [{n}, n_in] and the weights [{width}, n_in] and [n_out, {width}] on {self.device}, d_head 128")
-        _check_rotary(positions, n, cos_sin_cache, self.device)
+        _check_positions(positions, n, x.device)
         rows = torch.empty((2, n, width), dtype=x.dtype, device=x.device)     # q, then the attention's output
         y = torch.empty((n, wo.shape[0]), dtype=x.dtype, device=x.device)
         arr, ptr = _i32(tokens)
@@ -1027,11 +1021,11 @@ class Attention:
         """append_token_rotary with the projections folded in: the rows of x (what projection_takes accepts)
         times the three weights, q and k rotated, k and v written into the cache.  Returns q."""
         _check_projection(x, wq, wk, wv)
+        _check_rotary_table(cos_sin_cache, x.device)
         return self._project_append_rotary(tokens, x, wq, wk, wv, cos_sin_cache, positions)
 
     def _project_append_rotary(self, tokens, x, wq, wk, wv, cos_sin_cache, positions):
         """project_append_rotary() of rows and weights that projection_takes has accepted."""
-        import torch
         n = len(tokens)
         if self.tree.n_seqs != n:
             raise RuntimeError("num of seqs is not equal to num of tokens")
@@ -1039,7 +1033,7 @@ class Attention:
         if self.d_head != 128 or x.device != self.device or x.numel() != n * n_in or wq.size(0) != width or \
                 wk.size(0) != width or wv.size(0) != width:
             raise RuntimeError(f"x must be [{n}, n_in] and the weights [{width}, n_in] on {self.device}, d_head 128")
-        _check_rotary(positions, n, cos_sin_cache, self.device)
+        _check_positions(positions, n, x.device)
         self.reserve()
         self.refresh_kernel_context()
         q = torch.empty((n, self.n_heads, self.d_head), dtype=x.dtype, device=x.device)
@@ -1070,7 +1064,6 @@ class Attention:
         return seq_idx
 
     def forward(self, q, partition: int = 0):
-        import torch
         if not q.is_contiguous():
             raise RuntimeError("q is not contiguous")
         if q.dtype != torch.float16 or q.device != self.device or q.dim() != 3 or \

@@ -12,7 +12,7 @@ Weights are whatever the caller loads; tests use seeded random ones.
 from __future__ import annotations
 
 import math
-from typing import List, Sequence
+from typing import List, Optional, Sequence
 
 import torch
 from torch import nn
@@ -70,22 +70,22 @@ class LlamaChunkAttention(nn.Module):
         batch, n_tokens, d_hidden = hidden_states.shape
         projections = (self.q_proj, self.k_proj, self.v_proj)
         own_output = few_rows = False                  # which projections the framework's own kernel computes
-        if self.head_dim == 128 and capi.projection_pays(batch * n_tokens, d_hidden, d_hidden) and \
-                self._plain_rotary() and stock.linear_is_stock():
-            own_output = capi._projection_takes(hidden_states, *projections, self.o_proj)
-            few_rows = own_output or capi._projection_takes(hidden_states, *projections)
+        if self.head_dim == 128 and capi.projection_pays(batch * n_tokens, d_hidden, d_hidden) and stock.linear_is_stock():
+            table = self._plain_rotary(hidden_states.device)
+            own_output = table is not None and capi._projection_takes(hidden_states, *projections, self.o_proj)
+            few_rows = own_output or table is not None and capi._projection_takes(hidden_states, *projections)
         if few_rows:
             weights = [p.weight for p in projections]
         if few_rows and not prefill and capi.is_plain_cache(kv_cache):      # other caches have append_token_rotary only
             assert n_tokens == 1
             step = ([s[-1] for s in seqs], hidden_states, *weights)
-            rotary = (self.rotary_emb.cos_sin_cache, position_ids.reshape(batch).contiguous())
+            rotary = (table, position_ids.reshape(batch).contiguous())
             if own_output:
                 return kv_cache._layer_decode(*step, self.o_proj.weight, *rotary).view(batch, 1, -1)
             q3 = kv_cache._project_append_rotary(*step, *rotary)
             return self._output(kv_cache.forward(q3).view(batch, 1, d_hidden), kv_cache, False)
         if few_rows and prefill:
-            q, k, v = capi._qkv_rotary(hidden_states, *weights, position_ids.contiguous(), self.rotary_emb.cos_sin_cache)
+            q, k, v = capi._qkv_rotary(hidden_states, *weights, position_ids.contiguous(), table)
         else:
             q = self.q_proj(hidden_states)
             k = self.k_proj(hidden_states)
@@ -116,15 +116,15 @@ class LlamaChunkAttention(nn.Module):
         # (a cache of another class may return anything)
         return self._output(attn_output, kv_cache, own_output and capi._is_operand(attn_output, hidden_states.device))
 
-    def _plain_rotary(self) -> bool:
-        """The rotary module is the one this layer was built with, over whole heads, nothing hangs on it, and its table
-        is one that the projection kernels read (the operator takes narrower ones and any alignment)."""
+    def _plain_rotary(self, device: torch.device) -> Optional[torch.Tensor]:
+        """The rotary module's table, if the module is the one this layer was built with, over whole heads, nothing
+        hangs on it, and the projection kernels read such a table (the operator takes narrower ones and any
+        alignment)."""
         r = self.rotary_emb
-        if not (capi.is_bare(r, RotaryEmbedding) and stock.is_stock(RotaryEmbedding, _ROTARY_FORWARD) and r.is_neox_style and
-                r.rotary_dim == r.head_size == self.head_dim):
-            return False
-        table = r.cos_sin_cache
-        return table.dim() == 2 and table.shape[1] == self.head_dim and table.data_ptr() % 16 == 0
+        table = r.__dict__["_buffers"].get("cos_sin_cache")
+        plain = table is not None and capi.is_bare(r, RotaryEmbedding) and stock.is_stock(RotaryEmbedding, _ROTARY_FORWARD) and \
+            r.is_neox_style and r.rotary_dim == r.head_size == self.head_dim and capi.is_rotary_table(table, device)
+        return table if plain else None
 
     def _output(self, attn_output: torch.Tensor, kv_cache: capi.Attention, own: bool) -> torch.Tensor:
         output = capi._linear(attn_output, self.o_proj.weight) if own else self.o_proj(attn_output)

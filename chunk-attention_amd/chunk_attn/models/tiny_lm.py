@@ -31,6 +31,7 @@ class RMSNorm(nn.Module):
 
 
 _NORM_FORWARD = RMSNorm.forward
+_HOST = torch.device("cpu")
 
 
 def _pins(device: torch.device) -> bool:
@@ -82,7 +83,7 @@ class AttentionOnlyLM(nn.Module):
         # one upload, from pinned memory: the host does not wait for what the GPU still has to do (the device is
         # named: only host memory can be pinned, whatever the default device is)
         pinned = _pins(dev)
-        ids, pos = torch.tensor([input_ids, position_ids], dtype=torch.int64, device="cpu",
+        ids, pos = torch.tensor([input_ids, position_ids], dtype=torch.int64, device=_HOST,
                                 pin_memory=pinned).to(dev, non_blocking=pinned)
         hidden = self.embed_tokens(ids)
         token_lists = [s.tokens for s in seqs]

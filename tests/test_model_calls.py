@@ -174,10 +174,10 @@ def test_tables_that_only_the_operator_takes():
     from chunk_attn.llama_layer import LlamaChunkAttention
     layer = LlamaChunkAttention(256, 2, max_position_embeddings=8, device="cpu")
     flat = torch.zeros(8 * 128 + 1, dtype=torch.float16)
-    assert layer._plain_rotary()
+    assert layer._plain_rotary(flat.device) is layer.rotary_emb.cos_sin_cache
     for table, plain in ((flat[:-1].view(8, 128), True), (flat[1:].view(8, 128), False), (flat[:512].view(8, 64), False)):
         layer.rotary_emb.cos_sin_cache = table
-        assert layer._plain_rotary() == plain
+        assert (layer._plain_rotary(flat.device) is table) == plain
 
 
 # us on one GPU (MI355X), weights from memory

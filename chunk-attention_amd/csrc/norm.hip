@@ -50,8 +50,9 @@ __device__ __forceinline__ float first_pass8(h8& x, half_t* __restrict__ residua
 #pragma unroll
         for (int e = 0; e < 8; e++) {
             const float s = float(x[e]) + float(r[e]);
+            if constexpr (ADD == kAdd) ss += s * s;
             x[e] = half_t(s);
-            ss += (ADD == kAdd) ? s * s : float(x[e]) * float(x[e]);
+            if constexpr (ADD == kAddRounded) ss += float(x[e]) * float(x[e]);
         }
         *reinterpret_cast<h8*>(residual_piece) = x;
     } else {

@@ -113,8 +113,9 @@ class LlamaChunkAttention(nn.Module):
             kv_cache.append_token_rotary([s[-1] for s in seqs], q3, k3, v3, self.rotary_emb.cos_sin_cache,
                                          self.rotary_emb.is_neox_style, position_ids.reshape(batch).contiguous())
             attn_output = kv_cache.forward(q3).view(batch, 1, d_hidden)
-        # (a cache of another class may return anything)
-        return self._output(attn_output, kv_cache, own_output and capi._is_operand(attn_output, hidden_states.device))
+            # a cache of another class may return anything: another type, a subclass, something with a gradient
+            own_output = own_output and capi._projection_takes(attn_output, self.o_proj)
+        return self._output(attn_output, kv_cache, own_output)
 
     def _plain_rotary(self, device: torch.device) -> Optional[torch.Tensor]:
         """The rotary module's table, if the module is the one this layer was built with, over whole heads, nothing

@@ -278,6 +278,23 @@ def test_output_of_another_cache_is_not_taken_for_granted():
             layer(torch.zeros(1, 1, 256, dtype=torch.float16, device="cuda"), [[1] * 6], torch.full((1, 1), 5).cuda(), kv, False)
 
 
+def test_gradient_of_another_cache_goes_through_the_output_projection():
+    """A cache of another class may return something learned: with frozen weights its gradient is the product's."""
+    class Learned(capi.Attention):
+        def forward(self, q, partition=0):
+            return super().forward(q, partition) + self.offset
+
+    layer = LlamaChunkAttention(256, 2, device="cuda").requires_grad_(False)
+    kv = Learned(2, 128, 64, memory_mb=16, dtype=torch.float16, device=torch.device("cuda:0"))
+    kv.offset = torch.zeros(1, 2, 128, dtype=torch.float16, device="cuda", requires_grad=True)
+    layer(_draw(torch.Generator().manual_seed(1), 1, 5, 256), [[1] * 5], torch.arange(5)[None].cuda(), kv, True)
+    out = layer(_draw(torch.Generator().manual_seed(2), 1, 1, 256), [[1] * 6], torch.full((1, 1), 5).cuda(), kv, False)
+    out.sum().backward()
+    want = layer.o_proj.weight.double().sum(0)
+    # sums of 256 products with one in fp32, rounded to fp16
+    assert ((kv.offset.grad.double().view(-1) - want).abs() <= want.abs() * 2.0 ** -11 + 2.0 ** -14).all()
+
+
 @pytest.mark.parametrize("batch,heads,chunk", [(1, 2, 32), (9, 8, 64)])
 def test_folded_projections_with_the_output_projection_on_its_own(batch, heads, chunk):
     """A hook on the output projection alone: q, k and v still come from one launch with their append, in steps of

@@ -33,8 +33,9 @@ enum { kPlain = 0, kRotary = 1, kAppend = 2 };
 // has come goes through the wave's own LDS into the operands' layout (no barrier), W as the A operand, so
 // that a lane ends up with four neighbouring columns of one row; the eight partial tiles are added in LDS.
 //
-// What bounds it: with few rows the weights' bytes (16 rows or fewer, [32000, 4096]: 40 us, 6.6 TB/s; the
-// library 44), below that the launch and two round trips to memory (1024 x 1024: 3.3 us, the library 4.4; q, k
+// What bounds it: with few rows the weights' bytes ([32000, 4096] from memory on 1 row 46.5 us, 5.6 TB/s, on 8 rows
+// 49.9, on 16 59.6; the library 55.6 to 56.4; the same weight again and again 41 to 42, the library likewise),
+// below that the launch and two round trips to memory (1024 x 1024: 3.3 us, the library 4.4; q, k
 // and v together 4.3, as three library calls 13.3, the rotary launch not counted); with hundreds of rows
 // LDS, which every wave fills and reads for itself, and from some n_rows * n_in on a library product that
 // shares its tiles between waves is faster (projection_pays in capi.py has the line).

@@ -127,6 +127,12 @@ struct ca_ctx {
     size_t host_blob_cap[kStaging] = {};
     hipEvent_t host_blob_free[kStaging] = {};
     int next_host = 0;
+    bool direct = false;  // forwards over the current plan take the direct form, which reads no device tables
+    // Tables of such a plan are uploaded when something else first reads them (ensure_tables); until then they
+    // stand here.
+    bool upload_pending = false;
+    std::vector<char> pending_blob;
+    bool blob_in_graph = false;  // a captured upload writes dev_blob whenever its graph is replayed
     // offsets into dev_blob
     size_t off_shared = 0, off_stream = 0, off_slots = 0, off_seq_len = 0, off_part_ptr = 0,
            off_tail_slot = 0, off_tail_fill = 0;
@@ -248,8 +254,44 @@ ca::PlanParams plan_params(const ca_ctx* c, int partition) {
     return pp;
 }
 
-// Copies c->plan into a pinned staging buffer and queues its upload on `st`; sizes the
-// partial-row buffer for it.
+// Whether a forward over the current plan takes the direct form (launch_direct): a rule on what only a new plan
+// changes, so that equal caches take equal forms however their tables came about.  One workgroup per (sequence,
+// head) reads at what one compute unit takes in (some 130 GB/s, 4 us per 1000 tokens), and a second one on a unit
+// doubles that; the general path spreads a long run over the device but pays partial rows and a second launch.  us
+// per forward, general and direct (chunks of 64, sequences x heads, shared + own tokens): 4 x 12, 256 + 100, 6.8 and
+// 5.15; 8 x 32, 256 + 100, 9.6 and 6.65; 16 x 8, 640 + 120 (two rounds of the eight waves) 7.3 and 6.4; behind 768
+// tokens only launches of many workgroups gain, where the general path's tables grow too: 8 x 8, 800 + 150, 7.3 and 7.3,
+// but 4 x 32 9.85 and 9.15, 8 x 32 12.3 and 10.5; 16 x 12, 1280 + 100, 9.85 and 10.9; with chunks of 32 4 x 32, 768 +
+// 60, 8.9 and 9.1; 32 x 12 (384 workgroups), 512 + 100, 11.15 and 12.9.
+bool direct_form(const ca_ctx* c) {
+    const ca::Plan& p = c->plan;
+    if (p.path_stride == 0 || p.partition != 0 || c->schedule != 0 || c->seg_chunks > 0 || c->stream_chunks > 0) return false;
+    const int64_t wgs = int64_t(c->n_seqs) * c->H;
+    const int64_t tokens = int64_t(p.path_stride) * c->C;
+    return wgs <= c->n_cus && (tokens <= 768 || (tokens <= 1280 && c->C >= 64 && 2 * wgs >= c->n_cus));
+}
+
+int run_direct(ca_ctx* c, const ca::LaunchArgs& a, hipStream_t st) {
+    int32_t len[ca::kDirectSeqs];
+    for (int s = 0; s < c->n_seqs; s++) len[s] = c->plan.seq_len[s] + c->delta_tokens;
+    return launch_rc(ca::launch_direct(a, len, c->plan.paths.data(), c->n_seqs, c->plan.path_stride, st), "direct launch");
+}
+
+// The device tables of the current plan, for whatever reads them: uploads what upload_plan left out.
+int ensure_tables(ca_ctx* c, hipStream_t st) {
+    if (!c->upload_pending) return CA_OK;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    CA_HIP(hipStreamIsCapturing(st, &capture));
+    if (int rc = launch_rc(ca::launch_upload_args(c->dev_blob, c->pending_blob.data(), c->pending_blob.size(), st), "table upload")) return rc;
+    // Captured, it has not happened yet, and happens on every replay: still pending for everybody else, and no
+    // later tables may stand in this buffer (upload_plan).
+    if (capture == hipStreamCaptureStatusNone) c->upload_pending = false;
+    else c->blob_in_graph = true;
+    return CA_OK;
+}
+
+// Sizes the device buffers for c->plan and queues its upload on `st`, through a pinned staging buffer if it is
+// too large for a kernel argument.
 int upload_plan(ca_ctx* c, hipStream_t st) {
     ca::Plan& p = c->plan;
     size_t off = 0;
@@ -267,7 +309,37 @@ int upload_plan(ca_ctx* c, hipStream_t st) {
     c->off_tail_fill = place(p.tail_fill.size() * 4);
     const size_t total = std::max<size_t>(off, 64);  // a multiple of 64
 
+    if (c->blob_in_graph) {  // left to the graph
+        c->retired.push_back(c->dev_blob);
+        c->dev_blob = nullptr;
+        c->dev_blob_cap = 0;
+        c->blob_in_graph = false;
+    }
     if (int rc = ensure_dev(c, &c->dev_blob, &c->dev_blob_cap, total)) return rc;
+    const size_t part_bytes = std::max<size_t>(size_t(p.n_part_rows) * c->H * ca::PART_STRIDE * 4, 256);
+    if (int rc = ensure_dev(c, reinterpret_cast<char**>(&c->part), &c->part_cap, part_bytes)) return rc;
+    c->upload_pending = false;
+    c->direct = direct_form(c);
+    auto fill = [&](char* to) {
+        auto put = [&](size_t at, const void* src, size_t bytes) {
+            if (bytes) std::memcpy(to + at, src, bytes);
+        };
+        put(c->off_shared, p.shared_items.data(), p.shared_items.size() * sizeof(ca::WorkItem));
+        put(c->off_stream, p.stream_items.data(), p.stream_items.size() * sizeof(ca::WorkItem));
+        put(c->off_slots, p.slots.data(), p.slots.size() * 4);
+        put(c->off_seq_len, p.seq_len.data(), p.seq_len.size() * 4);
+        put(c->off_part_ptr, p.part_ptr.data(), p.part_ptr.size() * 4);
+        put(c->off_tail_slot, p.tail_slot.data(), p.tail_slot.size() * 4);
+        put(c->off_tail_fill, p.tail_fill.data(), p.tail_fill.size() * 4);
+    };
+    // Small tables travel as a kernel argument (no staging buffer, no event), those of a forward in direct
+    // form only if something asks for them.
+    if (total <= ca::kArgUploadBytes) {
+        c->pending_blob.resize(total);
+        fill(c->pending_blob.data());
+        c->upload_pending = true;
+        return c->direct ? CA_OK : ensure_tables(c, st);
+    }
     const int hb = c->next_host;
     c->next_host = (c->next_host + 1) % ca_ctx::kStaging;
     if (total > c->host_blob_cap[hb]) {
@@ -287,23 +359,12 @@ int upload_plan(ca_ctx* c, hipStream_t st) {
     // the staging buffer may still be the source of an earlier asynchronous upload
     CA_HIP(hipEventSynchronize(c->host_blob_free[hb]));
     char* hbuf = c->host_blob[hb];
-    auto put = [&](size_t at, const void* src, size_t bytes) {
-        if (bytes) std::memcpy(hbuf + at, src, bytes);
-    };
-    put(c->off_shared, p.shared_items.data(), p.shared_items.size() * sizeof(ca::WorkItem));
-    put(c->off_stream, p.stream_items.data(), p.stream_items.size() * sizeof(ca::WorkItem));
-    put(c->off_slots, p.slots.data(), p.slots.size() * 4);
-    put(c->off_seq_len, p.seq_len.data(), p.seq_len.size() * 4);
-    put(c->off_part_ptr, p.part_ptr.data(), p.part_ptr.size() * 4);
-    put(c->off_tail_slot, p.tail_slot.data(), p.tail_slot.size() * 4);
-    put(c->off_tail_fill, p.tail_fill.data(), p.tail_fill.size() * 4);
+    fill(hbuf);
     // a copy kernel, not hipMemcpyAsync: the copy engine's hand-over stalls the stream for
     // several microseconds in the middle of a decode step
     if (int rc = launch_rc(ca::launch_upload(c->dev_blob, hbuf, total, st), "table upload")) return rc;
     CA_HIP(hipEventRecord(c->host_blob_free[hb], st));
-
-    const size_t part_bytes = std::max<size_t>(size_t(p.n_part_rows) * c->H * ca::PART_STRIDE * 4, 256);
-    return ensure_dev(c, reinterpret_cast<char**>(&c->part), &c->part_cap, part_bytes);
+    return CA_OK;
 }
 
 // Builds the plan for `partition` from the context's rows and uploads it.
@@ -371,12 +432,14 @@ int collect_timing(ca_ctx* c) {
 }
 
 int run_shared(ca_ctx* c, const void* q, hipStream_t st) {
+    if (int rc = ensure_tables(c, st)) return rc;
     const ca::LaunchArgs a = launch_args(c, q, nullptr);
     return launch_rc(ca::launch_decode(a, static_cast<int>(c->plan.shared_items.size()), 0, false, st),
                      "chunk-first launch");
 }
 
 int run_stream(ca_ctx* c, const void* q, void* out, hipStream_t st) {
+    if (int rc = ensure_tables(c, st)) return rc;
     const ca::LaunchArgs a = launch_args(c, q, out);
     return launch_rc(ca::launch_decode(a, 0, static_cast<int>(c->plan.stream_items.size()), false, st),
                      "sequence-first launch");
@@ -390,6 +453,7 @@ int run_merge(ca_ctx* c, void* out, hipStream_t st) {
 
 int run_fused(ca_ctx* c, const void* q, void* out, hipStream_t st) {
     const ca::LaunchArgs a = launch_args(c, q, out);
+    if (c->direct) return run_direct(c, a, st);
     if (c->schedule == 0) {
         // both phases in one launch (shared and stream workgroups overlap), then the merge
         if (int rc = launch_rc(ca::launch_decode(a, static_cast<int>(c->plan.shared_items.size()),
@@ -555,7 +619,7 @@ int ca_attention(ca_ctx* c, const void* q, void* out, int n_seqs, int partition,
         if (!c->timing) return run_fused(c, q, out, st);
         if (int rc = collect_timing(c)) return rc;
         CA_HIP(hipEventRecord(c->ev[0], st));
-        if (c->timing == 1 && c->schedule == 0) {
+        if (c->timing == 1 && c->schedule == 0 && !c->direct) {
             // the forward as it normally runs: decode launch, then merge launch
             const ca::LaunchArgs a = launch_args(c, q, out);
             if (int rc = launch_rc(ca::launch_decode(a, static_cast<int>(c->plan.shared_items.size()),
@@ -563,7 +627,7 @@ int ca_attention(ca_ctx* c, const void* q, void* out, int n_seqs, int partition,
             CA_HIP(hipEventRecord(c->ev[1], st));
             CA_HIP(hipEventRecord(c->ev[2], st));
             if (int rc = run_merge(c, out, st)) return rc;
-        } else if (c->timing == 1) {
+        } else if (c->timing == 1 || c->direct) {  // one launch
             if (int rc = run_fused(c, q, out, st)) return rc;
             CA_HIP(hipEventRecord(c->ev[1], st));
             CA_HIP(hipEventRecord(c->ev[2], st));
@@ -599,6 +663,7 @@ int ca_attention_noalloc(ca_ctx* c, const void* q, void* out, int n_seqs, void* 
     }
     hipStream_t st = static_cast<hipStream_t>(stream);
     ca::LaunchArgs a = launch_args(c, q, out);
+    if (c->direct) return run_direct(c, a, st);
     a.part = scratch;  // every row that the merge reads is written by the decode launch first
     if (int rc = launch_rc(ca::launch_decode(a, static_cast<int>(c->plan.shared_items.size()),
                                              static_cast<int>(c->plan.stream_items.size()), false, st), "decode launch")) return rc;
@@ -609,11 +674,27 @@ int ca_attention_noalloc(ca_ctx* c, const void* q, void* out, int n_seqs, void* 
 static_assert(CA_NOALLOC_SCRATCH_BYTES == ca::kScratchBytes, "the header's scratch size and the kernels' must agree");
 
 namespace {
+// No two sequences end in the same chunk.
+bool ends_apart(const ca::Plan& p) {
+    return std::all_of(p.tail_width.begin(), p.tail_width.end(), [](int32_t w) { return w == 1; });
+}
+
 // The fused decode step: append and attention in the decode launch plus the merge launch.
 int decode_step(ca_ctx* c, const void* q, const void* k, const void* v, void* out, int n_seqs, hipStream_t st) {
     if (c->partition != 0 || c->schedule != c->plan_schedule) {
         if (int rc = build_and_upload(c, 0, st)) return rc;
     }
+    if (c->direct && ends_apart(c->plan)) {
+        // one launch: the workgroups of a sequence also write its new row
+        c->delta_tokens += 1;
+        ca::LaunchArgs a = launch_args(c, q, out);
+        a.k_new = k;
+        a.v_new = v;
+        const int rc = run_direct(c, a, st);
+        if (rc != CA_OK) c->delta_tokens -= 1;
+        return rc;
+    }
+    if (int rc = ensure_tables(c, st)) return rc;
     if (c->schedule == 0 && c->plan.tails_streamed) {
         // no append launch: the workgroup that streams a sequence's last chunk takes the new row
         // from k / v, and the merge launch writes the rows into the pool
@@ -711,6 +792,7 @@ int ca_append_kv(ca_ctx* c, const void* k, const void* v, int n_seqs, void* stre
         }
     }
     Range range("ca_append_kv");
+    if (int rc = ensure_tables(c, static_cast<hipStream_t>(stream))) return rc;
     const ca::LaunchArgs a = launch_args(c, nullptr, nullptr);
     return launch_rc(ca::launch_append(a, k, v, reinterpret_cast<const int32_t*>(c->dev_blob + c->off_tail_slot),
                                        reinterpret_cast<const int32_t*>(c->dev_blob + c->off_tail_fill),
@@ -881,6 +963,7 @@ int ca_qkv_rotary_append_kv(ca_ctx* c, const void* x, const void* wq, const void
             return fail(CA_ERR_STATE, "sequence " + std::to_string(s) + " has no free row in its last chunk: reserve and refresh first");
         }
     }
+    if (int rc = ensure_tables(c, static_cast<hipStream_t>(stream))) return rc;
     ca::ProjectArgs a = qkv_append_args(c, wq, wk, wv, positions, cos_sin_cache, max_position, q);
     a.tail_slot = reinterpret_cast<const int32_t*>(c->dev_blob + c->off_tail_slot);
     a.tail_fill = reinterpret_cast<const int32_t*>(c->dev_blob + c->off_tail_fill);
@@ -961,6 +1044,7 @@ int ca_rope_append_kv(ca_ctx* c, const int64_t* positions, void* q, const void* 
             return fail(CA_ERR_INVALID, "sequence " + std::to_string(s) + " is longer than the cos/sin cache");
         }
     }
+    if (int rc = ensure_tables(c, static_cast<hipStream_t>(stream))) return rc;
     const ca::LaunchArgs a = launch_args(c, nullptr, nullptr);
     ca::RotaryArgs r;
     r.positions = positions;
@@ -1228,6 +1312,7 @@ int ca_bench_decode_launch(ca_ctx* c, const void* q, void* out, int n_seqs, int 
     if (c->partition != 0 || c->schedule != 0 || c->plan_schedule != 0) {
         return fail(CA_ERR_STATE, "the tables were built for another partition or schedule");
     }
+    if (int rc = ensure_tables(c, static_cast<hipStream_t>(stream))) return rc;
     const ca::LaunchArgs a = launch_args(c, q, out);
     const int n_shared = what == 1 ? 0 : static_cast<int>(c->plan.shared_items.size());
     const int n_stream = what == 2 ? 0 : static_cast<int>(c->plan.stream_items.size());

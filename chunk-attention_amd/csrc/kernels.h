@@ -64,6 +64,11 @@ void* probe_sink_ptr(int device);
 // its output; otherwise only partial rows (and direct outputs) are written.
 int launch_decode(const LaunchArgs& a, int n_shared_items, int n_stream_items, bool fuse_merge,
                   hipStream_t st);
+// A small forward in one launch, without tables in memory: len[s] tokens of every sequence (a fused step's new one
+// among them: a.k_new / a.v_new, whose rows this launch also puts into the pool; no two sequences may then end in
+// one chunk), chunk k of its path at paths[s * stride + k], both host arrays.  At most kDirectSeqs sequences and
+// kDirectSlots = sequences x stride entries.
+int launch_direct(const LaunchArgs& a, const int32_t* len, const int32_t* paths, int n_seqs, int stride, hipStream_t st);
 // The second launch of a forward: merges the partial rows of every (sequence, head) when `merge`,
 // and, for a fused decode step (a.k_new set), writes the step's new K/V rows into the pool
 // (a.tail_slot / a.tail_fill, row tail_fill + delta_tokens - 1).
@@ -73,6 +78,10 @@ int launch_fill(int32_t* p, int n, int32_t value, hipStream_t st);
 // `st`.  For the table upload: a copy-engine transfer in the middle of a decode step costs the
 // stream several microseconds of hand-over between queues, a small kernel does not.
 int launch_upload(void* dst_dev, const void* src_pinned, size_t bytes, hipStream_t st);
+// The same for at most kArgUploadBytes of ordinary host memory, which travel as a kernel argument: `src` is free
+// when the call returns, and a captured launch keeps what it was captured with.
+constexpr size_t kArgUploadBytes = 3584;
+int launch_upload_args(void* dst_dev, const void* src, size_t bytes, hipStream_t st);
 // Measurement aid: n_wgs workgroups read `bytes` of device memory (from a 16-byte aligned
 // address) with non-temporal 16-byte loads and keep nothing; `sink` is 4 writable bytes of
 // device memory.

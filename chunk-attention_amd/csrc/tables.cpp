@@ -156,6 +156,34 @@ void build_stream_items(Plan& p, int chunk_size, const PlanParams& params) {
 
 }  // namespace
 
+namespace {
+bool paths_fit(int n_seqs, int stride) {
+    return n_seqs <= kDirectSeqs && stride >= 1 && stride <= kMaxItemChunks && n_seqs * stride <= kDirectSlots;
+}
+
+// The new last chunks of a roll-over behind the paths they extend.
+void roll_paths(Plan& p, const int32_t* seqs, const int32_t* new_slots, int n) {
+    if (p.path_stride == 0) return;
+    int stride = p.path_stride;
+    for (int i = 0; i < n; i++) stride = std::max(stride, p.path_len[seqs[i]] + 1);
+    if (!paths_fit(p.n_seqs, stride)) {
+        p.path_stride = 0;
+        p.paths.clear();
+        p.path_len.clear();
+        return;
+    }
+    if (stride != p.path_stride) {
+        std::vector<int32_t> wider(size_t(p.n_seqs) * stride, 0);
+        for (int s = 0; s < p.n_seqs; s++) {
+            std::copy_n(p.paths.begin() + size_t(s) * p.path_stride, p.path_len[s], wider.begin() + size_t(s) * stride);
+        }
+        p.paths = std::move(wider);
+        p.path_stride = stride;
+    }
+    for (int i = 0; i < n; i++) p.paths[size_t(seqs[i]) * stride + p.path_len[seqs[i]]++] = new_slots[i];
+}
+}  // namespace
+
 void build_plan(const ChunkRow* rows, int n_rows, int n_seqs, int chunk_size,
                 const PlanParams& params, Plan* out) {
     Plan& p = *out;
@@ -445,6 +473,21 @@ void build_plan(const ChunkRow* rows, int n_rows, int n_seqs, int chunk_size,
     p.hints.taper_chunks = taper_chunks;
 
     build_stream_items(p, chunk_size, params);
+
+    // ---- whole paths (direct form) ----------------------------------------------------------
+    if (n_seqs < 1 || n_seqs > kDirectSeqs) return;
+    std::vector<int> n_path(n_seqs, 0);
+    for (int i = 0; i < n_rows; i++) {
+        for (int s = rows[i].seq_begin; s < rows[i].seq_end; s++) n_path[s]++;
+    }
+    const int stride = *std::max_element(n_path.begin(), n_path.end());
+    if (!paths_fit(n_seqs, stride)) return;
+    p.path_stride = stride;
+    p.paths.assign(size_t(n_seqs) * stride, 0);
+    p.path_len.assign(n_seqs, 0);
+    for (int i = 0; i < n_rows; i++) {
+        for (int s = rows[i].seq_begin; s < rows[i].seq_end; s++) p.paths[size_t(s) * stride + p.path_len[s]++] = rows[i].slot;
+    }
 }
 
 void roll_tails(Plan* plan, int chunk_size, const PlanParams& params, int delta_tokens,
@@ -489,6 +532,7 @@ void roll_tails(Plan* plan, int chunk_size, const PlanParams& params, int delta_
         p.tail_width[s] = 1;
     }
     build_stream_items(p, chunk_size, params);
+    roll_paths(p, seqs, new_slots, n);
 }
 
 bool plan_is_stale(const Plan& plan, int percent, int64_t extra_tokens) {

@@ -89,6 +89,9 @@ constexpr int kWideMin = 96;    // chunks covering at least this many sequences 
 constexpr int kWideMinLong = 33;       // ... and from this many on (more than one M tile) when they belong to a long run:
 constexpr int kWideLongTokens = 2048;  // a run of at least this many tokens
 constexpr int32_t kItemWide = 1;
+// What the direct form takes: its tables travel as a kernel argument.
+constexpr int kDirectSeqs = 64;     // sequences
+constexpr int kDirectSlots = 768;   // sequences times chunks of the longest path
 
 struct Plan {
     int n_seqs = 0;
@@ -116,6 +119,12 @@ struct Plan {
     std::vector<std::vector<int32_t>> own;      // per sequence: slots of the chunks it streams, path order
     std::vector<int32_t> own_pos0;              // per sequence: path position of own[s][0]
     std::vector<int32_t> shared_parts;          // per sequence: partial rows written by shared items
+
+    // Every sequence's whole path, for the direct form of a small forward (kernels.h, DirectTable): chunk k of
+    // sequence s at paths[s * path_stride + k].  Empty when the tree does not fit that form.
+    int path_stride = 0;
+    std::vector<int32_t> paths;
+    std::vector<int32_t> path_len;              // chunks of every sequence
 };
 
 void build_plan(const ChunkRow* rows, int n_rows, int n_seqs, int chunk_size,

@@ -1,0 +1,118 @@
+"""The direct form of small forwards (one launch, a workgroup a (sequence, head), no device tables) against the
+general path and the oracle: lengths around its 64-token tiles and eight waves, every chunk size, heads and
+sequences around the lines of its rule, the fused decode step with its row write, and captured launches that are
+the first to read the device tables (which the direct form itself does not upload)."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_helpers import assert_close, dev, host_state, make_attention, oracle_output, to_dev
+
+pytestmark = pytest.mark.gpu
+
+
+def rand(rng, *shape):
+    return rng.standard_normal(shape).astype(np.float16)
+
+
+def build(rng, H, c, shared, privates, general=False, kv=None):
+    """kv: the rows of an earlier build, so that two caches hold the same."""
+    total = sum((shared + p) // c + 3 for p in privates)
+    attn = make_attention(H, c, total)
+    if general:
+        attn.ctx.set_plan(stream_chunks=4)    # explicit item sizes: the general path
+    kv = kv or [(rand(rng, shared + max(privates), H, 128), rand(rng, shared + max(privates), H, 128)) for _ in privates]
+    for s, p in enumerate(privates):
+        n = shared + p
+        k, v = (np.concatenate([kv[0][i][:shared], kv[s][i][shared:n]]) for i in range(2))
+        attn.add_seq(list(range(shared)) + [10_000 * (s + 1) + t for t in range(p)], to_dev(k), to_dev(v))
+    return attn, kv
+
+
+@pytest.mark.parametrize("H,c,shared,privates", [
+    (1, 64, 0, [1]), (12, 64, 256, [100, 75, 63, 1]), (5, 64, 64, [64, 65, 127, 447, 448, 449]),
+    (4, 32, 96, [1, 31, 32, 33, 64, 200]), (3, 128, 128, [1, 63, 64, 65, 127, 128, 300]),
+    (4, 64, 64, [7] * 64),                    # as many sequences and workgroups as it takes
+    (1, 64, 0, [5] * 20 + [700]),             # the large argument block
+    (32, 64, 1024, [130, 200, 10, 64, 1, 2, 3, 4]),   # long paths while half the compute units have a workgroup
+    (4, 64, 704, [64] * 3), (4, 64, 704, [65] * 3),   # both sides of the line on the path's length
+    (4, 64, 64, [7] * 65), (257, 64, 0, [30]),        # past the lines on sequences and workgroups
+])
+def test_direct_and_general_forwards_agree(H, c, shared, privates):
+    rng = np.random.default_rng(len(privates) + H)
+    attn, kv = build(rng, H, c, shared, privates)
+    other, _ = build(rng, H, c, shared, privates, True, kv)
+    q = rand(rng, len(privates), H, 128)
+    got, general = attn.forward(to_dev(q)), other.forward(to_dev(q))
+    # two roundings to fp16 of sums that differ by the general path's fp16 probabilities
+    assert_close(got, general.float().cpu().numpy())
+    assert_close(got, oracle_output(attn, q, exact=True))
+
+
+@pytest.mark.parametrize("c", [32, 64, 128])
+def test_fused_steps_write_their_rows_and_follow_rollovers(c):
+    rng = np.random.default_rng(c)
+    H, shared, privates = 4, 2 * c, [1, c - 2, c, c + 5]
+    fused, kv = build(rng, H, c, shared, privates)
+    apart, _ = build(rng, H, c, shared, privates, False, kv)
+    n = len(privates)
+    for step in range(c + 6):
+        tokens = [10 ** 6 + 100 * step + s for s in range(n)]
+        q, k, v = (to_dev(rand(rng, n, H, 128)) for _ in range(3))
+        out = fused.decode_step(tokens, q, k, v)
+        apart.append_token(tokens, k, v)
+        assert torch.equal(out, apart.forward(q))
+    rows_a, ka, va = host_state(fused)
+    rows_b, kb, vb = host_state(apart)
+    np.testing.assert_array_equal(rows_a, rows_b)
+    for slot, n_tok in {(r[0], r[1]) for r in rows_a.tolist()}:
+        np.testing.assert_array_equal(ka[slot][:, :n_tok], kb[slot][:, :n_tok])
+        np.testing.assert_array_equal(va[slot][:, :n_tok], vb[slot][:, :n_tok])
+
+
+def test_captured_append_before_any_upload():
+    """An append recorded into a graph brings the tables along; neither eager work nor later tables may depend on
+    whether the graph has run."""
+    rng = np.random.default_rng(3)
+    H, c, privates = 4, 64, [10, 20, 30]
+    attn, kv = build(rng, H, c, 64, privates)
+    q = rand(rng, 3, H, 128)
+    attn.refresh_kernel_context()
+    k, v = to_dev(rand(rng, 3, H, 128)), to_dev(rand(rng, 3, H, 128))
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        attn.ctx.append_kv(k.data_ptr(), v.data_ptr(), 3, torch.cuda.current_stream().cuda_stream)
+    attn.tree.append_token([1, 2, 3])
+    attn.ctx.delta_tokens = 1
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert_close(attn.forward(to_dev(q)), oracle_output(attn, q, exact=True))
+    # eager, after the capture: the tables are uploaded for it
+    attn.append_token([4, 5, 6], k, v)
+    assert_close(attn.forward(to_dev(q)), oracle_output(attn, q, exact=True))
+    # other tables, which a replay must leave alone: a replay writes the rows it was captured with and no more
+    attn.add_seq([7] * 40, to_dev(rand(rng, 40, H, 128)), to_dev(rand(rng, 40, H, 128)))
+    attn.append_token([8, 9, 10, 11], to_dev(rand(rng, 4, H, 128)), to_dev(rand(rng, 4, H, 128)))
+    graph.replay()
+    k4, v4 = to_dev(rand(rng, 4, H, 128)), to_dev(rand(rng, 4, H, 128))
+    attn.append_token([12, 13, 14, 15], k4, v4)
+    q4 = rand(rng, 4, H, 128)
+    assert_close(attn.forward(to_dev(q4)), oracle_output(attn, q4, exact=True))
+
+
+def test_phases_and_partitions_upload_what_they_read():
+    rng = np.random.default_rng(4)
+    attn, _ = build(rng, 4, 64, 128, [30, 70, 90])
+    q = rand(rng, 3, 4, 128)
+    want = oracle_output(attn, q, exact=True)
+    qd, out = to_dev(q), torch.empty(3, 4, 128, dtype=torch.float16, device=dev())
+    attn.refresh_kernel_context()
+    stream = torch.cuda.current_stream().cuda_stream
+    attn.ctx.attn_chunks_first(qd.data_ptr(), 3, stream)
+    attn.ctx.attn_seqs_first(qd.data_ptr(), out.data_ptr(), 3, stream)
+    assert_close(out, want)
+    for partition in (0, 1, 0, 2, 0):
+        assert_close(attn.forward(qd, partition), want)

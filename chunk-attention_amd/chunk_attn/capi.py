@@ -462,12 +462,12 @@ def projection_takes(x, *linears) -> bool:
     return stock.linear_is_stock() and _projection_takes(x, *linears)
 
 
-def _projection_takes(x, *linears) -> bool:
-    """projection_takes() once torch.nn.Linear is known to be as torch wrote it."""
+def _projection_takes(x, *linears, limit: int = 1 << 20) -> bool:
+    """projection_takes() once torch.nn.Linear is known to be as torch wrote it, for at most `limit` elements."""
     if type(x) is not torch.Tensor or x.dtype != torch.float16 or x.device.type != "cuda" or not x.is_contiguous():
         return False
     n_in = x.shape[-1]
-    if n_in == 0 or n_in % 64 or not 0 < x.numel() <= 1 << 20 or x.data_ptr() % 16:
+    if n_in == 0 or n_in % 64 or not 0 < x.numel() <= limit or x.data_ptr() % 16:
         return False
     grad = torch.is_grad_enabled()
     # whatever else may stand between a module and its product: hooks, subclasses, patched forwards, modes
@@ -504,6 +504,21 @@ def projection_pays(rows: int, n_in: int, n_out: int) -> bool:
     682 rows, 19 to 12, and 5120 x 5120 on 128 rows, 30 to 25 (q, k and v 64 to 99)."""
     weights = n_in * n_out
     return rows * n_out <= 1 << 20 and (weights <= 1 << 25 or rows <= 16 and weights <= 1 << 27)
+
+
+def shared_tiles_pay(rows: int, n_in: int, n_out: int, n_weights: int) -> bool:
+    """Whether rows [rows, n_in] times `n_weights` weights [n_out, n_in] are faster in the tiles that waves share than as
+    library products, where projection_pays does not say so already: the GPU's time decides.
+
+    The unit is a tile of 128 x 256, of which 256 are computed at a time.  One weight: while they fit at once (us here
+    and the library's: 4096 x 4096 on 1000 rows 34 to 40, on 1500 50 to 52, on 2048 58 to 64, on 2300 88 to 70; 2048 x
+    2048 on 3000 rows 28 to 31, on 4096 32 to 37, on 6000 53 to 47; 1024 x 1024 on 8192 rows 20 to 24).  q, k and v
+    with their rotation: up to three rounds (against three products and the rotary launch: 4096 x 4096 on 512 rows 52
+    to 86, on 2048 181 to 211, on 2300 220 to 222, on 2560 232 to 230; 2048 x 2048 on 4096 rows 101 to 120; 5120 x 5120
+    on 1000 rows 159 to 205, on 1600 269 to 271, on 2048 309 to 300; 1024 x 1024 on 8192 rows 64 to 81).  Weights of
+    more than 2^25 elements were not measured."""
+    tiles = -(-rows // 128) * -(-n_out // 256) * n_weights
+    return n_in * n_out <= 1 << 25 and tiles <= (256 if n_weights == 1 else 768)
 
 
 def _check_projection(x, *weights) -> None:

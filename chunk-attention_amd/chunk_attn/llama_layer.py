@@ -3,10 +3,10 @@
 Mirrors the reference's `LlamaChunkAttention`
 (src/chunk_attn/models/llama_hf/modeling_llama.py:16-113) and its rotary module
 (src/chunk_attn/models/llama_hf/rotary_embedding_vllm.py:43-147) with the same argument
-meaning.  For few rows (a decode batch, a short prompt) the three input projections and the rotary
-embedding are one launch, in the decode branch the KV append too; for many the projections are plain
-torch matmuls, and the rotary embedding of a decode step's query/key rows and the KV append are one
-launch (`Attention.append_token_rotary`).
+meaning.  Up to some thousand rows the three input projections and the rotary embedding are one
+launch, in the decode branch the KV append too; for more the projections are plain torch matmuls, and
+the rotary embedding of a decode step's query/key rows and the KV append are one launch
+(`Attention.append_token_rotary`).
 Weights are whatever the caller loads; tests use seeded random ones.
 """
 from __future__ import annotations
@@ -69,14 +69,19 @@ class LlamaChunkAttention(nn.Module):
         batch row i to be cache sequence i."""
         batch, n_tokens, d_hidden = hidden_states.shape
         projections = (self.q_proj, self.k_proj, self.v_proj)
-        own_output = few_rows = False                  # which projections the framework's own kernel computes
-        if self.head_dim == 128 and capi.projection_pays(batch * n_tokens, d_hidden, d_hidden) and stock.linear_is_stock():
+        own_output = own_input = False                 # which projections the framework's own kernels compute
+        rows = batch * n_tokens
+        few_rows = capi.projection_pays(rows, d_hidden, d_hidden)
+        if self.head_dim == 128 and (few_rows or prefill and capi.shared_tiles_pay(rows, d_hidden, d_hidden, 3)) and \
+                stock.linear_is_stock():
+            limit = hidden_states.numel()              # the two rules have looked at the size
             table = self._plain_rotary(hidden_states.device)
-            own_output = table is not None and capi._projection_takes(hidden_states, *projections, self.o_proj)
-            few_rows = own_output or table is not None and capi._projection_takes(hidden_states, *projections)
-        if few_rows:
+            own_output = table is not None and (few_rows or capi.shared_tiles_pay(rows, d_hidden, d_hidden, 1)) and \
+                capi._projection_takes(hidden_states, *projections, self.o_proj, limit=limit)
+            own_input = own_output or table is not None and capi._projection_takes(hidden_states, *projections, limit=limit)
+        if own_input:
             weights = [p.weight for p in projections]
-        if few_rows and not prefill and capi.is_plain_cache(kv_cache):      # other caches have append_token_rotary only
+        if own_input and not prefill and capi.is_plain_cache(kv_cache):     # other caches have append_token_rotary only
             assert n_tokens == 1
             step = ([s[-1] for s in seqs], hidden_states, *weights)
             rotary = (table, position_ids.reshape(batch).contiguous())
@@ -84,14 +89,14 @@ class LlamaChunkAttention(nn.Module):
                 return kv_cache._layer_decode(*step, self.o_proj.weight, *rotary).view(batch, 1, -1)
             q3 = kv_cache._project_append_rotary(*step, *rotary)
             return self._output(kv_cache.forward(q3).view(batch, 1, d_hidden), kv_cache, False)
-        if few_rows and prefill:
+        if own_input and prefill:
             q, k, v = capi._qkv_rotary(hidden_states, *weights, position_ids.contiguous(), table)
         else:
             q = self.q_proj(hidden_states)
             k = self.k_proj(hidden_states)
             v = self.v_proj(hidden_states)
         if prefill:
-            if not few_rows:
+            if not own_input:
                 q, k = self.rotary_emb(position_ids.contiguous(), q, k)
             shape = (batch, n_tokens, self.num_heads, self.head_dim)
             q4, k4, v4 = q.view(shape), k.view(shape), v.view(shape)

@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 #include "kernels.h"
 #include "rotary_math.h"
@@ -16,6 +17,7 @@ namespace ca {
 namespace {
 
 using rotary::half_t;
+using rotary::h4;
 using rotary::h8;
 typedef float f4 __attribute__((ext_vector_type(4)));
 
@@ -37,8 +39,8 @@ enum { kPlain = 0, kRotary = 1, kAppend = 2 };
 // 49.9, on 16 59.6; the library 55.6 to 56.4; the same weight again and again 41 to 42, the library likewise),
 // below that the launch and two round trips to memory (1024 x 1024: 3.3 us, the library 4.4; q, k
 // and v together 4.3, as three library calls 13.3, the rotary launch not counted); with hundreds of rows
-// LDS, which every wave fills and reads for itself, and from some n_rows * n_in on a library product that
-// shares its tiles between waves is faster (projection_pays in capi.py has the line).
+// LDS, which every wave fills and reads for itself: from there on the waves share their tiles
+// (project_tile_kernel; the line is at launch_mode).
 //
 // Columns of a rotary tile: half of them from the first half of a head, half their partners 64 further on.
 template <int MB, int NB, int R, int MODE>
@@ -226,17 +228,256 @@ int launch_tile(const ProjectArgs& a, hipStream_t st) {
     return e == hipSuccess ? 0 : static_cast<int>(e);
 }
 
+// ---- many rows: tiles that the waves of a workgroup share --------------------------------------------------------
+//
+// A workgroup computes BM rows by BN columns; stages of 64 k elements of its rows of x and of w reach LDS by direct
+// loads, NBUF - 1 stages ahead, and every wave reads the operands of its BM / WM x CW part from there, one k-step (32)
+// ahead of its products, with one barrier a stage.
+//
+// What bounds it: large products, power.  With every compute unit busy the clock falls to about 1.6 GHz (matrix ops
+// on registers alone then reach 1.70 PFLOP/s as 16 x 16 x 32, 1.55 as 32 x 32 x 16, which is why the operands here are
+// 16 wide), and every LDS read and fetched line lowers it further: q, k and v of 4096 with their rotation on 2048
+// rows 181 us, 1.14 PFLOP/s (three library products and the rotary launch 211; the same stages with all of their
+// loads requested in a row behind the barrier 219: a wave issues in order, and its products waited for the loads to
+// be taken; with 32 x 32 x 16 195).  One weight of 4096 on 2048 rows 57.6 (the library 64.1).  Smaller ones, the fill
+// of the pipeline and a stage's latency: 0.36 us a stage for 128 x 128, 0.56 for 128 x 256 (0.43 is the matrix cores').
+// Waves of 64 x 128 or 128 x 64, four to a workgroup, read less from LDS but leave one wave to a SIMD: 226 to 230
+// us where eight of 64 x 64 take 181; 256 x 256 tiles 210 to 218 (384 of them on 256 units).
+__device__ __forceinline__ void load_to_lds16(const char* src, half_t* dst) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                     (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+}
+
+constexpr int BK = 64;             // k elements of a stage: one 128-byte line of every row
+
+template <int BM, int BN, int NBUF, int WAVES, int NB, int MODE>
+__global__ __launch_bounds__(64 * WAVES, 2) void project_tile_kernel(const ProjectArgs a) {
+    constexpr int CW = 16 * NB;                      // columns of a wave
+    constexpr int WN = BN / CW, WM = WAVES / WN;
+    constexpr int TM = BM / WM;                      // rows of a wave
+    constexpr int MB = TM / 16;                      // its 16-row blocks
+    constexpr int STAGE = (BM + BN) * BK;            // halves of a stage: the rows of x, then the rows of w
+    constexpr int NLD = (BM + BN) / 8 / WAVES;       // loads of a wave a stage, eight rows each
+    constexpr int EP = CW + 8;                       // pitch of the output's way through LDS
+    __shared__ __attribute__((aligned(16))) half_t lds[NBUF * STAGE];
+    static_assert(WAVES * 32 * EP <= NBUF * STAGE && NLD * 8 * WAVES == BM + BN && MB % 2 == 0 && NBUF > 2, "");
+
+    const int tid = threadIdx.x;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = w / WN, wn = w % WN;
+    const int l = tid & 63, g = l >> 4, i = l & 15;
+    // Tiles in groups of eight row tiles, columns inside, dealt to the XCDs (block b runs on XCD b % 8) in
+    // contiguous ranges: what an XCD's 32 units work on at a time is about eight row tiles by four column tiles.
+    const int per_w = (a.N + BN - 1) / BN;
+    const int n_cb = per_w * a.n_w, n_rb = (a.M + BM - 1) / BM;
+    const int total = n_cb * n_rb;
+    const int xcd = blockIdx.x & 7, q8 = total >> 3, r8 = total & 7;
+    const int u = xcd * q8 + (xcd < r8 ? xcd : r8) + (blockIdx.x >> 3);
+    constexpr int GM = 8;
+    const int grp = u / (GM * n_cb), in_grp = u - grp * GM * n_cb;
+    const int g_rows = n_rb - grp * GM < GM ? n_rb - grp * GM : GM;
+    const int cb = in_grp / g_rows, rb = grp * GM + in_grp % g_rows;
+    const int which = cb / per_w, blk = cb - which * per_w;
+    const half_t* __restrict__ wt = static_cast<const half_t*>(which == 0 ? a.w[0] : which == 1 ? a.w[1] : a.w[2]);
+    const int row0 = rb * BM, col0 = blk * BN;
+    // Column of the weight behind row c of the tile's w part.  Rotary: a wave's columns are CW / 2 of a head's first
+    // half and their partners 64 further on, so that a lane holds both.
+    auto column = [&](int c) {
+        if (MODE == kPlain) return col0 + c;
+        const int part = (col0 + c) / CW, in = c % CW;
+        return part / (D / CW) * D + part % (D / CW) * (CW / 2) + in % (CW / 2) + in / (CW / 2) * (D / 2);
+    };
+
+    const char* xbase = reinterpret_cast<const char*>(static_cast<const half_t*>(a.x) + size_t(row0) * a.K);
+    const char* wbase = reinterpret_cast<const char*>(wt);
+    unsigned off[NLD];
+#pragma unroll
+    for (int r = 0; r < NLD; r++) {
+        const int lb = w * NLD + r;                  // rows 8 lb .. 8 lb + 7 of the stage
+        int row = 8 * lb + (l >> 3);
+        const int piece = (l & 7) ^ (l >> 3);        // piece c of row r stands at place c ^ (r & 7), as above
+        if (lb < BM / 8) {
+            if (row0 + row >= a.M) row = a.M - 1 - row0;          // computed, not stored
+        } else {
+            row = column(row - BM);
+            if (row >= a.N) row = a.N - 1;
+        }
+        off[r] = (unsigned(row) * unsigned(a.K) + 8 * piece) * 2;
+    }
+    // One load of stage t; `at`: the stage's buffer.
+    auto load = [&](int r, int t, int at) {
+        const int lb = w * NLD + r;
+        load_to_lds16((lb < BM / 8 ? xbase : wbase) + size_t(t) * (BK * 2) + off[r], &lds[at + lb * 8 * BK]);
+    };
+    auto fetch = [&](int t, int at) {
+#pragma unroll
+        for (int r = 0; r < NLD; r++) load(r, t, at);
+    };
+    f4 acc[MB][NB];
+#pragma unroll
+    for (int m = 0; m < MB; m++) {
+#pragma unroll
+        for (int n = 0; n < NB; n++) acc[m][n] = f4{ 0.f, 0.f, 0.f, 0.f };
+    }
+    h8 xf[2][MB], wf[2][NB];
+    const int xrow = (wm * TM + i) * BK, wrow = (BM + wn * CW + i) * BK;
+    // Operand o of k-step ks, w's blocks first.
+    auto operand = [&](int o, int at, int ks, int set) {
+        const half_t* p = &lds[at + 8 * ((4 * ks + g) ^ (i & 7))];
+        if (o < NB) wf[set][o] = *reinterpret_cast<const h8*>(p + wrow + o * 16 * BK);
+        else xf[set][o - NB] = *reinterpret_cast<const h8*>(p + xrow + (o - NB) * 16 * BK);
+    };
+    // The products of a k-step on operand set `set`.  Spread between them: the other set's operands (k-step ks of the
+    // stage at `at`, if MORE) and N loads of stage t.
+    auto step = [&](int set, auto more, int at, int ks, int t, int t_at, auto count) {
+        constexpr int PRODUCTS = MB * NB, OPS = MB + NB, N = decltype(count)::value;
+#pragma unroll
+        for (int k = 0; k < PRODUCTS; k++) {
+            if constexpr (decltype(more)::value) {
+#pragma unroll
+                for (int o = k * OPS / PRODUCTS; o < (k + 1) * OPS / PRODUCTS; o++) operand(o, at, ks, set ^ 1);
+            }
+#pragma unroll
+            for (int r = k * N / PRODUCTS; r < (k + 1) * N / PRODUCTS; r++) load(r, t, t_at);
+            const int m = k / NB, n = k % NB;
+            acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf[set][n], xf[set][m], acc[m][n], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+
+    const int n_t = a.K / BK;
+    // Every wave's loads but those of the newest `left` stages have landed, and every wave holds what it has read.
+    auto meet = [&](auto left) {
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(decltype(left)::value * NLD) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+#pragma unroll
+    for (int s = 0; s < NBUF - 1; s++) {
+        if (s < n_t) fetch(s, s * STAGE);
+    }
+    if (n_t >= NBUF - 1) meet(std::integral_constant<int, NBUF - 2>{});
+    else meet(std::integral_constant<int, 0>{});
+#pragma unroll
+    for (int o = 0; o < MB + NB; o++) operand(o, 0, 0, 0);
+    int at = 0, free_at = (NBUF - 1) * STAGE;
+    // Stage t.  LOADS: there is a stage t + NBUF - 1 to request; MORE: there is a stage t + 1.
+    auto stage_of = [&](int t, auto loads, auto more) {
+        constexpr bool LOADS = decltype(loads)::value;
+        step(0, std::true_type{}, at, 1, t + NBUF - 1, free_at, std::integral_constant<int, LOADS ? NLD : 0>{});
+        // The stage's last operands are in registers: behind the barrier its buffer is free, the next stage has
+        // landed, and this stage's last products cover the latency of its first operands.
+        meet(std::integral_constant<int, LOADS ? NBUF - 2 : 0>{});
+        free_at = at;
+        at = at + STAGE == NBUF * STAGE ? 0 : at + STAGE;
+        step(1, more, at, 0, 0, 0, std::integral_constant<int, 0>{});
+    };
+    int t = 0;
+    for (; t + NBUF - 1 < n_t; t++) stage_of(t, std::true_type{}, std::true_type{});
+    for (; t + 1 < n_t; t++) stage_of(t, std::false_type{}, std::true_type{});
+    stage_of(t, std::false_type{}, std::false_type{});
+    // the loop's last matrix ops are read behind a branch, where the compiler's own wait states do not reach
+    asm volatile("s_nop 15\n\ts_nop 15");
+    __builtin_amdgcn_sched_barrier(0);
+
+    // Lane (g, i) holds row i of a 16 x 16 block, columns 4g .. 4g + 3: rounded, and through the wave's own piece of
+    // LDS, 32 rows at a time, into whole lines.
+    half_t* stage = &lds[w * 32 * EP];
+    half_t* __restrict__ y = static_cast<half_t*>(which == 0 ? a.y[0] : which == 1 ? a.y[1] : a.y[2]);
+#pragma unroll
+    for (int m2 = 0; m2 < MB / 2; m2++) {
+        const int row_base = row0 + wm * TM + 32 * m2;
+#pragma unroll
+        for (int mm = 0; mm < 2; mm++) {
+            const int m = 2 * m2 + mm, row = row_base + 16 * mm + i;
+            const half_t* cs = nullptr;
+            if (MODE != kPlain && which < 2) {
+                cs = static_cast<const half_t*>(a.cos_sin_cache) +
+                     rotary::clamp_pos(a.positions[row < a.M ? row : a.M - 1], a.max_position) * D + (col0 + wn * CW) % D / 2;
+            }
+#pragma unroll
+            for (int n = 0; n < NB / 2; n++) {
+                const int c = 16 * n + 4 * g;
+                const f4 f0 = acc[m][n], f1 = acc[m][n + NB / 2];
+                h4 o0, o1;
+                if (MODE != kPlain && which < 2) {
+                    const h4 c4 = *reinterpret_cast<const h4*>(cs + c), s4 = *reinterpret_cast<const h4*>(cs + c + D / 2);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        o0[e] = half_t(rotary::rot_elem(f0[e], f1[e], float(c4[e]), float(s4[e]), true));
+                        o1[e] = half_t(rotary::rot_elem(f1[e], f0[e], float(c4[e]), float(s4[e]), false));
+                    }
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        o0[e] = half_t(f0[e]);
+                        o1[e] = half_t(f1[e]);
+                    }
+                }
+                *reinterpret_cast<h4*>(&stage[(16 * mm + i) * EP + c]) = o0;
+                *reinterpret_cast<h4*>(&stage[(16 * mm + i) * EP + CW / 2 + c]) = o1;
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int p = 0; p < CW / 16; p++) {
+            constexpr int PIECES = CW / 8;
+            const int r = p * (64 / PIECES) + l / PIECES, c = 8 * (l % PIECES);
+            const int row = row_base + r, n = column(wn * CW + c);
+            if (row >= a.M || n >= a.N) continue;
+            const h8 o = *reinterpret_cast<const h8*>(&stage[r * EP + c]);
+            half_t* dst = y + size_t(row) * a.N + n;
+            if (MODE == kAppend && which > 0) {
+                const int fill = a.tail_fill[row] + a.delta_tokens;
+                if (fill < 0 || fill >= a.C) continue;   // the host guarantees a free row; never write outside the chunk
+                dst = y + ((size_t(a.tail_slot[row]) * (a.N / D) + n / D) * a.C + fill) * D + n % D;
+            }
+            if (MODE != kPlain || a.vec8) {
+                *reinterpret_cast<h8*>(dst) = o;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    if (n + e < a.N) dst[e] = o[e];
+                }
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+template <int BM, int BN, int NBUF, int WAVES, int NB, int MODE>
+int launch_shared_tile(const ProjectArgs& a, hipStream_t st) {
+    const int64_t wgs = int64_t((a.N + BN - 1) / BN) * a.n_w * ((int64_t(a.M) + BM - 1) / BM);
+    if (wgs > 0x7fffffff) return -1;
+    hipLaunchKernelGGL((project_tile_kernel<BM, BN, NBUF, WAVES, NB, MODE>), dim3(static_cast<unsigned>(wgs)), dim3(64 * WAVES), 0, st, a);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? 0 : static_cast<int>(e);
+}
+
 // Tiles.  Up to 16 rows: 16 columns a workgroup (three weights of 4096 x 4096, 8 rows: 22.7 us against 26.3 with
 // 32 columns; one weight 8.4), three units on their way where a wave has more than two (otherwise they
-// would only be asked for again).  More rows: 64 x 64, unless that leaves a quarter of the 256 compute units
-// without a workgroup (one weight of 1024 x 1024, 252 rows: 4.7 us in 32 x 32 tiles, 13.7 in 64 x 64).
+// would only be asked for again).  More rows: 32 x 32 with k split over the waves while about one of them falls to each
+// of the 256 compute units, then the smallest shared tile of which that holds, each stage of it being the shorter
+// (us on the GPU, weights from memory, in 32 x 32, 64 x 64, 64 x 128, 128 x 128 tiles: one weight of 1024 on 252 rows
+// 4.3, 5.3, 6.5, 7.6; q, k and v of 1024 on 252 rows 8.6, 7.2, 8.9, 11.0, on 512 rows 15.1, 9.1, 9.4, 11.3; one of 4096
+// on 64 rows 11.4, 14.9, 19.1, 21.7, on 252 rows 19.6, 15.9, 19.5, 23.3; q, k and v of 4096 on 128 rows 38.8, 38.5, 32.7,
+// 41.9, on 192 rows 56.7, 51.3, 57.2, 38.1).  Where even 128 x 256 leaves a second round, the rounds decide, a stage of
+// 128 x 128 taking 0.36 us and one of 128 x 256 0.56 (q, k and v of 4096: 700 rows 95.5 and 99.8, 1500 rows 166 and
+// 161, 2048 rows 209 and 181).
 template <int MODE>
 int launch_mode(const ProjectArgs& a, hipStream_t st) {
     if (a.M <= 16) {
         return a.K > 2 * NW * UNIT ? launch_tile<1, 1, 3, MODE>(a, st) : launch_tile<1, 1, 2, MODE>(a, st);
     }
-    const int64_t big = int64_t((a.N + 63) / 64) * a.n_w * ((int64_t(a.M) + 63) / 64);
-    return big < 192 ? launch_tile<2, 2, 2, MODE>(a, st) : launch_tile<4, 4, 2, MODE>(a, st);
+    auto tiles = [&](int bm, int bn) { return int64_t((a.N + bn - 1) / bn) * a.n_w * ((int64_t(a.M) + bm - 1) / bm); };
+    constexpr int CUS = 256;
+    // (shared tiles reach their rows and columns with 32-bit offsets)
+    if (tiles(32, 32) <= CUS + CUS / 8 || int64_t(a.N) * a.K >= int64_t(1) << 30 || a.K > 1 << 22) return launch_tile<2, 2, 2, MODE>(a, st);
+    if (tiles(64, 64) <= CUS) return launch_shared_tile<64, 64, 4, 4, 2, MODE>(a, st);
+    if (tiles(64, 128) <= CUS) return launch_shared_tile<64, 128, 4, 8, 2, MODE>(a, st);
+    const int64_t square = (tiles(128, 128) + CUS - 1) / CUS, wide = (tiles(128, 256) + CUS - 1) / CUS;
+    if (square == 1 || square * 36 < wide * 56) return launch_shared_tile<128, 128, 4, 8, 2, MODE>(a, st);
+    return launch_shared_tile<128, 256, 3, 8, 4, MODE>(a, st);
 }
 
 }  // namespace

@@ -59,7 +59,28 @@ def test_qkv_rotary(rows, heads, n_in):
         _close(got, want.reshape(rows, -1), 2 * n_in)
 
 
-@pytest.mark.parametrize("batch,heads,chunk", [(1, 2, 32), (9, 8, 64), (17, 2, 128)])
+# shared tiles: 64 x 64, 64 x 128, 128 x 128, 128 x 256 by size, their last rows and columns, one to more stages than
+# buffers
+@pytest.mark.parametrize("rows,n_out,n_in", [
+    (17, 9224, 64), (290, 1024, 64), (512, 2048, 128), (500, 2047, 192), (321, 4096, 256), (700, 4104, 320), (129, 12288, 64),
+    (1500, 4096, 448), (2049, 4096, 192), (1023, 8000, 576)])
+def test_linear_in_shared_tiles(rows, n_out, n_in):
+    g = torch.Generator().manual_seed(rows + n_out)
+    x, w = _draw(g, rows, n_in), _draw(g, n_out, n_in, sigma=n_in ** -0.5)
+    guard = torch.full((rows * n_out + 64,), 3.0, dtype=torch.float16, device="cuda")
+    out = guard[:rows * n_out].view(rows, n_out)
+    capi._check(capi.load().ca_linear(x.data_ptr(), w.data_ptr(), out.data_ptr(), rows, n_out, n_in,
+                                      torch.cuda.current_stream().cuda_stream))
+    _close(out, x.double() @ w.double().t(), n_in)
+    assert (guard[rows * n_out:] == 3.0).all()
+
+
+@pytest.mark.parametrize("rows,heads,n_in", [(400, 8, 64), (129, 16, 320), (500, 12, 128), (300, 32, 192), (1030, 31, 256)])
+def test_qkv_rotary_in_shared_tiles(rows, heads, n_in):
+    test_qkv_rotary(rows, heads, n_in)
+
+
+@pytest.mark.parametrize("batch,heads,chunk", [(1, 2, 32), (9, 8, 64), (17, 2, 128), (70, 12, 64)])
 def test_layer_decode_writes_the_pool_as_the_library_path_does(batch, heads, chunk):
     """The folded step and the one with torch projections leave the same cache (but for fp16 roundings), over
     steps in which last chunks fill up, and refuse the same calls."""

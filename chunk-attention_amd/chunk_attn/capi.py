@@ -43,6 +43,11 @@ class PlanInfo(ctypes.Structure):
                 ("stream_per_wave", ctypes.c_int32), ("reserved", ctypes.c_int32)]
 
 
+class ModelLayer(ctypes.Structure):
+    _fields_ = [(name, ctypes.c_void_p) for name in ("ctx", "tree", "wq", "wk", "wv", "wo", "cos_sin_cache", "norm")] + \
+               [("max_position", ctypes.c_int32), ("norm_epsilon", ctypes.c_float)]
+
+
 # name -> (restype, argtypes); every symbol include/chunk_attn_hip.h declares
 SIGNATURES = {
     "ca_last_error": (ctypes.c_char_p, []),
@@ -90,6 +95,11 @@ SIGNATURES = {
     "ca_layer_decode": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, c_i32_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_int] +
                         [ctypes.c_void_p] * 4 + [ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int] +
                         [ctypes.c_void_p] * 4),
+    "ca_model_scratch_bytes": (ctypes.c_size_t, [ctypes.c_int64, ctypes.c_int]),
+    "ca_model_last_rows": (ctypes.c_size_t, [ctypes.c_int64, ctypes.c_int, ctypes.c_int]),
+    "ca_model_pass": (ctypes.c_int, [ctypes.POINTER(ModelLayer), ctypes.c_int, c_i32_p, c_i32_p] + [ctypes.c_int] * 3 +
+                      [ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_float, ctypes.c_int, ctypes.c_void_p,
+                       ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, c_i32_p, ctypes.c_void_p]),
     "ca_rope_append_kv": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
                                          ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_int,
                                          ctypes.c_int, ctypes.c_int, ctypes.c_void_p]),
@@ -469,12 +479,19 @@ def _projection_takes(x, *linears, limit: int = 1 << 20) -> bool:
     n_in = x.shape[-1]
     if n_in == 0 or n_in % 64 or not 0 < x.numel() <= limit or x.data_ptr() % 16:
         return False
+    if torch.is_grad_enabled() and x.requires_grad:
+        return False
+    return _linears_are_plain(n_in, x.device, linears)
+
+
+def _linears_are_plain(n_in: int, device, linears) -> bool:
+    """What each of the modules computes of fp16 rows [..., n_in] on the device is exactly their product with a weight
+    that the projection kernels read (torch.nn.Linear being as torch wrote it)."""
     grad = torch.is_grad_enabled()
     # whatever else may stand between a module and its product: hooks, subclasses, patched forwards, modes
-    if grad and x.requires_grad or torch.is_autocast_enabled() or not plain_call() or \
-            torch.nn.modules.module._has_any_global_hook():
+    if torch.is_autocast_enabled() or not plain_call() or torch.nn.modules.module._has_any_global_hook():
         return False
-    device, Linear, Parameter, half = x.device, torch.nn.Linear, torch.nn.Parameter, torch.float16
+    Linear, Parameter, half = torch.nn.Linear, torch.nn.Parameter, torch.float16
     for m in linears:
         if not is_bare(m, Linear):
             return False
@@ -596,6 +613,30 @@ def _qkv_rotary(x, wq, wk, wv, positions, cos_sin_cache):
     _launch(x.device, load().ca_qkv_rotary, x.data_ptr(), wq.data_ptr(), wk.data_ptr(), wv.data_ptr(), positions.data_ptr(),
             cos_sin_cache.data_ptr(), cos_sin_cache.shape[0], q.data_ptr(), k.data_ptr(), v.data_ptr(), rows, n // 128, n_in)
     return q, k, v
+
+
+def _model_pass(layers, tokens, positions, n_seqs: int, prefill: bool, embedding, norm, epsilon: float, head=None):
+    """A pass of the small model as one native call (see ca_model_pass).  layers: (cache, wq, wk, wv, wo, table, norm
+    weight, epsilon) of each; the caller has checked all of it (tiny_lm._plain_pass).  Returns (logits, or without a
+    head the last norm's rows; the sequence's index in every cache)."""
+    lib, device, hidden = load(), embedding.device, embedding.shape[1]
+    rows = len(tokens)
+    table = (ModelLayer * len(layers))(*[
+        (cache.ctx._h, cache.tree._h, wq.data_ptr(), wk.data_ptr(), wv.data_ptr(), wo.data_ptr(), t.data_ptr(), w.data_ptr(),
+         t.shape[0], eps) for cache, wq, wk, wv, wo, t, w, eps in layers])
+    ids, ids_ptr = _i32(tokens)
+    pos, pos_ptr = _i32(positions)
+    scratch = torch.empty(lib.ca_model_scratch_bytes(rows, hidden) // 2, dtype=torch.float16, device=device)
+    index = (ctypes.c_int32 * len(layers))()
+    logits = None if head is None else torch.empty((n_seqs, head.shape[0]), dtype=torch.float16, device=device)
+    _launch(device, lib.ca_model_pass, table, len(layers), ids_ptr, pos_ptr, n_seqs, rows // n_seqs, int(prefill),
+            embedding.data_ptr(), embedding.shape[0], norm.data_ptr(), epsilon, hidden, scratch.data_ptr(),
+            None if head is None else head.data_ptr(), 0 if head is None else head.shape[0],
+            None if head is None else logits.data_ptr(), index)
+    if head is None:
+        at = lib.ca_model_last_rows(rows, hidden, n_seqs) // 2
+        logits = scratch[at:at + n_seqs * hidden].view(n_seqs, hidden)
+    return logits, list(index)
 
 
 def max_chunks_for(memory_mb: int, chunk_size: int, n_heads: int, d_head: int, elem_bytes: int = 2) -> int:
@@ -1096,6 +1137,14 @@ class Attention:
         """(K, V) pool tensors viewed as [max_chunks, H, c, d]."""
         shape = (self.max_chunks, self.n_heads, self.chunk_size, self.d_head)
         return self.key_storage.view(shape), self.value_storage.view(shape)
+
+
+_ADD_SEQ = Attention.add_seq
+
+
+def is_plain_cache_to_fill(cache) -> bool:
+    """is_plain_cache, and nobody has replaced its add_seq either."""
+    return is_plain_cache(cache) and "add_seq" not in cache.__dict__ and Attention.add_seq is _ADD_SEQ
 
 
 _STEPS = ("append_token_rotary", "forward", "reserve", "refresh_kernel_context")      # of a decode pass

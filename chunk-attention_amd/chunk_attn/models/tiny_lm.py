@@ -6,8 +6,9 @@ scheduler and the decode path end to end with seeded weights; it is not a traine
 """
 from __future__ import annotations
 
+import array
 import math
-from typing import List
+from typing import List, Optional
 
 import torch
 from torch import nn
@@ -32,6 +33,12 @@ class RMSNorm(nn.Module):
 
 _NORM_FORWARD = RMSNorm.forward
 _HOST = torch.device("cpu")
+
+
+def _is_plain(w, shape, device: torch.device) -> bool:
+    """A parameter that kernels can read by its address."""
+    return type(w) is nn.Parameter and w.dtype is torch.float16 and w.device == device and w.shape == shape and \
+        w.is_contiguous() and w.data_ptr() % 16 == 0
 
 
 def _pins(device: torch.device) -> bool:
@@ -80,6 +87,19 @@ class AttentionOnlyLM(nn.Module):
             input_ids = [[s[-1]] for s in seqs]
             position_ids = [[len(s) - 1] for s in seqs]
         dev = self.embed_tokens.weight.device
+        joined = self._adds_in_norms()
+        layers = self._plain_pass(seqs, input_ids, kv_caches, prefill, dev) if joined else None
+        if layers:
+            head = self.lm_head.weight if capi.projection_pays(len(seqs), self.hidden_size, self.vocab_size) and \
+                capi._linears_are_plain(self.hidden_size, dev, (self.lm_head,)) else None
+            out, index = capi._model_pass(layers, [t for ids in input_ids for t in ids], [p for pos in position_ids for p in pos],
+                                          len(seqs), prefill, self.embed_tokens.weight, self.input_norms[0].weight,
+                                          self.input_norms[0].eps, head)
+            if prefill:
+                for layer, idx in zip(self.layers, index):
+                    layer.last_indices = [idx]
+                seqs[0].index = index[-1]
+            return out if head is not None else self.lm_head(out)
         # one upload, from pinned memory: the host does not wait for what the GPU still has to do (the device is
         # named: only host memory can be pinned, whatever the default device is)
         pinned = _pins(dev)
@@ -87,7 +107,6 @@ class AttentionOnlyLM(nn.Module):
                                 pin_memory=pinned).to(dev, non_blocking=pinned)
         hidden = self.embed_tokens(ids)
         token_lists = [s.tokens for s in seqs]
-        joined = self._adds_in_norms()
         normed = self.input_norms[0](hidden) if len(self.layers) else None
         for i, layer in enumerate(self.layers):
             out = layer(normed, token_lists, pos, kv_caches[i], prefill)
@@ -110,6 +129,41 @@ class AttentionOnlyLM(nn.Module):
                 capi._projection_takes(last, self.lm_head):
             return capi._linear(last, self.lm_head.weight)
         return self.lm_head(last)
+
+    def _plain_pass(self, seqs, input_ids, kv_caches, prefill: bool, dev: torch.device) -> Optional[list]:
+        """The layers as capi._model_pass takes them, if the pass is one that the native call computes as the modules
+        would (given _adds_in_norms): a decode step or one prompt, every layer's projections its own kernels' business,
+        caches and parameters plain, and no capture, under which ids are not uploaded either."""
+        hidden, n = self.hidden_size, len(self.layers)
+        if n == 0 or len(kv_caches) < n or not seqs or not input_ids[0] or (prefill and len(seqs) != 1) or dev.type != "cuda" or \
+                torch.cuda.is_current_stream_capturing():
+            return None
+        rows = len(seqs) * len(input_ids[0])
+        if not (capi.projection_pays(rows, hidden, hidden) or
+                prefill and capi.shared_tiles_pay(rows, hidden, hidden, 3) and capi.shared_tiles_pay(rows, hidden, hidden, 1)):
+            return None
+        try:
+            array.array("i", [t for ids in input_ids for t in ids])
+        except (TypeError, OverflowError):             # ids that are no 32-bit numbers: torch's business
+            return None
+        norms = (*self.input_norms, self.norm)
+        embedding = self.embed_tokens
+        if len(norms) != n + 1 or embedding.max_norm is not None or not _is_plain(embedding.weight, (self.vocab_size, hidden), dev) or \
+                not all([_is_plain(m.weight, (hidden,), dev) for m in norms]):
+            return None
+        plain_cache = capi.is_plain_cache_to_fill if prefill else capi.is_plain_cache
+        layers = []
+        for layer, norm, cache in zip(self.layers, norms[1:], kv_caches):
+            linears = (layer.q_proj, layer.k_proj, layer.v_proj, layer.o_proj)
+            table = layer._plain_rotary(dev) if layer.head_dim == 128 and layer.num_heads * 128 == hidden else None
+            if table is None or not capi._linears_are_plain(hidden, dev, linears) or not plain_cache(cache) or \
+                    cache.d_head != 128 or cache.n_heads != layer.num_heads or cache.device != dev:
+                return None
+            weights = [m.weight for m in linears]
+            if any([w.shape[0] != hidden for w in weights]):
+                return None
+            layers.append((cache, *weights, table, norm.weight, norm.eps))
+        return layers
 
     def _adds_in_norms(self) -> bool:
         """A layer's residual is added in the norm behind it, in place: nothing may want the tensors it overwrites

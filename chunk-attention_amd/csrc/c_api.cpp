@@ -1024,6 +1024,96 @@ int ca_layer_decode(ca_ctx* c, ca_tree* tree, const int32_t* tokens, int n_seqs,
     });
 }
 
+namespace {
+// Where a model pass keeps its rows: positions, residual, the norms' rows (and what the output projection leaves
+// there), q, k, v and the attention's output.
+struct ModelRows {
+    int64_t rows;
+    int hidden;
+    size_t row_bytes() const { return size_t(rows) * hidden * 2; }
+    size_t at(int buffer) const { return align_up(size_t(rows) * 8, 16) + size_t(buffer) * row_bytes(); }
+};
+}  // namespace
+
+size_t ca_model_scratch_bytes(int64_t n_rows, int hidden) {
+    return n_rows < 0 || hidden < 0 ? 0 : ModelRows{ n_rows, hidden }.at(6);
+}
+
+size_t ca_model_last_rows(int64_t n_rows, int hidden, int n_seqs) {
+    return ModelRows{ n_rows, hidden }.at(1) + size_t(n_rows - n_seqs) * hidden * 2;
+}
+
+int ca_model_pass(const ca_model_layer* layers, int n_layers, const int32_t* tokens, const int32_t* positions,
+                  int n_seqs, int n_tokens, int prefill, const void* embedding, int vocab, const void* norm,
+                  float norm_epsilon, int hidden, void* scratch, const void* head, int n_logits, void* logits,
+                  int32_t* seq_idx, void* stream) {
+    if (!layers || n_layers < 1 || !tokens || !positions || n_seqs < 1 || n_tokens < 1 || hidden < 128 || hidden % 128 != 0 ||
+        int64_t(n_seqs) * n_tokens > (1 << 24) || (prefill ? n_seqs != 1 || !seq_idx : n_tokens != 1)) {
+        return fail(CA_ERR_INVALID, "bad argument");
+    }
+    if (!embedding || !norm || !scratch || !aligned16(embedding) || !aligned16(norm) || !aligned16(scratch) || !(norm_epsilon >= 0.f)) {
+        return fail(CA_ERR_INVALID, "null or misaligned device pointer");
+    }
+    const int rows = n_seqs * n_tokens, H = hidden / 128;
+    for (int r = 0; r < rows; r++) {
+        if (tokens[r] < 0 || tokens[r] >= vocab) return fail(CA_ERR_INVALID, "token id " + std::to_string(tokens[r]) + " is outside the vocabulary");
+    }
+    const ModelRows at{ rows, hidden };
+    char* base = static_cast<char*>(scratch);
+    int64_t* pos = reinterpret_cast<int64_t*>(base);
+    char *residual = base + at.at(0), *x = base + at.at(1), *q = base + at.at(2), *k = base + at.at(3), *v = base + at.at(4),
+         *attn = base + at.at(5);
+    for (int i = 0; i < n_layers; i++) {
+        const ca_model_layer& layer = layers[i];
+        if (!layer.ctx || !layer.tree || layer.ctx->H != H) return fail(CA_ERR_INVALID, "a layer's cache does not fit the model");
+        if (int rc = check_attention_shape(layer.ctx)) return rc;
+        if (!layer.norm || !aligned16(layer.norm) || !(layer.norm_epsilon >= 0.f)) return fail(CA_ERR_INVALID, "null or misaligned device pointer");
+        ca::ProjectArgs in = qkv_append_args(layer.ctx, layer.wq, layer.wk, layer.wv, pos, layer.cos_sin_cache, layer.max_position, q);
+        if (int rc = check_project(in, x, rows, hidden, hidden)) return rc;
+        ca::ProjectArgs out;
+        out.n_w = 1;
+        out.w[0] = layer.wo;
+        out.y[0] = x;
+        if (int rc = check_project(out, attn, rows, hidden, hidden)) return rc;
+    }
+    if (head) {
+        ca::ProjectArgs out;
+        out.n_w = 1;
+        out.w[0] = head;
+        out.y[0] = logits;
+        if (int rc = check_project(out, x, n_seqs, n_logits, hidden)) return rc;
+    }
+    Range range("ca_model_pass");
+    return guarded([&]() -> int {
+        hipStream_t st = static_cast<hipStream_t>(stream);
+        if (int rc = launch_rc(ca::launch_embed_norm(embedding, tokens, positions, rows, residual, x, pos, norm, norm_epsilon, hidden, st), "embedding launch")) return rc;
+        std::vector<int32_t> slots;
+        for (int i = 0; i < n_layers; i++) {
+            const ca_model_layer& layer = layers[i];
+            ca_ctx* c = layer.ctx;
+            if (!prefill) {
+                if (int rc = ca_layer_decode(c, layer.tree, tokens, n_seqs, x, hidden, layer.wq, layer.wk, layer.wv, layer.wo, hidden,
+                                             pos, layer.cos_sin_cache, layer.max_position, q, attn, x, stream)) return rc;
+            } else {
+                if (int rc = ca_qkv_rotary(x, layer.wq, layer.wk, layer.wv, pos, layer.cos_sin_cache, layer.max_position, q, k, v, rows, H, hidden, stream)) return rc;
+                if (int rc = ca_causal_attention(q, k, v, attn, 1, n_tokens, H, 128, stream)) return rc;
+                int begin = 0, n_new = 0;
+                slots.resize(n_tokens / c->C + 2);
+                if (int rc = ca_tree_add_seq(layer.tree, tokens, n_tokens, &seq_idx[i], &begin, slots.data(), static_cast<int>(slots.size()), &n_new)) return rc;
+                ca_ctx_invalidate(c);
+                if (int rc = ca_scatter_kv(c, k, v, n_tokens, begin, slots.data(), n_new, stream)) return rc;
+                if (int rc = ca_linear(attn, layer.wo, x, rows, hidden, hidden, stream)) return rc;
+                if (int rc = settle(c, layer.tree, ca_tree_n_seqs(layer.tree), stream)) return rc;
+            }
+            // from the last layer on the last positions alone
+            const size_t skip = i + 1 == n_layers ? size_t(rows - n_seqs) * hidden * 2 : 0;
+            if (int rc = ca_add_rms_norm(x + skip, residual + skip, layer.norm, layer.norm_epsilon, i + 1 == n_layers ? n_seqs : rows, hidden, stream)) return rc;
+        }
+        if (!head) return CA_OK;
+        return ca_linear(base + ca_model_last_rows(rows, hidden, n_seqs), head, logits, n_seqs, n_logits, hidden, stream);
+    });
+}
+
 int ca_rope_append_kv(ca_ctx* c, const int64_t* positions, void* q, const void* k, const void* v,
                       const void* cos_sin_cache, int max_position, int rot_dim, int is_neox,
                       int n_seqs, void* stream) {

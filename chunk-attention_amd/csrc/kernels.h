@@ -128,6 +128,12 @@ int launch_rope_append(const LaunchArgs& a, const RotaryArgs& r, const void* k, 
 int launch_rms_norm(void* out, void* input, void* residual, const void* weight, float epsilon,
                     int64_t n_tokens, int hidden, bool vec8, bool mean_of_rounded, hipStream_t st);
 
+// Rows ids[r] of the embedding [vocab, hidden] into residual and, normalised, into out; positions[r] into
+// positions_out (ids and positions: host arrays; the others device, 16-byte aligned, hidden a multiple of 8).
+constexpr int kEmbedRows = 448;  // of one launch
+int launch_embed_norm(const void* embedding, const int32_t* ids, const int32_t* positions, int n_rows, void* residual,
+                      void* out, int64_t* positions_out, const void* weight, float epsilon, int hidden, hipStream_t st);
+
 // Causal attention of whole prompts: q, k, v, out [batch, n_tokens, n_heads, 128] fp16, contiguous and
 // 16-byte aligned; out must not overlap the inputs.
 int launch_causal_attention(const void* q, const void* k, const void* v, void* out, int batch, int n_tokens, int n_heads,

@@ -446,6 +446,35 @@ int ca_layer_decode(ca_ctx* ctx, ca_tree* tree, const int32_t* tokens, int n_seq
                     const int64_t* positions_dev, const void* cos_sin_cache, int max_position, void* q,
                     void* attn, void* y, void* stream);
 
+/* One layer of a model for ca_model_pass: its cache, its weights [hidden, hidden] each, its rotary table
+ * [max_position, 128], and the weight [hidden] and epsilon of the norm behind it. */
+typedef struct {
+    ca_ctx* ctx;
+    ca_tree* tree;
+    const void *wq, *wk, *wv, *wo;
+    const void* cos_sin_cache;
+    const void* norm;
+    int32_t max_position;
+    float norm_epsilon;
+} ca_model_layer;
+
+/* A pass of a pre-norm attention-only model (modeling_llama.py:206-235, without its MLP): embedding and first norm,
+ * then per layer the attention layer and the residual's addition in the norm behind it (ca_add_rms_norm), then, if
+ * `head` is not null, logits [n_seqs, n_logits] = last rows . head^T.
+ *   prefill == 0: one token per sequence of every cache (n_tokens is 1), per layer ca_layer_decode;
+ *   prefill == 1: one sequence (n_seqs is 1) of n_tokens tokens: ca_qkv_rotary, ca_causal_attention, ca_tree_add_seq,
+ *   ca_scatter_kv, ca_linear, room for the next token; seq_idx[layer] receives the sequence's index in that cache.
+ * tokens and positions: host, n_seqs * n_tokens; every id within the embedding [vocab, hidden].  hidden is the
+ * context's n_heads * 128.  scratch: ca_model_scratch_bytes(rows, hidden) bytes of device memory, 16-byte aligned;
+ * the last norm's rows start ca_model_last_rows(rows, hidden, n_seqs) bytes into it.  What a call refuses for its
+ * arguments leaves every cache as it was. */
+size_t ca_model_scratch_bytes(int64_t n_rows, int hidden);
+size_t ca_model_last_rows(int64_t n_rows, int hidden, int n_seqs);
+int ca_model_pass(const ca_model_layer* layers, int n_layers, const int32_t* tokens, const int32_t* positions,
+                  int n_seqs, int n_tokens, int prefill, const void* embedding, int vocab, const void* norm,
+                  float norm_epsilon, int hidden, void* scratch, const void* head, int n_logits, void* logits,
+                  int32_t* seq_idx, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -147,23 +147,23 @@ class AttentionOnlyLM(nn.Module):
         except (TypeError, OverflowError):             # ids that are no 32-bit numbers: torch's business
             return None
         norms = (*self.input_norms, self.norm)
-        embedding = self.embed_tokens
+        embedding, norm_weights = self.embed_tokens, [m._parameters.get("weight") for m in norms]
         if len(norms) != n + 1 or embedding.max_norm is not None or not _is_plain(embedding.weight, (self.vocab_size, hidden), dev) or \
-                not all([_is_plain(m.weight, (hidden,), dev) for m in norms]):
+                not all([_is_plain(w, (hidden,), dev) for w in norm_weights]):
             return None
+        # (by the modules' own dictionaries: __getattr__ costs as much as a launch here, a few dozen times a pass)
+        linears = [m[name] for m in [layer._modules for layer in self.layers] for name in ("q_proj", "k_proj", "v_proj", "o_proj")]
+        if not capi._linears_are_plain(hidden, dev, linears):
+            return None
+        weights = [m._parameters["weight"] for m in linears]
         plain_cache = capi.is_plain_cache_to_fill if prefill else capi.is_plain_cache
         layers = []
-        for layer, norm, cache in zip(self.layers, norms[1:], kv_caches):
-            linears = (layer.q_proj, layer.k_proj, layer.v_proj, layer.o_proj)
+        for i, (layer, cache) in enumerate(zip(self.layers, kv_caches)):
             table = layer._plain_rotary(dev) if layer.head_dim == 128 and layer.num_heads * 128 == hidden else None
-            if table is None or not capi._linears_are_plain(hidden, dev, linears) or not plain_cache(cache) or \
-                    cache.d_head != 128 or cache.n_heads != layer.num_heads or cache.device != dev:
+            if table is None or not plain_cache(cache) or cache.d_head != 128 or cache.n_heads != layer.num_heads or cache.device != dev:
                 return None
-            weights = [m.weight for m in linears]
-            if any([w.shape[0] != hidden for w in weights]):
-                return None
-            layers.append((cache, *weights, table, norm.weight, norm.eps))
-        return layers
+            layers.append((cache, *weights[4 * i:4 * i + 4], table, norm_weights[i + 1], norms[i + 1].eps))
+        return layers if all([w.size(0) == hidden for w in weights]) else None
 
     def _adds_in_norms(self) -> bool:
         """A layer's residual is added in the norm behind it, in place: nothing may want the tensors it overwrites

@@ -59,28 +59,7 @@ def test_qkv_rotary(rows, heads, n_in):
         _close(got, want.reshape(rows, -1), 2 * n_in)
 
 
-# shared tiles: 64 x 64, 64 x 128, 128 x 128, 128 x 256 by size, their last rows and columns, one to more stages than
-# buffers
-@pytest.mark.parametrize("rows,n_out,n_in", [
-    (17, 9224, 64), (290, 1024, 64), (512, 2048, 128), (500, 2047, 192), (321, 4096, 256), (700, 4104, 320), (129, 12288, 64),
-    (1500, 4096, 448), (2049, 4096, 192), (1023, 8000, 576)])
-def test_linear_in_shared_tiles(rows, n_out, n_in):
-    g = torch.Generator().manual_seed(rows + n_out)
-    x, w = _draw(g, rows, n_in), _draw(g, n_out, n_in, sigma=n_in ** -0.5)
-    guard = torch.full((rows * n_out + 64,), 3.0, dtype=torch.float16, device="cuda")
-    out = guard[:rows * n_out].view(rows, n_out)
-    capi._check(capi.load().ca_linear(x.data_ptr(), w.data_ptr(), out.data_ptr(), rows, n_out, n_in,
-                                      torch.cuda.current_stream().cuda_stream))
-    _close(out, x.double() @ w.double().t(), n_in)
-    assert (guard[rows * n_out:] == 3.0).all()
-
-
-@pytest.mark.parametrize("rows,heads,n_in", [(400, 8, 64), (129, 16, 320), (500, 12, 128), (300, 32, 192), (1030, 31, 256)])
-def test_qkv_rotary_in_shared_tiles(rows, heads, n_in):
-    test_qkv_rotary(rows, heads, n_in)
-
-
-@pytest.mark.parametrize("batch,heads,chunk", [(1, 2, 32), (9, 8, 64), (17, 2, 128), (70, 12, 64)])
+@pytest.mark.parametrize("batch,heads,chunk", [(1, 2, 32), (9, 8, 64), (17, 2, 128)])
 def test_layer_decode_writes_the_pool_as_the_library_path_does(batch, heads, chunk):
     """The folded step and the one with torch projections leave the same cache (but for fp16 roundings), over
     steps in which last chunks fill up, and refuse the same calls."""
@@ -216,46 +195,6 @@ def test_model_with_its_adds_in_the_norms_keeps_every_bit():
             seq.append(7)
             out[-1].append(model.logits([seq], caches, False))
     assert all(torch.equal(a, b) for a, b in zip(*out))
-
-
-@pytest.mark.parametrize("hidden,layers,prompts,chunk,vocab", [
-    (128, 1, [1, 5], 32, 40), (1024, 3, [449, 30, 449], 64, 300), (512, 2, [900, 65, 64, 63], 128, 1001)])
-def test_native_model_pass_keeps_every_bit(hidden, layers, prompts, chunk, vocab):
-    """One native call a pass against the modules' own calls (a hook on a norm keeps them): prompts on both sides of
-    the ids that one launch takes, decode steps over which last chunks fill up, the caches afterwards."""
-    from chunk_attn.models.sequence import Sequence
-    from chunk_attn.models.tiny_lm import AttentionOnlyLM
-    runs = []
-    for hooked in (False, True):
-        model = AttentionOnlyLM(vocab, hidden, hidden // 128, layers, chunk_size=chunk, memory_mb=32, seed=6)
-        if hooked:
-            model.norm.register_forward_hook(lambda m, a, out: None)
-        caches, running, out = model.create_kv_caches(), [], []
-        with torch.inference_mode():
-            for p in prompts:
-                seq = Sequence([t * 7 % vocab for t in range(p)])
-                assert hooked or model._plain_pass([seq], [seq.tokens], caches, True, torch.device("cuda:0")) is not None
-                out.append(model.logits([seq], caches, True))
-                running.insert(seq.index, seq)
-                assert all(layer.last_indices == [seq.index] for layer in model.layers)
-            for t in range(5):
-                for s, seq in enumerate(running):
-                    seq.append((11 * t + 3 * s) % vocab)
-                out.append(model.logits(running, caches, False))
-            if not hooked:
-                before = [c.tree.get_chunks() for c in caches]
-                for bad in (vocab, -1):
-                    with pytest.raises(RuntimeError, match="vocabulary"):
-                        model.logits([Sequence([0, bad])], caches, True)
-                assert all((a == c.tree.get_chunks()).all() for a, c in zip(before, caches))
-        rows = [c.tree.get_chunks() for c in caches]
-        pools = [[p[slot][:, :n].clone() for slot, n, _, _ in r for p in c.pool_views()] for r, c in zip(rows, caches)]
-        runs.append((out, rows, pools))
-    assert all(torch.equal(a, b) for a, b in zip(runs[0][0], runs[1][0]))
-    for a, b in zip(*(r[1] for r in runs)):
-        assert (a == b).all()
-    for a, b in zip(*(r[2] for r in runs)):
-        assert all(torch.equal(x, y) for x, y in zip(a, b))
 
 
 def test_projections_refuse_what_their_kernels_cannot_read():

@@ -83,9 +83,11 @@ __device__ __forceinline__ void load_to_lds16(const char* src, half_t* dst) {
 //
 // What bounds it: matrix ops (half of them the second P.V product below) and the vector ops of the softmax are
 // about equal, and each wave's run of them is one dependent chain; what hides a chain is another wave.  TILE 32
-// holds four workgroups a compute unit (118 registers, 32 KB), 64 two.  32 heads, 2048 tokens: 66 us, 8 x 300
-// tokens 22 us; 16 heads, 8 x 1000 tokens 66 us (32 rows a wave, 64 keys a tile, two workgroups a unit: 81, 40 and
-// 85).  Long runs of large ones are held back by the clock, which falls with what they draw (about 1.7 GHz).
+// holds four workgroups a compute unit (110 registers, 32 KB), 64 two.  32 heads, 2048 tokens: 63.4 us (66.2 with the
+// places of the tiles and the clamps at the prompt's end computed in every tile), 3000 tokens 120 (126), 8 x 300
+// tokens 21.8 us; 16 heads, 8 x 1000 tokens 62.6 (64.5).  Two blocks of 16 rows a wave, which halve the reads from LDS,
+// leave two waves to a SIMD: 67 to 85, 114 to 150, 21 to 30 and 62 to 87.  Long runs of large ones are held back by
+// the clock, which falls with what they draw (about 1.7 GHz).
 //
 // The probabilities are fp32; the matrix cores take fp16.  p = hi + lo with hi = fp16(p) and
 // lo = fp16(p - hi) carries 21 bits of p at the price of a second P.V product, and p is scaled by 2^8
@@ -144,11 +146,19 @@ __global__ __launch_bounds__(WG, TILE == 32 ? 4 : 2) void causal_attention_kerne
         const char* __restrict__ kg = reinterpret_cast<const char*>(k + base + size_t(TILE * t) * stride);
         const char* __restrict__ vg = reinterpret_cast<const char*>(v + base + size_t(TILE * t) * stride);
         const int left = n - 1 - TILE * t;
+        if (left >= TILE - 1) {
+#pragma unroll
+            for (int r = 0; r < RPW / 4; r++) {
+                load_to_lds16(kg + whole[r], &sm.k[buf][(RPW * w + 4 * r) * D]);
+                load_to_lds16(vg + whole[r], &sm.v[buf][(RPW * w + 4 * r) * D]);
+            }
+            return;
+        }
 #pragma unroll
         for (int r = 0; r < RPW / 4; r++) {
             unsigned off = whole[r];
             const int kr = RPW * w + 4 * r + g;
-            if (left < TILE - 1 && kr > left) off -= unsigned(kr - left) * unsigned(stride) * 2;
+            if (kr > left) off -= unsigned(kr - left) * unsigned(stride) * 2;
             load_to_lds16(kg + off, &sm.k[buf][(RPW * w + 4 * r) * D]);
             load_to_lds16(vg + off, &sm.v[buf][(RPW * w + 4 * r) * D]);
         }
@@ -160,20 +170,20 @@ __global__ __launch_bounds__(WG, TILE == 32 ? 4 : 2) void causal_attention_kerne
     auto tile_body = [&](int t, const half_t* __restrict__ kt, const half_t* __restrict__ vt, auto masked_tag) {
         constexpr bool MASKED = decltype(masked_tag)::value;   // some key of the tile lies after some row of the wave
         // The places of a row's pieces differ in a few bits of the address: one base a lane, the others by
-        // exclusive or, formed where they are used (hoisted out of the loop they cost twelve registers).
-        int kbase = place(i, g), vbase = place(4 * g + (i >> 2), (i >> 1) & 1) + 4 * (i & 1);
+        // exclusive or, formed where they are used (hoisted out of the loop they cost twelve registers); in bytes, so
+        // that nothing but the exclusive or is left of them.
+        int kbase = 2 * place(i, g), vbase = 2 * place(4 * g + (i >> 2), (i >> 1) & 1) + 8 * (i & 1);   // bytes
         asm volatile("" : "+v"(kbase), "+v"(vbase));
         f4 sc[TB];
 #pragma unroll
         for (int tb = 0; tb < TB; tb++) {
             h8 kop[4];
 #pragma unroll
-            for (int ks = 0; ks < 4; ks++) kop[ks] = *reinterpret_cast<const h8*>(&kt[16 * D * tb + (kbase ^ (32 * ks))]);
+            for (int ks = 0; ks < 4; ks++) kop[ks] = *reinterpret_cast<const h8*>(reinterpret_cast<const char*>(kt) + (kbase ^ (64 * ks)) + 32 * D * tb);
             f4 acc = f4{ 0.f, 0.f, 0.f, 0.f };
 #pragma unroll
             for (int ks = 0; ks < 4; ks++) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(kop[ks], qreg[ks], acc, 0, 0, 0);
             sc[tb] = acc;
-            __builtin_amdgcn_sched_barrier(0);
         }
         if constexpr (MASKED) {  // selects, not branches, between a matrix op and its first reader
 #pragma unroll
@@ -224,7 +234,7 @@ __global__ __launch_bounds__(WG, TILE == 32 ? 4 : 2) void causal_attention_kerne
                 h8 a[4];
 #pragma unroll
                 for (int d = 0; d < 4; d++) {                  // rows key and key + 16 are swizzled alike
-                    const half_t* p0 = &vt[32 * D * tp + (vbase ^ (16 * (4 * half + d)))];
+                    const half_t* p0 = reinterpret_cast<const half_t*>(reinterpret_cast<const char*>(vt) + (vbase ^ (32 * (4 * half + d))) + 64 * D * tp);
                     const h4 x = lds_read_tr(p0), y = lds_read_tr(p0 + 16 * D);
                     a[d] = h8{ x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3] };
                 }
@@ -245,13 +255,21 @@ __global__ __launch_bounds__(WG, TILE == 32 ? 4 : 2) void causal_attention_kerne
     };
     fetch_tile(0, 0);
     const int n_whole = q0 / TILE;                             // tiles that lie before every row of the workgroup
-    for (int t = 0; t < n_whole; t++) {
+    int t = 0;
+    for (; t + 1 < n_whole; t += 2) {                          // by two: the buffers' places are constants
         arrive(t);
-        tile_body(t, sm.k[t & 1], sm.v[t & 1], std::false_type{});
+        tile_body(t, sm.k[0], sm.v[0], std::false_type{});
+        arrive(t + 1);
+        tile_body(t + 1, sm.k[1], sm.v[1], std::false_type{});
+    }
+    if (t < n_whole) {
+        arrive(t);
+        tile_body(t, sm.k[0], sm.v[0], std::false_type{});
+        t++;
     }
     // The diagonal: waves whose rows all lie before a tile skip it.  Waves begin at multiples of 16, which
     // divides the tile: a wave that takes part has the tile's first key before or at every one of its rows.
-    for (int t = n_whole; t < n_tiles; t++) {
+    for (; t < n_tiles; t++) {
         arrive(t);
         if (TILE * t <= row0) tile_body(t, sm.k[t & 1], sm.v[t & 1], std::true_type{});
     }

@@ -20,6 +20,7 @@
 // that no 128-byte line holds data of two writers.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <cstring>
 #include <mutex>
@@ -1489,10 +1490,12 @@ __global__ __launch_bounds__(WG) void upload_kernel(uint4* __restrict__ dst, con
 
 // The same with what is uploaded as a kernel argument: nothing on the host to keep alive, no event, and no read
 // across the bus, which is what a launch of the kernel above waits for (2.1 us for 1 KB, 3.9 for 6).
+template <int BYTES>
 struct UploadBytes {
-    uint4 piece[kArgUploadBytes / 16];
+    uint4 piece[BYTES / 16];
 };
-__global__ __launch_bounds__(WG) void upload_args_kernel(uint4* __restrict__ dst, int n, const UploadBytes src) {
+template <int BYTES>
+__global__ __launch_bounds__(WG) void upload_args_kernel(uint4* __restrict__ dst, int n, const UploadBytes<BYTES> src) {
     const int idx = threadIdx.x;
     if (idx < n) dst[idx] = src.piece[idx];
 }
@@ -1565,15 +1568,18 @@ __global__ __launch_bounds__(WG) void scatter_kernel(const T* __restrict__ k, co
 
 // K/V rows to explicit places: row i of k and v goes to row targets.row[i] of chunk
 // targets.slot[i] (the beam-search step's row writes, one launch for all candidates).
-constexpr int PUT_ROWS = 64;
+// The argument blocks come in two sizes: what a launch of one beam's rows takes is written across the bus with every
+// launch (a beam search of 4, 61 such launches: 411 -> 324 us a pass).
+constexpr int PUT_ROWS = 64, FEW_ROWS = 8;
+template <int N>
 struct PutTargets {
-    int32_t slot[PUT_ROWS];
-    int32_t row[PUT_ROWS];
+    int32_t slot[N];
+    int32_t row[N];
 };
-template <typename T>
+template <typename T, int N>
 __global__ __launch_bounds__(WG) void put_rows_kernel(const T* __restrict__ k, const T* __restrict__ v,
                                                       T* __restrict__ kpool, T* __restrict__ vpool,
-                                                      PutTargets targets, int first, int n, int H, int C,
+                                                      PutTargets<N> targets, int first, int n, int H, int C,
                                                       int pieces) {
     const int idx = blockIdx.x * WG + threadIdx.x;
     if (idx >= n * H * pieces) return;
@@ -1589,16 +1595,18 @@ __global__ __launch_bounds__(WG) void put_rows_kernel(const T* __restrict__ k, c
 // pairs.skip[y][0..1] (-1: none) are left out, in source and destination alike: the same launch
 // writes them.  Workgroups with y >= n_pairs are the row writers: row i of k and v goes to row
 // put.row[i] of chunk put.slot[i] (what put_rows_kernel does).
-constexpr int COPY_PAIRS = 64;
+constexpr int COPY_PAIRS = 64, FEW_PAIRS = 8;
+template <int N>
 struct CopyPairs {
-    int32_t src[COPY_PAIRS];
-    int32_t dst[COPY_PAIRS];
-    int32_t skip[COPY_PAIRS][2];
+    int32_t src[N];
+    int32_t dst[N];
+    int32_t skip[N][2];
 };
+template <int NP, int NR>
 __global__ __launch_bounds__(WG) void copy_chunks_kernel(uint4* __restrict__ kpool, uint4* __restrict__ vpool,
-                                                         CopyPairs pairs, int n_pairs, int units_per_chunk,
+                                                         CopyPairs<NP> pairs, int n_pairs, int units_per_chunk,
                                                          int units_per_row, int C, const uint4* __restrict__ k,
-                                                         const uint4* __restrict__ v, PutTargets put, int n_put, int H) {
+                                                         const uint4* __restrict__ v, PutTargets<NR> put, int n_put, int H) {
     if (int(blockIdx.y) >= n_pairs) {
         const int idx = (blockIdx.y - n_pairs) * gridDim.x * WG + blockIdx.x * WG + threadIdx.x;
         if (idx >= n_put * H * units_per_row) return;
@@ -1836,15 +1844,20 @@ int launch_upload(void* dst_dev, const void* src_pinned, size_t bytes, hipStream
     return 0;
 }
 
+template <int BYTES>
+static int launch_upload_some(void* dst_dev, const void* src, size_t bytes, hipStream_t st) {
+    static_assert(BYTES / 16 <= WG, "one workgroup, one piece a thread");
+    UploadBytes<BYTES> b;
+    std::memcpy(b.piece, src, bytes);
+    hipLaunchKernelGGL(upload_args_kernel<BYTES>, dim3(1), dim3(WG), 0, st, static_cast<uint4*>(dst_dev), static_cast<int>(bytes / 16), b);
+    CA_LAUNCH_CHECK();
+    return 0;
+}
+
 int launch_upload_args(void* dst_dev, const void* src, size_t bytes, hipStream_t st) {
     if (bytes == 0) return 0;
     if (bytes % 16 != 0 || bytes > kArgUploadBytes) return -1;
-    static_assert(kArgUploadBytes / 16 <= WG, "one workgroup, one piece a thread");
-    UploadBytes b;
-    std::memcpy(b.piece, src, bytes);
-    hipLaunchKernelGGL(upload_args_kernel, dim3(1), dim3(WG), 0, st, static_cast<uint4*>(dst_dev), static_cast<int>(bytes / 16), b);
-    CA_LAUNCH_CHECK();
-    return 0;
+    return bytes <= 1024 ? launch_upload_some<1024>(dst_dev, src, bytes, st) : launch_upload_some<kArgUploadBytes>(dst_dev, src, bytes, st);
 }
 
 int launch_read_probe(const void* dev, size_t bytes, int n_wgs, void* sink, hipStream_t st) {
@@ -1909,77 +1922,96 @@ int launch_scatter(const LaunchArgs& a, const void* k, const void* v, int n_toke
     return 0;
 }
 
+namespace {
+// At most NP pairs and NR rows.
+template <int NP, int NR>
+int launch_copy_some(const LaunchArgs& a, const int32_t* src_dst, int m, const void* k, const void* v,
+                     const int32_t* slot_row, int n_rows, int n_put, int units, int units_per_row, hipStream_t st) {
+    CopyPairs<NP> pairs;
+    for (int i = 0; i < m; i++) {
+        pairs.src[i] = src_dst[2 * i];
+        pairs.dst[i] = src_dst[2 * i + 1];
+        pairs.skip[i][0] = pairs.skip[i][1] = -1;
+        // rows of this pair's chunks that the row writers own
+        for (int r = 0; r < n_rows; r++) {
+            const int slot = slot_row[2 * r], row = slot_row[2 * r + 1];
+            if (slot != pairs.src[i] && slot != pairs.dst[i]) continue;
+            if (pairs.skip[i][0] < 0 || pairs.skip[i][0] == row) {
+                pairs.skip[i][0] = row;
+            } else if (pairs.skip[i][1] < 0 || pairs.skip[i][1] == row) {
+                pairs.skip[i][1] = row;
+            } else {
+                return -1;  // more than two written rows in one pair's chunks: not a beam step
+            }
+        }
+    }
+    PutTargets<NR> put;
+    for (int i = 0; i < n_put; i++) {
+        put.slot[i] = slot_row[2 * i];
+        put.row[i] = slot_row[2 * i + 1];
+    }
+    // enough workgroups per pair to fill the device with a handful of pairs, two 16-byte
+    // pieces of each pool per thread at least
+    const int per_pair = std::max(1, std::min(128, (units + 2 * WG - 1) / (2 * WG)));
+    const int put_wgs = (n_put * a.H * units_per_row + per_pair * WG - 1) / (per_pair * WG);
+    hipLaunchKernelGGL((copy_chunks_kernel<NP, NR>), dim3(per_pair, m + put_wgs), dim3(WG), 0, st,
+                       static_cast<uint4*>(const_cast<void*>(a.kpool)), static_cast<uint4*>(const_cast<void*>(a.vpool)), pairs, m,
+                       units, units_per_row, a.C, static_cast<const uint4*>(k), static_cast<const uint4*>(v), put, n_put, a.H);
+    CA_LAUNCH_CHECK();
+    return 0;
+}
+
+template <typename T, int N>
+int launch_put_some(const LaunchArgs& a, const void* k, const void* v, const int32_t* slot_row, int first, int m,
+                    int pieces, hipStream_t st) {
+    PutTargets<N> t;
+    for (int i = 0; i < m; i++) {
+        t.slot[i] = slot_row[2 * (first + i)];
+        t.row[i] = slot_row[2 * (first + i) + 1];
+    }
+    const int total = m * a.H * pieces;
+    hipLaunchKernelGGL((put_rows_kernel<T, N>), dim3((total + WG - 1) / WG), dim3(WG), 0, st, static_cast<const T*>(k),
+                       static_cast<const T*>(v), static_cast<T*>(const_cast<void*>(a.kpool)),
+                       static_cast<T*>(const_cast<void*>(a.vpool)), t, first, m, a.H, a.C, pieces);
+    CA_LAUNCH_CHECK();
+    return 0;
+}
+}  // namespace
+
 int launch_copy_chunks(const LaunchArgs& a, const int32_t* src_dst, int n_pairs, const void* k, const void* v,
                        const int32_t* slot_row, int n_rows, hipStream_t st) {
     const size_t chunk_bytes = size_t(a.H) * a.C * a.d * 2;
     if (chunk_bytes % 16 != 0 || chunk_bytes / 16 > 0x7fffffff || (a.d * 2) % 16 != 0) return -1;
     if (n_rows > PUT_ROWS || (n_rows > 0 && (!k || !v || !slot_row))) return -1;
+    if (n_pairs == 0) return launch_put_rows(a, k, v, slot_row, n_rows, st);
     const int units = static_cast<int>(chunk_bytes / 16), units_per_row = a.d * 2 / 16;
-    uint4* kp = static_cast<uint4*>(const_cast<void*>(a.kpool));
-    uint4* vp = static_cast<uint4*>(const_cast<void*>(a.vpool));
-    PutTargets put;
-    for (int i = 0; i < PUT_ROWS; i++) {
-        put.slot[i] = (i < n_rows) ? slot_row[2 * i] : 0;
-        put.row[i] = (i < n_rows) ? slot_row[2 * i + 1] : 0;
-    }
-    // enough workgroups per pair to fill the device with a handful of pairs, two 16-byte
-    // pieces of each pool per thread at least
-    int per_pair = (units + 2 * WG - 1) / (2 * WG);
-    if (per_pair > 128) per_pair = 128;
-    if (per_pair < 1) per_pair = 1;
-    for (int i0 = 0; i0 < n_pairs || (i0 == 0 && n_rows > 0); i0 += COPY_PAIRS) {
-        const int m = (n_pairs - i0 < COPY_PAIRS) ? (n_pairs - i0) : COPY_PAIRS;
-        CopyPairs pairs;
-        for (int i = 0; i < COPY_PAIRS; i++) {
-            pairs.src[i] = (i < m) ? src_dst[2 * (i0 + i)] : 0;
-            pairs.dst[i] = (i < m) ? src_dst[2 * (i0 + i) + 1] : 0;
-            pairs.skip[i][0] = pairs.skip[i][1] = -1;
-            // rows of this pair's chunks that the row writers own
-            for (int r = 0; i < m && r < n_rows; r++) {
-                if (put.slot[r] != pairs.src[i] && put.slot[r] != pairs.dst[i]) continue;
-                if (pairs.skip[i][0] < 0 || pairs.skip[i][0] == put.row[r]) {
-                    pairs.skip[i][0] = put.row[r];
-                } else if (pairs.skip[i][1] < 0 || pairs.skip[i][1] == put.row[r]) {
-                    pairs.skip[i][1] = put.row[r];
-                } else {
-                    return -1;  // more than two written rows in one pair's chunks: not a beam step
-                }
-            }
-        }
+    for (int i0 = 0; i0 < n_pairs; i0 += COPY_PAIRS) {
+        const int m = std::min(n_pairs - i0, COPY_PAIRS);
         // the row writers ride along with the first launch
-        const int put_here = (i0 == 0) ? n_rows : 0;
-        const int put_wgs = (put_here * a.H * units_per_row + per_pair * WG - 1) / (per_pair * WG);
-        hipLaunchKernelGGL(copy_chunks_kernel, dim3(per_pair, m + put_wgs), dim3(WG), 0, st, kp, vp, pairs, m, units,
-                           units_per_row, a.C, static_cast<const uint4*>(k), static_cast<const uint4*>(v), put,
-                           put_here, a.H);
-        CA_LAUNCH_CHECK();
+        const int put_here = i0 == 0 ? n_rows : 0;
+        const int rc = m <= FEW_PAIRS && n_rows <= FEW_ROWS
+                         ? launch_copy_some<FEW_PAIRS, FEW_ROWS>(a, src_dst + 2 * i0, m, k, v, slot_row, n_rows, put_here, units, units_per_row, st)
+                         : launch_copy_some<COPY_PAIRS, PUT_ROWS>(a, src_dst + 2 * i0, m, k, v, slot_row, n_rows, put_here, units, units_per_row, st);
+        if (rc != 0) return rc;
     }
     return 0;
 }
 
 int launch_put_rows(const LaunchArgs& a, const void* k, const void* v, const int32_t* slot_row, int n,
                     hipStream_t st) {
-    void* kp = const_cast<void*>(a.kpool);
-    void* vp = const_cast<void*>(a.vpool);
+    const bool vec = a.d % 8 == 0;
+    const int pieces = vec ? a.d / 8 : a.d;
     for (int i0 = 0; i0 < n; i0 += PUT_ROWS) {
-        const int m = (n - i0 < PUT_ROWS) ? (n - i0) : PUT_ROWS;
-        PutTargets t;
-        for (int i = 0; i < PUT_ROWS; i++) {
-            t.slot[i] = (i < m) ? slot_row[2 * (i0 + i)] : 0;
-            t.row[i] = (i < m) ? slot_row[2 * (i0 + i) + 1] : 0;
-        }
-        if (a.d % 8 == 0) {
-            const int pieces = a.d / 8, total = m * a.H * pieces;
-            hipLaunchKernelGGL(put_rows_kernel<uint4>, dim3((total + WG - 1) / WG), dim3(WG), 0, st,
-                               static_cast<const uint4*>(k), static_cast<const uint4*>(v), static_cast<uint4*>(kp),
-                               static_cast<uint4*>(vp), t, i0, m, a.H, a.C, pieces);
+        const int m = std::min(n - i0, PUT_ROWS);
+        int rc;
+        if (m <= FEW_ROWS) {
+            rc = vec ? launch_put_some<uint4, FEW_ROWS>(a, k, v, slot_row, i0, m, pieces, st)
+                     : launch_put_some<uint16_t, FEW_ROWS>(a, k, v, slot_row, i0, m, pieces, st);
         } else {
-            const int pieces = a.d, total = m * a.H * pieces;
-            hipLaunchKernelGGL(put_rows_kernel<uint16_t>, dim3((total + WG - 1) / WG), dim3(WG), 0, st,
-                               static_cast<const uint16_t*>(k), static_cast<const uint16_t*>(v),
-                               static_cast<uint16_t*>(kp), static_cast<uint16_t*>(vp), t, i0, m, a.H, a.C, pieces);
+            rc = vec ? launch_put_some<uint4, PUT_ROWS>(a, k, v, slot_row, i0, m, pieces, st)
+                     : launch_put_some<uint16_t, PUT_ROWS>(a, k, v, slot_row, i0, m, pieces, st);
         }
-        CA_LAUNCH_CHECK();
+        if (rc != 0) return rc;
     }
     return 0;
 }

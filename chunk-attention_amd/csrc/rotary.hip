@@ -66,17 +66,17 @@ __global__ __launch_bounds__(WG) void rotary_vec_kernel(const int64_t* __restric
                                                         half_t* __restrict__ query,
                                                         half_t* __restrict__ key,
                                                         const half_t* __restrict__ cache,
-                                                        int64_t n_tokens, int n_heads, int n_kv_heads,
+                                                        int wgs_per_token, int n_heads, int n_kv_heads,
                                                         int head_size, int rot_dim, int max_position,
                                                         int64_t query_stride, int64_t key_stride) {
     const int embed = rot_dim / 2;
     const int units = IS_NEOX ? embed / 8 : rot_dim / 8;  // work units per head
-    const int64_t per_token = int64_t(n_heads + n_kv_heads) * units;
-    const int64_t idx = int64_t(blockIdx.x) * WG + threadIdx.x;
-    if (idx >= n_tokens * per_token) return;
-    const int64_t token = idx / per_token;
-    const int rem = static_cast<int>(idx % per_token);
-    const int head = rem / units, u = rem % units;
+    // Whole workgroups a token (the token of a workgroup is a scalar division; 64-bit divisions in every thread were
+    // as many vector ops as the rotation twice over: 2048 tokens of 32 + 32 heads 13.4 -> 12.4 us).
+    const int64_t token = blockIdx.x / unsigned(wgs_per_token);
+    const unsigned rem = (blockIdx.x % unsigned(wgs_per_token)) * WG + threadIdx.x;
+    const int head = rem / unsigned(units), u = rem % unsigned(units);
+    if (head >= n_heads + n_kv_heads) return;
     half_t* row = (head < n_heads) ? query + token * query_stride + int64_t(head) * head_size
                                    : key + token * key_stride + int64_t(head - n_heads) * head_size;
     const half_t* cs = cache + clamp_pos(positions[token], max_position) * rot_dim;
@@ -166,16 +166,17 @@ int launch_rotary(const RotaryArgs& r, hipStream_t st) {
                         aligned16(cache);
     if (pieces) {
         const int units = r.is_neox ? r.rot_dim / 16 : r.rot_dim / 8;
-        const int64_t total = r.n_tokens * int64_t(r.n_heads + r.n_kv_heads) * units;
-        if (total <= 0) return 0;
-        if (total > int64_t(0x7fffffff) * WG) return -1;
-        const dim3 grid(static_cast<unsigned>((total + WG - 1) / WG)), block(WG);
+        const int64_t per_token = (int64_t(r.n_heads + r.n_kv_heads) * units + WG - 1) / WG;
+        if (r.n_tokens * per_token <= 0) return 0;
+        if (r.n_tokens * per_token > 0x7fffffff) return -1;
+        const int wgs = static_cast<int>(per_token);
+        const dim3 grid(static_cast<unsigned>(r.n_tokens * per_token)), block(WG);
         if (r.is_neox) {
-            hipLaunchKernelGGL(rotary_vec_kernel<true>, grid, block, 0, st, r.positions, q, k, cache, r.n_tokens,
+            hipLaunchKernelGGL(rotary_vec_kernel<true>, grid, block, 0, st, r.positions, q, k, cache, wgs,
                                r.n_heads, r.n_kv_heads, r.head_size, r.rot_dim, r.max_position,
                                r.query_stride, r.key_stride);
         } else {
-            hipLaunchKernelGGL(rotary_vec_kernel<false>, grid, block, 0, st, r.positions, q, k, cache, r.n_tokens,
+            hipLaunchKernelGGL(rotary_vec_kernel<false>, grid, block, 0, st, r.positions, q, k, cache, wgs,
                                r.n_heads, r.n_kv_heads, r.head_size, r.rot_dim, r.max_position,
                                r.query_stride, r.key_stride);
         }

@@ -43,7 +43,10 @@ enum { kPlain = 0, kRotary = 1, kAppend = 2 };
 // (project_tile_kernel; the line is at launch_mode).
 //
 // Columns of a rotary tile: half of them from the first half of a head, half their partners 64 further on.
-template <int MB, int NB, int R, int MODE>
+// XR: rows of x that are fetched; of a block of 16 the others' products are of whatever stands in LDS, and not stored
+// (up to 8 rows a quarter of a unit's loads: q, k and v of 2048 on 1 row 9.1 -> 8.3 us, of 4096 20.9 -> 20.1, one weight
+// of 1024 3.0 -> 2.8).
+template <int MB, int NB, int R, int XR, int MODE>
 __global__ __launch_bounds__(WG) void project_kernel(const ProjectArgs a) {
     constexpr int MT = 16 * MB, NT = 16 * NB, PITCH = NT + 4;
     constexpr int ROWS = MT + NT;                    // rows of a unit: the tile's columns (rows of W), then its rows
@@ -69,7 +72,7 @@ __global__ __launch_bounds__(WG) void project_kernel(const ProjectArgs a) {
     // Load r of a unit brings rows 8r .. 8r+7, eight lanes to the 128 bytes of a row (requested in the
     // matrix cores' layout, neighbouring lanes would lie in different rows, and every lane would cost a
     // look-up of its own).
-    constexpr int NL = ROWS / 8;
+    constexpr int NL = (NT + XR) / 8;
     const half_t* src[NL];
 #pragma unroll
     for (int r = 0; r < NL; r++) {
@@ -218,12 +221,12 @@ __global__ __launch_bounds__(WG) void project_kernel(const ProjectArgs a) {
     }
 }
 
-template <int MB, int NB, int R, int MODE>
+template <int MB, int NB, int R, int XR, int MODE>
 int launch_tile(const ProjectArgs& a, hipStream_t st) {
     constexpr int MT = 16 * MB, NT = 16 * NB;
     const int64_t wgs = int64_t((a.N + NT - 1) / NT) * a.n_w * ((int64_t(a.M) + MT - 1) / MT);
     if (wgs > 0x7fffffff) return -1;
-    hipLaunchKernelGGL((project_kernel<MB, NB, R, MODE>), dim3(static_cast<unsigned>(wgs)), dim3(WG), 0, st, a);
+    hipLaunchKernelGGL((project_kernel<MB, NB, R, XR, MODE>), dim3(static_cast<unsigned>(wgs)), dim3(WG), 0, st, a);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? 0 : static_cast<int>(e);
 }
@@ -466,13 +469,16 @@ int launch_shared_tile(const ProjectArgs& a, hipStream_t st) {
 // 161, 2048 rows 209 and 181).
 template <int MODE>
 int launch_mode(const ProjectArgs& a, hipStream_t st) {
+    if (a.M <= 8) {
+        return a.K > 2 * NW * UNIT ? launch_tile<1, 1, 3, 8, MODE>(a, st) : launch_tile<1, 1, 2, 8, MODE>(a, st);
+    }
     if (a.M <= 16) {
-        return a.K > 2 * NW * UNIT ? launch_tile<1, 1, 3, MODE>(a, st) : launch_tile<1, 1, 2, MODE>(a, st);
+        return a.K > 2 * NW * UNIT ? launch_tile<1, 1, 3, 16, MODE>(a, st) : launch_tile<1, 1, 2, 16, MODE>(a, st);
     }
     auto tiles = [&](int bm, int bn) { return int64_t((a.N + bn - 1) / bn) * a.n_w * ((int64_t(a.M) + bm - 1) / bm); };
     constexpr int CUS = 256;
     // (shared tiles reach their rows and columns with 32-bit offsets)
-    if (tiles(32, 32) <= CUS + CUS / 8 || int64_t(a.N) * a.K >= int64_t(1) << 30 || a.K > 1 << 22) return launch_tile<2, 2, 2, MODE>(a, st);
+    if (tiles(32, 32) <= CUS + CUS / 8 || int64_t(a.N) * a.K >= int64_t(1) << 30 || a.K > 1 << 22) return launch_tile<2, 2, 2, 32, MODE>(a, st);
     if (tiles(64, 64) <= CUS) return launch_shared_tile<64, 64, 4, 4, 2, MODE>(a, st);
     if (tiles(64, 128) <= CUS) return launch_shared_tile<64, 128, 4, 8, 2, MODE>(a, st);
     const int64_t square = (tiles(128, 128) + CUS - 1) / CUS, wide = (tiles(128, 256) + CUS - 1) / CUS;

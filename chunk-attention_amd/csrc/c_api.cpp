@@ -127,7 +127,8 @@ struct ca_ctx {
     size_t host_blob_cap[kStaging] = {};
     hipEvent_t host_blob_free[kStaging] = {};
     int next_host = 0;
-    bool direct = false;  // forwards over the current plan take the direct form, which reads no device tables
+    bool direct = false;  // fused steps over the current plan take the direct form, which reads no device tables,
+    bool direct_forward = false;  // and so do plain forwards
     // Tables of such a plan are uploaded when something else first reads them (ensure_tables); until then they
     // stand here.
     bool upload_pending = false;
@@ -263,12 +264,23 @@ ca::PlanParams plan_params(const ca_ctx* c, int partition) {
 // tokens only launches of many workgroups gain, where the general path's tables grow too: 8 x 8, 800 + 150, 7.3 and 7.3,
 // but 4 x 32 9.85 and 9.15, 8 x 32 12.3 and 10.5; 16 x 12, 1280 + 100, 9.85 and 10.9; with chunks of 32 4 x 32, 768 +
 // 60, 8.9 and 9.1; 32 x 12 (384 workgroups), 512 + 100, 11.15 and 12.9.
+// A path of one chunk of 128 is one wave's in the general path, whose sums the direct form's two would round
+// otherwise: it stays there, for steps as for forwards.
 bool direct_form(const ca_ctx* c) {
     const ca::Plan& p = c->plan;
     if (p.path_stride == 0 || p.partition != 0 || c->schedule != 0 || c->seg_chunks > 0 || c->stream_chunks > 0) return false;
     const int64_t wgs = int64_t(c->n_seqs) * c->H;
     const int64_t tokens = int64_t(p.path_stride) * c->C;
+    if (c->C > 64 && p.path_stride == 1) return false;
     return wgs <= c->n_cus && (tokens <= 768 || (tokens <= 1280 && c->C >= 64 && 2 * wgs >= c->n_cus));
+}
+
+// Whether the general path, too, is one launch over at most a tile a wave: no partial rows, paths of up to four tiles
+// (chunks of 32 and 64; the same sums, bit for bit).  A plain forward then stays there: its arguments, which the host
+// writes on every call, are fewer (1 x 8, 30 tokens, 4.7 us from call to call, and 4.9 in the direct form; 20 x 12, 60
+// tokens, 4.65 and 4.9).
+bool one_launch_anyway(const ca_ctx* c) {
+    return c->plan.n_part_rows == 0 && c->C <= 64 && int64_t(c->plan.path_stride) * c->C <= 256;
 }
 
 int run_direct(ca_ctx* c, const ca::LaunchArgs& a, hipStream_t st) {
@@ -320,6 +332,7 @@ int upload_plan(ca_ctx* c, hipStream_t st) {
     if (int rc = ensure_dev(c, reinterpret_cast<char**>(&c->part), &c->part_cap, part_bytes)) return rc;
     c->upload_pending = false;
     c->direct = direct_form(c);
+    c->direct_forward = c->direct && !one_launch_anyway(c);
     auto fill = [&](char* to) {
         auto put = [&](size_t at, const void* src, size_t bytes) {
             if (bytes) std::memcpy(to + at, src, bytes);
@@ -338,7 +351,7 @@ int upload_plan(ca_ctx* c, hipStream_t st) {
         c->pending_blob.resize(total);
         fill(c->pending_blob.data());
         c->upload_pending = true;
-        return c->direct ? CA_OK : ensure_tables(c, st);
+        return c->direct_forward ? CA_OK : ensure_tables(c, st);
     }
     const int hb = c->next_host;
     c->next_host = (c->next_host + 1) % ca_ctx::kStaging;
@@ -453,7 +466,7 @@ int run_merge(ca_ctx* c, void* out, hipStream_t st) {
 
 int run_fused(ca_ctx* c, const void* q, void* out, hipStream_t st) {
     const ca::LaunchArgs a = launch_args(c, q, out);
-    if (c->direct) return run_direct(c, a, st);
+    if (c->direct_forward) return run_direct(c, a, st);
     if (c->schedule == 0) {
         // both phases in one launch (shared and stream workgroups overlap), then the merge
         if (int rc = launch_rc(ca::launch_decode(a, static_cast<int>(c->plan.shared_items.size()),
@@ -619,7 +632,7 @@ int ca_attention(ca_ctx* c, const void* q, void* out, int n_seqs, int partition,
         if (!c->timing) return run_fused(c, q, out, st);
         if (int rc = collect_timing(c)) return rc;
         CA_HIP(hipEventRecord(c->ev[0], st));
-        if (c->timing == 1 && c->schedule == 0 && !c->direct) {
+        if (c->timing == 1 && c->schedule == 0 && !c->direct_forward) {
             // the forward as it normally runs: decode launch, then merge launch
             const ca::LaunchArgs a = launch_args(c, q, out);
             if (int rc = launch_rc(ca::launch_decode(a, static_cast<int>(c->plan.shared_items.size()),
@@ -627,7 +640,7 @@ int ca_attention(ca_ctx* c, const void* q, void* out, int n_seqs, int partition,
             CA_HIP(hipEventRecord(c->ev[1], st));
             CA_HIP(hipEventRecord(c->ev[2], st));
             if (int rc = run_merge(c, out, st)) return rc;
-        } else if (c->timing == 1 || c->direct) {  // one launch
+        } else if (c->timing == 1 || c->direct_forward) {  // one launch
             if (int rc = run_fused(c, q, out, st)) return rc;
             CA_HIP(hipEventRecord(c->ev[1], st));
             CA_HIP(hipEventRecord(c->ev[2], st));
@@ -663,7 +676,7 @@ int ca_attention_noalloc(ca_ctx* c, const void* q, void* out, int n_seqs, void* 
     }
     hipStream_t st = static_cast<hipStream_t>(stream);
     ca::LaunchArgs a = launch_args(c, q, out);
-    if (c->direct) return run_direct(c, a, st);
+    if (c->direct_forward) return run_direct(c, a, st);
     a.part = scratch;  // every row that the merge reads is written by the decode launch first
     if (int rc = launch_rc(ca::launch_decode(a, static_cast<int>(c->plan.shared_items.size()),
                                              static_cast<int>(c->plan.stream_items.size()), false, st), "decode launch")) return rc;

@@ -305,6 +305,10 @@ struct StreamPathLds {
     float l[NW];
     int state;  // workgroup-uniform decision flags
 };
+// The direct form's item: a whole sequence, chunk k's slot in lane k of slotv.
+struct DirectItem {
+    int seq, n_chunks, len, slotv;
+};
 // K tiles use the same 288-byte row pitch: a 16-byte-per-lane read is served for lanes 0-7 of two
 // neighbouring 16-lane groups at a time, and with rows 288 B apart those sixteen pieces (rows i,
 // 16-byte columns g and g+1) fall into sixteen different 16-byte bank groups.  (272 B, which only
@@ -347,106 +351,6 @@ template <> union __attribute__((aligned(16))) DecodeLds<kMixNarrow> {
     StreamPathLds st;
 };
 
-// One 64-token sub-tile of a sequence: its loads, scores, online softmax and P.V.  kp / vp: the lane's place in
-// the chunks that supply it, vsub: its valid rows, prow: the wave's row of probabilities in LDS.
-template <int C, int STEP>
-__device__ __forceinline__ void stream_tile(const DecodeArgs& A, int seq, int h, int l, const h8& qv,
-                                            const size_t (&base)[C < 64 ? 64 / C : 1], int vsub,
-                                            bool new_here, float (&prow)[64], float& m_run, float& l_lane, float (&acc)[8]) {
-    constexpr bool APPEND = STEP != kForward;
-    constexpr int NL = 16;                         // 16-byte loads per lane
-    constexpr int LPC = C < 64 ? NL * C / 64 : NL; // of them that one chunk supplies
-    const int g = l >> 4, j = l & 15;
-    const float scale_log2 = A.scale_log2;
-    const bool masked = vsub < 64 || new_here;
-    constexpr int CPT = C < 64 ? 64 / C : 1;
-    const uint4* kp[CPT];
-    const uint4* vp[CPT];
-#pragma unroll
-    for (int cc = 0; cc < CPT; cc++) {
-        kp[cc] = reinterpret_cast<const uint4*>(A.kpool + base[cc]) + l;
-        vp[cc] = reinterpret_cast<const uint4*>(A.vpool + base[cc]) + l;
-    }
-    uint4 kr[NL], vr[NL];
-    if (!masked) {
-#pragma unroll
-        for (int i = 0; i < NL; i++) {
-            const uint4* p = kp[i / LPC] + 64 * (i % LPC);
-            kr[i] = A.stream_nt ? nt_load16(p) : *p;
-        }
-#pragma unroll
-        for (int i = 0; i < NL; i++) {
-            const uint4* p = vp[i / LPC] + 64 * (i % LPC);
-            vr[i] = A.stream_nt ? nt_load16(p) : *p;
-        }
-    } else {
-        // rows past the end of the sequence hold stale data: never read into the math
-        const int vmem = (APPEND && new_here) ? vsub - 1 : vsub;  // rows that the pool holds
-        // The newest token's pieces are requested in front of the tile's own loads: loads
-        // return in order, so they are there when the tile is, at no round trip of their own.
-        uint4 kn = make_uint4(0, 0, 0, 0), vn = make_uint4(0, 0, 0, 0);
-        if constexpr (APPEND) {
-            if (new_here) {
-                const size_t new_off = (size_t(seq) * A.H + h) * D;
-                kn = *(reinterpret_cast<const uint4*>(A.k_new + new_off) + j);
-                vn = *(reinterpret_cast<const uint4*>(A.v_new + new_off) + j);
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < NL; i++) {
-            const bool ok = 4 * i + g < vmem;
-            kr[i] = ok ? kp[i / LPC][64 * (i % LPC)] : make_uint4(0, 0, 0, 0);
-            vr[i] = ok ? vp[i / LPC][64 * (i % LPC)] : make_uint4(0, 0, 0, 0);
-        }
-        if constexpr (APPEND) {
-            if (new_here) {
-                // row vsub - 1 = 4 * i_new + g_new is the newest token: lanes (g_new, j) take
-                // piece j of it from the caller's rows, as if it had been loaded from the pool
-                const int i_new = (vsub - 1) >> 2;
-                const bool mine = ((vsub - 1) & 3) == g;
-#pragma unroll
-                for (int i = 0; i < NL; i++) {
-                    if (i == i_new && mine) {
-                        kr[i] = kn;
-                        vr[i] = vn;
-                    }
-                }
-            }
-        }
-    }
-    float sc[NL];
-#pragma unroll
-    for (int i = 0; i < NL; i++) {
-        sc[i] = dot8(*reinterpret_cast<const h8*>(&kr[i]), qv, 0.f);
-    }
-    // lane (g, j) now owns the score of row 4*(j % NL) + g
-    float s = reduce_rows16<NL>(sc, j) * scale_log2;
-    const int row = 4 * (j % NL) + g;
-    if (row >= vsub || j >= NL) s = NEG_INF;
-    const float m_new = fmaxf(m_run, wave_max(s));
-    const float alpha = fast_exp2(m_run - m_new);
-    const float p = fast_exp2(s - m_new);
-    m_run = m_new;
-    l_lane = l_lane * alpha + p;
-    prow[l] = p;
-#pragma unroll
-    for (int e = 0; e < 8; e++) acc[e] *= alpha;
-    __builtin_amdgcn_wave_barrier();
-    float pr[NL];
-#pragma unroll
-    for (int i = 0; i < NL; i += 4) {
-        const f4 t4 = *reinterpret_cast<const f4*>(&prow[16 * g + i]);
-        pr[i] = t4[0]; pr[i + 1] = t4[1]; pr[i + 2] = t4[2]; pr[i + 3] = t4[3];
-    }
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int i = 0; i < NL; i++) {
-        const h8 vv = *reinterpret_cast<const h8*>(&vr[i]);
-#pragma unroll
-        for (int e = 0; e < 8; e++) acc[e] = __builtin_fmaf(pr[i], float(vv[e]), acc[e]);
-    }
-}
-
 // ---------------------------------------------------------------------------------------
 // stream_path: an item = a run of one sequence's own chunks.  Wave w of the workgroup takes
 // tiles w, w+4, ... of the item (a tile = one chunk, or two chunks at chunk size 32) and reads
@@ -464,16 +368,30 @@ __device__ __forceinline__ void stream_tile(const DecodeArgs& A, int seq, int h,
 // that streams at the memory's speed cost it 9 % of its duration (256 sequences: 192 -> 209 us;
 // dirty lines leave the L2 in dribs and drabs and turn the memory bus around each time), the same
 // rows written by a launch of their own, or at the end of the merge launch, cost 1-3 us.
-template <int C, bool PER_WAVE, int STEP>
+//
+// DIRECT_NW waves (0: an ordinary item of NW): the direct form (direct_kernel).  The item, `direct`, is a whole
+// sequence, its slots come with it in the waves' registers, and a wave takes single 64-token tiles, also of a chunk
+// of 128.
+template <int C, bool PER_WAVE, int STEP, int DIRECT_NW = 0, typename LDS = StreamPathLds>
 __device__ __forceinline__ void stream_path(const DecodeArgs& A, const WorkItem* __restrict__ gi,
-                                            int h, StreamPathLds& sm) {
+                                            int h, LDS& sm, const DirectItem* direct = nullptr) {
+    constexpr bool DIRECT = DIRECT_NW > 0;
+    constexpr int NWV = DIRECT ? DIRECT_NW : NW;
     WorkItem it;  // header only: the inline slots are read from global memory where needed
-    it.seq_begin = gi->seq_begin; it.n_rows = gi->n_rows; it.slot_first = gi->slot_first;
-    it.n_chunks = gi->n_chunks; it.part_row = gi->part_row; it.pos0 = gi->pos0;
-    it.len0 = gi->len0; it.flags = gi->flags;
+    if constexpr (DIRECT) {
+        it.seq_begin = direct->seq; it.n_rows = 1; it.slot_first = 0; it.n_chunks = direct->n_chunks;
+        it.part_row = -1; it.pos0 = 0; it.len0 = direct->len; it.flags = 0;
+    } else {
+        it.seq_begin = gi->seq_begin; it.n_rows = gi->n_rows; it.slot_first = gi->slot_first;
+        it.n_chunks = gi->n_chunks; it.part_row = gi->part_row; it.pos0 = gi->pos0;
+        it.len0 = gi->len0; it.flags = gi->flags;
+    }
     const half_t* __restrict__ q = A.q;
+    const half_t* __restrict__ kpool = A.kpool;
+    const half_t* __restrict__ vpool = A.vpool;
     const int32_t* __restrict__ slots = A.slots;
     const int H = A.H;
+    const float scale_log2 = A.scale_log2;
     const bool coh = A.fuse_merge != 0;  // partial rows are read during this launch
     // A wave works on 64-token sub-tiles: one chunk at chunk size 64, half a chunk at 128, two
     // consecutive chunks of the item at 32 (their loads go out together, so a wave has the same
@@ -488,7 +406,9 @@ __device__ __forceinline__ void stream_path(const DecodeArgs& A, const WorkItem*
     const int tid = threadIdx.x;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave index, known uniform
     const int l = tid & 63, g = l >> 4, j = l & 15;
-    const int slotv = preload_slots(gi, it.slot_first, it.n_chunks, slots, l);
+    int slotv;
+    if constexpr (DIRECT) slotv = direct->slotv;
+    else slotv = preload_slots(gi, it.slot_first, it.n_chunks, slots, l);
     const int seq = it.seq_begin;
     const int len = it.len0 + A.delta_tokens;
 
@@ -553,7 +473,9 @@ __device__ __forceinline__ void stream_path(const DecodeArgs& A, const WorkItem*
     };
     bool tried = !can_fold;
 
-    for (int t = (PER_WAVE ? 0 : w) * CPT; t < it.n_chunks; t += (PER_WAVE ? 1 : NW) * CPT) {
+    constexpr int SPLIT = DIRECT ? NSUB : 1;       // steps that share a tile
+    for (int ts = (PER_WAVE ? 0 : w) * CPT; ts < it.n_chunks * SPLIT; ts += (PER_WAVE ? 1 : NWV) * CPT) {
+        const int t = SPLIT > 1 ? ts / SPLIT : ts;
         int valid = len - (it.pos0 + t) * C;
         if (valid <= 0) break;  // chunks are in path order: everything after is empty too
         // tokens of this tile: bounded by the sequence's end and by the item's last chunk (the
@@ -570,16 +492,100 @@ __device__ __forceinline__ void stream_path(const DecodeArgs& A, const WorkItem*
         }
 #pragma unroll
         for (int sub = 0; sub < NSUB; sub++) {
+            if (SPLIT > 1 && sub != ts % SPLIT) continue;
             const int vsub = valid - sub * SUB;  // valid rows in this sub-tile
             if (vsub <= 0) break;
             const bool new_here = tile_has_new && vsub <= SUB;  // the newest token is row vsub - 1
-            size_t at[CPT];
+            const bool masked = vsub < SUB || new_here;
+            // load i of the sub-tile: 1 KiB at offset (i % LPC) KiB of chunk i / LPC
+            const uint4* kp[CPT];
+            const uint4* vp[CPT];
 #pragma unroll
-            for (int cc = 0; cc < CPT; cc++) at[cc] = base[cc] + size_t(sub) * SUB * D;
-            stream_tile<C, STEP>(A, seq, h, l, qv, at, vsub, new_here, sm.p[w], m_run, l_lane, acc);
+            for (int cc = 0; cc < CPT; cc++) {
+                kp[cc] = reinterpret_cast<const uint4*>(kpool + base[cc] + size_t(sub) * SUB * D) + l;
+                vp[cc] = reinterpret_cast<const uint4*>(vpool + base[cc] + size_t(sub) * SUB * D) + l;
+            }
+            uint4 kr[NL], vr[NL];
+            if (!masked) {
+#pragma unroll
+                for (int i = 0; i < NL; i++) {
+                    const uint4* p = kp[i / LPC] + 64 * (i % LPC);
+                    kr[i] = A.stream_nt ? nt_load16(p) : *p;
+                }
+#pragma unroll
+                for (int i = 0; i < NL; i++) {
+                    const uint4* p = vp[i / LPC] + 64 * (i % LPC);
+                    vr[i] = A.stream_nt ? nt_load16(p) : *p;
+                }
+            } else {
+                // rows past the end of the sequence hold stale data: never read into the math
+                const int vmem = (APPEND && new_here) ? vsub - 1 : vsub;  // rows that the pool holds
+                // The newest token's pieces are requested in front of the tile's own loads: loads
+                // return in order, so they are there when the tile is, at no round trip of their own.
+                uint4 kn = make_uint4(0, 0, 0, 0), vn = make_uint4(0, 0, 0, 0);
+                if constexpr (APPEND) {
+                    if (new_here) {
+                        const size_t new_off = (size_t(seq) * H + h) * D;
+                        kn = *(reinterpret_cast<const uint4*>(A.k_new + new_off) + j);
+                        vn = *(reinterpret_cast<const uint4*>(A.v_new + new_off) + j);
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < NL; i++) {
+                    const bool ok = 4 * i + g < vmem;
+                    kr[i] = ok ? kp[i / LPC][64 * (i % LPC)] : make_uint4(0, 0, 0, 0);
+                    vr[i] = ok ? vp[i / LPC][64 * (i % LPC)] : make_uint4(0, 0, 0, 0);
+                }
+                if constexpr (APPEND) {
+                    if (new_here) {
+                        // row vsub - 1 = 4 * i_new + g_new is the newest token: lanes (g_new, j) take
+                        // piece j of it from the caller's rows, as if it had been loaded from the pool
+                        const int i_new = (vsub - 1) >> 2;
+                        const bool mine = ((vsub - 1) & 3) == g;
+#pragma unroll
+                        for (int i = 0; i < NL; i++) {
+                            if (i == i_new && mine) {
+                                kr[i] = kn;
+                                vr[i] = vn;
+                            }
+                        }
+                    }
+                }
+            }
+            float sc[NL];
+#pragma unroll
+            for (int i = 0; i < NL; i++) {
+                sc[i] = dot8(*reinterpret_cast<const h8*>(&kr[i]), qv, 0.f);
+            }
+            // lane (g, j) now owns the score of row 4*(j % NL) + g
+            float s = reduce_rows16<NL>(sc, j) * scale_log2;
 #ifdef CA_TIMELINE
             if (t == 0 && sub == 0) CA_STAMP(1);
 #endif
+            const int row = 4 * (j % NL) + g;
+            if (row >= vsub || j >= NL) s = NEG_INF;
+            const float m_new = fmaxf(m_run, wave_max(s));
+            const float alpha = fast_exp2(m_run - m_new);
+            const float p = fast_exp2(s - m_new);
+            m_run = m_new;
+            l_lane = l_lane * alpha + p;
+            sm.p[w][l] = p;
+#pragma unroll
+            for (int e = 0; e < 8; e++) acc[e] *= alpha;
+            __builtin_amdgcn_wave_barrier();
+            float pr[NL];
+#pragma unroll
+            for (int i = 0; i < NL; i += 4) {
+                const f4 t4 = *reinterpret_cast<const f4*>(&sm.p[w][16 * g + i]);
+                pr[i] = t4[0]; pr[i + 1] = t4[1]; pr[i + 2] = t4[2]; pr[i + 3] = t4[3];
+            }
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int i = 0; i < NL; i++) {
+                const h8 vv = *reinterpret_cast<const h8*>(&vr[i]);
+#pragma unroll
+                for (int e = 0; e < 8; e++) acc[e] = __builtin_fmaf(pr[i], float(vv[e]), acc[e]);
+            }
         }
         if (!tried) {
             tried = true;
@@ -637,14 +643,14 @@ __device__ __forceinline__ void stream_path(const DecodeArgs& A, const WorkItem*
     }
     __syncthreads();
 
-    // combine the four waves: thread tid < 128 owns output dim tid
+    // combine the waves: thread tid < 128 owns output dim tid
     float m = sm.m[0];
 #pragma unroll
-    for (int k = 1; k < NW; k++) m = fmaxf(m, sm.m[k]);
+    for (int k = 1; k < NWV; k++) m = fmaxf(m, sm.m[k]);
     float o = 0.f, lsum = 0.f;
     if (tid < D) {
 #pragma unroll
-        for (int k = 0; k < NW; k++) {
+        for (int k = 0; k < NWV; k++) {
             const float f = (sm.m[k] == NEG_INF) ? 0.f : fast_exp2(sm.m[k] - m);
             o += f * sm.o[k][tid];
             lsum += f * sm.l[k];
@@ -1335,7 +1341,7 @@ __global__ __launch_bounds__(WG, (MIX == kMixFull || MIX == kMixFullSmall || C =
 // w tiles w, w + 8, ..., and writes the output: shared chunks are read once per sequence (by workgroups of one
 // XCD, i.e. from one L2), in return there are no partial rows, no merge launch and no tables in memory --
 // lengths and chunk slots arrive as a kernel argument.  STEP kAppend: the workgroup also puts its head's part of
-// the new K and V row into the pool (nobody reads that row in this launch: see stream_tile).
+// the new K and V row into the pool (nobody reads that row in this launch: see stream_path).
 //
 // What bounds it: the launch, two round trips to memory (the argument block, then K and V) and, beyond a tile or two
 // a wave, what one compute unit takes in.  Eight waves: as many as 128 registers of K and V in flight a lane leave
@@ -1345,96 +1351,52 @@ __global__ __launch_bounds__(WG, (MIX == kMixFull || MIX == kMixFullSmall || C =
 constexpr int DIRECT_WAVES = 8;
 constexpr int DIRECT_WG = 64 * DIRECT_WAVES;
 template <int NS, int NSLOT>
-struct DirectArgs {
-    int32_t len[NS];       // tokens of every sequence, the new one of a fused step among them
+struct alignas(16) DirectArgs {
+    uint16_t len[NS];      // tokens of every sequence, the new one of a fused step among them
     int32_t slots[NSLOT];  // chunk k of sequence s at s * stride + k
 };
-using DirectSmall = DirectArgs<16, 112>;
+// 256 bytes, 1 KB and 3.2 KB: the host writes the whole block on every call, over the bus (20 sequences of one chunk
+// each 5.15 us from call to call with 3.3 KB, 5.0 with 1 KB, 4.9 with 256 bytes).
+using DirectSmall = DirectArgs<32, 48>;
+using DirectMedium = DirectArgs<kDirectSeqs, 224>;
 using DirectLarge = DirectArgs<kDirectSeqs, kDirectSlots>;
 
 template <int C, int STEP, typename TABLE>
 __global__ __launch_bounds__(DIRECT_WG) void direct_kernel(half_t* kpool, half_t* vpool, const half_t* q, half_t* out,
                                                            int n_seqs, int H, int stride, float scale_log2,
                                                            const half_t* k_new, const half_t* v_new, const TABLE t) {
-    constexpr bool APPEND = STEP != kForward;
-    constexpr int CPT = C < 64 ? 64 / C : 1;   // chunks of a 64-token tile
-    constexpr int TPC = C > 64 ? C / 64 : 1;   // tiles of a chunk
     __shared__ struct {
         float p[DIRECT_WAVES][64];
         float o[DIRECT_WAVES][D];
         float m[DIRECT_WAVES];
         float l[DIRECT_WAVES];
+        int state;
     } sm;
     // head-major: the sequences of one head, which share chunks, lie side by side on one XCD
     const int unit = xcd_unit(blockIdx.x, n_seqs * H);
     const int h = unit / n_seqs, seq = unit - h * n_seqs;
-    const int tid = threadIdx.x;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int l = tid & 63, g = l >> 4, j = l & 15;
-    const int slotv = l < stride ? t.slots[seq * stride + l] : 0;
-    const int len = t.len[seq];
-    const h8 qv = *reinterpret_cast<const h8*>(q + (size_t(seq) * H + h) * D + 8 * j);
+    const int l = threadIdx.x & 63;
+    // (by words: the scalar unit loads nothing narrower)
+    const int len = (reinterpret_cast<const uint32_t*>(t.len)[seq >> 1] >> (16 * (seq & 1))) & 0xffff;
+    const DirectItem item{ seq, (len + C - 1) / C, len, l < stride ? t.slots[seq * stride + l] : 0 };
     DecodeArgs A{};
+    A.q = q;
     A.kpool = kpool;
     A.vpool = vpool;
+    A.out = out;
     A.k_new = k_new;
     A.v_new = v_new;
     A.H = H;
     A.scale_log2 = scale_log2;
-
-    float m_run = NEG_INF, l_lane = 0.f;
-    float acc[8];
-#pragma unroll
-    for (int e = 0; e < 8; e++) acc[e] = 0.f;
-    for (int u = w; 64 * u < len; u += DIRECT_WAVES) {
-        const int valid = len - 64 * u < 64 ? len - 64 * u : 64;
-        const bool new_here = APPEND && len - 64 * u <= 64;
-        size_t at[CPT];
-#pragma unroll
-        for (int cc = 0; cc < CPT; cc++) {
-            int k = u * CPT / TPC + cc;
-            if (k * C >= len) k = u * CPT / TPC;   // a missing second chunk is never loaded
-            at[cc] = (size_t(chunk_slot(slotv, k)) * H + h) * size_t(C) * D + size_t(u % TPC) * 64 * D;
-        }
-        stream_tile<C, STEP>(A, seq, h, l, qv, at, valid, new_here, sm.p[w], m_run, l_lane, acc);
-    }
-    const float l_wave = wave_sum(l_lane);
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-        acc[e] += shfl_xor(acc[e], 16);
-        acc[e] += shfl_xor(acc[e], 32);
-    }
-    if (g == 0) {
-#pragma unroll
-        for (int e = 0; e < 8; e++) sm.o[w][8 * j + e] = acc[e];
-    }
-    if (l == 0) {
-        sm.m[w] = m_run;
-        sm.l[w] = l_wave;
-    }
-    if constexpr (APPEND) {
-        if (w == DIRECT_WAVES - 1 && g < 2) {      // lanes of group 0: K, of group 1: V
-            const int row = (len - 1) % C;
-            const size_t dst = ((size_t(chunk_slot(slotv, (len - 1) / C)) * H + h) * C + row) * D + 8 * j;
-            const half_t* src = (g == 0 ? k_new : v_new) + (size_t(seq) * H + h) * D + 8 * j;
-            *reinterpret_cast<h8*>((g == 0 ? kpool : vpool) + dst) = *reinterpret_cast<const h8*>(src);
+    if constexpr (STEP != kForward) {
+        if (threadIdx.x < 32) {                    // 16 lanes: K, 16 lanes: V
+            const int j = l & 15, row = (len - 1) % C;
+            const size_t dst = ((size_t(chunk_slot(item.slotv, (len - 1) / C)) * H + h) * C + row) * D + 8 * j;
+            const half_t* src = (l < 16 ? k_new : v_new) + (size_t(seq) * H + h) * D + 8 * j;
+            *reinterpret_cast<h8*>((l < 16 ? kpool : vpool) + dst) = *reinterpret_cast<const h8*>(src);
         }
     }
-    __syncthreads();
-    if (tid < D) {
-        float m = sm.m[0];
-#pragma unroll
-        for (int k = 1; k < DIRECT_WAVES; k++) m = fmaxf(m, sm.m[k]);
-        float o = 0.f, lsum = 0.f;
-#pragma unroll
-        for (int k = 0; k < DIRECT_WAVES; k++) {
-            const float f = (sm.m[k] == NEG_INF) ? 0.f : fast_exp2(sm.m[k] - m);
-            o += f * sm.o[k][tid];
-            lsum += f * sm.l[k];
-        }
-        const float r = lsum > 0.f ? 1.f / lsum : 0.f;
-        out[(size_t(seq) * H + h) * D + tid] = half_t(o * r);
-    }
+    stream_path<C, false, STEP, DIRECT_WAVES>(A, nullptr, h, sm, &item);
 }
 
 // What the merge launch of a fused decode step needs to write the step's new K/V rows.
@@ -1764,7 +1726,7 @@ template <typename TABLE>
 static int launch_direct_table(const LaunchArgs& a, const int32_t* len, const int32_t* paths, int n_seqs, int stride,
                                hipStream_t st) {
     TABLE t;
-    std::memcpy(t.len, len, sizeof(int32_t) * n_seqs);
+    std::copy_n(len, n_seqs, t.len);
     std::memcpy(t.slots, paths, sizeof(int32_t) * n_seqs * stride);
     half_t* kp = static_cast<half_t*>(const_cast<void*>(a.kpool));
     half_t* vp = static_cast<half_t*>(const_cast<void*>(a.vpool));
@@ -1797,9 +1759,10 @@ int launch_direct(const LaunchArgs& a, const int32_t* len, const int32_t* paths,
         return -1;
     }
     for (int s = 0; s < n_seqs; s++) {
-        if (int64_t(len[s]) > int64_t(stride) * a.C || len[s] < (a.k_new ? 1 : 0)) return -1;
+        if (int64_t(len[s]) > int64_t(stride) * a.C || len[s] > 0xffff || len[s] < (a.k_new ? 1 : 0)) return -1;
     }
-    if (n_seqs <= 16 && n_seqs * stride <= 112) return launch_direct_table<DirectSmall>(a, len, paths, n_seqs, stride, st);
+    if (n_seqs <= 32 && n_seqs * stride <= 48) return launch_direct_table<DirectSmall>(a, len, paths, n_seqs, stride, st);
+    if (n_seqs * stride <= 224) return launch_direct_table<DirectMedium>(a, len, paths, n_seqs, stride, st);
     return launch_direct_table<DirectLarge>(a, len, paths, n_seqs, stride, st);
 }
 

@@ -49,10 +49,12 @@ def test_direct_and_general_forwards_agree(H, c, shared, privates):
     assert_close(got, oracle_output(attn, q, exact=True))
 
 
-@pytest.mark.parametrize("c", [32, 64, 128])
-def test_fused_steps_write_their_rows_and_follow_rollovers(c):
+@pytest.mark.parametrize("c,H,shared,privates", [(c, 4, 2 * c, [1, c - 2, c, c + 5]) for c in (32, 64, 128)] + [
+    # nothing to merge: steps and forwards in different forms of one launch, up to and past four tiles
+    (32, 60, 0, [1, 33, 60, 222]), (64, 60, 0, [1, 60, 130, 250]), (128, 60, 0, [1, 100, 127, 126]), (64, 8, 0, [60]),
+])
+def test_fused_steps_write_their_rows_and_follow_rollovers(c, H, shared, privates):
     rng = np.random.default_rng(c)
-    H, shared, privates = 4, 2 * c, [1, c - 2, c, c + 5]
     fused, kv = build(rng, H, c, shared, privates)
     apart, _ = build(rng, H, c, shared, privates, False, kv)
     n = len(privates)

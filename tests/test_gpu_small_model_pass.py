@@ -43,3 +43,51 @@ def test_native_model_pass_keeps_every_bit(hidden, layers, prompts, chunk, vocab
         assert (a == b).all()
     for a, b in zip(*(r[2] for r in runs)):
         assert all(torch.equal(x, y) for x, y in zip(a, b))
+
+
+def test_what_the_native_pass_leaves_to_the_modules(monkeypatch):
+    from chunk_attn import capi
+    from chunk_attn.models.sequence import Sequence
+    from chunk_attn.models.tiny_lm import AttentionOnlyLM
+    dev = torch.device("cuda:0")
+    model = AttentionOnlyLM(60, 256, 2, 2, chunk_size=32, memory_mb=8, seed=7)
+    caches = model.create_kv_caches()
+    ids = list(range(40))
+
+    def taken(prefill=True, seqs=1, tokens=ids, kv=caches):
+        with torch.inference_mode():
+            return model._plain_pass([None] * seqs, [tokens] * seqs, kv, prefill, dev) is not None
+
+    assert taken() and taken(prefill=False, tokens=[3]) and taken(prefill=False, seqs=5, tokens=[3])
+    assert not taken(seqs=2) and not taken(tokens=[]) and not taken(seqs=0)       # several prompts, none
+    assert not taken(tokens=[2 ** 40]) and not taken(tokens=["a"])                # ids that are no 32-bit numbers
+    assert not taken(kv=caches[:1]) and not taken(kv=[caches[0], object()])
+    assert not taken(kv=[caches[0], capi.Attention(3, 128, 32, memory_mb=8, dtype=torch.float16, device=dev)])
+    assert not taken(tokens=[1] * 40000)                                          # beyond the tiles' line
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert not taken()
+    for make in (lambda: model.layers[1].v_proj.register_forward_hook(lambda *a: None),
+                 lambda: model.layers[0].rotary_emb.register_forward_pre_hook(lambda *a: None)):
+        handle = make()
+        assert not taken()
+        handle.remove()
+    caches[1].add_seq = lambda *a: 0
+    assert not taken() and taken(prefill=False, tokens=[3])
+    del caches[1].add_seq
+    with monkeypatch.context() as mp:
+        mp.setattr(capi.Attention, "add_seq", lambda *a: 0)
+        assert not taken()
+    with monkeypatch.context() as mp:
+        mp.setattr(model.embed_tokens, "max_norm", 1.0)
+        assert not taken()
+    with monkeypatch.context() as mp:
+        mp.setattr(model.norm, "weight", torch.nn.Parameter(torch.ones(256, device=dev), requires_grad=False))
+        assert not taken()                                                        # another type
+    with monkeypatch.context() as mp:
+        mp.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+        assert not taken()
+    assert taken()
+    with torch.enable_grad():                                                     # a gradient is wanted: not asked at all
+        assert not model._adds_in_norms()
+    with torch.inference_mode():
+        assert model.logits([Sequence(ids)], caches, True).shape == (1, 60)

@@ -68,25 +68,25 @@ __global__ __launch_bounds__(WG) void rotary_vec_kernel(const int64_t* __restric
                                                         half_t* __restrict__ query,
                                                         half_t* __restrict__ key,
                                                         const half_t* __restrict__ cache,
-                                                        int64_t n_tokens, int wgs_per_token, int tokens_per_wg,
-                                                        int n_heads, int n_kv_heads,
-                                                        int head_size, int rot_dim, int max_position,
+                                                        int64_t n_tokens, int split, int n_heads, int n_kv_heads,
+                                                        int rot_dim, int head_size, int max_position,
                                                         int64_t query_stride, int64_t key_stride) {
     const int embed = rot_dim / 2;
     const unsigned units = IS_NEOX ? embed / 8 : rot_dim / 8;  // work units per head
-    // Whole workgroups a token, or whole tokens a workgroup: the division of the workgroup's index is scalar, that of
+    // `split` whole workgroups a token, or whole tokens a workgroup: the division of the workgroup's index is scalar, that of
     // the thread's 32 bits wide (64-bit divisions in every thread were as many vector ops as the rotation twice over:
-    // 2048 tokens of 32 + 32 heads 13.4 -> 12.4 us).
+    // 2048 tokens of 32 + 32 heads 13.4 -> 12.4 us).  What the first load needs stands in the 14 argument dwords that
+    // arrive with the wave: behind them it cost small calls 0.8 us.
     const unsigned per_token = unsigned(n_heads + n_kv_heads) * units;
     int64_t token;
     unsigned rem;
     if constexpr (!SHARED_WG) {
-        token = blockIdx.x / unsigned(wgs_per_token);
-        rem = (blockIdx.x % unsigned(wgs_per_token)) * WG + threadIdx.x;
+        token = blockIdx.x / unsigned(split);
+        rem = (blockIdx.x % unsigned(split)) * WG + threadIdx.x;
     } else {
         const unsigned t = threadIdx.x / per_token;
-        if (t >= unsigned(tokens_per_wg)) return;
-        token = int64_t(blockIdx.x) * tokens_per_wg + t;
+        if (t >= unsigned(split)) return;
+        token = int64_t(blockIdx.x) * split + t;
         rem = threadIdx.x - t * per_token;
     }
     if (rem >= per_token || (SHARED_WG && token >= n_tokens)) return;
@@ -189,8 +189,8 @@ int launch_rotary(const RotaryArgs& r, hipStream_t st) {
         const dim3 grid(static_cast<unsigned>(blocks)), block(WG);
         const auto kernel = tokens > 1 ? (r.is_neox ? rotary_vec_kernel<true, true> : rotary_vec_kernel<false, true>)
                                        : (r.is_neox ? rotary_vec_kernel<true, false> : rotary_vec_kernel<false, false>);
-        hipLaunchKernelGGL(kernel, grid, block, 0, st, r.positions, q, k, cache, r.n_tokens, wgs, tokens, r.n_heads,
-                           r.n_kv_heads, r.head_size, r.rot_dim, r.max_position, r.query_stride, r.key_stride);
+        hipLaunchKernelGGL(kernel, grid, block, 0, st, r.positions, q, k, cache, r.n_tokens, tokens > 1 ? tokens : wgs,
+                           r.n_heads, r.n_kv_heads, r.rot_dim, r.head_size, r.max_position, r.query_stride, r.key_stride);
         CA_LAUNCH_CHECK();
         return 0;
     }

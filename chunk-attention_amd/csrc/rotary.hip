@@ -61,35 +61,21 @@ __global__ __launch_bounds__(WG) void rotary_kernel(const int64_t* __restrict__ 
 // rot_dim / 2 multiples of 8; GPT-J style rot_dim a multiple of 8; 16-byte aligned pointers): one
 // thread rotates 8 pairs (NeoX: the pieces at r0 and r0 + rot_dim/2) or 4 pairs (GPT-J: one
 // piece), so every load and store moves 16 bytes per lane.  Same arithmetic as rotary_kernel.
-// SHARED_WG: several tokens a workgroup, for tokens of fewer units than it has threads (as an argument instead of a
-// form of its own it cost the wide rows half of what the scalar division gives them).
-template <bool IS_NEOX, bool SHARED_WG>
+template <bool IS_NEOX>
 __global__ __launch_bounds__(WG) void rotary_vec_kernel(const int64_t* __restrict__ positions,
                                                         half_t* __restrict__ query,
                                                         half_t* __restrict__ key,
                                                         const half_t* __restrict__ cache,
-                                                        int64_t n_tokens, int split, int n_heads, int n_kv_heads,
-                                                        int rot_dim, int head_size, int max_position,
+                                                        int64_t n_tokens, int n_heads, int n_kv_heads,
+                                                        int head_size, int rot_dim, int max_position,
                                                         int64_t query_stride, int64_t key_stride) {
     const int embed = rot_dim / 2;
-    const unsigned units = IS_NEOX ? embed / 8 : rot_dim / 8;  // work units per head
-    // `split` whole workgroups a token, or whole tokens a workgroup: the division of the workgroup's index is scalar, that of
-    // the thread's 32 bits wide (64-bit divisions in every thread were as many vector ops as the rotation twice over:
-    // 2048 tokens of 32 + 32 heads 13.4 -> 12.4 us).  What the first load needs stands in the 14 argument dwords that
-    // arrive with the wave: behind them it cost small calls 0.8 us.
-    const unsigned per_token = unsigned(n_heads + n_kv_heads) * units;
-    int64_t token;
-    unsigned rem;
-    if constexpr (!SHARED_WG) {
-        token = blockIdx.x / unsigned(split);
-        rem = (blockIdx.x % unsigned(split)) * WG + threadIdx.x;
-    } else {
-        const unsigned t = threadIdx.x / per_token;
-        if (t >= unsigned(split)) return;
-        token = int64_t(blockIdx.x) * split + t;
-        rem = threadIdx.x - t * per_token;
-    }
-    if (rem >= per_token || (SHARED_WG && token >= n_tokens)) return;
+    const int units = IS_NEOX ? embed / 8 : rot_dim / 8;  // work units per head
+    const int64_t per_token = int64_t(n_heads + n_kv_heads) * units;
+    const int64_t idx = int64_t(blockIdx.x) * WG + threadIdx.x;
+    if (idx >= n_tokens * per_token) return;
+    const int64_t token = idx / per_token;
+    const int rem = static_cast<int>(idx % per_token);
     const int head = rem / units, u = rem % units;
     half_t* row = (head < n_heads) ? query + token * query_stride + int64_t(head) * head_size
                                    : key + token * key_stride + int64_t(head - n_heads) * head_size;
@@ -180,17 +166,19 @@ int launch_rotary(const RotaryArgs& r, hipStream_t st) {
                         aligned16(cache);
     if (pieces) {
         const int units = r.is_neox ? r.rot_dim / 16 : r.rot_dim / 8;
-        const int64_t per_token = int64_t(r.n_heads + r.n_kv_heads) * units;
-        if (r.n_tokens <= 0 || per_token <= 0) return 0;
-        if (per_token > 0x7fffffff - WG) return -1;
-        const int wgs = static_cast<int>((per_token + WG - 1) / WG), tokens = per_token < WG ? static_cast<int>(WG / per_token) : 1;
-        const int64_t blocks = tokens > 1 ? (r.n_tokens + tokens - 1) / tokens : r.n_tokens * wgs;
-        if (r.n_tokens > int64_t(0x7fffffff) * WG || blocks > 0x7fffffff) return -1;
-        const dim3 grid(static_cast<unsigned>(blocks)), block(WG);
-        const auto kernel = tokens > 1 ? (r.is_neox ? rotary_vec_kernel<true, true> : rotary_vec_kernel<false, true>)
-                                       : (r.is_neox ? rotary_vec_kernel<true, false> : rotary_vec_kernel<false, false>);
-        hipLaunchKernelGGL(kernel, grid, block, 0, st, r.positions, q, k, cache, r.n_tokens, tokens > 1 ? tokens : wgs,
-                           r.n_heads, r.n_kv_heads, r.rot_dim, r.head_size, r.max_position, r.query_stride, r.key_stride);
+        const int64_t total = r.n_tokens * int64_t(r.n_heads + r.n_kv_heads) * units;
+        if (total <= 0) return 0;
+        if (total > int64_t(0x7fffffff) * WG) return -1;
+        const dim3 grid(static_cast<unsigned>((total + WG - 1) / WG)), block(WG);
+        if (r.is_neox) {
+            hipLaunchKernelGGL(rotary_vec_kernel<true>, grid, block, 0, st, r.positions, q, k, cache, r.n_tokens,
+                               r.n_heads, r.n_kv_heads, r.head_size, r.rot_dim, r.max_position,
+                               r.query_stride, r.key_stride);
+        } else {
+            hipLaunchKernelGGL(rotary_vec_kernel<false>, grid, block, 0, st, r.positions, q, k, cache, r.n_tokens,
+                               r.n_heads, r.n_kv_heads, r.head_size, r.rot_dim, r.max_position,
+                               r.query_stride, r.key_stride);
+        }
         CA_LAUNCH_CHECK();
         return 0;
     }

@@ -129,8 +129,8 @@ struct ca_ctx {
     int next_host = 0;
     bool direct = false;  // fused steps over the current plan take the direct form, which reads no device tables,
     bool direct_forward = false;  // and so do plain forwards
-    // Tables of such a plan are uploaded when something else first reads them (ensure_tables); until then they
-    // stand here.
+    // Tables of such a plan, and those whose upload was only captured, are uploaded when something else first reads
+    // them (ensure_tables); until then they stand here.
     bool upload_pending = false;
     std::vector<char> pending_blob;
     bool blob_in_graph = false;  // a captured upload writes dev_blob whenever its graph is replayed
@@ -294,7 +294,11 @@ int ensure_tables(ca_ctx* c, hipStream_t st) {
     if (!c->upload_pending) return CA_OK;
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     CA_HIP(hipStreamIsCapturing(st, &capture));
-    if (int rc = launch_rc(ca::launch_upload_args(c->dev_blob, c->pending_blob.data(), c->pending_blob.size(), st), "table upload")) return rc;
+    const size_t total = c->pending_blob.size();
+    for (size_t at = 0; at < total; at += ca::kArgUploadBytes) {
+        const size_t n = std::min(total - at, ca::kArgUploadBytes);
+        if (int rc = launch_rc(ca::launch_upload_args(c->dev_blob + at, c->pending_blob.data() + at, n, st), "table upload")) return rc;
+    }
     // Captured, it has not happened yet, and happens on every replay: still pending for everybody else, and no
     // later tables may stand in this buffer (upload_plan).
     if (capture == hipStreamCaptureStatusNone) c->upload_pending = false;
@@ -346,8 +350,11 @@ int upload_plan(ca_ctx* c, hipStream_t st) {
         put(c->off_tail_fill, p.tail_fill.data(), p.tail_fill.size() * 4);
     };
     // Small tables travel as a kernel argument (no staging buffer, no event), those of a forward in direct
-    // form only if something asks for them.
-    if (total <= ca::kArgUploadBytes) {
+    // form only if something asks for them.  So do all tables under stream capture: a replay would read whatever the
+    // staging buffer holds by then, and its event could not be waited for any more.
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    CA_HIP(hipStreamIsCapturing(st, &capture));
+    if (total <= ca::kArgUploadBytes || capture != hipStreamCaptureStatusNone) {
         c->pending_blob.resize(total);
         fill(c->pending_blob.data());
         c->upload_pending = true;
@@ -467,6 +474,7 @@ int run_merge(ca_ctx* c, void* out, hipStream_t st) {
 int run_fused(ca_ctx* c, const void* q, void* out, hipStream_t st) {
     const ca::LaunchArgs a = launch_args(c, q, out);
     if (c->direct_forward) return run_direct(c, a, st);
+    if (int rc = ensure_tables(c, st)) return rc;
     if (c->schedule == 0) {
         // both phases in one launch (shared and stream workgroups overlap), then the merge
         if (int rc = launch_rc(ca::launch_decode(a, static_cast<int>(c->plan.shared_items.size()),
@@ -634,6 +642,7 @@ int ca_attention(ca_ctx* c, const void* q, void* out, int n_seqs, int partition,
         CA_HIP(hipEventRecord(c->ev[0], st));
         if (c->timing == 1 && c->schedule == 0 && !c->direct_forward) {
             // the forward as it normally runs: decode launch, then merge launch
+            if (int rc = ensure_tables(c, st)) return rc;
             const ca::LaunchArgs a = launch_args(c, q, out);
             if (int rc = launch_rc(ca::launch_decode(a, static_cast<int>(c->plan.shared_items.size()),
                                                      static_cast<int>(c->plan.stream_items.size()), false, st), "decode launch")) return rc;
@@ -677,6 +686,7 @@ int ca_attention_noalloc(ca_ctx* c, const void* q, void* out, int n_seqs, void* 
     hipStream_t st = static_cast<hipStream_t>(stream);
     ca::LaunchArgs a = launch_args(c, q, out);
     if (c->direct_forward) return run_direct(c, a, st);
+    if (int rc = ensure_tables(c, st)) return rc;  // a launch and no more: of tables that a captured refresh left behind
     a.part = scratch;  // every row that the merge reads is written by the decode launch first
     if (int rc = launch_rc(ca::launch_decode(a, static_cast<int>(c->plan.shared_items.size()),
                                              static_cast<int>(c->plan.stream_items.size()), false, st), "decode launch")) return rc;

@@ -1,0 +1,97 @@
+"""When device tables are brought to the device and on whose stream: tables built under stream capture, which are on
+the device only once the graph has run."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_helpers import assert_close, dev, make_attention, oracle_output, to_dev
+
+pytestmark = pytest.mark.gpu
+
+H, C = 4, 64
+
+
+def rand(rng, *shape):
+    return rng.standard_normal(shape).astype(np.float16)
+
+
+def cache(rng, shared, privates, general):
+    attn = make_attention(H, C, sum((shared + p) // C + 3 for p in privates))
+    if general:
+        attn.ctx.set_plan(stream_chunks=4)    # explicit item sizes: never the direct form
+    ks, vs = rand(rng, shared, H, 128), rand(rng, shared, H, 128)
+    for s, p in enumerate(privates):
+        k, v = np.concatenate([ks, rand(rng, p, H, 128)]), np.concatenate([vs, rand(rng, p, H, 128)])
+        attn.add_seq(list(range(shared)) + [10_000 * (s + 1) + t for t in range(p)], to_dev(k), to_dev(v))
+    return attn
+
+
+def stream():
+    return torch.cuda.current_stream().cuda_stream
+
+
+# tables of one kernel argument and of several; partition 1 of the first would be the direct form's in partition 0
+@pytest.mark.parametrize("privates,general", [([30, 70, 90], False), ([30, 70, 90], True), ([20 + 9 * s for s in range(70)], False)])
+@pytest.mark.parametrize("timing", [0, 1, 2])
+def test_eager_forwards_beside_tables_that_only_a_graph_uploads(privates, general, timing):
+    rng = np.random.default_rng(len(privates))
+    attn = cache(rng, 128, privates, general)
+    n = len(privates)
+    q = rand(rng, n, H, 128)
+    qd, want = to_dev(q), oracle_output(attn, q, exact=True)
+    for partition in (1, 2, 0):                        # buffers of every size are there: nothing is allocated below
+        attn.forward(qd, partition)
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=side):
+        captured = attn.forward(qd, 1)
+    attn.ctx.set_timing(timing)
+    assert_close(attn.forward(qd, 1), want)            # the graph has not run yet
+    for partition in (0, 2, 1, 0):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert_close(captured, want)
+        assert_close(attn.forward(qd, partition), want)
+    for _ in range(5):                                 # the staging buffers come round again
+        attn.refresh_kernel_context(force=True)
+        assert_close(attn.forward(qd), want)
+    graph.replay()
+    torch.cuda.synchronize()
+    assert_close(captured, want)
+
+
+@pytest.mark.parametrize("privates", [[30, 70, 90], [20 + 9 * s for s in range(70)]])
+def test_a_captured_refresh_leaves_every_reader_its_tables(privates):
+    rng = np.random.default_rng(1)
+    attn = cache(rng, 128, privates, True)
+    n = len(privates)
+    q, k, v = rand(rng, n, H, 128), to_dev(rand(rng, n, H, 128)), to_dev(rand(rng, n, H, 128))
+    qd, want = to_dev(q), oracle_output(attn, q, exact=True)
+    out = torch.empty(n, H, 128, dtype=torch.float16, device=dev())
+    attn.forward(qd)
+    side = torch.cuda.Stream()
+
+    def captured(call):
+        attn.refresh_kernel_context(force=True)        # whatever a graph owns is replaced outside the capture
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            attn.refresh_kernel_context(force=True)
+            call()
+        return graph
+
+    noalloc = lambda: attn.ctx.attention_noalloc(qd.data_ptr(), out.data_ptr(), n, stream())   # noqa: E731
+    graph = captured(noalloc)
+    noalloc()                                          # eagerly, before the graph has run
+    assert_close(out, want)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        assert_close(out, want)
+    captured(lambda: None)
+    attn.append_token(list(range(n)), k, v)
+    q2 = rand(rng, n, H, 128)
+    assert_close(attn.forward(to_dev(q2)), oracle_output(attn, q2, exact=True))
+    captured(lambda: None)
+    got = attn.decode_step(list(range(n)), to_dev(q2), k, v)
+    assert_close(got, oracle_output(attn, q2, exact=True))

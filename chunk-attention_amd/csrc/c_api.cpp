@@ -129,10 +129,12 @@ struct ca_ctx {
     int next_host = 0;
     bool direct = false;  // fused steps over the current plan take the direct form, which reads no device tables,
     bool direct_forward = false;  // and so do plain forwards
-    // Tables of such a plan, and those whose upload was only captured, are uploaded when something else first reads
-    // them (ensure_tables); until then they stand here.
+    // Tables of such a plan, and those whose upload was only captured, are uploaded by whoever else reads them
+    // (ensure_tables), and stand here.
     bool upload_pending = false;
     std::vector<char> pending_blob;
+    bool uploaded_late = false;  // some reader has done so, on this stream
+    hipStream_t late_stream = nullptr;
     bool blob_in_graph = false;  // a captured upload writes dev_blob whenever its graph is replayed
     // offsets into dev_blob
     size_t off_shared = 0, off_stream = 0, off_slots = 0, off_seq_len = 0, off_part_ptr = 0,
@@ -289,20 +291,27 @@ int run_direct(ca_ctx* c, const ca::LaunchArgs& a, hipStream_t st) {
     return launch_rc(ca::launch_direct(a, len, c->plan.paths.data(), c->n_seqs, c->plan.path_stride, st), "direct launch");
 }
 
-// The device tables of the current plan, for whatever reads them: uploads what upload_plan left out.
+// The device tables of the current plan, for whatever reads them on `st`: uploads what upload_plan left out.  A reader
+// on another stream need not be ordered behind the one that uploaded first (only behind the refresh), nor the replay of
+// a graph behind anything eager: each of them brings the tables itself.  Whoever writes them writes the same bytes.
 int ensure_tables(ca_ctx* c, hipStream_t st) {
     if (!c->upload_pending) return CA_OK;
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     CA_HIP(hipStreamIsCapturing(st, &capture));
+    const bool capturing = capture != hipStreamCaptureStatusNone;
+    // (every thread has a stream of its own behind that one handle)
+    if (!capturing && c->uploaded_late && c->late_stream == st && st != hipStreamPerThread) return CA_OK;
     const size_t total = c->pending_blob.size();
     for (size_t at = 0; at < total; at += ca::kArgUploadBytes) {
         const size_t n = std::min(total - at, ca::kArgUploadBytes);
         if (int rc = launch_rc(ca::launch_upload_args(c->dev_blob + at, c->pending_blob.data() + at, n, st), "table upload")) return rc;
     }
-    // Captured, it has not happened yet, and happens on every replay: still pending for everybody else, and no
-    // later tables may stand in this buffer (upload_plan).
-    if (capture == hipStreamCaptureStatusNone) c->upload_pending = false;
-    else c->blob_in_graph = true;
+    if (capturing) {
+        c->blob_in_graph = true;  // it happens on every replay: no later tables may stand in this buffer (upload_plan)
+    } else {
+        c->uploaded_late = true;
+        c->late_stream = st;
+    }
     return CA_OK;
 }
 
@@ -358,7 +367,12 @@ int upload_plan(ca_ctx* c, hipStream_t st) {
         c->pending_blob.resize(total);
         fill(c->pending_blob.data());
         c->upload_pending = true;
-        return c->direct_forward ? CA_OK : ensure_tables(c, st);
+        c->uploaded_late = false;
+        if (c->direct_forward) return CA_OK;
+        if (int rc = ensure_tables(c, st)) return rc;
+        // behind the refresh: all that a reader needs to be ordered behind
+        if (capture == hipStreamCaptureStatusNone) c->upload_pending = false;
+        return CA_OK;
     }
     const int hb = c->next_host;
     c->next_host = (c->next_host + 1) % ca_ctx::kStaging;

@@ -1,5 +1,5 @@
 """When device tables are brought to the device and on whose stream: tables built under stream capture, which are on
-the device only once the graph has run."""
+the device only once the graph has run, and those of small forwards, which whoever reads them uploads."""
 import numpy as np
 import pytest
 import torch
@@ -95,3 +95,63 @@ def test_a_captured_refresh_leaves_every_reader_its_tables(privates):
     captured(lambda: None)
     got = attn.decode_step(list(range(n)), to_dev(q2), k, v)
     assert_close(got, oracle_output(attn, q2, exact=True))
+
+
+def test_readers_on_streams_that_only_know_of_the_refresh():
+    """A small forward's tables are uploaded by their readers.  Two of them on streams of their own, both ordered behind
+    the refresh and in no order between themselves: the second must not count on the first one's upload, which is held
+    up here."""
+    rng = np.random.default_rng(2)
+    attn = cache(rng, 128, [30, 70, 90], False)
+    other = rand(rng, 40, H, 128)
+    attn.forward(to_dev(rand(rng, 3, H, 128)), 1)      # older tables in the buffer
+    attn.add_seq(list(range(5000, 5040)), to_dev(other), to_dev(other))
+    q, k, v = rand(rng, 4, H, 128), to_dev(rand(rng, 4, H, 128)), to_dev(rand(rng, 4, H, 128))
+    qd, want = to_dev(q), oracle_output(attn, q, exact=True)
+    first, second, back = (torch.cuda.Stream() for _ in range(3))
+    attn.refresh_kernel_context()
+    refreshed = torch.cuda.Event()
+    refreshed.record()
+    with torch.cuda.stream(first):
+        refreshed.wait()
+        torch.cuda._sleep(20_000_000)
+        attn.ctx.append_kv(k.data_ptr(), v.data_ptr(), 4, stream())     # rows that nobody attends yet
+    outs = []
+    for side in (second, back):
+        with torch.cuda.stream(side):
+            refreshed.wait()
+            out = torch.empty_like(qd)
+            attn.ctx.attn_chunks_first(qd.data_ptr(), 4, stream())
+            attn.ctx.attn_seqs_first(qd.data_ptr(), out.data_ptr(), 4, stream())
+            side.synchronize()
+            outs.append(out)
+    assert not first.query()                           # the first reader's upload is still to come
+    for out in outs:
+        assert_close(out, want)
+    torch.cuda.synchronize()
+    attn.tree.append_token([1, 2, 3, 4])
+    attn.ctx.delta_tokens = 1
+    assert_close(attn.forward(qd), oracle_output(attn, q, exact=True))
+
+
+def test_a_graph_brings_its_tables_whatever_was_uploaded_before():
+    """An append captured behind an eager one on the same stream, replayed on another."""
+    rng = np.random.default_rng(3)
+    attn = cache(rng, 128, [30, 70, 90], False)
+    q, k, v = rand(rng, 3, H, 128), to_dev(rand(rng, 3, H, 128)), to_dev(rand(rng, 3, H, 128))
+    qd = to_dev(q)
+    attn.forward(qd, 1)
+    attn.refresh_kernel_context(force=True)
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        attn.append_token([1, 2, 3], k, v)
+        side.synchronize()
+    with torch.cuda.graph(graph, stream=side):
+        attn.ctx.append_kv(v.data_ptr(), k.data_ptr(), 3, stream())
+    attn.tree.append_token([4, 5, 6])
+    attn.ctx.delta_tokens = 2
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert_close(attn.forward(qd), oracle_output(attn, q, exact=True))

@@ -287,7 +287,10 @@ bool one_launch_anyway(const ca_ctx* c) {
 
 int run_direct(ca_ctx* c, const ca::LaunchArgs& a, hipStream_t st) {
     int32_t len[ca::kDirectSeqs];
-    for (int s = 0; s < c->n_seqs; s++) len[s] = c->plan.seq_len[s] + c->delta_tokens;
+    // delta_tokens may be set beyond the room of a last chunk: that chunk's end is the end then, as in the general path
+    for (int s = 0; s < c->n_seqs; s++) {
+        len[s] = static_cast<int32_t>(std::min(int64_t(c->plan.seq_len[s]) + c->delta_tokens, int64_t(c->plan.path_len[s]) * c->C));
+    }
     return launch_rc(ca::launch_direct(a, len, c->plan.paths.data(), c->n_seqs, c->plan.path_stride, st), "direct launch");
 }
 

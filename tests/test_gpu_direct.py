@@ -118,3 +118,21 @@ def test_phases_and_partitions_upload_what_they_read():
     assert_close(out, want)
     for partition in (0, 1, 0, 2, 0):
         assert_close(attn.forward(qd, partition), want)
+
+
+@pytest.mark.parametrize("c", [32, 64, 128])
+def test_delta_tokens_past_the_room_of_last_chunks(c):
+    """Set beyond what a last chunk holds, delta_tokens ends at the chunk's end, whatever the neighbours' lengths."""
+    rng = np.random.default_rng(5)
+    privates = [c - 4, 2 * c + 22, 3 * c, 1]
+    attn, kv = build(rng, 4, c, c, privates)
+    other, _ = build(rng, 4, c, c, privates, True, kv)
+    for a in (attn, other):                                    # rows that nobody has written yet, the same in both
+        a.refresh_kernel_context()
+        for k, v, slot, n in [(*a.pool_views(), r[0], r[1]) for r in a.get_chunks().tolist()]:
+            k[slot][:, n:] = torch.arange(c - n, device=dev()).half()[None, :, None] / 64
+            v[slot][:, n:] = 1 - torch.arange(c - n, device=dev()).half()[None, :, None] / 64
+    q = to_dev(rand(rng, 4, 4, 128))
+    for delta in (0, 1, 4, 5, 11, c - 1, c, 5 * c, 1 << 20):
+        attn.ctx.delta_tokens = other.ctx.delta_tokens = delta
+        assert_close(attn.forward(q), other.forward(q).float().cpu().numpy())

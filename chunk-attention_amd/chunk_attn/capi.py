@@ -460,9 +460,11 @@ def _causal_attention(q, k, v):
 
 def is_bare(module, cls) -> bool:
     """The module is a `cls` and nothing hangs on it that a call would also run (hooks, a patched forward)."""
+    if type(module) is not cls:
+        return False
     own = module.__dict__
-    return type(module) is cls and not (own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"] or
-                                        own["_backward_pre_hooks"] or "forward" in own)
+    return not (own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"] or
+                own["_backward_pre_hooks"] or "forward" in own)
 
 
 def projection_takes(x, *linears) -> bool:
@@ -495,7 +497,10 @@ def _linears_are_plain(n_in: int, device, linears) -> bool:
     for m in linears:
         if not is_bare(m, Linear):
             return False
-        parameters = m.__dict__["_parameters"]
+        own = m.__dict__
+        if "weight" in own or "bias" in own:           # what hides the registered ones
+            return False
+        parameters = own["_parameters"]
         w = parameters.get("weight")
         if type(w) is not Parameter or parameters.get("bias", w) is not None or w.dtype is not half or \
                 w.device != device or w.dim() != 2 or w.shape[1] != n_in or not w.is_contiguous() or \

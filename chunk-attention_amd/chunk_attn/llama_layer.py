@@ -124,11 +124,11 @@ class LlamaChunkAttention(nn.Module):
 
     def _plain_rotary(self, device: torch.device) -> Optional[torch.Tensor]:
         """The rotary module's table, if the module is the one this layer was built with, over whole heads, nothing
-        hangs on it, and the projection kernels read such a table (the operator takes narrower ones and any
+        hangs on it or hides its table, and the projection kernels read such a table (the operator takes narrower ones and any
         alignment)."""
         r = self.rotary_emb
         table = r.__dict__["_buffers"].get("cos_sin_cache")
-        plain = table is not None and capi.is_bare(r, RotaryEmbedding) and stock.is_stock(RotaryEmbedding, _ROTARY_FORWARD) and \
+        plain = table is not None and "cos_sin_cache" not in r.__dict__ and capi.is_bare(r, RotaryEmbedding) and stock.is_stock(RotaryEmbedding, _ROTARY_FORWARD) and \
             r.is_neox_style and r.rotary_dim == r.head_size == self.head_dim and capi.is_rotary_table(table, device)
         return table if plain else None
 

@@ -33,6 +33,7 @@ class RMSNorm(nn.Module):
 
 _NORM_FORWARD = RMSNorm.forward
 _HOST = torch.device("cpu")
+_PROJECTIONS = ("q_proj", "k_proj", "v_proj", "o_proj")
 
 
 def _is_plain(w, shape, device: torch.device) -> bool:
@@ -147,12 +148,16 @@ class AttentionOnlyLM(nn.Module):
         except (TypeError, OverflowError):             # ids that are no 32-bit numbers: torch's business
             return None
         norms = (*self.input_norms, self.norm)
-        embedding, norm_weights = self.embed_tokens, [m._parameters.get("weight") for m in norms]
+        embedding, norm_weights = self.embed_tokens, [None if "weight" in m.__dict__ else m._parameters.get("weight") for m in norms]
         if len(norms) != n + 1 or embedding.max_norm is not None or not _is_plain(embedding.weight, (self.vocab_size, hidden), dev) or \
                 not all([_is_plain(w, (hidden,), dev) for w in norm_weights]):
             return None
-        # (by the modules' own dictionaries: __getattr__ costs as much as a launch here, a few dozen times a pass)
-        linears = [m[name] for m in [layer._modules for layer in self.layers] for name in ("q_proj", "k_proj", "v_proj", "o_proj")]
+        # (by the modules' own dictionaries: __getattr__ costs as much as a launch here, a few dozen times a pass; what
+        # hides a registered module, on the object or its class, is what the layer calls)
+        if not vars(LlamaChunkAttention).keys().isdisjoint(_PROJECTIONS) or \
+                not all([layer.__dict__.keys().isdisjoint(_PROJECTIONS) for layer in self.layers]):
+            return None
+        linears = [m.get(name) for m in [layer._modules for layer in self.layers] for name in _PROJECTIONS]
         if not capi._linears_are_plain(hidden, dev, linears):
             return None
         weights = [m._parameters["weight"] for m in linears]

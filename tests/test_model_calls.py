@@ -195,3 +195,70 @@ def test_projections_are_computed_here_while_the_host_gains_more(rows, n_in, n_o
     """A library call costs the host 9 us more than one here."""
     assert capi.projection_pays(rows, n_in, n_out) == pays
     assert here <= library + 9 if pays else here > library + 5
+
+
+class AnyGpu:
+    """A GPU that every tensor lies on."""
+    type = "cuda"
+    __hash__ = None
+
+    def __eq__(self, other):
+        return True
+
+    def __ne__(self, other):
+        return False
+
+
+def hide_projection(m, mp):
+    m.layers[1].__dict__["q_proj"] = lambda x: x
+
+
+def hide_output_projection(m, mp):
+    m.layers[0].__dict__["o_proj"] = m.layers[1].o_proj
+
+
+def function_for_a_deleted_projection(m, mp):
+    del m.layers[0].v_proj
+    m.layers[0].v_proj = torch.relu                            # a builtin: no dictionary of its own
+
+
+def hide_projections_of_the_class(m, mp):
+    mp.setattr(tiny_lm.LlamaChunkAttention, "k_proj", staticmethod(lambda x: x), raising=False)
+
+
+def hide_weight(m, mp):
+    m.layers[0].k_proj.__dict__["weight"] = m.layers[1].k_proj.weight
+
+
+def hide_bias(m, mp):
+    m.layers[0].o_proj.__dict__["bias"] = torch.ones(128, dtype=torch.float16)
+
+
+def hide_norm_weight(m, mp):
+    m.input_norms[1].__dict__["weight"] = m.norm.weight
+
+
+def hide_rotary_table(m, mp):
+    m.layers[1].rotary_emb.__dict__["cos_sin_cache"] = torch.zeros(64, 128, dtype=torch.float16)
+
+
+@pytest.mark.parametrize("hide", [
+    hide_projection, hide_output_projection, function_for_a_deleted_projection, hide_projections_of_the_class, hide_weight,
+    hide_bias, hide_norm_weight, hide_rotary_table])
+def test_native_pass_sees_what_hides_a_registered_module(monkeypatch, hide):
+    """Python finds an attribute of the object, and of its class, before the module or parameter of that name."""
+    import types
+    gpu = AnyGpu()
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(capi, "is_plain_cache", lambda c: True)
+    monkeypatch.setattr(capi, "is_plain_cache_to_fill", lambda c: True)
+    caches = [types.SimpleNamespace(d_head=128, n_heads=1, device=gpu)] * 2
+
+    def taken(m):
+        return [m._plain_pass([None], [[1, 2][:n]], caches, n == 2, gpu) is not None for n in (1, 2)]
+
+    with torch.no_grad():
+        m = AttentionOnlyLM(50, 128, 1, 2, max_position_embeddings=64, seed=3, device="cpu")
+        assert taken(m) == [True, True]
+        hide(m, monkeypatch)
+        assert taken(m) == [False, False]

@@ -1035,6 +1035,14 @@ int settle(ca_ctx* c, ca_tree* tree, int n_seqs, void* stream) {
 }
 }  // namespace
 
+namespace {
+// The tables are those of n_seqs sequences with a free row in every last chunk.
+bool has_room(const ca_ctx* c, int n_seqs) {
+    return c->valid && c->n_seqs == n_seqs && std::all_of(c->plan.tail_fill.begin(), c->plan.tail_fill.end(),
+                                                          [&](int32_t fill) { return fill + c->delta_tokens < c->C; });
+}
+}  // namespace
+
 int ca_layer_decode(ca_ctx* c, ca_tree* tree, const int32_t* tokens, int n_seqs, const void* x, int n_in,
                     const void* wq, const void* wk, const void* wv, const void* wo, int n_out,
                     const int64_t* positions, const void* cos_sin_cache, int max_position, void* q, void* attn,
@@ -1123,9 +1131,19 @@ int ca_model_pass(const ca_model_layer* layers, int n_layers, const int32_t* tok
         out.y[0] = logits;
         if (int rc = check_project(out, x, n_seqs, n_logits, hidden)) return rc;
     }
+    for (int i = 0; i < n_layers && !prefill; i++) {
+        if (ca_tree_n_seqs(layers[i].tree) != n_seqs) return fail(CA_ERR_INVALID, "num of seqs is not equal to num of tokens");
+    }
     Range range("ca_model_pass");
     return guarded([&]() -> int {
         hipStream_t st = static_cast<hipStream_t>(stream);
+        // nor may a layer's tables turn out to be another cache's, or without room, once earlier layers have moved on
+        for (int i = 0; i < n_layers && !prefill; i++) {
+            ca_ctx* c = layers[i].ctx;
+            if (has_room(c, n_seqs)) continue;
+            if (int rc = settle(c, layers[i].tree, n_seqs, stream)) return rc;
+            if (!has_room(c, n_seqs)) return fail(CA_ERR_STATE, "a layer's tables do not fit its cache: refresh first");
+        }
         if (int rc = launch_rc(ca::launch_embed_norm(embedding, tokens, positions, rows, residual, x, pos, norm, norm_epsilon, hidden, st), "embedding launch")) return rc;
         std::vector<int32_t> slots;
         for (int i = 0; i < n_layers; i++) {

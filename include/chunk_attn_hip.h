@@ -467,7 +467,7 @@ typedef struct {
  * tokens and positions: host, n_seqs * n_tokens; every id within the embedding [vocab, hidden].  hidden is the
  * context's n_heads * 128.  scratch: ca_model_scratch_bytes(rows, hidden) bytes of device memory, 16-byte aligned;
  * the last norm's rows start ca_model_last_rows(rows, hidden, n_seqs) bytes into it.  What a call refuses for its
- * arguments leaves every cache as it was. */
+ * arguments, or because a cache has other sequences than the pass, leaves every cache's tokens as they were. */
 size_t ca_model_scratch_bytes(int64_t n_rows, int hidden);
 size_t ca_model_last_rows(int64_t n_rows, int hidden, int n_seqs);
 int ca_model_pass(const ca_model_layer* layers, int n_layers, const int32_t* tokens, const int32_t* positions,

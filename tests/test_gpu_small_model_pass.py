@@ -91,3 +91,41 @@ def test_what_the_native_pass_leaves_to_the_modules(monkeypatch):
         assert not model._adds_in_norms()
     with torch.inference_mode():
         assert model.logits([Sequence(ids)], caches, True).shape == (1, 60)
+
+
+def test_refused_decode_passes_leave_every_cache_as_it_was():
+    """A later layer's cache that does not fit the pass is noticed before an earlier one takes the tokens."""
+    from chunk_attn.models.sequence import Sequence
+    from chunk_attn.models.tiny_lm import AttentionOnlyLM
+    model = AttentionOnlyLM(60, 256, 2, 3, chunk_size=32, memory_mb=8, seed=7)
+
+    def start():
+        caches, running = model.create_kv_caches(), []
+        for p in (10, 31, 40):
+            seq = Sequence([(t * 7 + p) % 60 for t in range(p)])
+            model.logits([seq], caches, True)
+            running.insert(seq.index, seq)
+        for seq in running:
+            seq.append(5)
+        return caches, running
+
+    def refused(caches, running, match):
+        before = [c.tree.get_chunks() for c in caches]
+        for _ in range(2):
+            with pytest.raises(RuntimeError, match=match):
+                model.logits(running, caches, False)
+            assert all((a == c.tree.get_chunks()).all() for a, c in zip(before, caches))
+
+    with torch.inference_mode():
+        caches, running = start()
+        caches[2].remove_seq(1)                        # other sequences in the tree
+        refused(caches, running, "num of seqs")
+        caches, running = start()
+        want = model.logits(running, caches, False)
+        caches, running = start()
+        rows = caches[1].tree.get_chunks()
+        first = rows[rows[:, 2] == 0]
+        caches[1].ctx.refresh(first, 1, torch.cuda.current_stream().cuda_stream)     # other sequences in the tables
+        refused(caches, running, "refresh first")
+        caches[1].refresh_kernel_context(force=True)
+        assert torch.equal(model.logits(running, caches, False), want)

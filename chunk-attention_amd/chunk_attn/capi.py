@@ -620,10 +620,11 @@ def _qkv_rotary(x, wq, wk, wv, positions, cos_sin_cache):
     return q, k, v
 
 
-def _model_pass(layers, tokens, positions, n_seqs: int, prefill: bool, embedding, norm, epsilon: float, head=None):
+def _model_pass(layers, tokens, positions, n_seqs: int, prefill: bool, embedding, norm, epsilon: float, head, index: list):
     """A pass of the small model as one native call (see ca_model_pass).  layers: (cache, wq, wk, wv, wo, table, norm
-    weight, epsilon) of each; the caller has checked all of it (tiny_lm._plain_pass).  Returns (logits, or without a
-    head the last norm's rows; the sequence's index in every cache)."""
+    weight, epsilon) of each; the caller has checked all of it (tiny_lm._plain_pass).  Returns the logits, or without a
+    head the last norm's rows; `index` receives the prompt's index in every cache, -1 where it was not inserted, also
+    when the pass fails."""
     lib, device, hidden = load(), embedding.device, embedding.shape[1]
     rows = len(tokens)
     table = (ModelLayer * len(layers))(*[
@@ -632,16 +633,19 @@ def _model_pass(layers, tokens, positions, n_seqs: int, prefill: bool, embedding
     ids, ids_ptr = _i32(tokens)
     pos, pos_ptr = _i32(positions)
     scratch = torch.empty(lib.ca_model_scratch_bytes(rows, hidden) // 2, dtype=torch.float16, device=device)
-    index = (ctypes.c_int32 * len(layers))()
+    inserted = (ctypes.c_int32 * len(layers))(*[-1] * len(layers))
     logits = None if head is None else torch.empty((n_seqs, head.shape[0]), dtype=torch.float16, device=device)
-    _launch(device, lib.ca_model_pass, table, len(layers), ids_ptr, pos_ptr, n_seqs, rows // n_seqs, int(prefill),
-            embedding.data_ptr(), embedding.shape[0], norm.data_ptr(), epsilon, hidden, scratch.data_ptr(),
-            None if head is None else head.data_ptr(), 0 if head is None else head.shape[0],
-            None if head is None else logits.data_ptr(), index)
+    try:
+        _launch(device, lib.ca_model_pass, table, len(layers), ids_ptr, pos_ptr, n_seqs, rows // n_seqs, int(prefill),
+                embedding.data_ptr(), embedding.shape[0], norm.data_ptr(), epsilon, hidden, scratch.data_ptr(),
+                None if head is None else head.data_ptr(), 0 if head is None else head.shape[0],
+                None if head is None else logits.data_ptr(), inserted)
+    finally:
+        index[:] = inserted
     if head is None:
         at = lib.ca_model_last_rows(rows, hidden, n_seqs) // 2
         logits = scratch[at:at + n_seqs * hidden].view(n_seqs, hidden)
-    return logits, list(index)
+    return logits
 
 
 def max_chunks_for(memory_mb: int, chunk_size: int, n_heads: int, d_head: int, elem_bytes: int = 2) -> int:

@@ -93,13 +93,16 @@ class AttentionOnlyLM(nn.Module):
         if layers:
             head = self.lm_head.weight if capi.projection_pays(len(seqs), self.hidden_size, self.vocab_size) and \
                 capi._linears_are_plain(self.hidden_size, dev, (self.lm_head,)) else None
-            out, index = capi._model_pass(layers, [t for ids in input_ids for t in ids], [p for pos in position_ids for p in pos],
-                                          len(seqs), prefill, self.embed_tokens.weight, self.input_norms[0].weight,
-                                          self.input_norms[0].eps, head)
-            if prefill:
-                for layer, idx in zip(self.layers, index):
-                    layer.last_indices = [idx]
-                seqs[0].index = index[-1]
+            index = []
+            try:
+                out = capi._model_pass(layers, [t for ids in input_ids for t in ids], [p for pos in position_ids for p in pos],
+                                       len(seqs), prefill, self.embed_tokens.weight, self.input_norms[0].weight,
+                                       self.input_norms[0].eps, head, index)
+            finally:                                   # a pass that failed has filled the caches in front of that layer
+                for layer, idx in zip(self.layers, index if prefill else ()):
+                    if idx >= 0:
+                        layer.last_indices = [idx]
+                        seqs[0].index = idx
             return out if head is not None else self.lm_head(out)
         # one upload, from pinned memory: the host does not wait for what the GPU still has to do (the device is
         # named: only host memory can be pinned, whatever the default device is)

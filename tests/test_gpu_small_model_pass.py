@@ -129,3 +129,28 @@ def test_refused_decode_passes_leave_every_cache_as_it_was():
         refused(caches, running, "refresh first")
         caches[1].refresh_kernel_context(force=True)
         assert torch.equal(model.logits(running, caches, False), want)
+
+
+@pytest.mark.parametrize("hooked", [False, True])
+@pytest.mark.parametrize("over", [5, 0])               # no chunk for the prompt's end; none for its next token
+def test_a_prompt_that_a_later_cache_cannot_take(hooked, over):
+    """The pass fails; where the prompt stands in the caches that took it is known, to remove it there."""
+    from chunk_attn import capi
+    from chunk_attn.models.sequence import Sequence
+    from chunk_attn.models.tiny_lm import AttentionOnlyLM
+    model = AttentionOnlyLM(60, 256, 2, 2, chunk_size=32, memory_mb=8, seed=7)
+    if hooked:                                         # the modules' own calls
+        model.norm.register_forward_hook(lambda m, a, out: None)
+    caches = model.create_kv_caches()
+    caches[1] = capi.Attention(2, 128, 32, memory_mb=1, dtype=torch.float16, device=torch.device("cuda:0"))
+    with torch.inference_mode():
+        model.logits([Sequence([59, 58])], [caches[0], model.create_kv_caches()[1]], True)     # index 0 is taken there
+        for layer in model.layers:
+            layer.last_indices = None
+        seq = Sequence([t % 50 for t in range(32 * caches[1].max_chunks + over)])
+        with pytest.raises(RuntimeError, match="capacity reached"):
+            model.logits([seq], caches, True)
+    assert caches[0].tree.n_seqs == 2 and model.layers[0].last_indices == [seq.index]
+    assert model.layers[1].last_indices is None
+    caches[0].remove_seq(model.layers[0].last_indices[0])
+    assert caches[0].tree.dump()[1][2][:2] == [59, 58]

@@ -666,7 +666,7 @@ int ca_attention(ca_ctx* c, const void* q, void* out, int n_seqs, int partition,
             CA_HIP(hipEventRecord(c->ev[1], st));
             CA_HIP(hipEventRecord(c->ev[2], st));
             if (int rc = run_merge(c, out, st)) return rc;
-        } else if (c->timing == 1 || c->direct_forward) {  // one launch
+        } else if (c->timing == 1) {  // one launch
             if (int rc = run_fused(c, q, out, st)) return rc;
             CA_HIP(hipEventRecord(c->ev[1], st));
             CA_HIP(hipEventRecord(c->ev[2], st));

@@ -268,8 +268,8 @@ int ca_ctx_set_schedule(ca_ctx* ctx, int mode);
 /* Timing of ca_attention with HIP events recorded on the stream the kernels are launched on
  * (the reference marks its phases with NVTX ranges, kernel_cuda.cu:1334-1433).
  * mode 0: off.  mode 1: ca_attention runs as it normally does with events around its launches;
- * ca_ctx_read_timing returns the accumulated milliseconds of the decode launch in *shared_ms
- * and of the merge launch in *merge_ms (*stream_ms stays 0).  mode 2: ca_attention runs as
+ * ca_ctx_read_timing returns the accumulated milliseconds of the decode launch (a small forward's only
+ * one) in *shared_ms and of the merge launch in *merge_ms (*stream_ms stays 0).  mode 2: ca_attention runs as
  * three separately timed launches (chunk-first, sequence-first, merge) and the three
  * accumulators are filled; for phase analysis, slower than the normal forward.  Every mode
  * writes the complete output. */

@@ -136,3 +136,20 @@ def test_delta_tokens_past_the_room_of_last_chunks(c):
     for delta in (0, 1, 4, 5, 11, c - 1, c, 5 * c, 1 << 20):
         attn.ctx.delta_tokens = other.ctx.delta_tokens = delta
         assert_close(attn.forward(q), other.forward(q).float().cpu().numpy())
+
+
+def test_timed_forwards_run_what_they_time():
+    """Mode 1: the forward as it is, here one launch; mode 2: the three phases."""
+    rng = np.random.default_rng(6)
+    attn, _ = build(rng, 12, 64, 256, [100, 75, 63, 1])
+    q = to_dev(rand(rng, 4, 12, 128))
+    plain, phases = attn.forward(q), torch.empty(4, 12, 128, dtype=torch.float16, device=dev())
+    stream = torch.cuda.current_stream().cuda_stream
+    attn.ctx.attn_chunks_first(q.data_ptr(), 4, stream)
+    attn.ctx.attn_seqs_first(q.data_ptr(), phases.data_ptr(), 4, stream)
+    assert not torch.equal(plain, phases)      # (the phases round probabilities of shared chunks to fp16)
+    for mode, want in ((1, plain), (2, phases), (0, plain)):
+        attn.ctx.set_timing(mode)
+        for _ in range(3):
+            assert torch.equal(attn.forward(q), want)
+        assert attn.ctx.read_timing()["calls"] == (3 if mode else 0)

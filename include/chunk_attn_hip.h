@@ -271,8 +271,8 @@ int ca_ctx_set_schedule(ca_ctx* ctx, int mode);
  * ca_ctx_read_timing returns the accumulated milliseconds of the decode launch (a small forward's only
  * one) in *shared_ms and of the merge launch in *merge_ms (*stream_ms stays 0).  mode 2: ca_attention runs as
  * three separately timed launches (chunk-first, sequence-first, merge) and the three
- * accumulators are filled; for phase analysis, slower than the normal forward.  Every mode
- * writes the complete output. */
+ * accumulators are filled; for phase analysis, slower than the normal forward (a small forward's own
+ * launch follows them).  Every mode writes the complete output, the same bits. */
 int ca_ctx_set_timing(ca_ctx* ctx, int mode);
 int ca_ctx_read_timing(ca_ctx* ctx, double* shared_ms, double* stream_ms, double* merge_ms,
                        int64_t* calls, int reset);

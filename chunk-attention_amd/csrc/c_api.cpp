@@ -147,6 +147,7 @@ struct ca_ctx {
 
     float* part = nullptr;
     size_t part_cap = 0;  // bytes
+    bool part_skipped = false;  // the last attention call was a direct launch, which has no partial rows
     int32_t* counters = nullptr;  // [n_seqs * H] partials finished per (sequence, head)
     size_t counters_cap = 0;      // bytes
     // Device buffers that were outgrown.  Launches already queued may still read them, and
@@ -291,6 +292,7 @@ int run_direct(ca_ctx* c, const ca::LaunchArgs& a, hipStream_t st) {
     for (int s = 0; s < c->n_seqs; s++) {
         len[s] = static_cast<int32_t>(std::min(int64_t(c->plan.seq_len[s]) + c->delta_tokens, int64_t(c->plan.path_len[s]) * c->C));
     }
+    c->part_skipped = true;
     return launch_rc(ca::launch_direct(a, len, c->plan.paths.data(), c->n_seqs, c->plan.path_stride, st), "direct launch");
 }
 
@@ -468,18 +470,24 @@ int collect_timing(ca_ctx* c) {
     return CA_OK;
 }
 
+// The decode launch over `n_shared` and `n_stream` of the plan's items, partial rows into the context's buffer.
+int run_items(ca_ctx* c, const ca::LaunchArgs& a, size_t n_shared, size_t n_stream, bool fuse_merge, const char* what, hipStream_t st) {
+    c->part_skipped = false;
+    return launch_rc(ca::launch_decode(a, static_cast<int>(n_shared), static_cast<int>(n_stream), fuse_merge, st), what);
+}
+
+int run_items(ca_ctx* c, const ca::LaunchArgs& a, bool fuse_merge, hipStream_t st) {
+    return run_items(c, a, c->plan.shared_items.size(), c->plan.stream_items.size(), fuse_merge, "decode launch", st);
+}
+
 int run_shared(ca_ctx* c, const void* q, hipStream_t st) {
     if (int rc = ensure_tables(c, st)) return rc;
-    const ca::LaunchArgs a = launch_args(c, q, nullptr);
-    return launch_rc(ca::launch_decode(a, static_cast<int>(c->plan.shared_items.size()), 0, false, st),
-                     "chunk-first launch");
+    return run_items(c, launch_args(c, q, nullptr), c->plan.shared_items.size(), 0, false, "chunk-first launch", st);
 }
 
 int run_stream(ca_ctx* c, const void* q, void* out, hipStream_t st) {
     if (int rc = ensure_tables(c, st)) return rc;
-    const ca::LaunchArgs a = launch_args(c, q, out);
-    return launch_rc(ca::launch_decode(a, 0, static_cast<int>(c->plan.stream_items.size()), false, st),
-                     "sequence-first launch");
+    return run_items(c, launch_args(c, q, out), 0, c->plan.stream_items.size(), false, "sequence-first launch", st);
 }
 
 int run_merge(ca_ctx* c, void* out, hipStream_t st) {
@@ -494,13 +502,10 @@ int run_fused(ca_ctx* c, const void* q, void* out, hipStream_t st) {
     if (int rc = ensure_tables(c, st)) return rc;
     if (c->schedule == 0) {
         // both phases in one launch (shared and stream workgroups overlap), then the merge
-        if (int rc = launch_rc(ca::launch_decode(a, static_cast<int>(c->plan.shared_items.size()),
-                                                 static_cast<int>(c->plan.stream_items.size()), false, st), "decode launch")) return rc;
+        if (int rc = run_items(c, a, false, st)) return rc;
         return run_merge(c, out, st);
     }
-    return launch_rc(ca::launch_decode(a, static_cast<int>(c->plan.shared_items.size()),
-                                       static_cast<int>(c->plan.stream_items.size()), true, st),
-                     "decode launch");
+    return run_items(c, a, true, st);
 }
 
 }  // namespace
@@ -660,9 +665,7 @@ int ca_attention(ca_ctx* c, const void* q, void* out, int n_seqs, int partition,
         if (c->timing == 1 && c->schedule == 0 && !c->direct_forward) {
             // the forward as it normally runs: decode launch, then merge launch
             if (int rc = ensure_tables(c, st)) return rc;
-            const ca::LaunchArgs a = launch_args(c, q, out);
-            if (int rc = launch_rc(ca::launch_decode(a, static_cast<int>(c->plan.shared_items.size()),
-                                                     static_cast<int>(c->plan.stream_items.size()), false, st), "decode launch")) return rc;
+            if (int rc = run_items(c, launch_args(c, q, out), false, st)) return rc;
             CA_HIP(hipEventRecord(c->ev[1], st));
             CA_HIP(hipEventRecord(c->ev[2], st));
             if (int rc = run_merge(c, out, st)) return rc;
@@ -680,7 +683,10 @@ int ca_attention(ca_ctx* c, const void* q, void* out, int n_seqs, int partition,
         CA_HIP(hipEventRecord(c->ev[3], st));
         c->ev_pending = true;
         // the phases round elsewhere than a small forward's one launch: timed or not, a forward has the same bits
-        if (c->timing == 2 && c->direct_forward) return run_fused(c, q, out, st);
+        if (c->timing == 2 && c->direct_forward) {
+            if (int rc = run_fused(c, q, out, st)) return rc;
+            c->part_skipped = false;  // the phases' rows
+        }
         return CA_OK;
     });
 }
@@ -746,8 +752,7 @@ int decode_step(ca_ctx* c, const void* q, const void* k, const void* v, void* ou
         a.v_new = v;
         a.tail_slot = reinterpret_cast<const int32_t*>(c->dev_blob + c->off_tail_slot);
         a.tail_fill = reinterpret_cast<const int32_t*>(c->dev_blob + c->off_tail_fill);
-        int rc = launch_rc(ca::launch_decode(a, static_cast<int>(c->plan.shared_items.size()),
-                                             static_cast<int>(c->plan.stream_items.size()), false, st), "decode launch");
+        int rc = run_items(c, a, false, st);
         // the merge launch also puts the new rows into the pool (after every read of this step)
         if (rc == CA_OK) rc = launch_rc(ca::launch_merge(a, c->n_seqs, c->plan.n_part_rows > 0, st), "merge launch");
         if (rc != CA_OK) c->delta_tokens -= 1;
@@ -1394,9 +1399,18 @@ int ca_ctx_ref_tables(const ca_ctx* c, int32_t* final_idx, int32_t* slots, int32
     });
 }
 
+namespace {
+int check_partials(const ca_ctx* c) {
+    if (!c->part_skipped) return CA_OK;
+    return fail(CA_ERR_STATE, "the last forward was a small one, whose single launch writes no partial rows: "
+                              "ca_attn_chunks_first and ca_attn_seqs_first do");
+}
+}  // namespace
+
 int ca_ctx_export_partials(ca_ctx* c, float* maxs, float* sums, float* attns, void* stream) {
     if (!c || !c->valid) return fail(CA_ERR_STATE, "kernel context is not valid");
     if (c->partition != 0) return fail(CA_ERR_STATE, "partials are exported for partition 0 only");
+    if (int rc = check_partials(c)) return rc;
     return guarded([&]() -> int {
         const ca::Plan& p = c->plan;
         // one item group per shared chunk, in shared-chunk order, is what the layout needs
@@ -1443,6 +1457,7 @@ int ca_ctx_export_partials(ca_ctx* c, float* maxs, float* sums, float* attns, vo
 
 int ca_ctx_read_partials_raw(ca_ctx* c, float* out, int64_t n_floats, void* stream) {
     if (!c || !out || n_floats < 0) return fail(CA_ERR_INVALID, "bad argument");
+    if (int rc = check_partials(c)) return rc;
     const int64_t have = int64_t(c->plan.n_part_rows) * c->H * ca::PART_STRIDE;
     const int64_t n = std::min(n_floats, have);
     hipStream_t st = static_cast<hipStream_t>(stream);
@@ -1463,10 +1478,8 @@ int ca_bench_decode_launch(ca_ctx* c, const void* q, void* out, int n_seqs, int 
         return fail(CA_ERR_STATE, "the tables were built for another partition or schedule");
     }
     if (int rc = ensure_tables(c, static_cast<hipStream_t>(stream))) return rc;
-    const ca::LaunchArgs a = launch_args(c, q, out);
-    const int n_shared = what == 1 ? 0 : static_cast<int>(c->plan.shared_items.size());
-    const int n_stream = what == 2 ? 0 : static_cast<int>(c->plan.stream_items.size());
-    return launch_rc(ca::launch_decode(a, n_shared, n_stream, false, static_cast<hipStream_t>(stream)), "decode launch");
+    return run_items(c, launch_args(c, q, out), what == 1 ? 0 : c->plan.shared_items.size(), what == 2 ? 0 : c->plan.stream_items.size(),
+                     false, "decode launch", static_cast<hipStream_t>(stream));
 }
 
 int ca_bench_read_probe(ca_ctx* c, const void* dev, size_t bytes, int wgs_per_cu, void* stream) {

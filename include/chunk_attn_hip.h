@@ -311,11 +311,12 @@ int ca_ctx_ref_tables(const ca_ctx* ctx, int32_t* final_idx, int32_t* slots, int
  * (kernel_cuda.cu:830-838): for shared chunk i with n covered sequences and row offset
  * off = offsets[i]:  maxs/sums[off*H + h*n + r], attns[(off*H + h*n + r)*d ...], maxima in
  * natural-log units of score/sqrt(d).  Needs tables built with shared_seg_chunks = 1 and
- * partition 0.  Synchronises the stream. */
+ * partition 0, and partial rows to copy: CA_ERR_STATE after a small forward that was one launch and wrote none
+ * (ca_attn_chunks_first and ca_attn_seqs_first always do).  Synchronises the stream. */
 int ca_ctx_export_partials(ca_ctx* ctx, float* maxs, float* sums, float* attns, void* stream);
 
 /* Raw copy of the partial-row buffer ([n_part_rows][n_heads][160] floats: max, sum, 2 unused,
- * 128 acc in base-2 units, 28 unused) to the host, for inspection.  Synchronises the stream. */
+ * 128 acc in base-2 units, 28 unused) to the host, for inspection; CA_ERR_STATE as above.  Synchronises the stream. */
 int ca_ctx_read_partials_raw(ca_ctx* ctx, float* out, int64_t n_floats, void* stream);
 
 /* ---- measurement aids: for benchmarks, not for callers --------------------------------- */

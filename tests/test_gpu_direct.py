@@ -7,6 +7,7 @@ import pytest
 import torch
 
 from gpu_helpers import assert_close, dev, host_state, make_attention, oracle_output, to_dev
+from oracle.attention_ref import textbook_partials
 
 pytestmark = pytest.mark.gpu
 
@@ -155,3 +156,29 @@ def test_timed_forwards_run_what_they_time():
     attn.ctx.attn_seqs_first(q.data_ptr(), out.data_ptr(), 4, stream)
     used = np.r_[0, 1, 4:132]
     np.testing.assert_array_equal(of_mode_2[:, :, used], attn.ctx.read_partials_raw()[:, :, used])
+
+
+def test_partial_rows_are_those_of_the_last_forward():
+    """A direct launch has none: none are handed out, least of all older ones."""
+    rng = np.random.default_rng(7)
+    attn, _ = build(rng, 3, 64, 64, [100, 75])
+    q = to_dev(rand(rng, 2, 3, 128))
+    stream = torch.cuda.current_stream().cuda_stream
+    phases = torch.empty_like(q)
+    for again in range(2):
+        attn.forward(q)
+        for read in (attn.ctx.read_partials_raw, attn.ctx.export_partials):
+            with pytest.raises(RuntimeError, match="no partial rows"):
+                read()
+        attn.ctx.attn_chunks_first(q.data_ptr(), 2, stream)
+        maxs, sums, attns = attn.ctx.export_partials()
+        rows, kp, vp = host_state(attn)
+        slot, n_tok, b, e = rows[0].tolist()
+        m, l, o = textbook_partials(q.float().cpu().numpy(), slot, n_tok, b, e, kp, vp)
+        np.testing.assert_allclose(maxs.reshape(m.shape), m, atol=1e-3, rtol=1e-3)      # as with explicit item sizes
+        np.testing.assert_allclose(sums.reshape(l.shape), l, atol=1e-3, rtol=2e-3)
+        np.testing.assert_allclose(attns.reshape(o.shape), o, atol=1e-2, rtol=1e-2)
+        attn.ctx.attn_seqs_first(q.data_ptr(), phases.data_ptr(), 2, stream)
+        assert np.isfinite(attn.ctx.read_partials_raw()[:, :, :2]).all()
+    attn.forward(q, 1)
+    assert attn.ctx.read_partials_raw().shape[1] == 3

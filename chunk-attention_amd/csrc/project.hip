@@ -477,8 +477,13 @@ int launch_mode(const ProjectArgs& a, hipStream_t st) {
     }
     auto tiles = [&](int bm, int bn) { return int64_t((a.N + bn - 1) / bn) * a.n_w * ((int64_t(a.M) + bm - 1) / bm); };
     constexpr int CUS = 256;
-    // (shared tiles reach their rows and columns with 32-bit offsets)
-    if (tiles(32, 32) <= CUS + CUS / 8 || int64_t(a.N) * a.K >= int64_t(1) << 30 || a.K > 1 << 22) return launch_tile<2, 2, 2, 32, MODE>(a, st);
+    if (tiles(32, 32) <= CUS + CUS / 8) return launch_tile<2, 2, 2, 32, MODE>(a, st);
+    // Shared tiles reach their rows and columns with 32-bit offsets.  Beyond them the largest tile with k split over
+    // the waves, where three quarters of the compute units get one (32768 x 32768 on 65, 252 and 1000 rows 779, 1544 and 6146 us; in
+    // 32 x 32 tiles 1134, 2960 and 11711).
+    if (int64_t(a.N) * a.K >= int64_t(1) << 30 || a.K > 1 << 22) {
+        return 4 * tiles(64, 64) < 3 * CUS ? launch_tile<2, 2, 2, 32, MODE>(a, st) : launch_tile<4, 4, 2, 64, MODE>(a, st);
+    }
     if (tiles(64, 64) <= CUS) return launch_shared_tile<64, 64, 4, 4, 2, MODE>(a, st);
     if (tiles(64, 128) <= CUS) return launch_shared_tile<64, 128, 4, 8, 2, MODE>(a, st);
     const int64_t square = (tiles(128, 128) + CUS - 1) / CUS, wide = (tiles(128, 256) + CUS - 1) / CUS;

@@ -33,3 +33,15 @@ def test_qkv_rotary_in_shared_tiles(rows, heads, n_in):
 
 def test_decode_of_more_rows_than_a_block():
     project.test_layer_decode_writes_the_pool_as_the_library_path_does(70, 12, 64)
+
+
+@pytest.mark.parametrize("rows", [20, 70])
+def test_linear_beyond_the_reach_of_shared_tiles(rows):
+    """2^30 weights and more: 64 x 64 tiles with k split over the waves."""
+    n_out, n_in = 16500, 65088
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    x = torch.randn(rows, n_in, generator=g, device="cuda", dtype=torch.float16)
+    w = torch.randn(n_out, n_in, generator=g, device="cuda", dtype=torch.float16).mul_(n_in ** -0.5)
+    got = capi.linear(x, w)
+    for c in range(0, n_out, 2500):
+        _close(got[:, c:c + 2500], x.double() @ w[c:c + 2500].double().t(), n_in)

@@ -472,6 +472,9 @@ __device__ __forceinline__ void stream_path(const DecodeArgs& A, const WorkItem*
         folded = true;
     };
     bool tried = !can_fold;
+    const bool alone = it.part_row < 0;  // the item is its sequence, its sums are the output
+    // What divides the sums where no weight is above zero: no tokens give zero, no finite score none.
+    const float r_empty = len > 0 ? __builtin_nanf("") : 0.f;
 
     constexpr int SPLIT = DIRECT ? NSUB : 1;       // steps that share a tile
     for (int ts = (PER_WAVE ? 0 : w) * CPT; ts < it.n_chunks * SPLIT; ts += (PER_WAVE ? 1 : NWV) * CPT) {
@@ -565,8 +568,10 @@ __device__ __forceinline__ void stream_path(const DecodeArgs& A, const WorkItem*
             const int row = 4 * (j % NL) + g;
             if (row >= vsub || j >= NL) s = NEG_INF;
             const float m_new = fmaxf(m_run, wave_max(s));
-            const float alpha = fast_exp2(m_run - m_new);
-            const float p = fast_exp2(s - m_new);
+            // Nothing but scores of minus infinity so far: weights of zero, whichever wave the tile falls to.
+            const float m_from = (alone && m_new == NEG_INF) ? 0.f : m_new;
+            const float alpha = fast_exp2(m_run - m_from);
+            const float p = fast_exp2(s - m_from);
             m_run = m_new;
             l_lane = l_lane * alpha + p;
             sm.p[w][l] = p;
@@ -619,7 +624,7 @@ __device__ __forceinline__ void stream_path(const DecodeArgs& A, const WorkItem*
         // lanes of group 0 hold dims 8j..8j+7 of the wave's (= the item's) result
         if (g == 0) {
             if (it.part_row < 0) {
-                const float r = l_wave > 0.f ? 1.f / l_wave : 0.f;
+                const float r = l_wave > 0.f ? 1.f / l_wave : r_empty;
                 h8 o8;
 #pragma unroll
                 for (int e = 0; e < 8; e++) o8[e] = half_t(acc[e] * r);
@@ -658,7 +663,7 @@ __device__ __forceinline__ void stream_path(const DecodeArgs& A, const WorkItem*
     }
     if (it.part_row < 0 || complete) {  // nothing (left) to merge: final output
         if (tid < D) {
-            const float r = lsum > 0.f ? 1.f / lsum : 0.f;
+            const float r = lsum > 0.f ? 1.f / lsum : r_empty;
             A.out[(size_t(seq) * H + h) * D + tid] = half_t(o * r);
         }
         if (complete && tid == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

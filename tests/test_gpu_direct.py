@@ -182,3 +182,62 @@ def test_partial_rows_are_those_of_the_last_forward():
         assert np.isfinite(attn.ctx.read_partials_raw()[:, :, :2]).all()
     attn.forward(q, 1)
     assert attn.ctx.read_partials_raw().shape[1] == 3
+
+
+def poison(attn, infinite):
+    """NaN in every row that no token stands in; key element 0 of token t of sequence s as infinite[s, t] says."""
+    kp, vp = attn.pool_views()
+    c = attn.chunk_size
+    for slot, n, _, _ in attn.get_chunks().tolist():
+        kp[slot][:, n:], vp[slot][:, n:] = float("nan"), float("nan")
+    paths = [[r[0] for r in attn.get_chunks().tolist() if r[2] <= s < r[3]] for s in range(attn.tree.n_seqs)]
+    for (s, t), value in infinite.items():
+        kp[paths[s][t // c]][:, t % c, 0] = value
+
+
+def same(got, want):
+    with np.errstate(invalid="ignore"):
+        np.testing.assert_allclose(got.float().cpu().numpy(), want, atol=2e-3, rtol=1e-2, equal_nan=True)
+
+
+@pytest.mark.filterwarnings("ignore:invalid value")
+@pytest.mark.parametrize("c", [32, 64, 128])
+def test_infinite_scores_and_stale_rows(c):
+    """A key whose score is minus infinity weighs nothing, also where a tile has no other and the tile is its wave's
+    first; a sequence of nothing else has no answer, nor one with a score of plus infinity.  Rows behind the last
+    token are not looked at."""
+    rng = np.random.default_rng(c)
+    low, high = -float("inf"), float("inf")
+    privates = [258, 400, 70, 700, 321, 300]
+    attn, _ = build(rng, 3, c, 0, privates)
+    poison(attn, {**{(0, t): low for t in (256, 257)}, **{(1, t): low for t in range(64, 192)}, **{(2, t): low for t in range(70)},
+                  (3, 5): high, **{(4, t): low for t in (0, 320)}, **{(5, t): low for t in range(1, 300)}})
+    q = np.abs(rand(rng, 6, 3, 128)) + np.float16(0.1)
+    want = oracle_output(attn, q, exact=True)
+    assert np.isnan(want[[2, 3]]).all() and np.isfinite(want[[0, 1, 4, 5]]).all()
+    same(attn.forward(to_dev(q)), want)
+
+
+@pytest.mark.filterwarnings("ignore:invalid value")
+@pytest.mark.parametrize("c", [32, 64, 128])
+def test_fused_steps_of_infinite_scores(c):
+    """Steps in direct form and forwards in the general one, over paths on which both are one launch: new tokens alone
+    in their tiles, with keys of minus infinity, and one that has no other token."""
+    rng = np.random.default_rng(c + 1)
+    privates = [64, 128, 190, 1, 250]
+    fused, kv = build(rng, 30, c, 0, privates)
+    apart, _ = build(rng, 30, c, 0, privates, False, kv)
+    for a in (fused, apart):
+        a.reserve()
+        poison(a, {(3, 0): -float("inf"), **{(4, t): -float("inf") for t in range(64)}})
+    for step in range(4):
+        q, k, v = (np.abs(rand(rng, 5, 30, 128)) + np.float16(0.1) for _ in range(3))
+        k[:4 if step < 2 else 2, :, 0] = -np.inf
+        q, k, v = map(to_dev, (q, k, v))
+        tokens = [10 ** 6 + 10 * step + s for s in range(5)]
+        out = fused.decode_step(tokens, q, k, v)
+        apart.append_token(tokens, k, v)
+        np.testing.assert_array_equal(out.cpu().numpy(), apart.forward(q).cpu().numpy())
+        want = oracle_output(fused, q.cpu().numpy(), exact=True)
+        assert np.isnan(want[3]).all() == (step < 2) and np.isfinite(np.delete(want, 3, 0)).all()
+        same(out, want)

@@ -141,6 +141,7 @@ SIGNATURES = {
     "ca_tables_plan_sizes": (ctypes.c_int, [ctypes.c_void_p, c_int_p]),
     "ca_tables_ref": (ctypes.c_int, [ctypes.c_void_p] + [c_i32_p] * 7),
     "ca_tables_plan": (ctypes.c_int, [ctypes.c_void_p] + [c_i32_p] * 7),
+    "ca_tables_paths": (ctypes.c_int, [ctypes.c_void_p, c_int_p, c_i32_p, c_i32_p]),
     "ca_tree_create": (ctypes.c_int, [ctypes.POINTER(ctypes.c_void_p), ctypes.c_int, ctypes.c_int,
                                       ctypes.c_int]),
     "ca_tree_destroy": (None, [ctypes.c_void_p]),
@@ -725,6 +726,12 @@ class HostTables:
         }
         _check(self._lib.ca_tables_plan(self._h, *[p[k].ctypes.data_as(c_i32_p) for k in (
             "shared_items", "stream_items", "slots", "seq_len", "part_ptr", "tail_slot", "tail_fill")]))
+        stride = ctypes.c_int()
+        _check(self._lib.ca_tables_paths(self._h, ctypes.byref(stride), None, None))
+        rows = info.n_seqs if stride.value else 0
+        p["path_stride"] = stride.value
+        p["paths"], p["path_len"] = np.zeros((rows, stride.value), np.int32), np.zeros(rows, np.int32)
+        _check(self._lib.ca_tables_paths(self._h, None, p["paths"].ctypes.data_as(c_i32_p), p["path_len"].ctypes.data_as(c_i32_p)))
         p["n_part_rows"] = info.n_part_rows
         p["shared_tokens"] = info.shared_tokens
         p["stream_tokens"] = info.stream_tokens

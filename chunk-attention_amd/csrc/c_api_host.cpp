@@ -169,6 +169,14 @@ int ca_tables_plan(const ca_tables* t, ca_work_item* shared_items, ca_work_item*
     return CA_OK;
 }
 
+int ca_tables_paths(const ca_tables* t, int* stride, int32_t* paths, int32_t* path_len) {
+    if (!t) return fail(CA_ERR_INVALID, "bad argument");
+    if (stride) *stride = t->plan.path_stride;
+    copy_i32(paths, t->plan.paths);
+    copy_i32(path_len, t->plan.path_len);
+    return CA_OK;
+}
+
 // ---- prefix-tree manager -------------------------------------------------------------------
 
 struct ca_tree {

@@ -376,6 +376,9 @@ int ca_tables_ref(const ca_tables* t, int32_t* final_idx, int32_t* slots, int32_
 int ca_tables_plan(const ca_tables* t, ca_work_item* shared_items, ca_work_item* stream_items,
                    int32_t* slots, int32_t* seq_len, int32_t* part_ptr, int32_t* tail_slot,
                    int32_t* tail_fill);
+/* whole paths, what a small forward in one launch takes instead: *stride 0 where the tree does not fit that
+ * form, else chunk k of sequence s at paths[s * *stride + k], path_len[s] of them (NULL = skip) */
+int ca_tables_paths(const ca_tables* t, int* stride, int32_t* paths, int32_t* path_len);
 
 /* ---- prefix-tree chunk manager -------------------------------------------------------- */
 

@@ -65,6 +65,9 @@ def test_fused_steps_write_their_rows_and_follow_rollovers(c, H, shared, private
         out = fused.decode_step(tokens, q, k, v)
         apart.append_token(tokens, k, v)
         assert torch.equal(out, apart.forward(q))
+        fills = {r[1] for r in fused.get_chunks().tolist() if r[3] - r[2] == 1}
+        if step < 2 or fills & {1, c}:                 # around roll-overs: also against what takes no work list of ours
+            assert_close(out, oracle_output(fused, q.cpu().numpy(), exact=True))
     rows_a, ka, va = host_state(fused)
     rows_b, kb, vb = host_state(apart)
     np.testing.assert_array_equal(rows_a, rows_b)
@@ -119,6 +122,20 @@ def test_phases_and_partitions_upload_what_they_read():
     assert_close(out, want)
     for partition in (0, 1, 0, 2, 0):
         assert_close(attn.forward(qd, partition), want)
+
+
+def test_stream_hint_and_side_streams_change_no_bit():
+    rng = np.random.default_rng(8)
+    attn, _ = build(rng, 12, 64, 256, [100, 75, 63, 1])
+    q = to_dev(rand(rng, 4, 12, 128))
+    want, side = attn.forward(q), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for hint in (1, 2, 0):
+        attn.ctx.set_stream_hint(hint)
+        with torch.cuda.stream(side):
+            got = attn.forward(q)
+        side.synchronize()
+        assert torch.equal(got, want)
 
 
 @pytest.mark.parametrize("c", [32, 64, 128])

@@ -428,3 +428,40 @@ def test_tiny_launches_count_the_segments_that_are_cut():
     rows = [(i, 32, 0, 16) for i in range(17)] + [(100 + s, 20, s, s + 1) for s in range(16)]
     plan = capi.build_tables(np.array(rows, np.int32), 16, 32, n_heads=16, n_cus=256)["plan"]
     assert len(set(plan["shared_items"][:, 4])) == 4
+
+
+def paths_of(rows, n_seqs):
+    return [[r[0] for r in rows.tolist() if r[2] <= s < r[3]] for s in range(n_seqs)]
+
+
+@pytest.mark.parametrize("c,shared,privates,fits", [
+    (4, 8, [1, 3, 4, 5, 17], True), (4, 0, [2], True), (2, 0, [3] * 64, True), (2, 0, [3] * 65, False),
+    (2, 0, [127], True), (2, 0, [127, 1], True), (2, 0, [129], False),                     # 64 chunks a path
+    (2, 8, [15] * 64, True), (2, 8, [15] * 63 + [17], False),                              # 768 slots in all
+])
+def test_whole_paths_through_rollovers(c, shared, privates, fits):
+    """What a small forward in one launch takes instead of work items: every sequence's chunks in path order, while
+    sequences and chunks are few enough, and nothing from the first table on that is past one of those lines."""
+    tree = capi.Tree(c, 4096)
+    n = len(privates)
+    for s, p in enumerate(privates):
+        tree.add_seq(list(range(shared)) + [1000 * (s + 1) + t for t in range(p)])
+    tree.reserve_tails()
+    live = capi.HostTables(tree.get_chunks(), n, c)
+    delta = 0
+    for step in range(2 * c + 2):
+        seqs, slots = tree.reserve_tails()
+        if seqs:
+            live.roll_tails(delta, seqs, slots)
+            delta = 0
+        want, plan = paths_of(tree.get_chunks(), n), live.plan()
+        stride = max(map(len, want))
+        held = n <= 64 and stride <= 64 and n * stride <= 768
+        if step == 0:
+            assert held == fits
+        assert plan["path_stride"] == (stride if held else 0)
+        assert plan["path_len"].tolist() == ([len(w) for w in want] if held else [])
+        for s in range(n if held else 0):
+            assert plan["paths"][s, :len(want[s])].tolist() == want[s] and not plan["paths"][s, len(want[s]):].any()
+        tree.append_token([10 ** 6 + step * 100 + s for s in range(n)])
+        delta += 1

@@ -537,7 +537,7 @@ def shared_tiles_pay(rows: int, n_in: int, n_out: int, n_weights: int) -> bool:
     and the library's: 4096 x 4096 on 1000 rows 34 to 40, on 1500 50 to 52, on 2048 58 to 64, on 2300 88 to 70; 2048 x
     2048 on 3000 rows 28 to 31, on 4096 32 to 37, on 6000 53 to 47; 1024 x 1024 on 8192 rows 20 to 24).  q, k and v
     with their rotation: up to three rounds (against three products and the rotary launch: 4096 x 4096 on 512 rows 52
-    to 86, on 2048 181 to 211, on 2300 220 to 222, on 2560 232 to 230; 2048 x 2048 on 4096 rows 101 to 120; 5120 x 5120
+    to 86, on 2048 181-193 to 209-212, on 2300 220 to 222, on 2560 232 to 230; 2048 x 2048 on 4096 rows 101 to 120; 5120 x 5120
     on 1000 rows 159 to 205, on 1600 269 to 271, on 2048 309 to 300; 1024 x 1024 on 8192 rows 64 to 81).  Weights of
     more than 2^25 elements were not measured."""
     tiles = -(-rows // 128) * -(-n_out // 256) * n_weights

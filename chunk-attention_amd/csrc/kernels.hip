@@ -1536,7 +1536,8 @@ __global__ __launch_bounds__(WG) void scatter_kernel(const T* __restrict__ k, co
 // K/V rows to explicit places: row i of k and v goes to row targets.row[i] of chunk
 // targets.slot[i] (the beam-search step's row writes, one launch for all candidates).
 // The argument blocks come in two sizes: what a launch of one beam's rows takes is written across the bus with every
-// launch (a beam search of 4, 61 such launches: 411 -> 324 us a pass).
+// launch (a beam search of 4, 61 such launches: 411 -> 324 us a pass on one machine; the host's part differs, 277 to
+// 385 us on others).
 constexpr int PUT_ROWS = 64, FEW_ROWS = 8;
 template <int N>
 struct PutTargets {

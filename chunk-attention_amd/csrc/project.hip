@@ -240,7 +240,7 @@ int launch_tile(const ProjectArgs& a, hipStream_t st) {
 // What bounds it: large products, power.  With every compute unit busy the clock falls to about 1.6 GHz (matrix ops
 // on registers alone then reach 1.70 PFLOP/s as 16 x 16 x 32, 1.55 as 32 x 32 x 16, which is why the operands here are
 // 16 wide), and every LDS read and fetched line lowers it further: q, k and v of 4096 with their rotation on 2048
-// rows 181 us, 1.14 PFLOP/s (three library products and the rotary launch 211; the same stages with all of their
+// rows 181 us, 1.14 PFLOP/s (187 to 193 on other machines; three library products and the rotary launch 209 to 212; the same stages with all of their
 // loads requested in a row behind the barrier 219: a wave issues in order, and its products waited for the loads to
 // be taken; with 32 x 32 x 16 195).  One weight of 4096 on 2048 rows 57.6 (the library 64.1).  Smaller ones, the fill
 // of the pipeline and a stage's latency: 0.36 us a stage for 128 x 128, 0.56 for 128 x 256 (0.43 is the matrix cores').

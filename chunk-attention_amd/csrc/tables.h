@@ -120,7 +120,7 @@ struct Plan {
     std::vector<int32_t> own_pos0;              // per sequence: path position of own[s][0]
     std::vector<int32_t> shared_parts;          // per sequence: partial rows written by shared items
 
-    // Every sequence's whole path, for the direct form of a small forward (kernels.h, DirectTable): chunk k of
+    // Every sequence's whole path, for the direct form of a small forward (launch_direct): chunk k of
     // sequence s at paths[s * path_stride + k].  Empty when the tree does not fit that form.
     int path_stride = 0;
     std::vector<int32_t> paths;

@@ -105,8 +105,8 @@ int ca_attention(ca_ctx* ctx, const void* q, void* out, int n_seqs, int partitio
  * schedule (it never rebuilds them).  All contexts on one GPU share the array: calls that
  * overlap on one GPU (different streams or threads) race; calls on one stream are safe.  Nothing
  * in the array needs clearing between calls (every row read is written first).
- * Under graph capture: delta_tokens and the table addresses are kernel arguments of the captured
- * launches, so a captured forward replays the sequence lengths it was captured with.  Capture
+ * Under graph capture: delta_tokens and the table addresses (a small forward's lengths and chunks) are kernel
+ * arguments of the captured launches, so a captured forward replays the sequence lengths it was captured with.  Capture
  * again after every ca_append_kv / ca_decode_step, ca_ctx_roll_tails or refresh. */
 #define CA_NOALLOC_SCRATCH_BYTES (32u << 20)
 int ca_attention_noalloc(ca_ctx* ctx, const void* q, void* out, int n_seqs, void* stream);
@@ -133,7 +133,8 @@ int ca_append_kv(ca_ctx* ctx, const void* k, const void* v, int n_seqs, void* st
  * last chunk is streamed per sequence (always, with trees built by ca_tree_* / the Attention class
  * and tpp_threshold >= 1) no append launch is made: the workgroup that streams a sequence's last
  * chunk takes the new row from k / v, and the merge launch writes the rows into the pool behind
- * its merges.  Otherwise the two launches are made here.  Same preconditions as ca_append_kv (a free row in every last chunk:
+ * its merges (a small step is one launch, which writes them itself).  Otherwise the append and the
+ * forward are launched one after the other.  Same preconditions as ca_append_kv (a free row in every last chunk:
  * reserve and refresh / ca_ctx_roll_tails first); delta_tokens is advanced by one on success. */
 int ca_decode_step(ca_ctx* ctx, const void* q, const void* k, const void* v, void* out, int n_seqs,
                    void* stream);
@@ -245,7 +246,8 @@ int ca_ctx_set_plan(ca_ctx* ctx, int shared_seg_chunks, int stream_chunks);
  * one forward attends more K/V than the 256 MiB last-level cache holds, plainly otherwise (a
  * caller that repeats forwards over a small cache finds part of it there again).  1: always with
  * the hint -- for a model whose layers each own a cache, so that nothing attended is still cached
- * when its layer comes round again.  2: never.  Results do not depend on it.  No counterpart in
+ * when its layer comes round again.  2: never.  A small forward that is one launch reads plainly whatever the
+ * hint.  Results do not depend on it.  No counterpart in
  * the reference (its kernels use plain loads, kernel_cuda.cu:885-1086). */
 int ca_ctx_set_stream_hint(ca_ctx* ctx, int mode);
 

@@ -960,13 +960,19 @@ int project(ca::ProjectArgs& a, const void* x, int M, int N, int K, void* stream
     if (M == 0) return CA_OK;
     return launch_rc(ca::launch_project(a, static_cast<hipStream_t>(stream)), "projection launch");
 }
-}  // namespace
 
-int ca_linear(const void* x, const void* w, void* y, int n_rows, int n_out, int n_in, void* stream) {
+ca::ProjectArgs linear_args(const void* w, void* y, const void* add = nullptr) {
     ca::ProjectArgs a;
     a.n_w = 1;
     a.w[0] = w;
     a.y[0] = y;
+    a.add = add;
+    return a;
+}
+}  // namespace
+
+int ca_linear(const void* x, const void* w, void* y, int n_rows, int n_out, int n_in, void* stream) {
+    ca::ProjectArgs a = linear_args(w, y);
     return project(a, x, n_rows, n_out, n_in, stream);
 }
 
@@ -998,9 +1004,15 @@ ca::ProjectArgs qkv_append_args(const ca_ctx* c, const void* wq, const void* wk,
 }
 }  // namespace
 
-int ca_qkv_rotary_append_kv(ca_ctx* c, const void* x, const void* wq, const void* wk, const void* wv,
-                            const int64_t* positions, const void* cos_sin_cache, int max_position, void* q,
-                            int n_in, int n_seqs, void* stream) {
+namespace {
+// norm: what the rows of x are normalised with first, if anything.
+struct RowNorm {
+    const void* weight = nullptr;
+    float epsilon = 0.f;
+};
+
+int qkv_append(ca_ctx* c, const void* x, const RowNorm& norm, const void* wq, const void* wk, const void* wv, const int64_t* positions,
+               const void* cos_sin_cache, int max_position, void* q, int n_in, int n_seqs, void* stream) {
     if (int rc = check_ready(c, q, n_seqs)) return rc;
     if (c->d != 128) return fail(CA_ERR_INVALID, "fused projection and append need d_head 128");
     if (n_seqs > 0 && !positions) return fail(CA_ERR_INVALID, "null device pointer");
@@ -1016,7 +1028,16 @@ int ca_qkv_rotary_append_kv(ca_ctx* c, const void* x, const void* wq, const void
     a.tail_fill = reinterpret_cast<const int32_t*>(c->dev_blob + c->off_tail_fill);
     a.delta_tokens = c->delta_tokens;
     a.C = c->C;
+    a.norm = norm.weight;
+    a.norm_epsilon = norm.epsilon;
     return project(a, x, n_seqs, c->H * 128, n_in, stream);
+}
+}  // namespace
+
+int ca_qkv_rotary_append_kv(ca_ctx* c, const void* x, const void* wq, const void* wk, const void* wv,
+                            const int64_t* positions, const void* cos_sin_cache, int max_position, void* q,
+                            int n_in, int n_seqs, void* stream) {
+    return qkv_append(c, x, {}, wq, wk, wv, positions, cos_sin_cache, max_position, q, n_in, n_seqs, stream);
 }
 
 namespace {
@@ -1050,10 +1071,12 @@ bool has_room(const ca_ctx* c, int n_seqs) {
 }
 }  // namespace
 
-int ca_layer_decode(ca_ctx* c, ca_tree* tree, const int32_t* tokens, int n_seqs, const void* x, int n_in,
-                    const void* wq, const void* wk, const void* wv, const void* wo, int n_out,
-                    const int64_t* positions, const void* cos_sin_cache, int max_position, void* q, void* attn,
-                    void* y, void* stream) {
+namespace {
+// norm: of the rows of x, if any; add: what the output projection is added to, if anything.
+int layer_decode(ca_ctx* c, ca_tree* tree, const int32_t* tokens, int n_seqs, const void* x, int n_in, const RowNorm& norm,
+                 const void* wq, const void* wk, const void* wv, const void* wo, int n_out, const void* add,
+                 const int64_t* positions, const void* cos_sin_cache, int max_position, void* q, void* attn,
+                 void* y, void* stream) {
     if (!c || !tree || !tokens || n_seqs <= 0) return fail(CA_ERR_INVALID, "bad argument");
     if (ca_tree_n_seqs(tree) != n_seqs) return fail(CA_ERR_INVALID, "num of seqs is not equal to num of tokens");
     // everything its calls would refuse, before the cache moves on: a refused call can be made again
@@ -1062,21 +1085,27 @@ int ca_layer_decode(ca_ctx* c, ca_tree* tree, const int32_t* tokens, int n_seqs,
     if (c->valid && c->delta_tokens < 0) return fail(CA_ERR_STATE, "delta_tokens is negative");
     ca::ProjectArgs in = qkv_append_args(c, wq, wk, wv, positions, cos_sin_cache, max_position, q);
     if (int rc = check_project(in, x, n_seqs, c->H * 128, n_in)) return rc;
-    ca::ProjectArgs out;
-    out.n_w = 1;
-    out.w[0] = wo;
-    out.y[0] = y;
+    ca::ProjectArgs out = linear_args(wo, y, add);
     if (int rc = check_project(out, attn, n_seqs, n_out, c->H * 128)) return rc;
     return guarded([&]() -> int {
         if (int rc = settle(c, tree, n_seqs, stream)) return rc;
-        if (int rc = ca_qkv_rotary_append_kv(c, x, wq, wk, wv, positions, cos_sin_cache, max_position, q, n_in, n_seqs, stream)) return rc;
+        if (int rc = qkv_append(c, x, norm, wq, wk, wv, positions, cos_sin_cache, max_position, q, n_in, n_seqs, stream)) return rc;
         int fresh = 0;
         if (int rc = ca_tree_append_token(tree, tokens, n_seqs, &fresh)) return rc;
         if (int rc = ca_ctx_set_delta_tokens(c, c->delta_tokens + 1)) return rc;
         if (int rc = ca_attention(c, q, attn, n_seqs, 0, stream)) return rc;
-        if (int rc = ca_linear(attn, wo, y, n_seqs, n_out, c->H * 128, stream)) return rc;
+        if (int rc = launch_rc(ca::launch_project(out, static_cast<hipStream_t>(stream)), "projection launch")) return rc;
         return settle(c, tree, n_seqs, stream);
     });
+}
+}  // namespace
+
+int ca_layer_decode(ca_ctx* c, ca_tree* tree, const int32_t* tokens, int n_seqs, const void* x, int n_in,
+                    const void* wq, const void* wk, const void* wv, const void* wo, int n_out,
+                    const int64_t* positions, const void* cos_sin_cache, int max_position, void* q, void* attn,
+                    void* y, void* stream) {
+    return layer_decode(c, tree, tokens, n_seqs, x, n_in, {}, wq, wk, wv, wo, n_out, nullptr, positions, cos_sin_cache, max_position,
+                        q, attn, y, stream);
 }
 
 namespace {
@@ -1125,17 +1154,11 @@ int ca_model_pass(const ca_model_layer* layers, int n_layers, const int32_t* tok
         if (!layer.norm || !aligned16(layer.norm) || !(layer.norm_epsilon >= 0.f)) return fail(CA_ERR_INVALID, "null or misaligned device pointer");
         ca::ProjectArgs in = qkv_append_args(layer.ctx, layer.wq, layer.wk, layer.wv, pos, layer.cos_sin_cache, layer.max_position, q);
         if (int rc = check_project(in, x, rows, hidden, hidden)) return rc;
-        ca::ProjectArgs out;
-        out.n_w = 1;
-        out.w[0] = layer.wo;
-        out.y[0] = x;
+        ca::ProjectArgs out = linear_args(layer.wo, residual, residual);
         if (int rc = check_project(out, attn, rows, hidden, hidden)) return rc;
     }
     if (head) {
-        ca::ProjectArgs out;
-        out.n_w = 1;
-        out.w[0] = head;
-        out.y[0] = logits;
+        ca::ProjectArgs out = linear_args(head, logits);
         if (int rc = check_project(out, x, n_seqs, n_logits, hidden)) return rc;
     }
     for (int i = 0; i < n_layers && !prefill; i++) {
@@ -1151,14 +1174,19 @@ int ca_model_pass(const ca_model_layer* layers, int n_layers, const int32_t* tok
             if (int rc = settle(c, layers[i].tree, n_seqs, stream)) return rc;
             if (!has_room(c, n_seqs)) return fail(CA_ERR_STATE, "a layer's tables do not fit its cache: refresh first");
         }
-        if (int rc = launch_rc(ca::launch_embed_norm(embedding, tokens, positions, rows, residual, x, pos, norm, norm_epsilon, hidden, st), "embedding launch")) return rc;
+        // A layer's residual stays in one buffer: its output projection adds to it, and what reads it next normalises it
+        // on the way (few rows) or finds it normalised in x (a launch of its own).
+        const bool norm_on_way = !prefill && ca::project_norms(rows, hidden);
+        if (int rc = launch_rc(ca::launch_embed_norm(embedding, tokens, positions, rows, residual, norm_on_way ? nullptr : x, pos, norm, norm_epsilon, hidden, st), "embedding launch")) return rc;
+        RowNorm row_norm{ norm, norm_epsilon };
         std::vector<int32_t> slots;
         for (int i = 0; i < n_layers; i++) {
             const ca_model_layer& layer = layers[i];
             ca_ctx* c = layer.ctx;
             if (!prefill) {
-                if (int rc = ca_layer_decode(c, layer.tree, tokens, n_seqs, x, hidden, layer.wq, layer.wk, layer.wv, layer.wo, hidden,
-                                             pos, layer.cos_sin_cache, layer.max_position, q, attn, x, stream)) return rc;
+                if (int rc = layer_decode(c, layer.tree, tokens, n_seqs, norm_on_way ? residual : x, hidden, norm_on_way ? row_norm : RowNorm{},
+                                          layer.wq, layer.wk, layer.wv, layer.wo, hidden, residual,
+                                          pos, layer.cos_sin_cache, layer.max_position, q, attn, residual, stream)) return rc;
             } else {
                 if (int rc = ca_qkv_rotary(x, layer.wq, layer.wk, layer.wv, pos, layer.cos_sin_cache, layer.max_position, q, k, v, rows, H, hidden, stream)) return rc;
                 if (int rc = ca_causal_attention(q, k, v, attn, 1, n_tokens, H, 128, stream)) return rc;
@@ -1167,15 +1195,24 @@ int ca_model_pass(const ca_model_layer* layers, int n_layers, const int32_t* tok
                 if (int rc = ca_tree_add_seq(layer.tree, tokens, n_tokens, &seq_idx[i], &begin, slots.data(), static_cast<int>(slots.size()), &n_new)) return rc;
                 ca_ctx_invalidate(c);
                 if (int rc = ca_scatter_kv(c, k, v, n_tokens, begin, slots.data(), n_new, stream)) return rc;
-                if (int rc = ca_linear(attn, layer.wo, x, rows, hidden, hidden, stream)) return rc;
+                ca::ProjectArgs out = linear_args(layer.wo, residual, residual);
+                if (int rc = project(out, attn, rows, hidden, hidden, stream)) return rc;
                 if (int rc = settle(c, layer.tree, ca_tree_n_seqs(layer.tree), stream)) return rc;
             }
-            // from the last layer on the last positions alone
-            const size_t skip = i + 1 == n_layers ? size_t(rows - n_seqs) * hidden * 2 : 0;
-            if (int rc = ca_add_rms_norm(x + skip, residual + skip, layer.norm, layer.norm_epsilon, i + 1 == n_layers ? n_seqs : rows, hidden, stream)) return rc;
+            row_norm = { layer.norm, layer.norm_epsilon };
+            if (i + 1 == n_layers || norm_on_way) continue;
+            if (int rc = ca_rms_norm(x, residual, layer.norm, layer.norm_epsilon, rows, hidden, stream)) return rc;
         }
-        if (!head) return CA_OK;
-        return ca_linear(base + ca_model_last_rows(rows, hidden, n_seqs), head, logits, n_seqs, n_logits, hidden, stream);
+        // from the last layer on the last positions alone
+        const size_t skip = size_t(rows - n_seqs) * hidden * 2;
+        ca::ProjectArgs out = linear_args(head, logits);
+        if (head && ca::project_norms(n_seqs, hidden)) {
+            out.norm = row_norm.weight;
+            out.norm_epsilon = row_norm.epsilon;
+            return project(out, residual + skip, n_seqs, n_logits, hidden, stream);
+        }
+        if (int rc = ca_rms_norm(x + skip, residual + skip, row_norm.weight, row_norm.epsilon, n_seqs, hidden, stream)) return rc;
+        return head ? project(out, x + skip, n_seqs, n_logits, hidden, stream) : CA_OK;
     });
 }
 

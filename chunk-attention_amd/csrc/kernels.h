@@ -129,7 +129,8 @@ int launch_rms_norm(void* out, void* input, void* residual, const void* weight, 
                     int64_t n_tokens, int hidden, bool vec8, bool mean_of_rounded, hipStream_t st);
 
 // Rows ids[r] of the embedding [vocab, hidden] into residual and, normalised, into out; positions[r] into
-// positions_out (ids and positions: host arrays; the others device, 16-byte aligned, hidden a multiple of 8).
+// positions_out (ids and positions: host arrays; the others device, 16-byte aligned, hidden a multiple of 8).  Without
+// an `out` nothing is normalised.
 constexpr int kEmbedRows = 448;  // of one launch
 int launch_embed_norm(const void* embedding, const int32_t* ids, const int32_t* positions, int n_rows, void* residual,
                       void* out, int64_t* positions_out, const void* weight, float epsilon, int hidden, hipStream_t st);
@@ -144,6 +145,9 @@ int launch_causal_attention(const void* q, const void* k, const void* v, void* o
 // 128) the heads of y[0] and y[1] are turned by the angles of the rows' positions (NeoX style over the
 // whole head of 128, cos_sin_cache [max_position, 128]) before they are rounded; with tail_slot set, y[1] and
 // y[2] are the K and the V pool and row m goes to row tail_fill[m] + delta_tokens of chunk tail_slot[m].
+// norm: the rows of x are normalised first, as launch_rms_norm does with that weight, bit for bit (project_norms
+// says whether it can be; not with positions alone, nor with add).  add ([M, N], 16-byte aligned like y[0], which it may be; one weight, N a multiple of 8, no
+// positions): added to the products once they are rounded.
 struct ProjectArgs {
     const void* x = nullptr;
     const void* w[3] = { nullptr, nullptr, nullptr };
@@ -156,7 +160,11 @@ struct ProjectArgs {
     const int32_t* tail_slot = nullptr;  // [M]
     const int32_t* tail_fill = nullptr;
     int delta_tokens = 0, C = 0;
+    const void* norm = nullptr;          // [K], 16-byte aligned
+    float norm_epsilon = 0.f;
+    const void* add = nullptr;
 };
+bool project_norms(int M, int K);
 int launch_project(const ProjectArgs& a, hipStream_t st);
 
 }  // namespace ca

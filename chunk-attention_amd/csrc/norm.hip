@@ -15,12 +15,14 @@
 #include <cstdint>
 
 #include "kernels.h"
+#include "norm_math.h"
 
 namespace ca {
 namespace {
 
-typedef _Float16 half_t;
-typedef half_t h8 __attribute__((ext_vector_type(8)));
+using norm::h8;
+using norm::half_t;
+using norm::scaled8;
 
 constexpr int WG = 256;
 enum { kNoAdd = 0, kAdd = 1, kAddRounded = 2 };   // what a row is added to first, and which sums the mean is of
@@ -56,17 +58,9 @@ __device__ __forceinline__ float first_pass8(h8& x, half_t* __restrict__ residua
         }
         *reinterpret_cast<h8*>(residual_piece) = x;
     } else {
-#pragma unroll
-        for (int e = 0; e < 8; e++) ss += float(x[e]) * float(x[e]);
+        ss = norm::sum_of_squares8(x);
     }
     return ss;
-}
-
-__device__ __forceinline__ h8 second_pass8(const h8 x, const h8 w, float inv) {
-    h8 y;
-#pragma unroll
-    for (int e = 0; e < 8; e++) y[e] = half_t(float(x[e]) * inv) * w[e];
-    return y;
 }
 
 template <int VEC, int ADD>
@@ -95,19 +89,19 @@ __global__ __launch_bounds__(WG) void rms_norm_kernel(half_t* __restrict__ out, 
             h8 x = *reinterpret_cast<const h8*>(input + row + idx);
             ss += first_pass8<ADD>(x, ADD ? residual + row + idx : nullptr);
         }
-        const float inv = __builtin_amdgcn_rsqf(block_sum(ss, sm) / float(hidden) + epsilon);
+        const float inv = norm::inverse_rms(block_sum(ss, sm), hidden, epsilon);
 #pragma unroll
         for (int it = 0; it < KEEP; it++) {
             const int idx = (threadIdx.x + it * WG) * 8;
             if (idx < hidden) {
                 *reinterpret_cast<h8*>(dst + row + idx) =
-                  second_pass8(kept[it], *reinterpret_cast<const h8*>(weight + idx), inv);
+                  scaled8(kept[it], *reinterpret_cast<const h8*>(weight + idx), inv);
             }
         }
         // (with ADD, a thread re-reads here only what it wrote above itself)
         for (int idx = (threadIdx.x + KEEP * WG) * 8; idx < hidden; idx += WG * 8) {
             *reinterpret_cast<h8*>(dst + row + idx) =
-              second_pass8(*reinterpret_cast<const h8*>(src + row + idx), *reinterpret_cast<const h8*>(weight + idx), inv);
+              scaled8(*reinterpret_cast<const h8*>(src + row + idx), *reinterpret_cast<const h8*>(weight + idx), inv);
         }
     } else {
         for (int idx = threadIdx.x; idx < hidden; idx += WG) {
@@ -119,7 +113,7 @@ __global__ __launch_bounds__(WG) void rms_norm_kernel(half_t* __restrict__ out, 
             }
             ss += s * s;
         }
-        const float inv = __builtin_amdgcn_rsqf(block_sum(ss, sm) / float(hidden) + epsilon);
+        const float inv = norm::inverse_rms(block_sum(ss, sm), hidden, epsilon);
         for (int idx = threadIdx.x; idx < hidden; idx += WG) {
             dst[row + idx] = half_t(float(src[row + idx]) * inv) * weight[idx];
         }
@@ -127,7 +121,7 @@ __global__ __launch_bounds__(WG) void rms_norm_kernel(half_t* __restrict__ out, 
 }
 
 // A model's first launch: row r of the embedding of tokens.id[r], into `residual` and normalised into `out` (bit for
-// bit what a gather and rms_norm give), and tokens.position[r] where the layers read it.  The ids travel as a kernel
+// bit what a gather and rms_norm give; not at all without an `out`), and tokens.position[r] where the layers read it.  The ids travel as a kernel
 // argument: no pinned upload, no gather and no norm of their own in front of the first layer (8 rows of 1024: 3.3 us
 // for four launches of 2.5 to 6).  One workgroup a row; rows of whole 16-byte pieces.
 struct EmbedTokens {
@@ -162,17 +156,18 @@ __global__ __launch_bounds__(WG) void embed_norm_kernel(const half_t* __restrict
         *reinterpret_cast<h8*>(residual + row + idx) = x;
         ss += first_pass8<kNoAdd>(x, nullptr);
     }
-    const float inv = __builtin_amdgcn_rsqf(block_sum(ss, sm) / float(hidden) + epsilon);
+    if (!out) return;
+    const float inv = norm::inverse_rms(block_sum(ss, sm), hidden, epsilon);
 #pragma unroll
     for (int it = 0; it < KEEP; it++) {
         const int idx = (threadIdx.x + it * WG) * 8;
         if (idx < hidden) {
-            *reinterpret_cast<h8*>(out + row + idx) = second_pass8(kept[it], *reinterpret_cast<const h8*>(weight + idx), inv);
+            *reinterpret_cast<h8*>(out + row + idx) = scaled8(kept[it], *reinterpret_cast<const h8*>(weight + idx), inv);
         }
     }
     for (int idx = (threadIdx.x + KEEP * WG) * 8; idx < hidden; idx += WG * 8) {
         *reinterpret_cast<h8*>(out + row + idx) =
-          second_pass8(*reinterpret_cast<const h8*>(src + idx), *reinterpret_cast<const h8*>(weight + idx), inv);
+          scaled8(*reinterpret_cast<const h8*>(src + idx), *reinterpret_cast<const h8*>(weight + idx), inv);
     }
 }
 
@@ -190,7 +185,7 @@ int launch_embed_norm(const void* embedding, const int32_t* ids, const int32_t* 
         }
         const size_t at = size_t(r0) * hidden;
         hipLaunchKernelGGL(embed_norm_kernel, dim3(n), dim3(WG), 0, st, static_cast<const half_t*>(embedding),
-                           static_cast<half_t*>(residual) + at, static_cast<half_t*>(out) + at, positions_out + r0,
+                           static_cast<half_t*>(residual) + at, out ? static_cast<half_t*>(out) + at : nullptr, positions_out + r0,
                            static_cast<const half_t*>(weight), epsilon, hidden, tokens);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return static_cast<int>(e);

@@ -5,12 +5,14 @@
 //   plain     any row-major weights [N, K]: output projection, language-model head
 //   rotary    q, k and v of a layer, q and k turned by their positions' angles before they are rounded
 //   append    the same for a decode step: k and v go straight to the free row of each sequence's last chunk
+//   add       plain, added to other rows once rounded: output projection and residual
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
 #include <type_traits>
 
 #include "kernels.h"
+#include "norm_math.h"
 #include "rotary_math.h"
 
 namespace ca {
@@ -26,7 +28,8 @@ constexpr int NW = 8;              // waves of a workgroup: each sums its share 
 constexpr int WG = 64 * NW;
 constexpr int UNIT = 64;           // k elements a wave takes at a time: one 128-byte line of every row
 
-enum { kPlain = 0, kRotary = 1, kAppend = 2 };
+enum { kPlain = 0, kRotary = 1, kAppend = 2, kAdd = 3 };
+constexpr bool turns(int mode) { return mode == kRotary || mode == kAppend; }
 
 // A workgroup owns 16 * MB rows and 16 * NB columns.  Few rows (a decode batch, one prompt) make this a
 // read of the weights: what counts is that all of their bytes are on request at once, so the tile is
@@ -46,7 +49,12 @@ enum { kPlain = 0, kRotary = 1, kAppend = 2 };
 // XR: rows of x that are fetched; of a block of 16 the others' products are of whatever stands in LDS, and not stored
 // (up to 8 rows a quarter of a unit's loads: q, k and v of 2048 on 1 row 9.1 -> 8.3 us, of 4096 20.9 -> 20.1, one weight
 // of 1024 3.0 -> 2.8).
-template <int MB, int NB, int R, int XR, int MODE>
+//
+// NORM: x is normalised on its way.  Between them the eight waves hold a whole row in registers (at most R units
+// each), so its squares cost one exchange over LDS, in the order in which rms_norm adds them (pieces 32, 16, ... 1
+// apart, then by 512 elements: the same bits), while the weights are still on their way (q, k and v of 1024 on 8 rows 4.6 -> 5.4
+// us, and the norm's launch of 2.6 in front is gone).
+template <int MB, int NB, int R, int XR, int MODE, bool NORM>
 __global__ __launch_bounds__(WG) void project_kernel(const ProjectArgs a) {
     constexpr int MT = 16 * MB, NT = 16 * NB, PITCH = NT + 4;
     constexpr int ROWS = MT + NT;                    // rows of a unit: the tile's columns (rows of W), then its rows
@@ -54,6 +62,8 @@ __global__ __launch_bounds__(WG) void project_kernel(const ProjectArgs a) {
         half_t stage[NW][ROWS * UNIT];
         float red[NW][MT][PITCH];
     } sm;
+    // squares of the x pieces of a unit: [unit of the wave][load][wave][lane]
+    __shared__ float squares[NORM ? R * (XR / 8) * NW * 64 : 1];
     const int tid = threadIdx.x;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l = tid & 63, g = l >> 4, i = l & 15;
@@ -66,7 +76,7 @@ __global__ __launch_bounds__(WG) void project_kernel(const ProjectArgs a) {
     // column c of the tile in the weight
     constexpr int HALF = NT / 2;
     constexpr int PER_HEAD = D / NT;                 // rotary tiles of a head
-    const int col0 = (MODE == kPlain) ? blk * NT : (blk / PER_HEAD) * D + (blk % PER_HEAD) * HALF;
+    const int col0 = !turns(MODE) ? blk * NT : (blk / PER_HEAD) * D + (blk % PER_HEAD) * HALF;
     const int row0 = rb * MT;
 
     // Load r of a unit brings rows 8r .. 8r+7, eight lanes to the 128 bytes of a row (requested in the
@@ -78,7 +88,7 @@ __global__ __launch_bounds__(WG) void project_kernel(const ProjectArgs a) {
     for (int r = 0; r < NL; r++) {
         if (8 * r < NT) {
             const int c = 8 * r + (l >> 3);
-            int n = (MODE == kPlain || c < HALF) ? col0 + c : col0 + c + D / 2 - HALF;
+            int n = (!turns(MODE) || c < HALF) ? col0 + c : col0 + c + D / 2 - HALF;
             if (n >= a.N) n = a.N - 1;               // computed, not stored
             src[r] = wt + size_t(n) * a.K + 8 * (l & 7);
         } else {
@@ -93,6 +103,11 @@ __global__ __launch_bounds__(WG) void project_kernel(const ProjectArgs a) {
 #pragma unroll
         for (int nb = 0; nb < NB; nb++) acc[mb][nb] = f4{ 0.f, 0.f, 0.f, 0.f };
     }
+    // what is added to this thread's eight products at the end: asked for now
+    static_assert(MT * NT / 8 <= WG, "one piece of the output a thread");
+    h8 added;
+    const bool adds = MODE == kAdd && tid < MT * NT / 8 && row0 + tid / (NT / 8) < a.M && col0 + 8 * (tid % (NT / 8)) < a.N;
+    if (adds) added = *reinterpret_cast<const h8*>(static_cast<const half_t*>(a.add) + size_t(row0 + tid / (NT / 8)) * a.N + col0 + 8 * (tid % (NT / 8)));
 
     const int units = a.K / UNIT;
     const int mine = (units - w + NW - 1) / NW;      // of them this wave's: w, w + NW, ...
@@ -130,7 +145,55 @@ __global__ __launch_bounds__(WG) void project_kernel(const ProjectArgs a) {
             }
         }
     };
-    if (mine > 0) {
+    if constexpr (NORM) {                            // at most R units a wave: all of them now
+        constexpr int XL = XR / 8;                   // loads of x a unit, behind those of w
+        h8 weight[R];
+        if (mine > 0) {
+#pragma unroll
+            for (int r = 0; r < R; r++) {            // x first: it is waited for first
+                const int k0 = (w + NW * (r < mine ? r : mine - 1)) * UNIT;
+#pragma unroll
+                for (int n = 0; n < XL; n++) st[r][NL - XL + n] = *reinterpret_cast<const h8*>(src[NL - XL + n] + k0);
+                weight[r] = *reinterpret_cast<const h8*>(static_cast<const half_t*>(a.norm) + k0 + 8 * (l & 7));
+            }
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const int k0 = (w + NW * (r < mine ? r : mine - 1)) * UNIT;
+#pragma unroll
+                for (int n = 0; n < NL - XL; n++) st[r][n] = *reinterpret_cast<const h8*>(src[n] + k0);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+#pragma unroll
+            for (int n = 0; n < XL; n++) {
+                squares[((r * XL + n) * NW + w) * 64 + l] = r < mine ? norm::sum_of_squares8(st[r][NL - XL + n]) : 0.f;
+            }
+        }
+        __syncthreads();
+        float inv[XL];
+#pragma unroll
+        for (int n = 0; n < XL; n++) {
+            float sum = 0.f;
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const float* s = &squares[(r * XL + n) * NW * 64 + l];
+                float v = ((s[0] + s[4 * 64]) + (s[2 * 64] + s[6 * 64])) + ((s[64] + s[5 * 64]) + (s[3 * 64] + s[7 * 64]));
+#pragma unroll
+                for (int m = 4; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
+                sum = r == 0 ? v : sum + v;
+            }
+            inv[n] = norm::inverse_rms(sum, a.K, a.norm_epsilon);
+        }
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            if (r < mine) {
+#pragma unroll
+                for (int n = 0; n < XL; n++) st[r][NL - XL + n] = norm::scaled8(st[r][NL - XL + n], weight[r], inv[n]);
+                multiply(st[r]);
+            }
+        }
+    } else if (mine > 0) {
 #pragma unroll
         for (int r = 0; r + 1 < R; r++) load(r, st[r]);
         for (int u = 0; u < mine; u += R) {
@@ -162,16 +225,20 @@ __global__ __launch_bounds__(WG) void project_kernel(const ProjectArgs a) {
     }
     __syncthreads();
 
-    if constexpr (MODE == kPlain) {
+    if constexpr (!turns(MODE)) {
         half_t* __restrict__ y = static_cast<half_t*>(which == 0 ? a.y[0] : which == 1 ? a.y[1] : a.y[2]);
         for (int u = tid; u < MT * NT / 8; u += WG) {
             const int r = u / (NT / 8), c = 8 * (u % (NT / 8));
             if (row0 + r >= a.M || col0 + c >= a.N) continue;
             half_t* dst = y + size_t(row0 + r) * a.N + col0 + c;
-            if (a.vec8) {
+            if (MODE == kAdd || a.vec8) {
                 h8 o;
 #pragma unroll
                 for (int e = 0; e < 8; e++) o[e] = half_t(red[0][r][c + e]);
+                if (MODE == kAdd) {
+#pragma unroll
+                    for (int e = 0; e < 8; e++) o[e] = half_t(float(o[e]) + float(added[e]));
+                }
                 *reinterpret_cast<h8*>(dst) = o;
             } else {
                 for (int e = 0; e < 8 && col0 + c + e < a.N; e++) dst[e] = half_t(red[0][r][c + e]);
@@ -221,12 +288,12 @@ __global__ __launch_bounds__(WG) void project_kernel(const ProjectArgs a) {
     }
 }
 
-template <int MB, int NB, int R, int XR, int MODE>
+template <int MB, int NB, int R, int XR, int MODE, bool NORM = false>
 int launch_tile(const ProjectArgs& a, hipStream_t st) {
     constexpr int MT = 16 * MB, NT = 16 * NB;
     const int64_t wgs = int64_t((a.N + NT - 1) / NT) * a.n_w * ((int64_t(a.M) + MT - 1) / MT);
     if (wgs > 0x7fffffff) return -1;
-    hipLaunchKernelGGL((project_kernel<MB, NB, R, XR, MODE>), dim3(static_cast<unsigned>(wgs)), dim3(WG), 0, st, a);
+    hipLaunchKernelGGL((project_kernel<MB, NB, R, XR, MODE, NORM>), dim3(static_cast<unsigned>(wgs)), dim3(WG), 0, st, a);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? 0 : static_cast<int>(e);
 }
@@ -286,7 +353,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void project_tile_kernel(const Proje
     // Column of the weight behind row c of the tile's w part.  Rotary: a wave's columns are CW / 2 of a head's first
     // half and their partners 64 further on, so that a lane holds both.
     auto column = [&](int c) {
-        if (MODE == kPlain) return col0 + c;
+        if (!turns(MODE)) return col0 + c;
         const int part = (col0 + c) / CW, in = c % CW;
         return part / (D / CW) * D + part % (D / CW) * (CW / 2) + in % (CW / 2) + in / (CW / 2) * (D / 2);
     };
@@ -390,11 +457,20 @@ __global__ __launch_bounds__(64 * WAVES, 2) void project_tile_kernel(const Proje
 #pragma unroll
     for (int m2 = 0; m2 < MB / 2; m2++) {
         const int row_base = row0 + wm * TM + 32 * m2;
+        constexpr int PIECES = CW / 8;
+        h8 added[CW / 16];          // asked for before the sums go through LDS
+        if constexpr (MODE == kAdd) {
+#pragma unroll
+            for (int p = 0; p < CW / 16; p++) {
+                const int row = row_base + p * (64 / PIECES) + l / PIECES, n = column(wn * CW + 8 * (l % PIECES));
+                if (row < a.M && n < a.N) added[p] = *reinterpret_cast<const h8*>(static_cast<const half_t*>(a.add) + size_t(row) * a.N + n);
+            }
+        }
 #pragma unroll
         for (int mm = 0; mm < 2; mm++) {
             const int m = 2 * m2 + mm, row = row_base + 16 * mm + i;
             const half_t* cs = nullptr;
-            if (MODE != kPlain && which < 2) {
+            if (turns(MODE) && which < 2) {
                 cs = static_cast<const half_t*>(a.cos_sin_cache) +
                      rotary::clamp_pos(a.positions[row < a.M ? row : a.M - 1], a.max_position) * D + (col0 + wn * CW) % D / 2;
             }
@@ -403,7 +479,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void project_tile_kernel(const Proje
                 const int c = 16 * n + 4 * g;
                 const f4 f0 = acc[m][n], f1 = acc[m][n + NB / 2];
                 h4 o0, o1;
-                if (MODE != kPlain && which < 2) {
+                if (turns(MODE) && which < 2) {
                     const h4 c4 = *reinterpret_cast<const h4*>(cs + c), s4 = *reinterpret_cast<const h4*>(cs + c + D / 2);
 #pragma unroll
                     for (int e = 0; e < 4; e++) {
@@ -424,18 +500,21 @@ __global__ __launch_bounds__(64 * WAVES, 2) void project_tile_kernel(const Proje
         __builtin_amdgcn_wave_barrier();
 #pragma unroll
         for (int p = 0; p < CW / 16; p++) {
-            constexpr int PIECES = CW / 8;
             const int r = p * (64 / PIECES) + l / PIECES, c = 8 * (l % PIECES);
             const int row = row_base + r, n = column(wn * CW + c);
             if (row >= a.M || n >= a.N) continue;
-            const h8 o = *reinterpret_cast<const h8*>(&stage[r * EP + c]);
+            h8 o = *reinterpret_cast<const h8*>(&stage[r * EP + c]);
+            if constexpr (MODE == kAdd) {
+#pragma unroll
+                for (int e = 0; e < 8; e++) o[e] = half_t(float(o[e]) + float(added[p][e]));
+            }
             half_t* dst = y + size_t(row) * a.N + n;
             if (MODE == kAppend && which > 0) {
                 const int fill = a.tail_fill[row] + a.delta_tokens;
                 if (fill < 0 || fill >= a.C) continue;   // the host guarantees a free row; never write outside the chunk
                 dst = y + ((size_t(a.tail_slot[row]) * (a.N / D) + n / D) * a.C + fill) * D + n % D;
             }
-            if (MODE != kPlain || a.vec8) {
+            if (turns(MODE) || MODE == kAdd || a.vec8) {
                 *reinterpret_cast<h8*>(dst) = o;
             } else {
 #pragma unroll
@@ -469,6 +548,9 @@ int launch_shared_tile(const ProjectArgs& a, hipStream_t st) {
 // 161, 2048 rows 209 and 181).
 template <int MODE>
 int launch_mode(const ProjectArgs& a, hipStream_t st) {
+    if constexpr (MODE == kPlain || MODE == kAppend) {
+        if (a.norm) return a.M <= 8 ? launch_tile<1, 1, 2, 8, MODE, true>(a, st) : launch_tile<1, 1, 2, 16, MODE, true>(a, st);
+    }
     if (a.M <= 8) {
         return a.K > 2 * NW * UNIT ? launch_tile<1, 1, 3, 8, MODE>(a, st) : launch_tile<1, 1, 2, 8, MODE>(a, st);
     }
@@ -493,10 +575,15 @@ int launch_mode(const ProjectArgs& a, hipStream_t st) {
 
 }  // namespace
 
+// One block of rows, two units a wave.
+bool project_norms(int M, int K) { return M <= 16 && K <= 2 * NW * UNIT; }
+
 int launch_project(const ProjectArgs& a, hipStream_t st) {
     if (a.M <= 0 || a.N <= 0) return 0;
     if (a.K <= 0 || a.K % UNIT != 0 || a.n_w < 1 || a.n_w > 3 || a.M > 0x7fffff00) return -1;
-    if (!a.positions) return launch_mode<kPlain>(a, st);
+    if (a.norm && (!project_norms(a.M, a.K) || a.add || (a.positions && !a.tail_slot))) return -1;
+    if (a.add && (a.n_w != 1 || a.positions || !a.vec8)) return -1;
+    if (!a.positions) return a.add ? launch_mode<kAdd>(a, st) : launch_mode<kPlain>(a, st);
     if (a.N % D != 0 || a.n_w != 3) return -1;
     return a.tail_slot ? launch_mode<kAppend>(a, st) : launch_mode<kRotary>(a, st);
 }

@@ -154,3 +154,35 @@ def test_a_prompt_that_a_later_cache_cannot_take(hooked, over):
     assert model.layers[1].last_indices is None
     caches[0].remove_seq(model.layers[0].last_indices[0])
     assert caches[0].tree.dump()[1][2][:2] == [59, 58]
+
+
+@pytest.mark.parametrize("hidden,prompts", [
+    (1024, [3] * 9), (1024, [2] * 16), (384, [5, 1, 9]),   # both numbers of rows that are normalised on their way
+    (1024, [2] * 17), (1152, [7, 40])])                     # more rows, longer ones: a launch of its own
+def test_norms_on_the_way_keep_every_bit(hidden, prompts):
+    """Rows normalised by the projection that reads them, and sums that the output projection writes, against the
+    modules' own launches, with weights and an epsilon that show in the result."""
+    from chunk_attn.models.sequence import Sequence
+    from chunk_attn.models.tiny_lm import AttentionOnlyLM
+    runs = []
+    for hooked in (False, True):
+        model = AttentionOnlyLM(333, hidden, hidden // 128, 2, chunk_size=32, memory_mb=32, seed=8)
+        g = torch.Generator().manual_seed(hidden)
+        with torch.no_grad():
+            for norm in (*model.input_norms, model.norm):
+                norm.weight.copy_(torch.randn(hidden, generator=g))
+                norm.eps = 0.3
+        if hooked:
+            model.norm.register_forward_hook(lambda m, a, out: None)
+        caches, running, out = model.create_kv_caches(), [], []
+        with torch.inference_mode():
+            for i, n in enumerate(prompts):
+                seq = Sequence([(7 * t + 50 * i) % 333 for t in range(n)])
+                out.append(model.logits([seq], caches, True))
+                running.insert(seq.index, seq)
+            for t in range(2):
+                for s, seq in enumerate(running):
+                    seq.append((11 * t + 3 * s) % 333)
+                out.append(model.logits(running, caches, False))
+        runs.append(out)
+    assert all(torch.equal(a, b) for a, b in zip(*runs)) and all(torch.isfinite(a).all() for a in runs[0])

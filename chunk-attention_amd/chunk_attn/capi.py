@@ -86,6 +86,8 @@ SIGNATURES = {
                                        ctypes.c_int64, ctypes.c_int, ctypes.c_void_p]),
     "ca_causal_attention": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
                                            ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p]),
+    "ca_prefill_attention": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, c_i32_p, ctypes.c_int, ctypes.c_int] +
+                             [ctypes.c_void_p] * 4 + [c_i32_p, ctypes.c_void_p]),
     "ca_linear": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_int,
                                  ctypes.c_int, ctypes.c_void_p]),
     "ca_qkv_rotary": (ctypes.c_int, [ctypes.c_void_p] * 6 + [ctypes.c_int] + [ctypes.c_void_p] * 3 +
@@ -983,6 +985,23 @@ class Attention:
             self.ctx.scatter_kv(k.data_ptr(), v.data_ptr(), len(tokens), tok_begin, slots, self._stream())
         self.ctx.invalidate()
         return idx
+
+    def _prefill_attention(self, prompts, q, k, v):
+        """causal_attention() of what causal_attention_takes has accepted, [batch, n, n_heads, 128], and add_seq() of every
+        prompt, the copies in the attention's launch.  (output, indices), or None, with nothing done, where prompts
+        or tensors are not the cache's: add_seq says what is wrong with them."""
+        batch, n = q.shape[:2]
+        if batch == 0 or n == 0 or tuple(q.shape[2:]) != (self.n_heads, self.d_head) or q.device != self.device or \
+                len(prompts) != batch or any([type(p) is not list or len(p) != n for p in prompts]):
+            return None
+        try:
+            flat = array.array("i", [t for p in prompts for t in p])
+        except (TypeError, OverflowError):
+            return None
+        out, index = torch.empty_like(q), (ctypes.c_int32 * batch)()
+        _launch(q.device, self.ctx._lib.ca_prefill_attention, self.ctx._h, self.tree._h, (ctypes.c_int32 * len(flat)).from_buffer(flat),
+                batch, n, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), index)
+        return out, list(index)
 
     def remove_seq(self, seq_idx: int) -> None:
         self.tree.remove_seq(seq_idx)

@@ -100,7 +100,11 @@ class LlamaChunkAttention(nn.Module):
                 q, k = self.rotary_emb(position_ids.contiguous(), q, k)
             shape = (batch, n_tokens, self.num_heads, self.head_dim)
             q4, k4, v4 = q.view(shape), k.view(shape), v.view(shape)
-            if hidden_states.dtype == torch.float16 and capi.causal_attention_takes(q4, k4, v4):
+            takes = hidden_states.dtype == torch.float16 and capi.causal_attention_takes(q4, k4, v4)
+            both = kv_cache._prefill_attention(seqs, q4, k4, v4) if takes and capi.is_plain_cache_to_fill(kv_cache) else None
+            if both is not None:
+                attn_output, self.last_indices = both[0].view(batch, n_tokens, d_hidden), both[1]
+            elif takes:
                 attn_output = capi._causal_attention(q4, k4, v4).view(batch, n_tokens, d_hidden)
             else:
                 # what the kernel does not take (a gradient is wanted, another head size): plain fp32 torch math
@@ -109,8 +113,9 @@ class LlamaChunkAttention(nn.Module):
                 future = torch.ones(n_tokens, n_tokens, dtype=torch.bool, device=scores.device).triu(1)
                 attn = torch.softmax(scores.masked_fill(future, float("-inf")), dim=-1) @ vh
                 attn_output = attn.transpose(1, 2).reshape(batch, n_tokens, d_hidden).to(hidden_states.dtype)
-            self.last_indices = [kv_cache.add_seq(list(seqs[i]), k4[i].contiguous(), v4[i].contiguous())
-                                 for i in range(batch)]
+            if both is None:
+                self.last_indices = [kv_cache.add_seq(list(seqs[i]), k4[i].contiguous(), v4[i].contiguous())
+                                     for i in range(batch)]
         else:
             assert n_tokens == 1
             shape = (batch, self.num_heads, self.head_dim)

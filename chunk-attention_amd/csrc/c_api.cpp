@@ -917,18 +917,70 @@ int ca_add_rms_norm(void* input, void* residual, const void* weight, float epsil
     return add_and_norm(input, residual, weight, epsilon, n_tokens, hidden_size, true, stream);
 }
 
-int ca_causal_attention(const void* q, const void* k, const void* v, void* out, int batch, int n_tokens,
-                        int n_heads, int d_head, void* stream) {
+namespace {
+int check_causal(ca::CausalArgs& a, const void* q, const void* k, const void* v, void* out, int batch, int n_tokens, int n_heads) {
     if (batch < 0 || n_tokens < 0 || n_heads <= 0) return fail(CA_ERR_INVALID, "bad argument");
-    if (d_head != 128) return fail(CA_ERR_INVALID, "causal attention needs d_head 128");
+    a.q = q; a.k = k; a.v = v; a.out = out;
+    a.batch = batch; a.n_tokens = n_tokens; a.n_heads = n_heads;
+    a.scale_log2 = 1.4426950408889634f / std::sqrt(128.f);
     if (batch == 0 || n_tokens == 0) return CA_OK;
     if (!q || !k || !v || !out) return fail(CA_ERR_INVALID, "null device pointer");
     if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(out)) {
         return fail(CA_ERR_INVALID, "q, k, v and out must be 16-byte aligned");
     }
-    const float scale_log2 = 1.4426950408889634f / std::sqrt(float(d_head));
-    return launch_rc(ca::launch_causal_attention(q, k, v, out, batch, n_tokens, n_heads, scale_log2,
-                                                 static_cast<hipStream_t>(stream)), "causal attention launch");
+    return CA_OK;
+}
+}  // namespace
+
+int ca_causal_attention(const void* q, const void* k, const void* v, void* out, int batch, int n_tokens,
+                        int n_heads, int d_head, void* stream) {
+    ca::CausalArgs a;
+    if (batch >= 0 && n_tokens >= 0 && n_heads > 0 && d_head != 128) return fail(CA_ERR_INVALID, "causal attention needs d_head 128");
+    if (int rc = check_causal(a, q, k, v, out, batch, n_tokens, n_heads)) return rc;
+    return launch_rc(ca::launch_causal_attention(a, static_cast<hipStream_t>(stream)), "causal attention launch");
+}
+
+int ca_prefill_attention(ca_ctx* c, ca_tree* tree, const int32_t* tokens, int batch, int n_tokens, const void* q,
+                         const void* k, const void* v, void* out, int32_t* seq_idx, void* stream) {
+    if (!c || !tree || !tokens || !seq_idx || batch < 1 || n_tokens < 1) return fail(CA_ERR_INVALID, "bad argument");
+    if (int rc = check_attention_shape(c)) return rc;
+    ca::CausalArgs a;
+    if (int rc = check_causal(a, q, k, v, out, batch, n_tokens, c->H)) return rc;
+    if (!ca::causal_attention_fits(batch, n_tokens, c->H)) return launch_rc(-1, "causal attention launch");
+    return guarded([&]() -> int {
+        std::vector<ca::CopyChunk> chunks;
+        std::vector<int32_t> slots(n_tokens / c->C + 2);
+        int rc = CA_OK;
+        for (int s = 0; s < batch && rc == CA_OK; s++) {
+            int begin = 0, n_new = 0;
+            rc = ca_tree_add_seq(tree, tokens + size_t(s) * n_tokens, n_tokens, &seq_idx[s], &begin, slots.data(),
+                                 static_cast<int>(slots.size()), &n_new);
+            if (rc != CA_OK) break;
+            ca_ctx_invalidate(c);
+            if (n_new > static_cast<int>(slots.size())) return fail(CA_ERR_STATE, "the tree's chunks are not the context's");
+            for (int i = 0; i < n_new && begin + i * c->C < n_tokens; i++) {
+                const int at = begin + i * c->C;
+                if (slots[i] < 0 || slots[i] >= c->max_chunks) return fail(CA_ERR_INVALID, "slot outside the pool");
+                chunks.push_back({ slots[i], s * n_tokens + at, std::min(c->C, n_tokens - at) });
+            }
+        }
+        // (a prompt that the cache cannot take leaves those in front of it with their rows; the message is the tree's)
+        const std::string why = rc != CA_OK ? ca_last_error() : "";
+        a.kpool = c->k_pool;
+        a.vpool = c->v_pool;
+        a.C = c->C;
+        hipStream_t st = static_cast<hipStream_t>(stream);
+        for (size_t i = 0; i < chunks.size() || i == 0; i += ca::kCausalChunks) {
+            a.chunks = chunks.data() + i;
+            a.n_chunks = static_cast<int>(std::min(chunks.size() - i, size_t(ca::kCausalChunks)));
+            if (i == 0) {
+                if (int e = launch_rc(ca::launch_causal_attention(a, st), "causal attention launch")) return e;
+            } else if (int e = launch_rc(ca::launch_copy_in(a, st), "scatter launch")) {
+                return e;
+            }
+        }
+        return rc == CA_OK ? rc : fail(rc, why);
+    });
 }
 
 namespace {
@@ -1179,7 +1231,6 @@ int ca_model_pass(const ca_model_layer* layers, int n_layers, const int32_t* tok
         const bool norm_on_way = !prefill && ca::project_norms(rows, hidden);
         if (int rc = launch_rc(ca::launch_embed_norm(embedding, tokens, positions, rows, residual, norm_on_way ? nullptr : x, pos, norm, norm_epsilon, hidden, st), "embedding launch")) return rc;
         RowNorm row_norm{ norm, norm_epsilon };
-        std::vector<int32_t> slots;
         for (int i = 0; i < n_layers; i++) {
             const ca_model_layer& layer = layers[i];
             ca_ctx* c = layer.ctx;
@@ -1189,12 +1240,7 @@ int ca_model_pass(const ca_model_layer* layers, int n_layers, const int32_t* tok
                                           pos, layer.cos_sin_cache, layer.max_position, q, attn, residual, stream)) return rc;
             } else {
                 if (int rc = ca_qkv_rotary(x, layer.wq, layer.wk, layer.wv, pos, layer.cos_sin_cache, layer.max_position, q, k, v, rows, H, hidden, stream)) return rc;
-                if (int rc = ca_causal_attention(q, k, v, attn, 1, n_tokens, H, 128, stream)) return rc;
-                int begin = 0, n_new = 0;
-                slots.resize(n_tokens / c->C + 2);
-                if (int rc = ca_tree_add_seq(layer.tree, tokens, n_tokens, &seq_idx[i], &begin, slots.data(), static_cast<int>(slots.size()), &n_new)) return rc;
-                ca_ctx_invalidate(c);
-                if (int rc = ca_scatter_kv(c, k, v, n_tokens, begin, slots.data(), n_new, stream)) return rc;
+                if (int rc = ca_prefill_attention(c, layer.tree, tokens, 1, n_tokens, q, k, v, attn, &seq_idx[i], stream)) return rc;
                 ca::ProjectArgs out = linear_args(layer.wo, residual, residual);
                 if (int rc = project(out, attn, rows, hidden, hidden, stream)) return rc;
                 if (int rc = settle(c, layer.tree, ca_tree_n_seqs(layer.tree), stream)) return rc;

@@ -136,9 +136,29 @@ int launch_embed_norm(const void* embedding, const int32_t* ids, const int32_t* 
                       void* out, int64_t* positions_out, const void* weight, float epsilon, int hidden, hipStream_t st);
 
 // Causal attention of whole prompts: q, k, v, out [batch, n_tokens, n_heads, 128] fp16, contiguous and
-// 16-byte aligned; out must not overlap the inputs.
-int launch_causal_attention(const void* q, const void* k, const void* v, void* out, int batch, int n_tokens, int n_heads,
-                            float scale_log2, hipStream_t st);
+// 16-byte aligned; out must not overlap the inputs.  With n_chunks > 0 (at most kCausalChunks) the launch also copies
+// rows of k and v into the chunks of a cache of as many heads of 128: n rows from row `row` on (of batch * n_tokens) to
+// rows 0 .. n - 1 of chunk `slot`.
+struct CopyChunk {
+    int32_t slot, row, n;
+};
+constexpr int kCausalChunks = 64;
+struct CausalArgs {
+    const void* q = nullptr;
+    const void* k = nullptr;
+    const void* v = nullptr;
+    void* out = nullptr;
+    int batch = 0, n_tokens = 0, n_heads = 0;
+    float scale_log2 = 0.f;
+    void* kpool = nullptr;
+    void* vpool = nullptr;
+    int C = 0;
+    const CopyChunk* chunks = nullptr;   // host memory
+    int n_chunks = 0;
+};
+bool causal_attention_fits(int batch, int n_tokens, int n_heads);
+int launch_causal_attention(const CausalArgs& a, hipStream_t st);
+int launch_copy_in(const CausalArgs& a, hipStream_t st);   // the copies alone
 
 // y[j] = x . w[j]^T for up to three weights: x [M, K], w[j] [N, K], fp16, contiguous and 16-byte aligned, K a
 // multiple of 64; fp32 sums.  positions == nullptr: y[j] is [M, N].  Otherwise (three weights, N a multiple of

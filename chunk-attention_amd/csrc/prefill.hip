@@ -17,6 +17,7 @@ typedef half_t h2 __attribute__((ext_vector_type(2)));
 typedef half_t h4 __attribute__((ext_vector_type(4)));
 typedef half_t h8 __attribute__((ext_vector_type(8)));
 typedef float f4 __attribute__((ext_vector_type(4)));
+typedef unsigned u4 __attribute__((ext_vector_type(4)));
 
 constexpr int D = 128;
 constexpr int WG = 256;
@@ -76,6 +77,58 @@ __device__ __forceinline__ void load_to_lds16(const char* src, half_t* dst) {
                                      (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
 }
 
+// Up to N chunks' rows of k and v for a cache's pools, copied in the attention's launch by the workgroups behind its own:
+// they need the memory, which the attention leaves idle, and start as its first workgroups end.  As a launch of their own
+// the rows of 2048 tokens of 32 heads took 11.2 us behind the attention's 64.2, together they take 69.5.
+template <int N>
+struct CopyIn {
+    u4* kpool;
+    u4* vpool;
+    int C, chunk_wgs;                                          // workgroups of a chunk
+    CopyChunk chunk[N];
+};
+template <>
+struct CopyIn<0> {};
+
+// Threads that copy one chunk: a thread one piece of 16 bytes of up to four neighbouring tokens.
+constexpr int COPY_TOKENS = 4, PIECES = D / 8;
+__host__ __device__ __forceinline__ int copy_threads(int H, int C) { return (C + COPY_TOKENS - 1) / COPY_TOKENS * H * PIECES; }
+
+// Workgroup u of those that copy.  All of a thread's loads are on request before its first store.
+template <int N>
+__device__ __forceinline__ void copy_rows(const half_t* __restrict__ k, const half_t* __restrict__ v, int H, const CopyIn<N>& in, int u) {
+    const int e = u / in.chunk_wgs;
+    const unsigned id = unsigned(u - e * in.chunk_wgs) * WG + threadIdx.x, row_pieces = unsigned(H) * PIECES;
+    const unsigned quad = id / row_pieces, at = id - quad * row_pieces;
+    const int t0 = int(quad) * COPY_TOKENS, n = in.chunk[e].n;
+    if (t0 >= n) return;
+    const u4* __restrict__ ks = reinterpret_cast<const u4*>(k) + (size_t(in.chunk[e].row) + t0) * row_pieces + at;
+    const u4* __restrict__ vs = reinterpret_cast<const u4*>(v) + (size_t(in.chunk[e].row) + t0) * row_pieces + at;
+    const size_t to = ((size_t(in.chunk[e].slot) * H + at / PIECES) * in.C + t0) * PIECES + at % PIECES;
+    u4 kr[COPY_TOKENS], vr[COPY_TOKENS];
+#pragma unroll
+    for (int j = 0; j < COPY_TOKENS; j++) {          // past the last row that one again: no branch between the loads
+        const size_t row = size_t(t0 + j < n ? j : n - 1 - t0) * row_pieces;
+        kr[j] = ks[row];
+        vr[j] = vs[row];
+    }
+    asm volatile("" ::: "memory");                   // (a load that only a branch below needs would move there)
+#pragma unroll
+    for (int j = 0; j < COPY_TOKENS; j++) {
+        if (t0 + j < n) {
+            in.kpool[to + j * PIECES] = kr[j];
+            in.vpool[to + j * PIECES] = vr[j];
+        }
+    }
+}
+
+// The chunks that the attention's launch has no room for.
+template <int N>
+__global__ __launch_bounds__(WG) void copy_in_kernel(const half_t* __restrict__ k, const half_t* __restrict__ v, int H,
+                                                     const CopyIn<N> in) {
+    copy_rows(k, v, H, in, blockIdx.x);
+}
+
 // A workgroup attends 64 query rows of one (sequence, head): wave w owns 16 of them and keeps their Q^T
 // operands and output accumulators in registers; TILE-key tiles of K and V go through LDS, the next tile on
 // its way into a second buffer.  S^T = K.Q^T leaves each lane with four keys of one row, which is the operand
@@ -95,10 +148,17 @@ __device__ __forceinline__ void load_to_lds16(const char* src, half_t* dst) {
 // bits the output is as far off as with fp32 products: its own rounding to fp16 is what remains.
 // The maximum a row's scores are taken relative to moves only when it would grow by more than 2^7 (p stays
 // below 2^15, inside fp16): the accumulators are rescaled a few times a row instead of at most tiles.
-template <int TILE>
+template <int TILE, int N>
 __global__ __launch_bounds__(WG, TILE == 32 ? 4 : 2) void causal_attention_kernel(
     const half_t* __restrict__ q, const half_t* __restrict__ k, const half_t* __restrict__ v, half_t* __restrict__ out,
-    int n, int H, int n_bh, int n_blocks, float scale_log2) {
+    int n, int H, int n_bh, int n_blocks, float scale_log2, const CopyIn<N> in) {
+    const int n_wgs = n_bh * n_blocks;
+    if constexpr (N > 0) {
+        if (int(blockIdx.x) >= n_wgs) {
+            copy_rows(k, v, H, in, blockIdx.x - n_wgs);
+            return;
+        }
+    }
     constexpr int TB = TILE / 16;                              // 16-key blocks of a tile
     constexpr int TP = TILE / 32;                              // pairs of them
     constexpr int RPW = TILE / NW;                             // rows of a tile that a wave brings
@@ -108,7 +168,7 @@ __global__ __launch_bounds__(WG, TILE == 32 ? 4 : 2) void causal_attention_kerne
     // Every second 256 workgroups (one per compute unit) are taken in reverse, in steps of 8 so that the
     // XCD does not change: a compute unit gets a long and a short block instead of two long ones.
     int b = blockIdx.x;
-    if (((b >> 8) & 1) && (b | 255) < int(gridDim.x)) b = (b & ~255) | ((31 - ((b >> 3) & 31)) << 3) | (b & 7);
+    if (((b >> 8) & 1) && (b | 255) < n_wgs) b = (b & ~255) | ((31 - ((b >> 3) & 31)) << 3) | (b & 7);
     const int bh = b % n_bh;
     const int block = n_blocks - 1 - b / n_bh;
     const int seq = bh / H, h = bh - seq * H;
@@ -288,32 +348,71 @@ __global__ __launch_bounds__(WG, TILE == 32 ? 4 : 2) void causal_attention_kerne
     }
 }
 
-}  // namespace
+template <int N>
+CopyIn<N> copies(const CausalArgs& a) {
+    CopyIn<N> in;
+    in.kpool = static_cast<u4*>(a.kpool);
+    in.vpool = static_cast<u4*>(a.vpool);
+    in.C = a.C;
+    in.chunk_wgs = (copy_threads(a.n_heads, a.C) + WG - 1) / WG;
+    for (int i = 0; i < N; i++) in.chunk[i] = i < a.n_chunks ? a.chunks[i] : CopyChunk{ 0, 0, 0 };
+    return in;
+}
 
-int launch_causal_attention(const void* q, const void* k, const void* v, void* out, int batch, int n_tokens, int n_heads,
-                            float scale_log2, hipStream_t st) {
-    if (batch <= 0 || n_tokens <= 0 || n_heads <= 0) return 0;
-    const int64_t n_bh = int64_t(batch) * n_heads;
-    const int64_t blocks = (n_tokens + ROWS - 1) / ROWS;
-    if (n_bh * blocks > 0x7fffff00 || n_tokens > 0x7fffff00 - ROWS) return -1;
-    const dim3 grid(static_cast<unsigned>(n_bh * blocks)), block(WG);
-    const half_t* qh = static_cast<const half_t*>(q);
-    const half_t* kh = static_cast<const half_t*>(k);
-    const half_t* vh = static_cast<const half_t*>(v);
-    half_t* oh = static_cast<half_t*>(out);
+template <int N>
+int launch(const CausalArgs& a, hipStream_t st) {
+    const int n_bh = a.batch * a.n_heads, blocks = (a.n_tokens + ROWS - 1) / ROWS;
+    const half_t* q = static_cast<const half_t*>(a.q);
+    const half_t* k = static_cast<const half_t*>(a.k);
+    const half_t* v = static_cast<const half_t*>(a.v);
+    half_t* out = static_cast<half_t*>(a.out);
+    CopyIn<N> in;
+    int64_t wgs = int64_t(n_bh) * blocks;
+    if constexpr (N > 0) {
+        in = copies<N>(a);
+        wgs += int64_t(a.n_chunks) * in.chunk_wgs;
+        if (wgs > 0x7fffffff) return -1;
+    }
+    const dim3 grid(static_cast<unsigned>(wgs)), block(WG);
     // Tiles of 32 keys let four workgroups share a compute unit, tiles of 64 two, with half as many barriers: worth
     // more while few workgroups are left over from two a unit, the longer the prompt the more (us with 64 and 32 keys
     // a tile, workgroups in brackets: 1004 tokens x 16 heads [256] 21.9, 24.8; 1516 x 16 [384] 33.5, 37.6; 1004 x 32
     // [512] 23.5, 25.8; 4 x 236 x 32 [512] 9.5, 9.3; 4 x 556 x 16 [576] 15.8, 17.1; 4 x 300 x 32 [640] 12.4, 11.8;
     // 4 x 620 x 16 [640] 17.6, 18.9; 4 x 364 x 32 [768] 15.9, 14.3; 1516 x 32 [768] 37.7, 42.0; 2028 x 32 [1024]
     // 64.0, 61.5).
-    if (n_bh * blocks > (n_tokens < 600 ? 576 : 768)) {
-        hipLaunchKernelGGL(causal_attention_kernel<32>, grid, block, 0, st, qh, kh, vh, oh, n_tokens, n_heads, int(n_bh),
-                           int(blocks), scale_log2);
+    if (int64_t(n_bh) * blocks > (a.n_tokens < 600 ? 576 : 768)) {
+        hipLaunchKernelGGL((causal_attention_kernel<32, N>), grid, block, 0, st, q, k, v, out, a.n_tokens, a.n_heads, n_bh, blocks,
+                           a.scale_log2, in);
     } else {
-        hipLaunchKernelGGL(causal_attention_kernel<64>, grid, block, 0, st, qh, kh, vh, oh, n_tokens, n_heads, int(n_bh),
-                           int(blocks), scale_log2);
+        hipLaunchKernelGGL((causal_attention_kernel<64, N>), grid, block, 0, st, q, k, v, out, a.n_tokens, a.n_heads, n_bh, blocks,
+                           a.scale_log2, in);
     }
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? 0 : static_cast<int>(e);
+}
+
+}  // namespace
+
+bool causal_attention_fits(int batch, int n_tokens, int n_heads) {
+    const int64_t blocks = (int64_t(n_tokens) + ROWS - 1) / ROWS;
+    return int64_t(batch) * n_heads <= 0x7fffff00 / blocks && n_tokens <= 0x7fffff00 - ROWS;
+}
+
+int launch_causal_attention(const CausalArgs& a, hipStream_t st) {
+    if (a.batch <= 0 || a.n_tokens <= 0 || a.n_heads <= 0) return 0;
+    if (!causal_attention_fits(a.batch, a.n_tokens, a.n_heads) || a.n_chunks > kCausalChunks) return -1;
+    if (a.n_chunks == 0) return launch<0>(a, st);
+    return a.n_chunks <= 8 ? launch<8>(a, st) : launch<kCausalChunks>(a, st);
+}
+
+int launch_copy_in(const CausalArgs& a, hipStream_t st) {
+    if (a.n_chunks <= 0 || a.n_heads <= 0) return 0;
+    if (a.n_chunks > kCausalChunks) return -1;
+    const CopyIn<kCausalChunks> in = copies<kCausalChunks>(a);
+    const int64_t wgs = int64_t(a.n_chunks) * in.chunk_wgs;
+    if (wgs > 0x7fffffff) return -1;
+    hipLaunchKernelGGL(copy_in_kernel<kCausalChunks>, dim3(static_cast<unsigned>(wgs)), dim3(WG), 0, st, static_cast<const half_t*>(a.k),
+                       static_cast<const half_t*>(a.v), a.n_heads, in);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? 0 : static_cast<int>(e);
 }

@@ -452,6 +452,14 @@ int ca_layer_decode(ca_ctx* ctx, ca_tree* tree, const int32_t* tokens, int n_seq
                     const int64_t* positions_dev, const void* cos_sin_cache, int max_position, void* q,
                     void* attn, void* y, void* stream);
 
+/* The prefill branch's attention on a cache: ca_tree_add_seq for each of `batch` prompts of n_tokens tokens
+ * (tokens [batch, n_tokens], host; seq_idx[s] receives what it gives), ca_causal_attention over them, and in the same
+ * launch the rows of k and v that ca_scatter_kv would copy for each (chunks past the first 64 follow in launches of
+ * their own).  The context's tables are invalid afterwards.  A prompt that the cache cannot take is an error; those in
+ * front of it stay, with their rows. */
+int ca_prefill_attention(ca_ctx* ctx, ca_tree* tree, const int32_t* tokens, int batch, int n_tokens, const void* q,
+                         const void* k, const void* v, void* out, int32_t* seq_idx, void* stream);
+
 /* One layer of a model for ca_model_pass: its cache, its weights [hidden, hidden] each, its rotary table
  * [max_position, 128], and the weight [hidden] and epsilon of the norm behind it. */
 typedef struct {
@@ -468,8 +476,7 @@ typedef struct {
  * then per layer the attention layer and the residual's addition in the norm behind it (ca_add_rms_norm), then, if
  * `head` is not null, logits [n_seqs, n_logits] = last rows . head^T.
  *   prefill == 0: one token per sequence of every cache (n_tokens is 1), per layer ca_layer_decode;
- *   prefill == 1: one sequence (n_seqs is 1) of n_tokens tokens: ca_qkv_rotary, ca_causal_attention, ca_tree_add_seq,
- *   ca_scatter_kv, ca_linear, room for the next token; seq_idx[layer] receives the sequence's index in that cache.
+ *   prefill == 1: one sequence (n_seqs is 1) of n_tokens tokens: ca_qkv_rotary, ca_prefill_attention, ca_linear, room for the next token; seq_idx[layer] receives the sequence's index in that cache.
  * tokens and positions: host, n_seqs * n_tokens; every id within the embedding [vocab, hidden].  hidden is the
  * context's n_heads * 128.  scratch: ca_model_scratch_bytes(rows, hidden) bytes of device memory, 16-byte aligned;
  * the last norm's rows start ca_model_last_rows(rows, hidden, n_seqs) bytes into it.  What a call refuses for its

@@ -8,6 +8,7 @@ import torch
 from chunk_attn import capi
 
 pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
 
 
 def reference(q, k, v):
@@ -95,3 +96,52 @@ def test_infinite_and_undefined_scores(batch, n, heads):
     assert torch.isnan(want).any(-1).sum() == (n - 120) + (n - 130) + 1
     ok = ~torch.isnan(want)
     assert ((out - want).abs() <= want.abs() * 2.0 ** -11 + 6 * 2.0 ** -16)[ok].all()
+
+
+@pytest.mark.parametrize("batch,n,heads,chunk,same", [
+    (1, 1, 1, 32, 0), (1, 63, 3, 64, 0), (2, 64, 8, 64, 0), (3, 65, 2, 32, 40), (2, 256, 8, 64, 256), (8, 130, 2, 32, 64),
+    (1, 2048, 2, 32, 0), (2, 1061, 1, 32, 700), (3, 300, 5, 128, 150)])
+def test_attention_and_insertion_in_one_launch(batch, n, heads, chunk, same):
+    """Prompts that share `same` tokens, with up to 64 chunks and more, into a cache that holds one already: output,
+    indices, tree and every row of the pools as from the separate calls."""
+    g = torch.Generator(device=DEV).manual_seed(batch * n + heads)
+    q, k, v = (torch.empty((batch, n, heads, 128), dtype=torch.float16, device=DEV).normal_(generator=g) for _ in range(3))
+    first = torch.empty((chunk + 3, heads, 128), dtype=torch.float16, device=DEV).normal_(generator=g)
+    prompts = [list(range(min(same, n))) + [1000 * (s + 1) + t for t in range(n - same)] for s in range(batch)]
+    found = []
+    for joined in (True, False):
+        cache = capi.Attention(heads, 128, chunk, memory_mb=64, dtype=torch.float16, device=torch.device(DEV))
+        for pool in cache.pool_views():
+            pool.zero_()
+        cache.add_seq(list(range(chunk + 3)), first, first)
+        if joined:
+            out, index = cache._prefill_attention(prompts, q, k, v)
+        else:
+            out, index = capi.causal_attention(q, k, v), [cache.add_seq(p, k[i], v[i]) for i, p in enumerate(prompts)]
+        assert not cache.ctx.valid
+        found.append((out, index, cache.tree.get_chunks(), cache.pool_views(), cache))
+    a, b = found
+    assert torch.equal(a[0], b[0]) and a[1] == b[1] and (a[2] == b[2]).all()
+    assert all(torch.equal(x, y) for x, y in zip(a[3], b[3]))
+
+
+def test_a_prompt_the_cache_cannot_take_leaves_those_before_it_with_their_rows():
+    k = torch.randn((2, 400, 16, 128), device=DEV).half()
+    cache = capi.Attention(16, 128, 64, memory_mb=4, dtype=torch.float16, device=torch.device(DEV))   # 8 chunks
+    for pool in cache.pool_views():
+        pool.zero_()
+    with pytest.raises(RuntimeError):
+        cache._prefill_attention([list(range(400)), list(range(1000, 1400))], k, k, k)
+    rows = [(slot, m) for slot, m, begin, _ in cache.tree.get_chunks() if begin == 0]
+    assert sum(m for _, m in rows) == 400
+    for pool in cache.pool_views():
+        assert torch.equal(torch.cat([pool[slot][:, :m] for slot, m in rows[:7]], dim=1).transpose(0, 1), k[0])
+
+
+def test_prompts_that_are_not_the_caches_are_left_to_the_separate_calls():
+    q = torch.zeros((1, 40, 2, 128), device=DEV).half()
+    cache = capi.Attention(2, 128, 64, memory_mb=2, dtype=torch.float16, device=torch.device(DEV))
+    for prompts in ([], [list(range(39))], [tuple(range(40))], [[1 << 40] * 40], [[0.5] * 40], [list(range(40))] * 2):
+        assert cache._prefill_attention(prompts, q, q, q) is None
+    assert cache._prefill_attention([list(range(40))], *[q[:, :, :1].contiguous()] * 3) is None
+    assert cache.tree.n_seqs == 0

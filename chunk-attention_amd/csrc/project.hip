@@ -8,6 +8,7 @@
 //   add       plain, added to other rows once rounded: output projection and residual
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <type_traits>
 
@@ -536,6 +537,254 @@ int launch_shared_tile(const ProjectArgs& a, hipStream_t st) {
     return e == hipSuccess ? 0 : static_cast<int>(e);
 }
 
+// ---- q, k and v of many rows: tiles of 256 x 384 and 128 x 384 -----------------------------------------------------
+//
+// The three weights' columns are one row of heads here, of which a workgroup takes three by 256 (MB 8) or 128 (MB 4)
+// rows: q, k and v of 4096 on 2048 rows are 256 tiles of 256 x 384, one for each compute unit, where 128 x 256 makes
+// three rounds of 48 KB a stage for 4 MFLOP.
+// Eight waves of 128 x 96 (64 x 96), two to a SIMD: 192 accumulators of 256 registers, so that a k-step's operands do
+// not fit twice.  The six of w stay for a stage and are replaced one by one behind their last product, those of x are
+// read two rows of products ahead into four places in turn.  A stage's last reads lie two such rows before its end, and
+// what follows them is covered by those rows' products: the barrier behind which its buffer is free and the next
+// stage's first operands.  Four stages of 32 k elements fill the LDS: a load has three stages' time to land, and a stage's
+// are spread over all of its products (a wave issues in order: in a row, the products wait for them to be taken).
+// A wave's columns are three pairs of 16, a head's first half and the partners 64 further on; pair p of the launch is
+// pair p % 4 of head p / 4, counted over the weights.
+//
+// What bounds it: the clock, as above, and 0.3 us of 64 k elements' 1.8 the loads.  4096 x 4096 on 2048 rows 189 -> 161
+// us, 1.28 PFLOP/s; on 1024 rows (128 x 384) 118 -> 103; 2048 x 2048 on 3000 rows 87 -> 70.  Two stages of 64 took
+// 166, and the results' way out as straight code for every accumulator 170 (20 KB of it, fetched once by each wave).
+constexpr int HN = 384;
+constexpr int HK = 32;             // k elements of a stage: one k-step
+
+template <int MB>
+__global__ __launch_bounds__(512, 2) void project_heads_kernel(const ProjectArgs a) {
+#ifdef __HIP_DEVICE_COMPILE__                        // (the host's pass knows no buffer resources, and drops a template that has one)
+    constexpr int HM = 32 * MB, WN = 4, NB = 6, PAIRS = NB / 2, CW = 16 * NB, TM = 16 * MB;
+    constexpr int STAGE = (HM + HN) * HK * 2;        // bytes
+    constexpr int NBUF = 4;
+    constexpr int XL = HM / 128, WL = HN / 128;      // loads of a wave a stage, sixteen rows each
+    constexpr int NLD = XL + WL, EARLY = 2;           // the first two behind the barrier, the others over the next stage
+    constexpr int EP = CW + 4;                       // pitch of the sums' way through LDS
+    __shared__ __attribute__((aligned(16))) char lds[NBUF * STAGE];
+    static_assert(NLD >= EARLY && MB % 4 == 0 && 8 * 32 * EP * 4 + HM * 4 <= NBUF * STAGE, "");
+
+    const int tid = threadIdx.x;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = w / WN, wn = w % WN;
+    const int l = tid & 63, g = l >> 4, i = l & 15;
+    // tiles to XCDs as above
+    const int heads = a.N / D, all_heads = 3 * heads;
+    const int n_cb = heads, n_rb = (a.M + HM - 1) / HM;
+    const int total = n_cb * n_rb;
+    const int xcd = blockIdx.x & 7, q8 = total >> 3, r8 = total & 7;
+    const int u = xcd * q8 + (xcd < r8 ? xcd : r8) + (blockIdx.x >> 3);
+    constexpr int GM = 8;
+    const int grp = u / (GM * n_cb), in_grp = u - grp * GM * n_cb;
+    const int g_rows = n_rb - grp * GM < GM ? n_rb - grp * GM : GM;
+    const int cb = in_grp / g_rows, rb = grp * GM + in_grp % g_rows;
+    const int row0 = rb * HM;
+    const int pair0 = cb * (HN / 32);                // the tile's first pair
+
+    // A wave's loads of a stage: rows 16 (XL w + r) .. + 15 of x, then rows 16 (WL w + r) .. + 15 of the tile's columns.
+    // As buffer loads: a lane's part of the address is 32 bits (64 would not fit beside the accumulators).  Piece c of
+    // row r stands at place c ^ (r >> 2 & 1) * 2: eight rows at two neighbouring pieces lie in different banks.
+    int lane_row = l >> 2;
+    const int piece = (l & 3) ^ ((l >> 4 & 1) << 1);
+    const unsigned last_row = a.M - 1 - row0;        // rows behind it repeat it: computed, not stored
+    auto buffer = [](const void* p) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, -1, 0x00020000); };
+    const auto xsrc = buffer(static_cast<const half_t*>(a.x) + size_t(row0) * a.K);
+    const half_t* wsrc[WL];
+#pragma unroll
+    for (int r = 0; r < WL; r++) {
+        const int part = WL * w + r, block = part % NB;
+        const int pair = pair0 + part / NB * PAIRS + block % PAIRS, head = pair >> 2, which = head / heads;
+        const int col = (head - which * heads) * D + (pair & 3) * 16 + block / PAIRS * (D / 2);
+        wsrc[r] = static_cast<const half_t*>(which == 0 ? a.w[0] : which == 1 ? a.w[1] : a.w[2]) + size_t(col) * a.K;
+    }
+    const unsigned woff = unsigned(lane_row) * (unsigned(a.K) * 2) + 16 * piece;
+    auto load = [&](int r, int t, int at) {          // `at`: the stage's buffer
+        auto* dst = (__attribute__((address_space(3))) void*)(lds + at + (r < XL ? XL * w + r : HM / 16 + WL * w + r - XL) * 1024);
+        if (r < XL) {
+            const unsigned row = min(unsigned(lane_row + 16 * (XL * w + r)), last_row);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(xsrc, dst, 16, row * (unsigned(a.K) * 2) + 16 * piece, t * (HK * 2), 0, 0);
+            return;
+        }
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(buffer(wsrc[r - XL]), dst, 16, woff, t * (HK * 2), 0, 0);
+    };
+
+    f4 acc[MB][NB];
+#pragma unroll
+    for (int m = 0; m < MB; m++) {
+#pragma unroll
+        for (int n = 0; n < NB; n++) acc[m][n] = f4{ 0.f, 0.f, 0.f, 0.f };
+    }
+    h8 xf[4], wf[NB];
+    const int lane = i * (HK * 2) + 16 * (g ^ ((i >> 2 & 1) << 1));
+    int xat = wm * TM * (HK * 2) + lane, wat = (HM + wn * CW) * (HK * 2) + lane;
+    auto read = [&](int at) { return *reinterpret_cast<const h8*>(lds + at); };
+
+    const int n_t = a.K / HK;
+    // Every wave's loads but its newest `left` have landed, and every wave holds what it has read.
+    auto meet = [&](auto left) {
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(decltype(left)::value) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+#pragma unroll
+    for (int s = 0; s < NBUF; s++) {
+#pragma unroll
+        for (int r = 0; r < (s < NBUF - 1 ? NLD : EARLY); r++) {
+            if (s < n_t) load(r, s, s * STAGE);
+        }
+    }
+    if (n_t >= NBUF) meet(std::integral_constant<int, 2 * NLD + EARLY>{});
+    else meet(std::integral_constant<int, 0>{});
+#pragma unroll
+    for (int n = 0; n < NB; n++) wf[n] = read(wat + n * 1024);
+    xf[0] = read(xat);
+    xf[1] = read(xat + 1024);
+    int here = 0;
+    // Stage t in the buffer at `here`.  MORE: there is a stage t + 1; LATE: a stage t + 3, whose last load is still to be
+    // asked for; LOADS: a stage t + 4.
+    auto stage_of = [&](int t, auto more, auto late, auto loads) {
+        constexpr bool MORE = decltype(more)::value, LATE = decltype(late)::value, LOADS = decltype(loads)::value;
+        const int next = here + STAGE == NBUF * STAGE ? 0 : here + STAGE, before = here == 0 ? (NBUF - 1) * STAGE : here - STAGE;
+        asm volatile("" : "+v"(lane_row));           // the offsets in x are formed where they are used: kept, they are registers
+#pragma unroll
+        for (int m = 0; m < MB; m++) {
+            if (m == MB - 2 && MORE) {
+                meet(std::integral_constant<int, LATE ? 2 * NLD : 0>{});
+                xat += next - here;
+                wat += next - here;
+            }
+#pragma unroll
+            for (int n = 0; n < NB; n++) {
+                acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf[n], xf[m & 3], acc[m][n], 0, 0, 0);
+                if (n == 0 && (m + 2 < MB || MORE)) xf[(m + 2) & 3] = read(xat + (m + 2) % MB * 1024);
+                if (m == MB - 1 && MORE) wf[n] = read(wat + n * 1024);
+                constexpr int FREE = (MB - 2) * NB, TAIL = 2 * NB;
+                const int k = m * NB + n;
+#pragma unroll
+                for (int r = 0; r < NLD; r++) {
+                    if (LATE && r >= EARLY && k == (2 * (r - EARLY) + 1) * FREE / (2 * (NLD - EARLY > 0 ? NLD - EARLY : 1))) load(r, t + NBUF - 1, before);
+                    if (LOADS && r < EARLY && k - FREE == (2 * r + 1) * TAIL / (2 * EARLY)) load(r, t + NBUF, here);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        here = next;
+    };
+    const auto yes = std::true_type{};
+    const auto no = std::false_type{};
+    int t = 0;
+    for (; t + NBUF < n_t; t++) stage_of(t, yes, yes, yes);
+    if (t + NBUF == n_t) stage_of(t++, yes, yes, no);
+    for (; t + 1 < n_t; t++) stage_of(t, yes, no, no);
+    // the rows' positions: on their way during the last stage, then where every lane finds them
+    const int64_t own = tid < HM ? a.positions[row0 + tid < a.M ? row0 + tid : a.M - 1] : 0;
+    stage_of(t, no, no, no);
+    // the loop's last matrix ops are read behind a branch, where the compiler's own wait states do not reach
+    asm volatile("s_nop 15\n\ts_nop 15");
+    __builtin_amdgcn_sched_barrier(0);
+    __syncthreads();                                 // every wave is done with the last stage's operands
+    int* position = reinterpret_cast<int*>(lds + 8 * 32 * EP * 4);
+    if (tid < HM) position[tid] = static_cast<int>(rotary::clamp_pos(own, a.max_position));
+    __syncthreads();
+
+    // Lane (g, i) holds row i of a 16 x 16 block, columns 4g .. 4g + 3: through the wave's own piece of LDS, 32 rows at a
+    // time, to lanes that hold eight columns of a row and their partners.  One piece of code for all of
+    // them: what is run once is fetched once, and straight code for every accumulator took 6 us longer.
+    float* sums = reinterpret_cast<float*>(lds) + w * 32 * EP;
+    const int pair_w = pair0 + wn * PAIRS;           // the wave's first pair
+    auto put = [&](auto block) {
+        constexpr int M2 = decltype(block)::value;
+#pragma unroll
+        for (int mm = 0; mm < 2; mm++) {
+#pragma unroll
+            for (int n = 0; n < NB; n++) *reinterpret_cast<f4*>(&sums[(16 * mm + i) * EP + 16 * n + 4 * g]) = acc[2 * M2 + mm][n];
+        }
+    };
+#pragma unroll 1
+    for (int m2 = 0; m2 < MB / 2; m2++) {
+        if (m2 == 0) put(std::integral_constant<int, 0>{});
+        if (m2 == 1) put(std::integral_constant<int, 1>{});
+        if constexpr (MB > 4) {
+            if (m2 == 2) put(std::integral_constant<int, 2>{});
+            if (m2 == 3) put(std::integral_constant<int, 3>{});
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int p = 0; p < PAIRS; p++) {
+            const int at = p * 64 + l, r = at / (2 * PAIRS), q = at % (2 * PAIRS);
+            const int in_tile = wm * TM + 32 * m2 + r, pair = pair_w + (q >> 1), head = pair >> 2;
+            const int which = head >= 2 * heads ? 2 : head >= heads ? 1 : 0, d0 = (pair & 3) * 16 + 8 * (q & 1);
+            const half_t* cs = static_cast<const half_t*>(a.cos_sin_cache) + size_t(position[in_tile]) * D + d0;
+            const h8 c8 = *reinterpret_cast<const h8*>(cs), s8 = *reinterpret_cast<const h8*>(cs + D / 2);
+            const float* f = &sums[r * EP + 8 * q];
+            float f0[8], f1[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                f0[e] = f[e];
+                f1[e] = f[CW / 2 + e];
+            }
+            h8 o0, o1;
+            if (which < 2) {
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    o0[e] = half_t(rotary::rot_elem(f0[e], f1[e], float(c8[e]), float(s8[e]), true));
+                    o1[e] = half_t(rotary::rot_elem(f1[e], f0[e], float(c8[e]), float(s8[e]), false));
+                }
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    o0[e] = half_t(f0[e]);
+                    o1[e] = half_t(f1[e]);
+                }
+            }
+            if (row0 + in_tile < a.M) {
+                half_t* dst = static_cast<half_t*>(which == 0 ? a.y[0] : which == 1 ? a.y[1] : a.y[2]) +
+                              size_t(row0 + in_tile) * a.N + (head - which * heads) * D + d0;
+                *reinterpret_cast<h8*>(dst) = o0;
+                *reinterpret_cast<h8*>(dst + D / 2) = o1;
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+#endif
+}
+
+template <int MB>
+int launch_heads(const ProjectArgs& a, hipStream_t st) {
+    constexpr int HM = 32 * MB;
+    const int64_t wgs = int64_t(a.N) / D * ((int64_t(a.M) + HM - 1) / HM);
+    if (wgs > 0x7fffffff) return -1;
+    hipLaunchKernelGGL(project_heads_kernel<MB>, dim3(static_cast<unsigned>(wgs)), dim3(512), 0, st, a);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? 0 : static_cast<int>(e);
+}
+
+// Which of them q, k and v take beside the tiles of 128 x 128 and 128 x 256, of which there are `square` and `wide` rounds:
+// the one that the rounds make the shortest; 0 for none.  A round takes so long for each 64 k elements, and at its ends (in
+// 1/64 us; the last, partial one of 256 x 384 less, for the clock is higher then).  Measured with each (us in 128 x 128 or
+// 128 x 256, 128 x 384, 256 x 384): 4096 x 4096 on 500 rows 62, 96, 121, on 700 102, 97, 119, on 1024 118, 103, 126, on 1200
+// 117, 188, 126, on 1500 161, 190, 132, on 2048 189, 216, 161, on 2300 221, 257, 278; 2048 x 2048 on 1000 rows 30, 38, 61, on
+// 1500 53, 42, 62, on 2048 56, 51, 63, on 3000 87, 85, 70; 1024 x 1024 on 2000 rows 19, 24, 38, on 4096 35, 30, 40, on 7000
+// 55, 53, 46; 5120 x 5120 on 1000 rows 159, 266, 178, on 1300 222, 259, 181.
+int heads_shape(const ProjectArgs& a, int64_t square, int64_t wide) {
+    constexpr int CUS = 256;
+    const int64_t stages = a.K / 64, heads = a.N / D;
+    if (square == 1) return 0;
+    auto cost = [&](int64_t tiles, int round, int empty, int ends) {
+        const int64_t full = tiles / CUS, rest = tiles % CUS;
+        return full * (stages * round + ends) + (rest ? stages * (empty + (round - empty) * rest / CUS) + ends : 0);
+    };
+    const int64_t others = std::min(square * (stages * 39 + 160), wide * (stages * 59 + 160));
+    const int64_t tall = cost(heads * ((int64_t(a.M) + 255) / 256), 160, 115, 576);
+    const int64_t flat = cost(heads * ((int64_t(a.M) + 127) / 128), 105, 94, 192);
+    return std::min(tall, flat) >= others ? 0 : tall < flat ? 8 : 4;
+}
+
 // Tiles.  Up to 16 rows: 16 columns a workgroup (three weights of 4096 x 4096, 8 rows: 22.7 us against 26.3 with
 // 32 columns; one weight 8.4), three units on their way where a wave has more than two (otherwise they
 // would only be asked for again).  More rows: 32 x 32 with k split over the waves while about one of them falls to each
@@ -569,6 +818,10 @@ int launch_mode(const ProjectArgs& a, hipStream_t st) {
     if (tiles(64, 64) <= CUS) return launch_shared_tile<64, 64, 4, 4, 2, MODE>(a, st);
     if (tiles(64, 128) <= CUS) return launch_shared_tile<64, 128, 4, 8, 2, MODE>(a, st);
     const int64_t square = (tiles(128, 128) + CUS - 1) / CUS, wide = (tiles(128, 256) + CUS - 1) / CUS;
+    if constexpr (MODE == kRotary) {
+        const int shape = heads_shape(a, square, wide);
+        if (shape) return shape == 8 ? launch_heads<8>(a, st) : launch_heads<4>(a, st);
+    }
     if (square == 1 || square * 36 < wide * 56) return launch_shared_tile<128, 128, 4, 8, 2, MODE>(a, st);
     return launch_shared_tile<128, 256, 3, 8, 4, MODE>(a, st);
 }

@@ -31,6 +31,13 @@ def test_qkv_rotary_in_shared_tiles(rows, heads, n_in):
     project.test_qkv_rotary(rows, heads, n_in)
 
 
+# tiles of three heads: 128 rows (one to more stages than buffers, last rows, a grid that the XCDs do not divide), 256 rows
+@pytest.mark.parametrize("rows,heads,n_in", [(1300, 16, 64), (1409, 16, 128), (1291, 17, 192), (2047, 12, 320),
+                                             (1290, 32, 1024), (2000, 31, 1088), (6900, 8, 1024)])
+def test_qkv_rotary_in_tiles_of_three_heads(rows, heads, n_in):
+    project.test_qkv_rotary(rows, heads, n_in)
+
+
 def test_decode_of_more_rows_than_a_block():
     project.test_layer_decode_writes_the_pool_as_the_library_path_does(70, 12, 64)
 

@@ -78,7 +78,7 @@ def build_pybind() -> str:
                                                      "-I" + sysconfig.get_paths()["include"],
                                                      "-I" + os.path.join(ROOT, "include"), "-I" + CSRC,
                                                      "-I/opt/rocm/include"]
-    srcs = [os.path.join(CSRC, f) for f in ("attention.cpp", "python_exports.cpp")]
+    srcs = [os.path.join(CSRC, f) for f in ("attention.cpp", "module_checks.cpp", "python_exports.cpp")]
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
            "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=chunk_attn_c",
            "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI)] + incs + srcs + [

@@ -3,7 +3,8 @@
 `Tree` wraps the prefix-tree manager handle, `KernelContext` the device-side context, and
 `Attention` composes both over a torch-allocated fp16 KV pool with the same methods as the
 pybind11 class (add_seq / append_token / forward / remove_seq / reserve /
-refresh_kernel_context), for hosts that cannot load the C++ extension module.
+refresh_kernel_context).  What stands between a module and its kernel is looked at by the C++ extension
+module (chunk_attn_c.modules).
 
 There is no CPU fallback: loading fails if the library has not been built, and every device
 entry point reports an error when no HIP device is present.
@@ -19,6 +20,7 @@ import numpy as np
 import torch
 
 from . import stock
+from .lib.chunk_attn_c import modules
 
 _LIB_PATH = os.environ.get("CHUNK_ATTN_HIP_LIB") or os.path.join(
     os.path.dirname(os.path.abspath(__file__)), "lib", "libchunkattn_hip.so")
@@ -463,11 +465,7 @@ def _causal_attention(q, k, v):
 
 def is_bare(module, cls) -> bool:
     """The module is a `cls` and nothing hangs on it that a call would also run (hooks, a patched forward)."""
-    if type(module) is not cls:
-        return False
-    own = module.__dict__
-    return not (own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"] or
-                own["_backward_pre_hooks"] or "forward" in own)
+    return modules.all_bare(cls, (module,))
 
 
 def projection_takes(x, *linears) -> bool:
@@ -492,24 +490,16 @@ def _projection_takes(x, *linears, limit: int = 1 << 20) -> bool:
 def _linears_are_plain(n_in: int, device, linears) -> bool:
     """What each of the modules computes of fp16 rows [..., n_in] on the device is exactly their product with a weight
     that the projection kernels read (torch.nn.Linear being as torch wrote it)."""
-    grad = torch.is_grad_enabled()
+    return plain_weights(-1, n_in, device, linears) is not None
+
+
+def plain_weights(n_out: int, n_in: int, device, linears):
+    """(addresses of the weights [n_out (-1: any), n_in], the weights) of linears that are all as _linears_are_plain says,
+    None otherwise."""
     # whatever else may stand between a module and its product: hooks, subclasses, patched forwards, modes
     if torch.is_autocast_enabled() or not plain_call() or torch.nn.modules.module._has_any_global_hook():
-        return False
-    Linear, Parameter, half = torch.nn.Linear, torch.nn.Parameter, torch.float16
-    for m in linears:
-        if not is_bare(m, Linear):
-            return False
-        own = m.__dict__
-        if "weight" in own or "bias" in own:           # what hides the registered ones
-            return False
-        parameters = own["_parameters"]
-        w = parameters.get("weight")
-        if type(w) is not Parameter or parameters.get("bias", w) is not None or w.dtype is not half or \
-                w.device != device or w.dim() != 2 or w.shape[1] != n_in or not w.is_contiguous() or \
-                w.data_ptr() % 16 or (grad and w.requires_grad):
-            return False
-    return True
+        return None
+    return modules.linear_weights(linears, torch.nn.Linear, torch.nn.Parameter, n_out, n_in, device, torch.is_grad_enabled())
 
 
 def projection_pays(rows: int, n_in: int, n_out: int) -> bool:
@@ -624,15 +614,13 @@ def _qkv_rotary(x, wq, wk, wv, positions, cos_sin_cache):
 
 
 def _model_pass(layers, tokens, positions, n_seqs: int, prefill: bool, embedding, norm, epsilon: float, head, index: list):
-    """A pass of the small model as one native call (see ca_model_pass).  layers: (cache, wq, wk, wv, wo, table, norm
-    weight, epsilon) of each; the caller has checked all of it (tiny_lm._plain_pass).  Returns the logits, or without a
+    """A pass of the small model as one native call (see ca_model_pass).  layers: of each its cache and a
+    ModelLayer's other fields; the caller has checked all of it (tiny_lm._plain_pass).  Returns the logits, or without a
     head the last norm's rows; `index` receives the prompt's index in every cache, -1 where it was not inserted, also
     when the pass fails."""
     lib, device, hidden = load(), embedding.device, embedding.shape[1]
     rows = len(tokens)
-    table = (ModelLayer * len(layers))(*[
-        (cache.ctx._h, cache.tree._h, wq.data_ptr(), wk.data_ptr(), wv.data_ptr(), wo.data_ptr(), t.data_ptr(), w.data_ptr(),
-         t.shape[0], eps) for cache, wq, wk, wv, wo, t, w, eps in layers])
+    table = (ModelLayer * len(layers))(*[(cache.ctx._h, cache.tree._h, *rest) for cache, *rest in layers])
     ids, ids_ptr = _i32(tokens)
     pos, pos_ptr = _i32(positions)
     scratch = torch.empty(lib.ca_model_scratch_bytes(rows, hidden) // 2, dtype=torch.float16, device=device)

@@ -42,6 +42,11 @@ class RotaryEmbedding(nn.Module):
 _ROTARY_FORWARD = RotaryEmbedding.forward
 
 
+def plain_rotaries(layers, device: torch.device) -> Optional[List[torch.Tensor]]:
+    """The layers' rotary tables, if every one is as LlamaChunkAttention._plain_rotary says."""
+    return capi.modules.rotary_tables(layers, RotaryEmbedding, device) if stock.is_stock(RotaryEmbedding, _ROTARY_FORWARD) else None
+
+
 class LlamaChunkAttention(nn.Module):
     """q/k/v projections -> rotary -> (prefill: causal attention + add_seq | decode: append +
     chunk attention) -> output projection."""
@@ -131,11 +136,8 @@ class LlamaChunkAttention(nn.Module):
         """The rotary module's table, if the module is the one this layer was built with, over whole heads, nothing
         hangs on it or hides its table, and the projection kernels read such a table (the operator takes narrower ones and any
         alignment)."""
-        r = self.rotary_emb
-        table = r.__dict__["_buffers"].get("cos_sin_cache")
-        plain = table is not None and "cos_sin_cache" not in r.__dict__ and capi.is_bare(r, RotaryEmbedding) and stock.is_stock(RotaryEmbedding, _ROTARY_FORWARD) and \
-            r.is_neox_style and r.rotary_dim == r.head_size == self.head_dim and capi.is_rotary_table(table, device)
-        return table if plain else None
+        tables = plain_rotaries((self,), device)
+        return tables[0] if tables else None
 
     def _output(self, attn_output: torch.Tensor, kv_cache: capi.Attention, own: bool) -> torch.Tensor:
         output = capi._linear(attn_output, self.o_proj.weight) if own else self.o_proj(attn_output)

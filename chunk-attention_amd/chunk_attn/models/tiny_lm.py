@@ -14,7 +14,7 @@ import torch
 from torch import nn
 
 from .. import capi, stock
-from ..llama_layer import LlamaChunkAttention, layer_is_stock
+from ..llama_layer import LlamaChunkAttention, layer_is_stock, plain_rotaries
 from .sequence import Sequence
 
 
@@ -36,10 +36,9 @@ _HOST = torch.device("cpu")
 _PROJECTIONS = ("q_proj", "k_proj", "v_proj", "o_proj")
 
 
-def _is_plain(w, shape, device: torch.device) -> bool:
-    """A parameter that kernels can read by its address."""
-    return type(w) is nn.Parameter and w.dtype is torch.float16 and w.device == device and w.shape == shape and \
-        w.is_contiguous() and w.data_ptr() % 16 == 0
+def _addresses(parameters, shape, device: torch.device) -> Optional[List[int]]:
+    """Of parameters that kernels can read by their address; None if one is not."""
+    return capi.modules.parameter_addresses(parameters, nn.Parameter, shape, device)
 
 
 def _pins(device: torch.device) -> bool:
@@ -87,19 +86,21 @@ class AttentionOnlyLM(nn.Module):
         else:
             input_ids = [[s[-1]] for s in seqs]
             position_ids = [[len(s) - 1] for s in seqs]
-        dev = self.embed_tokens.weight.device
+        embedding = self.embed_tokens.weight
+        dev = embedding.device
         joined = self._adds_in_norms()
-        layers = self._plain_pass(seqs, input_ids, kv_caches, prefill, dev) if joined else None
-        if layers:
-            head = self.lm_head.weight if capi.projection_pays(len(seqs), self.hidden_size, self.vocab_size) and \
-                capi._linears_are_plain(self.hidden_size, dev, (self.lm_head,)) else None
+        plain = self._plain_pass(seqs, input_ids, kv_caches, prefill, dev) if joined else None
+        if plain is not None:
+            layers, kept = plain                       # (kept to the end of the call: addresses alone hold nothing)
+            lm_head, first = self.lm_head, self.input_norms[0]
+            head = lm_head.weight if capi.projection_pays(len(seqs), self.hidden_size, self.vocab_size) and \
+                capi._linears_are_plain(self.hidden_size, dev, (lm_head,)) else None
             index = []
             try:
                 out = capi._model_pass(layers, [t for ids in input_ids for t in ids], [p for pos in position_ids for p in pos],
-                                       len(seqs), prefill, self.embed_tokens.weight, self.input_norms[0].weight,
-                                       self.input_norms[0].eps, head, index)
+                                       len(seqs), prefill, embedding, first.weight, first.eps, head, index)
             finally:                                   # a pass that failed has filled the caches in front of that layer
-                for layer, idx in zip(self.layers, index if prefill else ()):
+                for layer, idx in zip(self.layers, index) if prefill else ():
                     if idx >= 0:
                         layer.last_indices = [idx]
                         seqs[0].index = idx
@@ -134,10 +135,10 @@ class AttentionOnlyLM(nn.Module):
             return capi._linear(last, self.lm_head.weight)
         return self.lm_head(last)
 
-    def _plain_pass(self, seqs, input_ids, kv_caches, prefill: bool, dev: torch.device) -> Optional[list]:
-        """The layers as capi._model_pass takes them, if the pass is one that the native call computes as the modules
-        would (given _adds_in_norms): a decode step or one prompt, every layer's projections its own kernels' business,
-        caches and parameters plain, and no capture, under which ids are not uploaded either."""
+    def _plain_pass(self, seqs, input_ids, kv_caches, prefill: bool, dev: torch.device) -> Optional[tuple]:
+        """(the layers as capi._model_pass takes them, what their addresses are of), if the pass is one that the native call
+        computes as the modules would (given _adds_in_norms): a decode step or one prompt, every layer's projections its
+        own kernels' business, caches and parameters plain, and no capture, under which ids are not uploaded either."""
         hidden, n = self.hidden_size, len(self.layers)
         if n == 0 or len(kv_caches) < n or not seqs or not input_ids[0] or (prefill and len(seqs) != 1) or dev.type != "cuda" or \
                 torch.cuda.is_current_stream_capturing():
@@ -150,39 +151,45 @@ class AttentionOnlyLM(nn.Module):
             array.array("i", [t for ids in input_ids for t in ids])
         except (TypeError, OverflowError):             # ids that are no 32-bit numbers: torch's business
             return None
-        norms = (*self.input_norms, self.norm)
-        embedding, norm_weights = self.embed_tokens, [None if "weight" in m.__dict__ else m._parameters.get("weight") for m in norms]
-        if len(norms) != n + 1 or embedding.max_norm is not None or not _is_plain(embedding.weight, (self.vocab_size, hidden), dev) or \
-                not all([_is_plain(w, (hidden,), dev) for w in norm_weights]):
+        norms, modules = (*self.input_norms, self.norm), list(self.layers)
+        gains = [None if "weight" in m.__dict__ else m._parameters.get("weight") for m in norms]
+        norm_weights, embedding = _addresses(gains, (hidden,), dev), self.embed_tokens
+        if len(norms) != n + 1 or embedding.max_norm is not None or norm_weights is None or \
+                _addresses((embedding.weight,), (self.vocab_size, hidden), dev) is None:
             return None
         # (by the modules' own dictionaries: __getattr__ costs as much as a launch here, a few dozen times a pass; what
         # hides a registered module, on the object or its class, is what the layer calls)
         if not vars(LlamaChunkAttention).keys().isdisjoint(_PROJECTIONS) or \
-                not all([layer.__dict__.keys().isdisjoint(_PROJECTIONS) for layer in self.layers]):
+                not all([layer.__dict__.keys().isdisjoint(_PROJECTIONS) for layer in modules]):
             return None
-        linears = [m.get(name) for m in [layer._modules for layer in self.layers] for name in _PROJECTIONS]
-        if not capi._linears_are_plain(hidden, dev, linears):
+        weights = capi.plain_weights(hidden, hidden, dev, [own.get(name) for own in [layer._modules for layer in modules] for name in _PROJECTIONS])
+        if weights is None:
             return None
-        weights = [m._parameters["weight"] for m in linears]
+        tables = plain_rotaries(modules, dev)
+        if tables is None:
+            return None
         plain_cache = capi.is_plain_cache_to_fill if prefill else capi.is_plain_cache
-        layers = []
-        for i, (layer, cache) in enumerate(zip(self.layers, kv_caches)):
-            table = layer._plain_rotary(dev) if layer.head_dim == 128 and layer.num_heads * 128 == hidden else None
-            if table is None or not plain_cache(cache) or cache.d_head != 128 or cache.n_heads != layer.num_heads or cache.device != dev:
+        addresses, tensors = weights
+        layers, kept = [], (tensors, gains, tables)
+        for i, (layer, cache, table) in enumerate(zip(modules, kv_caches, tables)):
+            heads = layer.num_heads
+            if layer.head_dim != 128 or heads * 128 != hidden or not plain_cache(cache) or cache.d_head != 128 or \
+                    cache.n_heads != heads or cache.device != dev:
                 return None
-            layers.append((cache, *weights[4 * i:4 * i + 4], table, norm_weights[i + 1], norms[i + 1].eps))
-        return layers if all([w.size(0) == hidden for w in weights]) else None
+            layers.append((cache, *addresses[4 * i:4 * i + 4], table.data_ptr(), norm_weights[i + 1], table.shape[0], norms[i + 1].eps))
+        return layers, kept
 
     def _adds_in_norms(self) -> bool:
         """A layer's residual is added in the norm behind it, in place: nothing may want the tensors it overwrites
         (a gradient, a hook, a mode that sees them, a forward-mode tangent of them), and the norms must be the plain
         ones."""
+        bare, layers = capi.modules.all_bare, list(self.layers)
         return capi.plain_call() and not torch.is_grad_enabled() and \
             stock.embedding_is_stock() and stock.linear_is_stock() and layer_is_stock() and \
             stock.is_stock(RMSNorm, _NORM_FORWARD) and \
             not torch.nn.modules.module._has_any_global_hook() and capi.is_bare(self.embed_tokens, nn.Embedding) and \
-            all([capi.is_bare(m, LlamaChunkAttention) and capi.is_bare(m.o_proj, nn.Linear) for m in self.layers]) and \
-            all([capi.is_bare(m, RMSNorm) for m in (*self.input_norms, self.norm)])
+            bare(LlamaChunkAttention, layers) and capi.modules.children_bare(nn.Linear, layers, "o_proj") and \
+            bare(RMSNorm, (*self.input_norms, self.norm))
 
     @torch.no_grad()
     def forward(self, seqs: List[Sequence], kv_caches, prefill: bool) -> List[int]:

@@ -5,6 +5,7 @@
 #include <torch/extension.h>
 
 #include "attention.h"
+#include "module_checks.h"
 
 namespace py = pybind11;
 using GPT::Attention;
@@ -80,4 +81,13 @@ PYBIND11_MODULE(chunk_attn_c, m) {
             "Apply Root Mean Square (RMS) Normalization to the input tensor.");
     ops.def("fused_add_rms_norm", &GPT::fused_add_rms_norm, py::arg("input"), py::arg("residual"),
             py::arg("weight"), py::arg("epsilon"), "In-place fused Add and RMS Normalization");
+
+    py::module modules = m.def_submodule("modules", "what kernels that stand in for modules look at first");
+    modules.def("all_bare", &GPT::all_bare, py::arg("cls"), py::arg("modules"));
+    modules.def("children_bare", &GPT::children_bare, py::arg("cls"), py::arg("modules"), py::arg("name"));
+    modules.def("rotary_tables", &GPT::rotary_tables, py::arg("layers"), py::arg("rotary"), py::arg("device"));
+    modules.def("linear_weights", &GPT::linear_weights, py::arg("modules"), py::arg("linear"), py::arg("parameter"),
+                py::arg("n_out"), py::arg("n_in"), py::arg("device"), py::arg("grad"));
+    modules.def("parameter_addresses", &GPT::parameter_addresses, py::arg("tensors"), py::arg("parameter"),
+                py::arg("shape"), py::arg("device"));
 }

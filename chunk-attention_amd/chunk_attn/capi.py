@@ -42,7 +42,7 @@ class PlanInfo(ctypes.Structure):
                 ("max_seq_n_chunks", ctypes.c_int32), ("n_shared_items", ctypes.c_int32),
                 ("n_stream_items", ctypes.c_int32), ("n_part_rows", ctypes.c_int32),
                 ("shared_tokens", ctypes.c_int64), ("stream_tokens", ctypes.c_int64),
-                ("stream_per_wave", ctypes.c_int32), ("stream_per_head", ctypes.c_int32)]
+                ("stream_per_wave", ctypes.c_int32), ("reserved", ctypes.c_int32)]
 
 
 class ModelLayer(ctypes.Structure):
@@ -725,7 +725,7 @@ class HostTables:
         p["n_part_rows"] = info.n_part_rows
         p["shared_tokens"] = info.shared_tokens
         p["stream_tokens"] = info.stream_tokens
-        p["stream_per_wave"], p["stream_per_head"] = info.stream_per_wave, info.stream_per_head
+        p["stream_per_wave"] = info.stream_per_wave
         return p
 
 

@@ -201,7 +201,6 @@ ca::LaunchArgs launch_args(const ca_ctx* c, const void* q, void* out) {
     a.n_cus = c->n_cus;
     a.scale_log2 = 1.4426950408889634f / std::sqrt(static_cast<float>(c->d));
     a.stream_per_wave = c->plan.stream_per_wave;
-    a.stream_per_head = c->plan.hints.per_head;
     a.shared_narrow = c->plan.shared_narrow;
     // 256 MiB of Infinity Cache on this part.  A forward that attends more than that cannot find
     // its K/V there again on the next step, and plain loads top out near 6.3 TB/s against
@@ -1458,7 +1457,7 @@ int ca_ctx_plan_info(const ca_ctx* c, ca_plan_info* info) {
         info->shared_tokens = c->plan.shared_tokens;
         info->stream_tokens = c->plan.stream_tokens;
         info->stream_per_wave = c->plan.stream_per_wave ? 1 : 0;
-        info->stream_per_head = c->plan.hints.per_head ? 1 : 0;
+        info->reserved = 0;
         return CA_OK;
     });
 }

@@ -123,7 +123,7 @@ int ca_tables_info(const ca_tables* t, ca_plan_info* info) {
     info->shared_tokens = t->plan.shared_tokens;
     info->stream_tokens = t->plan.stream_tokens;
     info->stream_per_wave = t->plan.stream_per_wave ? 1 : 0;
-    info->stream_per_head = t->plan.hints.per_head ? 1 : 0;
+    info->reserved = 0;
     return CA_OK;
 }
 

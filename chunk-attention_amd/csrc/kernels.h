@@ -35,9 +35,6 @@ struct LaunchArgs {
     // Every wave of a stream workgroup takes a stream item of its own (four consecutive items per
     // workgroup): set by the plan when there are many short runs.  Not with fuse_merge.
     bool stream_per_wave = false;
-    // Every wave of a stream workgroup takes a head of its own of one item, which is a whole sequence (four consecutive
-    // heads per workgroup; the heads a multiple of four).  Not with fuse_merge, nor with shared items.
-    bool stream_per_head = false;
     // No shared item of the work list covers more than 16 sequences and none is wide: the launch
     // can take the form of the kernel without the 32-row and wide matrix-core paths.
     bool shared_narrow = false;

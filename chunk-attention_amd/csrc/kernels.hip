@@ -369,12 +369,10 @@ template <> union __attribute__((aligned(16))) DecodeLds<kMixNarrow> {
 // dirty lines leave the L2 in dribs and drabs and turn the memory bus around each time), the same
 // rows written by a launch of their own, or at the end of the merge launch, cost 1-3 us.
 //
-// WHOLE (with PER_WAVE): the item is all that its sequence streams, however long (whole_kernel).
-//
 // DIRECT_NW waves (0: an ordinary item of NW): the direct form (direct_kernel).  The item, `direct`, is a whole
 // sequence, its slots come with it in the waves' registers, and a wave takes single 64-token tiles, also of a chunk
 // of 128.
-template <int C, bool PER_WAVE, int STEP, int DIRECT_NW = 0, bool WHOLE = false, typename LDS = StreamPathLds>
+template <int C, bool PER_WAVE, int STEP, int DIRECT_NW = 0, typename LDS = StreamPathLds>
 __device__ __forceinline__ void stream_path(const DecodeArgs& A, const WorkItem* __restrict__ gi,
                                             int h, LDS& sm, const DirectItem* direct = nullptr) {
     constexpr bool DIRECT = DIRECT_NW > 0;
@@ -478,29 +476,9 @@ __device__ __forceinline__ void stream_path(const DecodeArgs& A, const WorkItem*
     // What divides the sums where no weight is above zero: no tokens give zero, no finite score none.
     const float r_empty = len > 0 ? __builtin_nanf("") : 0.f;
 
-    // WHOLE: the sums of four tiles at a time, which keeps the chains of additions as short as with tiles in turn
-    float far[8], far_l = 0.f, far_scale = 1.f;
-    if constexpr (WHOLE) {
-#pragma unroll
-        for (int e = 0; e < 8; e++) far[e] = 0.f;
-    }
-    auto fold_far = [&]() {
-#pragma unroll
-        for (int e = 0; e < 8; e++) {
-            far[e] = __builtin_fmaf(far[e], far_scale, acc[e]);
-            acc[e] = 0.f;
-        }
-        far_l = __builtin_fmaf(far_l, far_scale, l_lane);
-        l_lane = 0.f;
-        far_scale = 1.f;
-    };
-
     constexpr int SPLIT = DIRECT ? NSUB : 1;       // steps that share a tile
     for (int ts = (PER_WAVE ? 0 : w) * CPT; ts < it.n_chunks * SPLIT; ts += (PER_WAVE ? 1 : NWV) * CPT) {
         const int t = SPLIT > 1 ? ts / SPLIT : ts;
-        if constexpr (WHOLE) {                         // the lanes hold 64 slots
-            if (t > 0 && t % 64 == 0) slotv = t + l < it.n_chunks ? slots[it.slot_first + t + l] : 0;
-        }
         int valid = len - (it.pos0 + t) * C;
         if (valid <= 0) break;  // chunks are in path order: everything after is empty too
         // tokens of this tile: bounded by the sequence's end and by the item's last chunk (the
@@ -513,7 +491,7 @@ __device__ __forceinline__ void stream_path(const DecodeArgs& A, const WorkItem*
 #pragma unroll
         for (int cc = 0; cc < CPT; cc++) {
             const int tc = (cc < n_here) ? t + cc : t;  // a missing second chunk is never loaded
-            base[cc] = (size_t(chunk_slot(slotv, WHOLE ? tc % 64 : tc)) * H + h) * size_t(C) * D;
+            base[cc] = (size_t(chunk_slot(slotv, tc)) * H + h) * size_t(C) * D;
         }
 #pragma unroll
         for (int sub = 0; sub < NSUB; sub++) {
@@ -596,7 +574,6 @@ __device__ __forceinline__ void stream_path(const DecodeArgs& A, const WorkItem*
             const float p = fast_exp2(s - m_from);
             m_run = m_new;
             l_lane = l_lane * alpha + p;
-            if constexpr (WHOLE) far_scale *= alpha;
             sm.p[w][l] = p;
 #pragma unroll
             for (int e = 0; e < 8; e++) acc[e] *= alpha;
@@ -614,9 +591,6 @@ __device__ __forceinline__ void stream_path(const DecodeArgs& A, const WorkItem*
 #pragma unroll
                 for (int e = 0; e < 8; e++) acc[e] = __builtin_fmaf(pr[i], float(vv[e]), acc[e]);
             }
-        }
-        if constexpr (WHOLE) {
-            if (t / CPT % 4 == 3) fold_far();
         }
         if (!tried) {
             tried = true;
@@ -639,12 +613,6 @@ __device__ __forceinline__ void stream_path(const DecodeArgs& A, const WorkItem*
     }
     const bool complete = can_fold && sm.state;
 
-    if constexpr (WHOLE) {
-        fold_far();
-        l_lane = far_l;
-#pragma unroll
-        for (int e = 0; e < 8; e++) acc[e] = far[e];
-    }
     // wave result: rows are spread over the four 16-lane groups
     const float l_wave = wave_sum(l_lane);
 #pragma unroll
@@ -1374,29 +1342,6 @@ __global__ __launch_bounds__(WG, (MIX == kMixFull || MIX == kMixFullSmall || C =
 }
 
 // ---------------------------------------------------------------------------------------
-// whole_kernel: unshared sequences, a workgroup four consecutive heads of one, a wave one head from the first chunk to
-// the last.  The planner says when (head_per_wave in tables.cpp).  What bounds it: the memory's rate, and its rate for
-// this pattern is higher than for tiles in turn (64 KB in a run and pool where those are 16 KB a wave from chunks of
-// their own; no partial rows between the reads, which cost many times their bytes): 64 sequences of 4096 tokens, 32
-// heads, 655 -> 614 us, 7.0 TB/s.
-// ---------------------------------------------------------------------------------------
-template <int C, int STEP>
-__global__ __launch_bounds__(WG, 2) void whole_kernel(const WorkItem* stream_items, const half_t* kpool, const half_t* vpool,
-                                                      const half_t* q, int H, int delta_tokens, int flags, float scale_log2,
-                                                      const DecodeRest rest) {
-    DecodeArgs A{};
-    A.q = q; A.kpool = kpool; A.vpool = vpool; A.out = rest.out; A.part = rest.part;
-    A.slots = rest.slots; A.part_ptr = rest.part_ptr; A.counters = rest.counters;
-    A.delta_tokens = delta_tokens; A.H = H; A.scale_log2 = scale_log2;
-    A.stream_nt = (flags & kFlagStreamNt) ? 1 : 0;
-    A.k_new = rest.k_new; A.v_new = rest.v_new;
-    __shared__ StreamPathLds sm;
-    const int groups = H / NW, item = blockIdx.x / groups;
-    const int h = NW * (blockIdx.x - item * groups) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    stream_path<C, true, STEP, 0, true>(A, stream_items + item, h, sm);
-}
-
-// ---------------------------------------------------------------------------------------
 // direct_kernel: a small forward as one launch.  One workgroup of eight waves attends a whole (sequence, head), wave
 // w tiles w, w + 8, ..., and writes the output: shared chunks are read once per sequence (by workgroups of one
 // XCD, i.e. from one L2), in return there are no partial rows, no merge launch and no tables in memory --
@@ -1734,13 +1679,12 @@ static DecodeArgs decode_args(const LaunchArgs& a) {
 
 int launch_decode(const LaunchArgs& a, int n_shared_items, int n_stream_items, bool fuse_merge,
                   hipStream_t st) {
-    if ((a.stream_per_wave || a.stream_per_head) && fuse_merge) return -1;  // waves on their own never meet at a barrier
-    if (a.stream_per_head && (n_shared_items > 0 || a.H % NW != 0)) return -1;
+    if (a.stream_per_wave && fuse_merge) return -1;  // waves on their own never meet at a barrier
     const bool append = a.k_new != nullptr;
     if (append && (!a.v_new || fuse_merge)) return -1;
     const int step = append ? kAppend : kForward;
     const int stream_groups = a.stream_per_wave ? (n_stream_items + NW - 1) / NW : n_stream_items;
-    const int64_t wgs = int64_t(n_shared_items + stream_groups) * (a.stream_per_head ? a.H / NW : a.H);
+    const int64_t wgs = int64_t(n_shared_items + stream_groups) * a.H;
     if (wgs <= 0) return 0;
     DecodeArgs d = decode_args(a);
     d.n_shared_wgs = n_shared_items * a.H;
@@ -1751,23 +1695,6 @@ int launch_decode(const LaunchArgs& a, int n_shared_items, int n_stream_items, b
     const DecodeRest rest{ d.slots, d.out, d.part, d.part_ptr, d.counters, d.k_new, d.v_new };
     const int flags = (d.fuse_merge ? kFlagFuseMerge : 0) | (d.stream_per_wave ? kFlagPerWave : 0) |
                       (d.stream_nt ? kFlagStreamNt : 0);
-    if (a.stream_per_head) {
-#define CA_WHOLE_LAUNCH(CS, STEP)                                                                                      \
-    hipLaunchKernelGGL((whole_kernel<CS, STEP>), grid, block, 0, st, d.stream_items, d.kpool, d.vpool, d.q, d.H,       \
-                       d.delta_tokens, flags, d.scale_log2, rest)
-        switch (2 * a.C + (step == kForward ? 0 : 1)) {
-            case 64: CA_WHOLE_LAUNCH(32, kForward); break;
-            case 65: CA_WHOLE_LAUNCH(32, kAppend); break;
-            case 128: CA_WHOLE_LAUNCH(64, kForward); break;
-            case 129: CA_WHOLE_LAUNCH(64, kAppend); break;
-            case 256: CA_WHOLE_LAUNCH(128, kForward); break;
-            case 257: CA_WHOLE_LAUNCH(128, kAppend); break;
-            default: return -1;
-        }
-#undef CA_WHOLE_LAUNCH
-        CA_LAUNCH_CHECK();
-        return 0;
-    }
     // the lightest form of the kernel that holds every path this launch takes
     // (two workgroups of the full forms fit a compute unit; up to a quarter more than that still gain: 48 sequences x
     // 12 heads, 512 shared tokens, 624 workgroups 12.65 -> 12.35 us, but 24 x 32 heads, 1024, 832 workgroups 15.0 -> 15.3)

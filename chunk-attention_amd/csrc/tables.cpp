@@ -113,7 +113,7 @@ void build_stream_items(Plan& p, int chunk_size, const PlanParams& params) {
         int max_tiles = 0;
         for (const WorkItem& it : p.stream_items) max_tiles = std::max(max_tiles, ceil_div(it.n_chunks * chunk_size, 64));
         const int64_t tasks = int64_t(p.stream_items.size()) * std::max(params.n_heads, 1);
-        p.stream_per_wave = !p.hints.per_head && params.allow_per_wave && !p.stream_items.empty() && max_tiles <= 3 &&
+        p.stream_per_wave = params.allow_per_wave && !p.stream_items.empty() && max_tiles <= 3 &&
                             tasks >= int64_t(3) * 2 * params.n_cus;
     }
 
@@ -147,40 +147,13 @@ void build_stream_items(Plan& p, int chunk_size, const PlanParams& params) {
     // what the kernels assume about every item
     for (const auto* list : { &p.shared_items, &p.stream_items }) {
         for (const WorkItem& it : *list) {
-            if (it.n_chunks < 1 || (it.n_chunks > kMaxItemChunks && !(p.hints.per_head && list == &p.stream_items))) {
+            if (it.n_chunks < 1 || it.n_chunks > kMaxItemChunks) {
                 throw std::logic_error("tables: work item with an unsupported number of chunks");
             }
         }
     }
 }
 
-}  // namespace
-
-namespace {
-constexpr int kWholeSequence = 1 << 20;   // chunks of a stream item: all that a sequence streams
-
-// Whether the waves of a stream workgroup take a head each of a whole sequence, in place of tiles of a head in turn: four
-// heads' pieces of a chunk are one run of memory, nothing is added over the waves, and a sequence leaves no partial
-// row behind (nor needs a merge launch).  But the launch is then as long as its longest sequence, in rounds of two
-// workgroups a compute unit, of which a last one that fills less than half of the device is as long as a half full
-// one: worth it where nothing is shared, the sequences are long and of about one length, and the rounds come out.
-// Measured (us per forward, tiles in turn and a head a wave; chunks of 64, 32 heads, sequences x own tokens): 64 x
-// 4096 655 and 614, 64 x 2000 333 and 315, 56 x 2000 (0.9 rounds) 294 and 280, 32 x 4096 (a half) 338 and 323, 96 x 2000
-// (one and a half) 495 and 466, 128 x 1000 335 and 324, 64 x 1000 166 and 164; 256 x 3000 of 8 heads 477 and 468; chunks of
-// 32 and 128, 64 x 2000, 334 and 319, 321 and 313; lengths between 1800 and 2000 308 and 302.  Outside the rule: 66 x
-// 2000 346 and 383, 7 x 4096 79 and 177, 64 x between 1000 and 2000 244 and 255, 128 x 300 94 and 97.
-bool head_per_wave(const Plan& p, int chunk_size, const PlanParams& params) {
-    if (!params.allow_per_wave || params.partition != 0 || !p.shared_items.empty() || p.n_seqs < 1 || params.n_heads % 4 != 0) return false;
-    int64_t total = 0, longest = 0;
-    for (int s = 0; s < p.n_seqs; s++) {
-        const int64_t tokens = p.seq_len[s] - int64_t(p.own_pos0[s]) * chunk_size;
-        total += tokens;
-        longest = std::max(longest, tokens);
-    }
-    if (total < int64_t(1000) * p.n_seqs || total * 20 < longest * 19 * p.n_seqs) return false;
-    const int64_t wgs = int64_t(p.n_seqs) * params.n_heads / 4, round = 2 * params.n_cus, rest = wgs % round;
-    return wgs >= round / 2 && (rest == 0 || 2 * rest >= round);
-}
 }  // namespace
 
 namespace {
@@ -435,12 +408,10 @@ void build_plan(const ChunkRow* rows, int n_rows, int n_seqs, int chunk_size,
     p.own_pos0.assign(n_seqs, 0);
     p.shared_parts = n_parts;
     int64_t stream_chunk_total = 0;
-    int n_streamed_twice = 0;       // chunks that more than one sequence streams
     {
         std::vector<int> last_pos(n_seqs, -1);
         for (int i = 0; i < n_rows; i++) {
             if (is_shared(rows[i])) continue;
-            n_streamed_twice += rows[i].seq_end - rows[i].seq_begin > 1;
             for (int s = rows[i].seq_begin; s < rows[i].seq_end; s++) {
                 // the chunks a sequence streams are the tail end of its path: consecutive positions
                 if (p.own[s].empty()) {
@@ -492,15 +463,12 @@ void build_plan(const ChunkRow* rows, int n_rows, int n_seqs, int chunk_size,
         }
         if (stream_chunks / 2 >= min_chunks) taper_chunks = stream_chunks / 2;
     }
-    p.hints.per_head = params.stream_chunks <= 0 && n_streamed_twice == 0 && head_per_wave(p, chunk_size, params);
+    stream_chunks = std::min(stream_chunks, kMaxItemChunks - 1);  // an item may take one chunk more
+    if (taper_chunks >= stream_chunks) taper_chunks = 0;          // (after the cap: nothing to taper)
     if (params.keep) {
         stream_chunks = params.keep->stream_chunks;
         taper_chunks = params.keep->taper_chunks;
-        p.hints.per_head = params.keep->per_head && params.allow_per_wave && params.n_heads % 4 == 0 && p.shared_items.empty();
     }
-    if (p.hints.per_head) stream_chunks = kWholeSequence;
-    else stream_chunks = std::min(stream_chunks, kMaxItemChunks - 1);  // an item may take one chunk more
-    if (taper_chunks >= stream_chunks || p.hints.per_head) taper_chunks = 0;   // (after the cap: nothing to taper)
     p.hints.stream_chunks = stream_chunks;
     p.hints.taper_chunks = taper_chunks;
 

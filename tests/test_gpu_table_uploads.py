@@ -155,3 +155,19 @@ def test_a_graph_brings_its_tables_whatever_was_uploaded_before():
         graph.replay()
         torch.cuda.synchronize()
         assert_close(attn.forward(qd), oracle_output(attn, q, exact=True))
+
+
+# tables of one to four kernel arguments and past them (about 100 bytes a sequence), some refreshes ahead of the device
+@pytest.mark.parametrize("n", [30, 38, 75, 112, 148, 190])
+def test_tables_of_several_kernel_arguments(n):
+    rng = np.random.default_rng(n)
+    attn = cache(rng, 64, [3 + 5 * s % 61 for s in range(n)], True)
+    steps = []
+    for step in range(9):                              # every step another sequence's last chunk rolls over
+        q, k, v = (rand(rng, n, H, 128) for _ in range(3))
+        steps.append((q, attn.decode_step([50_000_000 + 1000 * step + s for s in range(n)], to_dev(q), to_dev(k), to_dev(v))))
+        if step < 8:
+            attn.refresh_kernel_context(force=True)
+    q, out = steps[-1]
+    assert_close(out, oracle_output(attn, q, exact=True))
+    assert_close(attn.forward(to_dev(q)), oracle_output(attn, q, exact=True))

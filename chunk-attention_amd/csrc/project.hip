@@ -815,7 +815,9 @@ int launch_mode(const ProjectArgs& a, hipStream_t st) {
     if (int64_t(a.N) * a.K >= int64_t(1) << 30 || a.K > 1 << 22) {
         return 4 * tiles(64, 64) < 3 * CUS ? launch_tile<2, 2, 2, 32, MODE>(a, st) : launch_tile<4, 4, 2, 64, MODE>(a, st);
     }
-    if (tiles(64, 64) <= CUS) return launch_shared_tile<64, 64, 4, 4, 2, MODE>(a, st);
+    // (five buffers: one weight of 4096 from memory on 100 and 200 rows 18.4 and 19.0 us with four, 16.8 and 17.0 with five, 16.9
+    // to 17.5 with six to ten; the larger tiles gain nothing from a fifth)
+    if (tiles(64, 64) <= CUS) return launch_shared_tile<64, 64, 5, 4, 2, MODE>(a, st);
     if (tiles(64, 128) <= CUS) return launch_shared_tile<64, 128, 4, 8, 2, MODE>(a, st);
     const int64_t square = (tiles(128, 128) + CUS - 1) / CUS, wide = (tiles(128, 256) + CUS - 1) / CUS;
     if constexpr (MODE == kRotary) {

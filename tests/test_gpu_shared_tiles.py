@@ -26,6 +26,11 @@ def test_linear_in_shared_tiles(rows, n_out, n_in):
     assert (guard[rows * n_out:] == 3.0).all()
 
 
+@pytest.mark.parametrize("n_in", [256, 320, 384])            # one stage less than buffers, as many, one more
+def test_linear_in_the_smallest_shared_tiles(n_in):
+    test_linear_in_shared_tiles(300, 2050, n_in)
+
+
 @pytest.mark.parametrize("rows,heads,n_in", [(400, 8, 64), (129, 16, 320), (500, 12, 128), (300, 32, 192), (1030, 31, 256)])
 def test_qkv_rotary_in_shared_tiles(rows, heads, n_in):
     project.test_qkv_rotary(rows, heads, n_in)

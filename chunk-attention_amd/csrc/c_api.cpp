@@ -449,10 +449,14 @@ int check_ready(ca_ctx* c, const void* q, int n_seqs) {
     return CA_OK;
 }
 
+int check_head_dim(const ca_ctx* c) {
+    return c->d == 128 ? CA_OK : fail(CA_ERR_INVALID, "unsupported head dim " + std::to_string(c->d));
+}
+
 // The attention kernels exist for the shapes the reference's GPU kernels take
 // (kernel_cuda.cu:1199, 1256-1265 there); like there, other shapes fail when attention is asked for.
 int check_attention_shape(const ca_ctx* c) {
-    if (c->d != 128) return fail(CA_ERR_INVALID, "unsupported head dim " + std::to_string(c->d));
+    if (int rc = check_head_dim(c)) return rc;
     if (c->C != 32 && c->C != 64 && c->C != 128) {
         return fail(CA_ERR_INVALID, "unsupported chunk_size " + std::to_string(c->C));
     }
@@ -946,7 +950,7 @@ int ca_causal_attention(const void* q, const void* k, const void* v, void* out, 
 int ca_prefill_attention(ca_ctx* c, ca_tree* tree, const int32_t* tokens, int batch, int n_tokens, const void* q,
                          const void* k, const void* v, void* out, int32_t* seq_idx, void* stream) {
     if (!c || !tree || !tokens || !seq_idx || batch < 1 || n_tokens < 1) return fail(CA_ERR_INVALID, "bad argument");
-    if (int rc = check_attention_shape(c)) return rc;
+    if (int rc = check_head_dim(c)) return rc;       // (a cache of any chunk size can be filled)
     ca::CausalArgs a;
     if (int rc = check_causal(a, q, k, v, out, batch, n_tokens, c->H)) return rc;
     if (!ca::causal_attention_fits(batch, n_tokens, c->H)) return launch_rc(-1, "causal attention launch");
@@ -1205,7 +1209,7 @@ int ca_model_pass(const ca_model_layer* layers, int n_layers, const int32_t* tok
     for (int i = 0; i < n_layers; i++) {
         const ca_model_layer& layer = layers[i];
         if (!layer.ctx || !layer.tree || layer.ctx->H != H) return fail(CA_ERR_INVALID, "a layer's cache does not fit the model");
-        if (int rc = check_attention_shape(layer.ctx)) return rc;
+        if (int rc = prefill ? check_head_dim(layer.ctx) : check_attention_shape(layer.ctx)) return rc;
         if (!layer.norm || !aligned16(layer.norm) || !(layer.norm_epsilon >= 0.f)) return fail(CA_ERR_INVALID, "null or misaligned device pointer");
         ca::ProjectArgs in = qkv_append_args(layer.ctx, layer.wq, layer.wk, layer.wv, pos, layer.cos_sin_cache, layer.max_position, q);
         if (int rc = check_project(in, x, rows, hidden, hidden)) return rc;

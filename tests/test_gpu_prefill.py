@@ -145,3 +145,36 @@ def test_prompts_that_are_not_the_caches_are_left_to_the_separate_calls():
         assert cache._prefill_attention(prompts, q, q, q) is None
     assert cache._prefill_attention([list(range(40))], *[q[:, :, :1].contiguous()] * 3) is None
     assert cache.tree.n_seqs == 0
+
+
+@pytest.mark.parametrize("chunk", [48, 20])
+def test_prefill_into_chunks_of_a_size_that_no_decode_attention_takes(chunk):
+    """Such a cache is filled like any other, by the attention's own launch, by the layer and by the small model; only a
+    decode forward over it is refused."""
+    from chunk_attn.llama_layer import LlamaChunkAttention
+    from chunk_attn.models.sequence import Sequence
+    from chunk_attn.models.tiny_lm import AttentionOnlyLM
+    test_attention_and_insertion_in_one_launch(2, 3 * chunk + 7, 2, chunk, chunk + 3)
+    prompts = [[100 * s + t for t in range(2 * chunk + 5)] for s in range(2)]
+    layer = LlamaChunkAttention(256, 2, max_position_embeddings=256)
+    x = torch.randn((2, 2 * chunk + 5, 256), device=DEV).half()
+    positions = torch.arange(2 * chunk + 5, device=DEV).expand(2, -1).contiguous()
+    with torch.inference_mode():
+        outs, rows = [], []
+        for size in (chunk, 64):
+            cache = capi.Attention(2, 128, size, memory_mb=8, dtype=torch.float16, device=torch.device(DEV))
+            outs.append(layer(x, prompts, positions, cache, True))
+            assert layer.last_indices == [0, 1]
+            rows.append([torch.cat([pool[slot][:, :m] for slot, m, b, e in cache.get_chunks() if b <= s < e], dim=1)
+                         for s in range(2) for pool in cache.pool_views()])
+            if size == chunk:
+                with pytest.raises(RuntimeError, match="unsupported chunk_size"):
+                    cache.forward(torch.zeros((2, 2, 128), device=DEV).half())
+        assert torch.equal(*outs) and all(torch.equal(a, b) for a, b in zip(*rows))
+        logits = []
+        for size, hooked in ((chunk, False), (chunk, True), (64, False)):
+            model = AttentionOnlyLM(60, 256, 2, 2, chunk_size=size, memory_mb=8, seed=7)
+            if hooked:                                       # the modules' own calls
+                model.norm.register_forward_hook(lambda m, a, out: None)
+            logits.append(model.logits([Sequence(list(range(50)))], model.create_kv_caches(), True))
+        assert torch.equal(logits[0], logits[1]) and torch.equal(logits[0], logits[2])

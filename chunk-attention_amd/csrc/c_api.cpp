@@ -957,22 +957,38 @@ int ca_prefill_attention(ca_ctx* c, ca_tree* tree, const int32_t* tokens, int ba
     return guarded([&]() -> int {
         std::vector<ca::CopyChunk> chunks;
         std::vector<int32_t> slots(n_tokens / c->C + 2);
+        chunks.reserve(size_t(batch) * slots.size());
         int rc = CA_OK;
+        std::string why;
         for (int s = 0; s < batch && rc == CA_OK; s++) {
             int begin = 0, n_new = 0;
             rc = ca_tree_add_seq(tree, tokens + size_t(s) * n_tokens, n_tokens, &seq_idx[s], &begin, slots.data(),
                                  static_cast<int>(slots.size()), &n_new);
-            if (rc != CA_OK) break;
+            if (rc != CA_OK) {
+                why = ca_last_error();
+                break;
+            }
             ca_ctx_invalidate(c);
-            if (n_new > static_cast<int>(slots.size())) return fail(CA_ERR_STATE, "the tree's chunks are not the context's");
-            for (int i = 0; i < n_new && begin + i * c->C < n_tokens; i++) {
+            // a tree whose chunks are not the context's
+            const char* wrong = nullptr;
+            if (n_new != (n_tokens - begin + c->C - 1) / c->C) {
+                wrong = "the tree's chunks do not hold as many tokens as the context's";
+            } else if (std::any_of(slots.begin(), slots.begin() + n_new, [&](int32_t slot) { return slot < 0 || slot >= c->max_chunks; })) {
+                wrong = "slot outside the pool";
+            }
+            if (wrong) {
+                (void)ca_tree_remove_seq(tree, seq_idx[s]);
+                seq_idx[s] = -1;
+                rc = CA_ERR_INVALID;
+                why = wrong;
+                break;
+            }
+            for (int i = 0; i < n_new; i++) {
                 const int at = begin + i * c->C;
-                if (slots[i] < 0 || slots[i] >= c->max_chunks) return fail(CA_ERR_INVALID, "slot outside the pool");
                 chunks.push_back({ slots[i], s * n_tokens + at, std::min(c->C, n_tokens - at) });
             }
         }
-        // (a prompt that the cache cannot take leaves those in front of it with their rows; the message is the tree's)
-        const std::string why = rc != CA_OK ? ca_last_error() : "";
+        // a prompt that the cache cannot take leaves those in front of it with their rows
         a.kpool = c->k_pool;
         a.vpool = c->v_pool;
         a.C = c->C;

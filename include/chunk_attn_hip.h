@@ -455,8 +455,9 @@ int ca_layer_decode(ca_ctx* ctx, ca_tree* tree, const int32_t* tokens, int n_seq
 /* The prefill branch's attention on a cache: ca_tree_add_seq for each of `batch` prompts of n_tokens tokens
  * (tokens [batch, n_tokens], host; seq_idx[s] receives what it gives), ca_causal_attention over them, and in the same
  * launch the rows of k and v that ca_scatter_kv would copy for each (chunks past the first 64 follow in launches of
- * their own).  The context's tables are invalid afterwards.  A prompt that the cache cannot take is an error; those in
- * front of it stay, with their rows. */
+ * their own).  The context's chunks may have any size.  Its tables are invalid afterwards.  A prompt that the cache cannot
+ * take, or for which the tree gives chunks that are not the context's, is an error and not in the tree (seq_idx[s] is -1 for
+ * the latter); those in front of it stay, with their rows. */
 int ca_prefill_attention(ca_ctx* ctx, ca_tree* tree, const int32_t* tokens, int batch, int n_tokens, const void* q,
                          const void* k, const void* v, void* out, int32_t* seq_idx, void* stream);
 

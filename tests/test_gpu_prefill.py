@@ -178,3 +178,34 @@ def test_prefill_into_chunks_of_a_size_that_no_decode_attention_takes(chunk):
                 model.norm.register_forward_hook(lambda m, a, out: None)
             logits.append(model.logits([Sequence(list(range(50)))], model.create_kv_caches(), True))
         assert torch.equal(logits[0], logits[1]) and torch.equal(logits[0], logits[2])
+
+
+@pytest.mark.parametrize("tree_chunk,tree_chunks,match", [
+    (128, 16, "as many tokens"), (32, 16, "as many tokens"), (64, 16, "outside the pool")])
+def test_a_tree_whose_chunks_are_not_the_contexts(tree_chunk, tree_chunks, match):
+    """Larger chunks, smaller ones, more of them than the pool has: the prompt that shows it is refused and not in the
+    tree; those before it stay, with their rows."""
+    import ctypes
+    n, fits = 100 if tree_chunk > 64 else 64, tree_chunk == 64
+    k = torch.randn((4, n, 2, 128), device=DEV).half()
+    cache = capi.Attention(2, 128, 64, memory_mb=1, dtype=torch.float16, device=torch.device(DEV))
+    pool_chunks = 4                                          # of the pool, for the context: two prompts and their tails
+    ctx = capi.KernelContext(2, 128, 64, cache.key_storage.data_ptr(), cache.value_storage.data_ptr(), pool_chunks)
+    tree = capi.Tree(tree_chunk, tree_chunks)
+    for pool in cache.pool_views():
+        pool.zero_()
+    prompts = [1000 * s + t for s in range(4) for t in range(n)]
+    out, index = torch.empty_like(k), (ctypes.c_int32 * 4)(*[7] * 4)
+    with pytest.raises(RuntimeError, match=match):
+        capi._launch(k.device, ctx._lib.ca_prefill_attention, ctx._h, tree._h, (ctypes.c_int32 * len(prompts))(*prompts), 4, n,
+                     k.data_ptr(), k.data_ptr(), k.data_ptr(), out.data_ptr(), index)
+    taken = 2 if fits else 0
+    assert tree.n_seqs == taken and list(index) == list(range(taken)) + [-1] + [7] * (3 - taken)
+    rows = tree.get_chunks()
+    for s in range(taken):
+        (slot,) = [slot for slot, m, b, _ in rows if b == s and m > 0]
+        for pool in cache.pool_views():
+            assert torch.equal(pool[slot].transpose(0, 1), k[s])
+    assert all(not pool[slot].any() for pool in cache.pool_views() for slot in range(cache.max_chunks)
+               if slot not in [r[0] for r in rows])
+    assert torch.equal(out, capi.causal_attention(k, k, k))

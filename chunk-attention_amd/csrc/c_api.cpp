@@ -1278,6 +1278,7 @@ int ca_model_pass(const ca_model_layer* layers, int n_layers, const int32_t* tok
         if (head && ca::project_norms(n_seqs, hidden)) {
             out.norm = row_norm.weight;
             out.norm_epsilon = row_norm.epsilon;
+            out.normed = x + skip;                   // the last norm's rows, head or not
             return project(out, residual + skip, n_seqs, n_logits, hidden, stream);
         }
         if (int rc = ca_rms_norm(x + skip, residual + skip, row_norm.weight, row_norm.epsilon, n_seqs, hidden, stream)) return rc;

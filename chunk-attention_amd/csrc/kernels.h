@@ -166,8 +166,10 @@ int launch_copy_in(const CausalArgs& a, hipStream_t st);   // the copies alone
 // whole head of 128, cos_sin_cache [max_position, 128]) before they are rounded; with tail_slot set, y[1] and
 // y[2] are the K and the V pool and row m goes to row tail_fill[m] + delta_tokens of chunk tail_slot[m].
 // norm: the rows of x are normalised first, as launch_rms_norm does with that weight, bit for bit (project_norms
-// says whether it can be; not with positions alone, nor with add).  add ([M, N], 16-byte aligned like y[0], which it may be; one weight, N a multiple of 8, no
-// positions): added to the products once they are rounded.
+// says whether they can be; without positions or with tail_slot, not with add).  normed ([M, K], 16-byte aligned, apart from
+// the operands; norm and no positions): receives the normalised rows, too.
+// add ([M, N], 16-byte aligned like y[0], which it may be; one weight, N a multiple of 8, no positions): added to the
+// products once they are rounded.
 struct ProjectArgs {
     const void* x = nullptr;
     const void* w[3] = { nullptr, nullptr, nullptr };
@@ -182,6 +184,7 @@ struct ProjectArgs {
     int delta_tokens = 0, C = 0;
     const void* norm = nullptr;          // [K], 16-byte aligned
     float norm_epsilon = 0.f;
+    void* normed = nullptr;
     const void* add = nullptr;
 };
 bool project_norms(int M, int K);

@@ -190,7 +190,13 @@ __global__ __launch_bounds__(WG) void project_kernel(const ProjectArgs a) {
         for (int r = 0; r < R; r++) {
             if (r < mine) {
 #pragma unroll
-                for (int n = 0; n < XL; n++) st[r][NL - XL + n] = norm::scaled8(st[r][NL - XL + n], weight[r], inv[n]);
+                for (int n = 0; n < XL; n++) {
+                    st[r][NL - XL + n] = norm::scaled8(st[r][NL - XL + n], weight[r], inv[n]);
+                    if (MODE == kPlain && blockIdx.x == 0 && a.normed && 8 * n + (l >> 3) < a.M) {   // (one block of rows)
+                        half_t* to = static_cast<half_t*>(a.normed) + size_t(8 * n + (l >> 3)) * a.K + (w + NW * r) * UNIT + 8 * (l & 7);
+                        *reinterpret_cast<h8*>(to) = st[r][NL - XL + n];
+                    }
+                }
                 multiply(st[r]);
             }
         }
@@ -837,6 +843,7 @@ int launch_project(const ProjectArgs& a, hipStream_t st) {
     if (a.M <= 0 || a.N <= 0) return 0;
     if (a.K <= 0 || a.K % UNIT != 0 || a.n_w < 1 || a.n_w > 3 || a.M > 0x7fffff00) return -1;
     if (a.norm && (!project_norms(a.M, a.K) || a.add || (a.positions && !a.tail_slot))) return -1;
+    if (a.normed && (!a.norm || a.positions)) return -1;
     if (a.add && (a.n_w != 1 || a.positions || !a.vec8)) return -1;
     if (!a.positions) return a.add ? launch_mode<kAdd>(a, st) : launch_mode<kPlain>(a, st);
     if (a.N % D != 0 || a.n_w != 3) return -1;

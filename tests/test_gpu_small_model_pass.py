@@ -186,3 +186,49 @@ def test_norms_on_the_way_keep_every_bit(hidden, prompts):
                 out.append(model.logits(running, caches, False))
         runs.append(out)
     assert all(torch.equal(a, b) for a, b in zip(*runs)) and all(torch.isfinite(a).all() for a in runs[0])
+
+
+@pytest.mark.parametrize("hidden,prompts", [(256, [40, 3]), (1024, [2] * 8), (1024, [3] * 9), (384, [1] * 16), (1024, [2] * 17), (1152, [7, 40])])
+def test_the_last_norms_rows_are_in_the_scratch_with_a_head_too(hidden, prompts):
+    """Where ca_model_last_rows says, after prompts and decode passes, whoever normalised them; guard rows behind stay."""
+    import ctypes
+    from chunk_attn import capi
+    from chunk_attn.models.sequence import Sequence
+    from chunk_attn.models.tiny_lm import AttentionOnlyLM
+    dev, lib = torch.device("cuda:0"), capi.load()
+    model = AttentionOnlyLM(60, hidden, hidden // 128, 2, chunk_size=32, memory_mb=32, seed=9)
+    g = torch.Generator().manual_seed(hidden)
+    with torch.no_grad():
+        for norm in (*model.input_norms, model.norm):
+            norm.weight.copy_(torch.randn(hidden, generator=g))
+
+    def rows_of(caches, seqs, ids, positions, prefill, head):
+        layers, kept = model._plain_pass(seqs, ids, caches, prefill, dev)
+        table = (capi.ModelLayer * len(layers))(*[(cache.ctx._h, cache.tree._h, *rest) for cache, *rest in layers])
+        tokens, places = sum(ids, []), sum(positions, [])
+        n, i32 = len(tokens), ctypes.c_int32 * len(tokens)
+        scratch = torch.full((lib.ca_model_scratch_bytes(n, hidden) // 2 + 64,), 5.0, dtype=torch.float16, device=dev)
+        logits = torch.empty((len(seqs), 60), dtype=torch.float16, device=dev)
+        capi._launch(dev, lib.ca_model_pass, table, len(layers), i32(*tokens), i32(*places), len(seqs), n // len(seqs), int(prefill),
+                     model.embed_tokens.weight.data_ptr(), 60, model.input_norms[0].weight.data_ptr(), model.input_norms[0].eps,
+                     hidden, scratch.data_ptr(), model.lm_head.weight.data_ptr() if head else None, 60 if head else 0,
+                     logits.data_ptr() if head else None, (ctypes.c_int32 * len(layers))())
+        assert (scratch[-64:] == 5.0).all()
+        at = lib.ca_model_last_rows(n, hidden, len(seqs)) // 2
+        rows = scratch[at:at + len(seqs) * hidden].view(len(seqs), hidden)
+        if head:                                         # (what a pass with a head is for)
+            assert torch.equal(logits, capi.linear(rows.clone(), model.lm_head.weight))
+        return rows
+
+    with torch.inference_mode():
+        found = []
+        for head in (False, True):
+            caches, rows = model.create_kv_caches(), []
+            for s, n in enumerate(prompts):
+                ids = [(7 * t + 5 * s) % 60 for t in range(n)]
+                rows.append(rows_of(caches, [Sequence(ids)], [ids], [list(range(n))], True, head))
+            for t in range(2):
+                ids = [[(11 * t + 3 * s) % 60] for s in range(len(prompts))]
+                rows.append(rows_of(caches, [None] * len(prompts), ids, [[9 + t]] * len(prompts), False, head))
+            found.append(rows)
+        assert all(torch.equal(a, b) and torch.isfinite(a).all() for a, b in zip(*found))

@@ -233,7 +233,7 @@ __global__ __launch_bounds__(WG) void project_kernel(const ProjectArgs a) {
     __syncthreads();
 
     if constexpr (!turns(MODE)) {
-        half_t* __restrict__ y = static_cast<half_t*>(which == 0 ? a.y[0] : which == 1 ? a.y[1] : a.y[2]);
+        half_t* y = static_cast<half_t*>(which == 0 ? a.y[0] : which == 1 ? a.y[1] : a.y[2]);
         for (int u = tid; u < MT * NT / 8; u += WG) {
             const int r = u / (NT / 8), c = 8 * (u % (NT / 8));
             if (row0 + r >= a.M || col0 + c >= a.N) continue;
@@ -460,7 +460,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void project_tile_kernel(const Proje
     // Lane (g, i) holds row i of a 16 x 16 block, columns 4g .. 4g + 3: rounded, and through the wave's own piece of
     // LDS, 32 rows at a time, into whole lines.
     half_t* stage = &lds[w * 32 * EP];
-    half_t* __restrict__ y = static_cast<half_t*>(which == 0 ? a.y[0] : which == 1 ? a.y[1] : a.y[2]);
+    half_t* y = static_cast<half_t*>(which == 0 ? a.y[0] : which == 1 ? a.y[1] : a.y[2]);
 #pragma unroll
     for (int m2 = 0; m2 < MB / 2; m2++) {
         const int row_base = row0 + wm * TM + 32 * m2;

@@ -6,7 +6,10 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("hidden,layers,prompts,chunk,vocab", [
-    (128, 1, [1, 5], 32, 40), (1024, 3, [449, 30, 449], 64, 300), (512, 2, [900, 65, 64, 63], 128, 1001)])
+    (128, 1, [1, 5], 32, 40), (1024, 3, [449, 30, 449], 64, 300), (512, 2, [900, 65, 64, 63], 128, 1001),
+    # residuals in the output projection's tiles of 128 x 128 and 64 x 128, and of 128 x 256; more new chunks than one
+    # launch copies
+    (1024, 1, [3001, 1100], 32, 60), (1536, 2, [660, 2000], 64, 60), (2048, 1, [2100], 64, 60)])
 def test_native_model_pass_keeps_every_bit(hidden, layers, prompts, chunk, vocab):
     """One native call a pass against the modules' own calls (a hook on a norm keeps them): prompts on both sides of
     the ids that one launch takes, decode steps over which last chunks fill up, the caches afterwards."""

@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 import torch
 
+from chunk_attn.capi import HostTables
 from gpu_helpers import assert_close, dev, make_attention, oracle_output, to_dev
 
 pytestmark = pytest.mark.gpu
@@ -157,17 +158,41 @@ def test_a_graph_brings_its_tables_whatever_was_uploaded_before():
         assert_close(attn.forward(qd), oracle_output(attn, q, exact=True))
 
 
-# tables of one to four kernel arguments and past them (about 100 bytes a sequence), some refreshes ahead of the device
-@pytest.mark.parametrize("n", [30, 38, 75, 112, 148, 190])
-def test_tables_of_several_kernel_arguments(n):
-    rng = np.random.default_rng(n)
-    attn = cache(rng, 64, [3 + 5 * s % 61 for s in range(n)], True)
-    steps = []
-    for step in range(9):                              # every step another sequence's last chunk rolls over
-        q, k, v = (rand(rng, n, H, 128) for _ in range(3))
-        steps.append((q, attn.decode_step([50_000_000 + 1000 * step + s for s in range(n)], to_dev(q), to_dev(k), to_dev(v))))
-        if step < 8:
-            attn.refresh_kernel_context(force=True)
-    q, out = steps[-1]
-    assert_close(out, oracle_output(attn, q, exact=True))
-    assert_close(attn.forward(to_dev(q)), oracle_output(attn, q, exact=True))
+def table_bytes(attn, n):
+    """Of the blob that a refresh brings to the device: its seven tables in whole 64-byte lines."""
+    plan = HostTables(attn.tree.get_chunks(), n, C, stream_chunks=4, n_heads=H).plan()
+    return sum(-(-plan[name].nbytes // 64) * 64 for name in ("shared_items", "stream_items", "slots", "seq_len", "part_ptr",
+                                                             "tail_slot", "tail_fill"))
+
+
+# tables of one to four kernel arguments of 3.5 KB and past them
+@pytest.mark.parametrize("n,arguments", [(30, 1), (38, 1), (75, 2), (112, 3), (148, 4), (190, 5)])
+def test_tables_of_several_kernel_arguments(n, arguments):
+    """Every step another sequence's last chunk rolls over.  A device that is asked for all steps before it has run the first
+    one, each with tables of its own in the same buffer, gives what one step at a time does."""
+    runs = []
+    for ahead in (False, True):
+        rng = np.random.default_rng(n)
+        attn = cache(rng, 64, [3 + 5 * s % 61 for s in range(n)], True)
+        inputs = [[rand(rng, n, H, 128) for _ in range(3)] for _ in range(9)]
+        on_device = [[to_dev(t) for t in step] for step in inputs]
+        attn.refresh_kernel_context(force=True)        # buffers: nothing is allocated below
+        torch.cuda.synchronize()
+        if ahead:
+            torch.cuda._sleep(60_000_000)
+            slept = torch.cuda.Event()
+            slept.record()
+        outs = []
+        for step in range(9):
+            outs.append(attn.decode_step([50_000_000 + 1000 * step + s for s in range(n)], *on_device[step]))
+            if not ahead:
+                assert_close(outs[-1], oracle_output(attn, inputs[step][0], exact=True))
+                assert -(-table_bytes(attn, n) // 3584) == arguments
+            if step < 8:
+                attn.refresh_kernel_context(force=True)
+        if ahead and arguments <= 4:                   # (larger ones wait for a staging buffer)
+            assert not slept.query()
+        torch.cuda.synchronize()
+        runs.append(outs)
+    assert all(torch.equal(a, b) for a, b in zip(*runs))
+    assert_close(attn.forward(on_device[-1][0]), oracle_output(attn, inputs[-1][0], exact=True))

@@ -92,6 +92,7 @@ SIGNATURES = {
                              [ctypes.c_void_p] * 4 + [c_i32_p, ctypes.c_void_p]),
     "ca_linear": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_int,
                                  ctypes.c_int, ctypes.c_void_p]),
+    "ca_projection_tile": (ctypes.c_int, [ctypes.c_int] * 4 + [ctypes.POINTER(ctypes.c_int)] * 2),
     "ca_qkv_rotary": (ctypes.c_int, [ctypes.c_void_p] * 6 + [ctypes.c_int] + [ctypes.c_void_p] * 3 +
                       [ctypes.c_int] * 3 + [ctypes.c_void_p]),
     "ca_qkv_rotary_append_kv": (ctypes.c_int, [ctypes.c_void_p] * 7 + [ctypes.c_int, ctypes.c_void_p, ctypes.c_int,
@@ -525,13 +526,17 @@ def shared_tiles_pay(rows: int, n_in: int, n_out: int, n_weights: int) -> bool:
     """Whether rows [rows, n_in] times `n_weights` weights [n_out, n_in] are faster in the tiles that waves share than as
     library products, where projection_pays does not say so already: the GPU's time decides.
 
-    The unit is a tile of 128 x 256, of which 256 are computed at a time.  One weight: while they fit at once (us here
-    and the library's: 4096 x 4096 on 1000 rows 34 to 40, on 1500 50 to 52, on 2048 58 to 64, on 2300 88 to 70; 2048 x
-    2048 on 3000 rows 28 to 31, on 4096 32 to 37, on 6000 53 to 47; 1024 x 1024 on 8192 rows 20 to 24).  q, k and v
-    with their rotation: up to three rounds (against three products and the rotary launch: 4096 x 4096 on 512 rows 52
-    to 86, on 2048 181-193 to 209-212, on 2300 220 to 222, on 2560 232 to 230; 2048 x 2048 on 4096 rows 101 to 120; 5120 x 5120
-    on 1000 rows 159 to 205, on 1600 269 to 271, on 2048 309 to 300; 1024 x 1024 on 8192 rows 64 to 81).  Weights of
-    more than 2^25 elements were not measured."""
+    The line counts tiles of 128 x 256, of which 256 are computed at a time, whatever tile a launch takes.  us here and
+    the library's, weights from memory.  One weight, while they fit at once: 4096 x 4096 on 1000 rows 38 and 42, on 1500 57
+    and 55, on 2048 66 and 72, on 2300 98 and 74; 2048 x 2048 on 3000 rows 30 and 32, on 4096 36 and 39, on 6000 59 and
+    50; 5120 x 5120 on 1000 rows 76 and 69, on 1300 75 and 80, on 1600 121 and 93; 1024 x 1024 on 8192 rows 24 and 26, on 16000
+    42 and 35.  q, k and v with their rotation, against three products and the rotary launch, up to three rounds: 4096 x 4096
+    on 512 rows 67 and 110, on 1024 114 and 143, on 2048 180 and 234; 2048 x 2048 on 3000 rows 82 and 105, on 4096 96 and
+    131; 5120 x 5120 on 1000 rows 169 and 226, on 1300 206 and 266; 1024 x 1024 on 8192 rows 55 and 85.  Behind the line the two
+    are level (4096 x 4096 on 2300 rows 244 and 245, on 3072 310 and 311, on 4096 349 and 341; 2048 x 2048 on 6000 168 and 167;
+    5120 x 5120 on 1600 295 and 307, on 2048 331 and 335), but for whole rounds of the tiles of three heads, which are faster
+    here and not taken: 2048 x 2048 on 8192 rows 190 and 197, 1024 x 1024 on 16384 108 and 128.  Weights of more than 2^25
+    elements were not measured."""
     tiles = -(-rows // 128) * -(-n_out // 256) * n_weights
     return n_in * n_out <= 1 << 25 and tiles <= (256 if n_weights == 1 else 768)
 

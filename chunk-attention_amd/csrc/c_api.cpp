@@ -365,10 +365,11 @@ int upload_plan(ca_ctx* c, hipStream_t st) {
     };
     // Tables of up to four kernel arguments travel as those: no staging buffer, no event, and the host never waits for the
     // buffer of the fourth refresh before, which put a batch's whole backlog between its last steps and the next
-    // admissions (32 sequences, 1024 shared + 300 tokens and 48 steps, tables of some 5 KB: 1745 -> 1648 us a pass; 64 sequences
-    // of 12 heads with chunks of 32, 13 KB, 1852 to 1960 -> 1654 to 1821; a launch of 3.5 KB takes 1.2 us, one from pinned
-    // memory 4).  Those of a forward in direct form only if something asks for them.  So do all tables under stream capture: a replay would read whatever the
-    // staging buffer holds by then, and its event could not be waited for any more.
+    // admissions (32 sequences, 1024 shared + 300 tokens and 48 steps, tables of some 5 KB: 1745 -> 1648 us a pass where the
+    // host is that far ahead, level where it is not, as on a batch's first pass; the copies themselves take what the one
+    // from pinned memory did, 4 us in a trace).  Those of a forward in direct form only if something asks for them.  So do
+    // all tables under stream capture: a replay would read whatever the staging buffer holds by then, and its event could
+    // not be waited for any more.
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     CA_HIP(hipStreamIsCapturing(st, &capture));
     if (total <= 4 * ca::kArgUploadBytes || capture != hipStreamCaptureStatusNone) {
@@ -1065,6 +1066,21 @@ int ca_qkv_rotary(const void* x, const void* wq, const void* wk, const void* wv,
     return project(a, x, n_rows, n_heads * 128, n_in, stream);
 }
 
+int ca_projection_tile(int n_rows, int n_out, int n_in, int rotary, int* tile_rows, int* tile_cols) {
+    if (n_rows <= 0 || n_out <= 0 || n_in <= 0 || n_in % 64 != 0 || (rotary && n_out % 128 != 0) || !tile_rows || !tile_cols) {
+        return fail(CA_ERR_INVALID, "bad argument");
+    }
+    ca::ProjectArgs a;
+    const int64_t somewhere = 0;
+    a.n_w = rotary ? 3 : 1;
+    a.positions = rotary ? &somewhere : nullptr;
+    a.M = n_rows;
+    a.N = n_out;
+    a.K = n_in;
+    ca::project_tile(a, tile_rows, tile_cols);
+    return CA_OK;
+}
+
 namespace {
 ca::ProjectArgs qkv_append_args(const ca_ctx* c, const void* wq, const void* wk, const void* wv, const int64_t* positions,
                                 const void* cos_sin_cache, int max_position, void* q) {
@@ -1184,8 +1200,8 @@ int ca_layer_decode(ca_ctx* c, ca_tree* tree, const int32_t* tokens, int n_seqs,
 }
 
 namespace {
-// Where a model pass keeps its rows: positions, residual, the norms' rows (and what the output projection leaves
-// there), q, k, v and the attention's output.
+// Where a model pass keeps its rows: positions, residual (to which the output projections add), the norms' rows where
+// a launch of its own writes them and the last norm's, q, k, v and the attention's output.
 struct ModelRows {
     int64_t rows;
     int hidden;

@@ -188,6 +188,7 @@ struct ProjectArgs {
     const void* add = nullptr;
 };
 bool project_norms(int M, int K);
+void project_tile(const ProjectArgs& a, int* rows, int* cols);   // what a workgroup of its launch computes (M, N, K, n_w > 0)
 int launch_project(const ProjectArgs& a, hipStream_t st);
 
 }  // namespace ca

@@ -801,40 +801,60 @@ int heads_shape(const ProjectArgs& a, int64_t square, int64_t wide) {
 // 41.9, on 192 rows 56.7, 51.3, 57.2, 38.1).  Where even 128 x 256 leaves a second round, the rounds decide, a stage of
 // 128 x 128 taking 0.36 us and one of 128 x 256 0.56 (q, k and v of 4096: 700 rows 95.5 and 99.8, 1500 rows 166 and
 // 161, 2048 rows 209 and 181).
+enum Tile { kRows8, kRows16, k32x32, k64x64Split, k64x64, k64x128, k128x128, k128x256, kHeads128, kHeads256 };
+
+Tile tile_of(const ProjectArgs& a, bool rotary) {
+    if (a.M <= 16) return a.M <= 8 ? kRows8 : kRows16;
+    auto tiles = [&](int bm, int bn) { return int64_t((a.N + bn - 1) / bn) * a.n_w * ((int64_t(a.M) + bm - 1) / bm); };
+    constexpr int CUS = 256;
+    if (tiles(32, 32) <= CUS + CUS / 8) return k32x32;
+    // Shared tiles reach their rows and columns with 32-bit offsets.  Beyond them the largest tile with k split over
+    // the waves, where three quarters of the compute units get one (32768 x 32768 on 65, 252 and 1000 rows 779, 1544 and 6146 us; in
+    // 32 x 32 tiles 1134, 2960 and 11711).
+    if (int64_t(a.N) * a.K >= int64_t(1) << 30 || a.K > 1 << 22) return 4 * tiles(64, 64) < 3 * CUS ? k32x32 : k64x64Split;
+    if (tiles(64, 64) <= CUS) return k64x64;
+    if (tiles(64, 128) <= CUS) return k64x128;
+    const int64_t square = (tiles(128, 128) + CUS - 1) / CUS, wide = (tiles(128, 256) + CUS - 1) / CUS;
+    const int shape = rotary ? heads_shape(a, square, wide) : 0;
+    if (shape) return shape == 8 ? kHeads256 : kHeads128;
+    return square == 1 || square * 36 < wide * 56 ? k128x128 : k128x256;
+}
+
 template <int MODE>
 int launch_mode(const ProjectArgs& a, hipStream_t st) {
     if constexpr (MODE == kPlain || MODE == kAppend) {
         if (a.norm) return a.M <= 8 ? launch_tile<1, 1, 2, 8, MODE, true>(a, st) : launch_tile<1, 1, 2, 16, MODE, true>(a, st);
     }
-    if (a.M <= 8) {
-        return a.K > 2 * NW * UNIT ? launch_tile<1, 1, 3, 8, MODE>(a, st) : launch_tile<1, 1, 2, 8, MODE>(a, st);
-    }
-    if (a.M <= 16) {
-        return a.K > 2 * NW * UNIT ? launch_tile<1, 1, 3, 16, MODE>(a, st) : launch_tile<1, 1, 2, 16, MODE>(a, st);
-    }
-    auto tiles = [&](int bm, int bn) { return int64_t((a.N + bn - 1) / bn) * a.n_w * ((int64_t(a.M) + bm - 1) / bm); };
-    constexpr int CUS = 256;
-    if (tiles(32, 32) <= CUS + CUS / 8) return launch_tile<2, 2, 2, 32, MODE>(a, st);
-    // Shared tiles reach their rows and columns with 32-bit offsets.  Beyond them the largest tile with k split over
-    // the waves, where three quarters of the compute units get one (32768 x 32768 on 65, 252 and 1000 rows 779, 1544 and 6146 us; in
-    // 32 x 32 tiles 1134, 2960 and 11711).
-    if (int64_t(a.N) * a.K >= int64_t(1) << 30 || a.K > 1 << 22) {
-        return 4 * tiles(64, 64) < 3 * CUS ? launch_tile<2, 2, 2, 32, MODE>(a, st) : launch_tile<4, 4, 2, 64, MODE>(a, st);
-    }
+    const bool long_k = a.K > 2 * NW * UNIT;
+    switch (tile_of(a, MODE == kRotary)) {
+    case kRows8: return long_k ? launch_tile<1, 1, 3, 8, MODE>(a, st) : launch_tile<1, 1, 2, 8, MODE>(a, st);
+    case kRows16: return long_k ? launch_tile<1, 1, 3, 16, MODE>(a, st) : launch_tile<1, 1, 2, 16, MODE>(a, st);
+    case k32x32: return launch_tile<2, 2, 2, 32, MODE>(a, st);
+    case k64x64Split: return launch_tile<4, 4, 2, 64, MODE>(a, st);
     // (five buffers: one weight of 4096 from memory on 100 and 200 rows 18.4 and 19.0 us with four, 16.8 and 17.0 with five, 16.9
     // to 17.5 with six to ten; the larger tiles gain nothing from a fifth)
-    if (tiles(64, 64) <= CUS) return launch_shared_tile<64, 64, 5, 4, 2, MODE>(a, st);
-    if (tiles(64, 128) <= CUS) return launch_shared_tile<64, 128, 4, 8, 2, MODE>(a, st);
-    const int64_t square = (tiles(128, 128) + CUS - 1) / CUS, wide = (tiles(128, 256) + CUS - 1) / CUS;
-    if constexpr (MODE == kRotary) {
-        const int shape = heads_shape(a, square, wide);
-        if (shape) return shape == 8 ? launch_heads<8>(a, st) : launch_heads<4>(a, st);
+    case k64x64: return launch_shared_tile<64, 64, 5, 4, 2, MODE>(a, st);
+    case k64x128: return launch_shared_tile<64, 128, 4, 8, 2, MODE>(a, st);
+    case k128x128: return launch_shared_tile<128, 128, 4, 8, 2, MODE>(a, st);
+    case k128x256: return launch_shared_tile<128, 256, 3, 8, 4, MODE>(a, st);
+    case kHeads128:
+        if constexpr (MODE == kRotary) return launch_heads<4>(a, st);
+        break;
+    case kHeads256:
+        if constexpr (MODE == kRotary) return launch_heads<8>(a, st);
+        break;
     }
-    if (square == 1 || square * 36 < wide * 56) return launch_shared_tile<128, 128, 4, 8, 2, MODE>(a, st);
-    return launch_shared_tile<128, 256, 3, 8, 4, MODE>(a, st);
+    return -1;
 }
 
 }  // namespace
+
+void project_tile(const ProjectArgs& a, int* rows, int* cols) {
+    constexpr int shape[][2] = { { 16, 16 }, { 16, 16 }, { 32, 32 }, { 64, 64 }, { 64, 64 }, { 64, 128 }, { 128, 128 }, { 128, 256 }, { 128, HN }, { 256, HN } };
+    const Tile t = tile_of(a, a.positions && !a.tail_slot);
+    *rows = shape[t][0];
+    *cols = shape[t][1];
+}
 
 // One block of rows, two units a wave.
 bool project_norms(int M, int K) { return M <= 16 && K <= 2 * NW * UNIT; }

@@ -1,6 +1,6 @@
 // The arithmetic of the rotary position embedding, shared by the rotary kernels and by the decode
 // kernel's fused step (which rotates the new query and key rows in registers): fp16 data, fp32
-// arithmetic rounded once.  cos_sin_cache row p holds cos(p * f_r), r < rot_dim/2, then
+// arithmetic, one rounding to fp16.  cos_sin_cache row p holds cos(p * f_r), r < rot_dim/2, then
 // sin(p * f_r).  NeoX style pairs element r with r + rot_dim/2; GPT-J style pairs 2r with 2r+1.
 // Elements past rot_dim pass through unchanged.
 // (reference: cpp/chunk_attn/pos_encoding_kernels.cu:24-92)
@@ -25,6 +25,9 @@ __device__ __forceinline__ int64_t clamp_pos(int64_t p, int max_position) {
 // Every kernel forms the rotation with the same two fp32 operations per element, a rounded
 // product and a fused multiply-add:
 //   x' = fma(x, cos, -(y * sin)),  y' = fma(y, cos, x * sin)
+// What is rounded to fp16 next is the fp32 result or, where the compiler forms v_fma_mixlo_f16 or v_fma_mixhi_f16, the exact
+// sum: which, it chooses for every element of every kernel, so that an element may differ in its last bit with the kernel that
+// computed it.  Either is off by half a unit of fp16, but for 2^-13 of one in the first case.
 __device__ __forceinline__ float rot_elem(float own, float other, float c, float s, bool is_x) {
     const float t = other * s;
     return __builtin_fmaf(own, c, is_x ? -t : t);

@@ -194,6 +194,11 @@ int ca_qkv_rotary_append_kv(ca_ctx* ctx, const void* x, const void* wq, const vo
                             const int64_t* positions_dev, const void* cos_sin_cache, int max_position, void* q,
                             int n_in, int n_seqs, void* stream);
 
+/* Which tile a workgroup computes in ca_linear (rotary 0) or ca_qkv_rotary (1; its three weights' columns are counted as
+ * one row) of such a size: the rule on rows, columns and k that the launch follows, for tests and measurements.  16 rows mean up to
+ * 16, 32 x 32 and 64 x 64 also tiles with k split over the waves. */
+int ca_projection_tile(int n_rows, int n_out, int n_in, int rotary, int* tile_rows, int* tile_cols);
+
 /* The decode step of the reference's attention layer
  * (src/chunk_attn/models/llama_hf/modeling_llama.py:62,91-95: rotary_embedding on the new
  * query/key rows, then append_token -> append_kv) as one launch: q [n_seqs, n_heads, d_head]
@@ -474,14 +479,15 @@ typedef struct {
 } ca_model_layer;
 
 /* A pass of a pre-norm attention-only model (modeling_llama.py:206-235, without its MLP): embedding and first norm,
- * then per layer the attention layer and the residual's addition in the norm behind it (ca_add_rms_norm), then, if
- * `head` is not null, logits [n_seqs, n_logits] = last rows . head^T.
+ * then per layer the attention layer, its output added to the residual, and the norm behind it (the bits of ca_linear and
+ * ca_add_rms_norm), then, if `head` is not null, logits [n_seqs, n_logits] = last rows . head^T.
  *   prefill == 0: one token per sequence of every cache (n_tokens is 1), per layer ca_layer_decode;
- *   prefill == 1: one sequence (n_seqs is 1) of n_tokens tokens: ca_qkv_rotary, ca_prefill_attention, ca_linear, room for the next token; seq_idx[layer] receives the sequence's index in that cache.
+ *   prefill == 1: one sequence (n_seqs is 1) of n_tokens tokens: ca_qkv_rotary, ca_prefill_attention, ca_linear, room for
+ *   the next token; seq_idx[layer] receives the sequence's index in that cache.
  * tokens and positions: host, n_seqs * n_tokens; every id within the embedding [vocab, hidden].  hidden is the
  * context's n_heads * 128.  scratch: ca_model_scratch_bytes(rows, hidden) bytes of device memory, 16-byte aligned;
- * the last norm's rows start ca_model_last_rows(rows, hidden, n_seqs) bytes into it.  What a call refuses for its
- * arguments, or because a cache has other sequences than the pass, leaves every cache's tokens as they were. */
+ * the last norm's rows start ca_model_last_rows(rows, hidden, n_seqs) bytes into it, with a head and without.  What a call
+ * refuses for its arguments, or because a cache has other sequences than the pass, leaves every cache's tokens as they were. */
 size_t ca_model_scratch_bytes(int64_t n_rows, int hidden);
 size_t ca_model_last_rows(int64_t n_rows, int hidden, int n_seqs);
 int ca_model_pass(const ca_model_layer* layers, int n_layers, const int32_t* tokens, const int32_t* positions,

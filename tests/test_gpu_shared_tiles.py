@@ -31,12 +31,13 @@ def test_linear_in_the_smallest_shared_tiles(n_in):
     test_linear_in_shared_tiles(300, 2050, n_in)
 
 
-@pytest.mark.parametrize("rows,heads,n_in", [(400, 8, 64), (129, 16, 320), (500, 12, 128), (300, 32, 192), (1030, 31, 256)])
+@pytest.mark.parametrize("rows,heads,n_in", [(250, 8, 384), (400, 8, 64), (129, 16, 320), (500, 12, 128), (300, 32, 192), (1030, 31, 256)])
 def test_qkv_rotary_in_shared_tiles(rows, heads, n_in):
     project.test_qkv_rotary(rows, heads, n_in)
 
 
 # tiles of three heads: 128 rows (one to more stages than buffers, last rows, a grid that the XCDs do not divide), 256 rows
+# (test_projection_rules holds the rule to these tiles)
 @pytest.mark.parametrize("rows,heads,n_in", [(1300, 16, 64), (1409, 16, 128), (1291, 17, 192), (2047, 12, 320),
                                              (1290, 32, 1024), (2000, 31, 1088), (6900, 8, 1024)])
 def test_qkv_rotary_in_tiles_of_three_heads(rows, heads, n_in):
